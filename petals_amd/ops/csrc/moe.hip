@@ -18,6 +18,7 @@
 
 #include "common.h"
 #include "gemv_reduce.h"
+#include "paged.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 
@@ -222,28 +223,67 @@ __global__ __launch_bounds__(WAVE) void gemv_nf4_moe_kernel(
 
 // ------------------------------------------------- grouped GEMM (prefill)
 //
-// Prefill-time grouped GEMM over expert-sorted (token, slot) pairs: the host
-// (fused_moe.py) sorts the R = T*k pairs by expert with each expert's segment
-// padded to a multiple of MT rows, so every MT-row tile belongs to ONE expert
-// (tile_expert[tile], -1 = pure padding). Each workgroup computes an
-// MT x NT C tile with mfma_f32_16x16x32_bf16: the expert's B tile (KT x NT)
-// is staged per k-step into LDS TRANSPOSED with the attention kernel's XOR
-// swizzle (prefill_attn.hip VT_BYTE) so B-fragments are contiguous
-// ds_read_b128 rows; NF4 weights are dequantized on the way into LDS, so the
-// packed form (4.25 b/param) is what crosses HBM — no dense dequant pass.
-// Replaces the per-expert dense-matmul loop for prefill (each expert's
-// weights are read ceil(rows_e/MT) times instead of once per token).
+// Grouped GEMM over expert-sorted (token, slot) pairs: the caller sorts the R = T*k
+// pairs by expert with each expert's segment padded to a multiple of MT rows, so every
+// MT-row tile belongs to ONE expert (tile_expert[tile], -1 = pure padding).
+//
+// Up to four tiles of one expert (128 rows) and 256 columns are a workgroup's: an
+// expert's weights are read once per 128 of its rows, and the rows once per 256 columns.
+// With a tile of 32 rows and 128 columns each, weights crossed the caches four times as
+// often and every product waited for a transposing store of its weights. Both products of
+// a layer of 8 experts, width 4096 and inner size 14336: with 290 rows an expert from 6.06
+// to 1.73 ms (135 to 472 TFLOP/s), with 71 from 2.09 to 0.80 ms (weights at 3.5 TB/s).
+//
+// 8 waves of 64 x 64; K in steps of 64, staged in two LDS buffers while the next step's
+// loads are in flight. The product is W^T X^T, so that a lane ends with 4 neighbouring
+// columns of one row. Weights lie in LDS as in memory and are read by transposing loads;
+// NF4 weights are dequantized on the way, so that their packed form is what is read.
+// LDS rows are 128 (X) and 512 (W) bytes: their 16-byte groups are permuted by the row, so
+// that the 16 rows that a load touches lie in different banks.
+//
+// Workgroups are dealt to the 8 chiplets in turn; a chiplet takes every eighth run of
+// columns and all row groups of it one after the other: they find its weights in its L2.
 
-#define MOE_MT 32        // C tile rows (2 MFMA row blocks)
-#define MOE_NT 128       // C tile cols (4 waves x 2 MFMA col blocks)
-#define MOE_KT 64        // k (in-dim) step staged in LDS
-#define MOE_KPAD 8       // LDS k padding (elements)
+#define MOE_MT 32   // rows of a tile of one expert
+#define MOE_BM 128  // rows of a workgroup
+#define MOE_BN 256  // columns of a workgroup
+#define MOE_BK 64   // k step
+#define MOE_X_BYTES (MOE_BM * MOE_BK * 2)
+#define MOE_W_BYTES (MOE_BK * MOE_BN * 2)
+#define MOE_LDS (2 * (MOE_X_BYTES + MOE_W_BYTES))
 
-#define BT_BYTE(n, k_byte) \
-  ((((unsigned)(n)) * ((MOE_KT + MOE_KPAD) * 2) + (unsigned)(k_byte)) ^ ((((unsigned)(n) >> 3) & 7u) << 4))
+// where 16-byte group c of a row lies
+__device__ __forceinline__ int moe_x_at(int row, int c) { return row * (MOE_BK * 2) + ((c ^ ((row >> 1) & 7)) << 4); }
+__device__ __forceinline__ int moe_w_at(int row, int c) {
+  return row * (MOE_BN * 2) + ((c ^ (((row & 3) | ((row >> 1) & 4)) << 1)) << 4);
+}
+
+// The first tile of the which-th group: tiles come in runs of one expert, a run's groups
+// have four tiles, its last one maybe fewer. -1: there are not so many. Uniform over a wave.
+__device__ __forceinline__ int moe_group_tile(const int* __restrict__ tile_expert, int n_tiles, int which) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  int seen = 0, run = 0;  // groups so far; first tile of the run that reaches into this chunk
+  for (int base = 0; base < n_tiles; base += WAVE) {
+    const int i = base + lane;
+    const int e = i < n_tiles ? tile_expert[i] : -1;
+    const int before = i > 0 && i <= n_tiles ? tile_expert[i - 1] : -1;
+    const unsigned long long starts = __ballot(e != before || i == 0);
+    const unsigned long long upto = starts & (~0ull >> (WAVE - 1 - lane));
+    const int first = upto ? base + WAVE - 1 - __clzll((long long)upto) : run;
+    const unsigned long long leads = __ballot(e >= 0 && ((i - first) & 3) == 0);
+    const int n = __popcll(leads);
+    if (which < seen + n) {
+      const bool mine = ((leads >> lane) & 1) && __popcll(leads & ((1ull << lane) - 1)) == which - seen;
+      return base + __ffsll((long long)__ballot(mine)) - 1;
+    }
+    seen += n;
+    if (starts) run = base + WAVE - 1 - __clzll((long long)starts);
+  }
+  return -1;
+}
 
 template <bool NF4>
-__global__ __launch_bounds__(256) void moe_gemm_kernel(
+__global__ __launch_bounds__(512) void moe_gemm_kernel(
     const unsigned short* __restrict__ wt_all,      // [E, in, out] bf16 (NF4: null)
     const unsigned char* __restrict__ packed_all,   // [E, in, out/2] u8 (bf16: null)
     const unsigned short* __restrict__ absmax_all,  // [E, in, out/64] bf16 (bf16: null)
@@ -253,132 +293,141 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(
     unsigned short* __restrict__ c,                 // [R, out] bf16
     int in_dim,
     int out_dim,
-    int k_per_tok) {
-  const int tile = blockIdx.x;
+    int k_per_tok,
+    int n_tiles,
+    int experts,
+    int groups) {
+  extern __shared__ unsigned char smem[];
+  __shared__ float2 lut2[NF4 ? 256 : 1];
+  const int slot = blockIdx.x >> 3;
+  const int n0 = ((slot / groups) * 8 + (blockIdx.x & 7)) * MOE_BN;
+  if (n0 >= out_dim) return;
+  const int tile = moe_group_tile(tile_expert, n_tiles, slot % groups);
+  if (tile < 0) return;
   const int e = tile_expert[tile];
-  if (e < 0) return;  // pure-padding tile
-  const int n0 = blockIdx.y * MOE_NT;
+  if (e >= experts) return;
+  int rows = MOE_MT;  // of this group
+  while (rows < MOE_BM && tile + rows / MOE_MT < n_tiles && tile_expert[tile + rows / MOE_MT] == e) rows += MOE_MT;
 
-  const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
-  const int lane = tid & (WAVE - 1);
-  const int col = lane & 15;
-  const int hi = lane >> 4;
+  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
+  const int col = lane & 15, hi = lane >> 4;
+  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;  // this wave's rows and columns
+  if (NF4 && tid < 256) lut2[tid] = make_float2(MOE_NF4_LUT[tid & 0xF], MOE_NF4_LUT[tid >> 4]);
 
-  __shared__ float2 lut2[256];
-  if (NF4) {
-    for (int i = tid; i < 256; i += 256)
-      lut2[i] = make_float2(MOE_NF4_LUT[i & 0xF], MOE_NF4_LUT[i >> 4]);
+  // loads of a step: two 16-byte groups of X, and four of W or 32 packed weights, per thread
+  constexpr int XN = MOE_BM * MOE_BK / 8 / 512, WN = NF4 ? 1 : MOE_BK * MOE_BN / 8 / 512;
+  const unsigned short* xp[XN];
+#pragma unroll
+  for (int i = 0; i < XN; ++i) {
+    const int row = (tid + i * 512) / 8;
+    const int pr = row < rows ? sorted_pairs[tile * MOE_MT + row] : -1;
+    xp[i] = pr < 0 ? nullptr : x + (size_t)(pr / k_per_tok) * in_dim + (tid & 7) * 8;
   }
-  __shared__ unsigned char bt_raw[MOE_NT * (MOE_KT + MOE_KPAD) * 2];
-
-  // this lane's A rows (2 row blocks): token index per MFMA A row
-  int tok[2];
-  int cpair[2][4];  // C rows: pair ids for rows rb*16 + hi*4 + r
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const int pr = sorted_pairs[tile * MOE_MT + rb * 16 + col];
-    tok[rb] = pr >= 0 ? pr / k_per_tok : -1;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      cpair[rb][r] = sorted_pairs[tile * MOE_MT + rb * 16 + hi * 4 + r];
-  }
-
-  f32x4_moe acc[2][2];
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) acc[rb][nb] = f32x4_moe{0.f, 0.f, 0.f, 0.f};
-
   const size_t w_stride = (size_t)in_dim * out_dim;
+  const int wc = NF4 ? (tid & 7) * 32 : (tid & 31) * 8;  // first column and row of this thread's weights
+  const int wr = NF4 ? tid >> 3 : tid >> 5;
+  const bool w_live = n0 + wc < out_dim;  // out_dim is a multiple of 128
+  const unsigned short* wp = NF4 ? nullptr : wt_all + e * w_stride + (size_t)wr * out_dim + n0 + wc;
+  const unsigned char* pp = NF4 ? packed_all + (e * w_stride + (size_t)wr * out_dim + n0 + wc) / 2 : nullptr;
+  const unsigned short* sp = NF4 ? absmax_all + (e * w_stride + (size_t)wr * out_dim + n0 + wc) / 64 : nullptr;
 
-  for (int kt = 0; kt < in_dim; kt += MOE_KT) {
-    // ---- stage B tile [MOE_KT k][MOE_NT n] transposed+swizzled into LDS
-    __syncthreads();
-    {
-      const int krow = kt + (tid >> 2);          // 64 rows, 4 threads per row
-      const int nloc = (tid & 3) * 32;           // 32 n values per thread
-      if (NF4) {
-        // 16 packed bytes -> 32 values; one absmax block per thread
-        unsigned int pk4[4] = {0u, 0u, 0u, 0u};
-        float am = 0.f;
-        if (krow < in_dim && n0 + nloc < out_dim) {
-          const unsigned char* prow =
-              packed_all + (size_t)e * (w_stride >> 1) + (size_t)krow * (out_dim >> 1) + ((n0 + nloc) >> 1);
-          const uint4 p = *reinterpret_cast<const uint4*>(prow);
-          pk4[0] = p.x; pk4[1] = p.y; pk4[2] = p.z; pk4[3] = p.w;
-          am = bf16_to_f32(absmax_all[(size_t)e * (w_stride >> 6) + (size_t)krow * (out_dim >> 6) + ((n0 + nloc) >> 6)]);
-        }
-        const int kb = (krow - kt) * 2;  // k byte offset in LDS rows
+  short8 xn[XN], wnext[WN];
+  uint4 pk = {0u, 0u, 0u, 0u};
+  unsigned short am = 0;
 #pragma unroll
-        for (int w4 = 0; w4 < 4; ++w4)
+  for (int i = 0; i < XN; ++i) xn[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const float2 w2 = lut2[(pk4[w4] >> (8 * b)) & 0xFFu];
-            const int n = nloc + w4 * 8 + b * 2;
-            *reinterpret_cast<unsigned short*>(&bt_raw[BT_BYTE(n, kb)]) = f32_to_bf16(w2.x * am);
-            *reinterpret_cast<unsigned short*>(&bt_raw[BT_BYTE(n + 1, kb)]) = f32_to_bf16(w2.y * am);
-          }
+  for (int i = 0; i < WN; ++i) wnext[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+  auto fetch = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < XN; ++i)
+      if (xp[i]) xn[i] = *reinterpret_cast<const short8*>(xp[i] + kt);
+    if (w_live) {
+      if constexpr (NF4) {
+        pk = *reinterpret_cast<const uint4*>(pp + (size_t)kt * out_dim / 2);
+        am = sp[(size_t)kt * out_dim / 64];
       } else {
-        const int kb = (krow - kt) * 2;
 #pragma unroll
-        for (int c8 = 0; c8 < 4; ++c8) {
-          short8 w8 = {0, 0, 0, 0, 0, 0, 0, 0};
-          if (krow < in_dim && n0 + nloc + c8 * 8 < out_dim)
-            w8 = *reinterpret_cast<const short8*>(
-                wt_all + (size_t)e * w_stride + (size_t)krow * out_dim + n0 + nloc + c8 * 8);
-#pragma unroll
-          for (int v = 0; v < 8; ++v)
-            *reinterpret_cast<unsigned short*>(&bt_raw[BT_BYTE(nloc + c8 * 8 + v, kb)]) =
-                (unsigned short)w8[v];
-        }
+        for (int i = 0; i < WN; ++i)
+          wnext[i] = *reinterpret_cast<const short8*>(wp + (size_t)(kt + i * 16) * out_dim);
       }
     }
-    __syncthreads();
+  };
+  auto stage = [&](unsigned char* buf) {
+#pragma unroll
+    for (int i = 0; i < XN; ++i) *reinterpret_cast<short8*>(buf + moe_x_at((tid + i * 512) / 8, tid & 7)) = xn[i];
+    unsigned char* w = buf + MOE_X_BYTES;
+    if constexpr (NF4) {
+      const float scale = bf16_to_f32(am);
+      const unsigned int words[4] = {pk.x, pk.y, pk.z, pk.w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        short8 v;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const float2 two = lut2[(words[q] >> (8 * b)) & 0xFFu];
+          v[2 * b] = (short)f32_to_bf16(two.x * scale);
+          v[2 * b + 1] = (short)f32_to_bf16(two.y * scale);
+        }
+        *reinterpret_cast<short8*>(w + moe_w_at(wr, wc / 8 + q)) = v;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < WN; ++i) *reinterpret_cast<short8*>(w + moe_w_at(wr + i * 16, wc / 8)) = wnext[i];
+    }
+  };
 
-    // ---- MFMA: 2 k-chunks x 2 row blocks x 2 col blocks
+  f32x4_moe acc[4][4];  // [columns][rows]
 #pragma unroll
-    for (int kc = 0; kc < MOE_KT / 32; ++kc) {
-      bf16x8_moe a_frag[2];
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        if (tok[rb] >= 0 && kt + kc * 32 + hi * 8 + 8 <= in_dim) {
-          a_frag[rb] = *reinterpret_cast<const bf16x8_moe*>(
-              x + (size_t)tok[rb] * in_dim + kt + kc * 32 + hi * 8);
-        } else if (tok[rb] >= 0 && kt + kc * 32 + hi * 8 < in_dim) {
-          short vs[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-          for (int v = 0; v < 8 && kt + kc * 32 + hi * 8 + v < in_dim; ++v)
-            vs[v] = (short)x[(size_t)tok[rb] * in_dim + kt + kc * 32 + hi * 8 + v];
-          a_frag[rb] = bf16x8_moe{vs[0], vs[1], vs[2], vs[3], vs[4], vs[5], vs[6], vs[7]};
-        } else {
-          a_frag[rb] = bf16x8_moe{0, 0, 0, 0, 0, 0, 0, 0};
-        }
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_moe{0.f, 0.f, 0.f, 0.f};
+
+  fetch(0);
+  if (NF4) __syncthreads();  // the table
+  stage(smem);
+  __syncthreads();
+  int which = 0;
+  for (int kt = 0; kt < in_dim; kt += MOE_BK, which ^= 1) {
+    const bool more = kt + MOE_BK < in_dim;
+    if (more) fetch(kt + MOE_BK);
+    const unsigned char* xb = smem + which * (MOE_X_BYTES + MOE_W_BYTES);
+    const unsigned char* wb = xb + MOE_X_BYTES;
+#pragma unroll
+    for (int kc = 0; kc < MOE_BK / 32; ++kc) {
+      bf16x8_moe xf[4], wf[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        xf[j] = *reinterpret_cast<const bf16x8_moe*>(xb + moe_x_at(wm + j * 16 + col, kc * 4 + hi));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // rows hi*8 + col/4 and 4 below, which are permuted alike; 4 columns a lane
+        const int row = kc * 32 + hi * 8 + col / 4, group = (wn + i * 16) / 8 + ((col >> 1) & 1);
+        wf[i] = load_keys(reinterpret_cast<const unsigned short*>(wb + moe_w_at(row, group) + (col & 1) * 8), MOE_BN);
       }
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        const int n = wave * 32 + nb * 16 + col;
-        const bf16x8_moe b_frag =
-            *reinterpret_cast<const bf16x8_moe*>(&bt_raw[BT_BYTE(n, kc * 64 + hi * 16)]);
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-          acc[rb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_frag[rb], b_frag, acc[rb][nb], 0, 0, 0);
-      }
+        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
     }
+    if (more) stage(smem + (which ^ 1) * (MOE_X_BYTES + MOE_W_BYTES));
+    __syncthreads();
   }
 
-  // ---- write C (bf16, original pair rows): C row = hi*4 + r within block
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int j = 0; j < 4; ++j) {
+    const int row = wm + j * 16 + col;
+    const int pr = row < rows ? sorted_pairs[tile * MOE_MT + row] : -1;
+    if (pr < 0) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int pr = cpair[rb][r];
-      if (pr < 0) continue;
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        const int n = n0 + wave * 32 + nb * 16 + col;
-        if (n < out_dim) c[(size_t)pr * out_dim + n] = f32_to_bf16(acc[rb][nb][r]);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int n = n0 + wn + i * 16 + hi * 4;
+      if (n < out_dim)
+        *reinterpret_cast<v4s*>(c + (size_t)pr * out_dim + n) =
+            v4s{(short)f32_to_bf16(acc[i][j][0]), (short)f32_to_bf16(acc[i][j][1]), (short)f32_to_bf16(acc[i][j][2]),
+                (short)f32_to_bf16(acc[i][j][3])};
     }
+  }
 }
 
 // ------------------------------------------------------------------- host
@@ -410,28 +459,37 @@ torch::Tensor moe_gemm(
   TORCH_CHECK(x.size(1) == in_dim);
   // staging loads are 16B/32-value vectors: callers fall back to the dense
   // path for geometries outside these alignments (fused_moe.py)
-  TORCH_CHECK(out_dim % MOE_NT == 0, "moe_gemm needs out_dim % 128 == 0");
-  TORCH_CHECK(in_dim % MOE_KT == 0, "moe_gemm needs in_dim % 64 == 0");
-  const int Rp = sorted_pairs.size(0);
+  TORCH_CHECK(out_dim % 128 == 0, "moe_gemm needs out_dim % 128 == 0");
+  TORCH_CHECK(in_dim % MOE_BK == 0, "moe_gemm needs in_dim % 64 == 0");
+  const long Rp = sorted_pairs.size(0);
   TORCH_CHECK(Rp % MOE_MT == 0 && tile_expert.size(0) == Rp / MOE_MT);
 
   auto c = torch::empty({n_rows, (long)out_dim}, x.options());
-  dim3 grid(Rp / MOE_MT, (out_dim + MOE_NT - 1) / MOE_NT);
+  const long n_tiles = Rp / MOE_MT, experts = nf4 ? packed_all->size(0) : wt_all->size(0);
+  // an expert's last group may have one tile
+  const long groups = std::min(n_tiles, (n_tiles + 3 * experts) / 4);
+  if (groups == 0) return c;
+  const long columns = (out_dim + MOE_BN - 1) / MOE_BN;
+  const long blocks = groups * ((columns + 7) / 8) * 8;
+  TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
   auto stream = at::cuda::getCurrentCUDAStream();
+#define MOE_GEMM(NF4, W, P, S)                                                                              \
+  do {                                                                                                      \
+    static const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_kernel<NF4>), \
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS); \
+    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                 \
+    moe_gemm_kernel<NF4><<<blocks, 512, MOE_LDS, stream>>>(                                                 \
+        W, P, S, reinterpret_cast<const unsigned short*>(x.data_ptr()), sorted_pairs.data_ptr<int>(),       \
+        tile_expert.data_ptr<int>(), reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim,      \
+        (int)k_per_tok, (int)n_tiles, (int)experts, (int)groups);                                           \
+  } while (0)
   if (nf4) {
-    moe_gemm_kernel<true><<<grid, 256, 0, stream>>>(
-        nullptr, packed_all->data_ptr<unsigned char>(),
-        reinterpret_cast<const unsigned short*>(absmax_all->data_ptr()),
-        reinterpret_cast<const unsigned short*>(x.data_ptr()),
-        sorted_pairs.data_ptr<int>(), tile_expert.data_ptr<int>(),
-        reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim, (int)k_per_tok);
+    MOE_GEMM(true, nullptr, packed_all->data_ptr<unsigned char>(),
+             reinterpret_cast<const unsigned short*>(absmax_all->data_ptr()));
   } else {
-    moe_gemm_kernel<false><<<grid, 256, 0, stream>>>(
-        reinterpret_cast<const unsigned short*>(wt_all->data_ptr()), nullptr, nullptr,
-        reinterpret_cast<const unsigned short*>(x.data_ptr()),
-        sorted_pairs.data_ptr<int>(), tile_expert.data_ptr<int>(),
-        reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim, (int)k_per_tok);
+    MOE_GEMM(false, reinterpret_cast<const unsigned short*>(wt_all->data_ptr()), nullptr, nullptr);
   }
+#undef MOE_GEMM
   HIP_CHECK_LAST();
   return c;
 }

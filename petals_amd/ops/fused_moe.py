@@ -31,7 +31,7 @@ from petals_amd.ops.fused_decode import (
 )
 
 
-MOE_GEMM_MT = 32  # moe_gemm C-tile rows (ops/csrc/moe.hip MOE_MT)
+MOE_GEMM_MT = 32  # rows of a tile of one expert (ops/csrc/moe.hip MOE_MT)
 
 
 def sort_pairs_by_expert(selected: torch.Tensor, num_experts: int):
