@@ -27,8 +27,8 @@ SRC_DIR = os.path.join(PKG_DIR, "csrc")
 EXTENSIONS = {
     "core": (
         "_hip_ops.so", "petals_amd_hip_ops", "_build",
-        ["bindings.cpp", "elementwise.hip", "gemv.hip", "attention.hip", "nf4.hip", "int8.hip", "prefill_attn.hip",
-         "moe.hip"],
+        ["bindings.cpp", "elementwise.hip", "gemv.hip", "attention.hip", "nf4.hip", "nf4_tiles.hip", "int8.hip",
+         "prefill_attn.hip", "moe.hip"],
     ),
     "latent": (
         "_hip_latent.so", "petals_amd_hip_latent", os.path.join("_build", "latent"),

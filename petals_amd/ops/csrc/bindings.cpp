@@ -48,12 +48,17 @@ torch::Tensor sumsq_rows(torch::Tensor x);
 torch::Tensor gemv_bf16_moe(
     torch::Tensor wt_all, torch::Tensor x, torch::Tensor sel, int64_t k_per_tok,
     torch::Tensor workspace, int64_t epilogue, int64_t splits_override, double limit, double alpha);
-torch::Tensor gemv_nf4_moe(
-    torch::Tensor packed_all, torch::Tensor absmax_all, torch::Tensor x, torch::Tensor sel,
-    int64_t k_per_tok, torch::Tensor workspace, int64_t epilogue, int64_t splits_override);
+std::vector<torch::Tensor> nf4_tile(torch::Tensor packed, torch::Tensor absmax);
+torch::Tensor nf4_untile(torch::Tensor tiles, torch::Tensor scales, int64_t in_dim);
+torch::Tensor gemv_nf4_tiles(
+    torch::Tensor tiles, torch::Tensor scales, int64_t in_dim, torch::Tensor x, torch::Tensor workspace,
+    c10::optional<torch::Tensor> residual, int64_t epilogue, c10::optional<torch::Tensor> bias);
+torch::Tensor gemv_nf4_tiles_moe(
+    torch::Tensor tiles, torch::Tensor scales, int64_t in_dim, torch::Tensor x, torch::Tensor sel,
+    int64_t k_per_tok, torch::Tensor workspace, int64_t epilogue);
 torch::Tensor moe_gemm(
-    c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> packed_all,
-    c10::optional<torch::Tensor> absmax_all, torch::Tensor x, torch::Tensor sorted_pairs,
+    c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> nf4_all,
+    c10::optional<torch::Tensor> scales_all, torch::Tensor x, torch::Tensor sorted_pairs,
     torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -98,13 +103,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("wt_all"), py::arg("x"), py::arg("sel"), py::arg("k_per_tok"),
         py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0);
-  m.def("gemv_nf4_moe", &gemv_nf4_moe,
-        "device-routed MoE gemv: stacked NF4 expert weights, expert ids from a device tensor",
-        py::arg("packed_all"), py::arg("absmax_all"), py::arg("x"), py::arg("sel"),
-        py::arg("k_per_tok"), py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0);
+  m.def("nf4_tile", &nf4_tile, "NF4 in the order of the matrix cores: (packed, absmax) -> (tiles, scales)");
+  m.def("nf4_untile", &nf4_untile, "(tiles, scales) -> bf16 [in, out]");
+  m.def("gemv_nf4_tiles", &gemv_nf4_tiles, "few rows times NF4 tiles, with epilogue",
+        py::arg("tiles"), py::arg("scales"), py::arg("in_dim"), py::arg("x"), py::arg("workspace"),
+        py::arg("residual"), py::arg("epilogue"), py::arg("bias") = py::none());
+  m.def("gemv_nf4_tiles_moe", &gemv_nf4_tiles_moe,
+        "device-routed MoE gemv: stacked NF4 tiles, expert ids from a device tensor",
+        py::arg("tiles"), py::arg("scales"), py::arg("in_dim"), py::arg("x"), py::arg("sel"),
+        py::arg("k_per_tok"), py::arg("workspace"), py::arg("epilogue"));
   m.def("moe_gemm", &moe_gemm,
         "grouped MFMA GEMM over expert-sorted (token, slot) pairs (prefill; NF4 dequant fused "
         "into the LDS B-tile staging)",
-        py::arg("wt_all"), py::arg("packed_all"), py::arg("absmax_all"), py::arg("x"),
+        py::arg("wt_all"), py::arg("nf4_all"), py::arg("scales_all"), py::arg("x"),
         py::arg("sorted_pairs"), py::arg("tile_expert"), py::arg("k_per_tok"), py::arg("n_rows"));
 }

@@ -10,8 +10,8 @@ torch::Tensor gemv_bf16_moe(
     torch::Tensor wt_all, torch::Tensor x, torch::Tensor sel, int64_t k_per_tok,
     torch::Tensor workspace, int64_t epilogue, int64_t splits_override, double limit, double alpha);
 torch::Tensor moe_gemm(
-    c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> packed_all,
-    c10::optional<torch::Tensor> absmax_all, torch::Tensor x, torch::Tensor sorted_pairs,
+    c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> nf4_all,
+    c10::optional<torch::Tensor> scales_all, torch::Tensor x, torch::Tensor sorted_pairs,
     torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows);
 torch::Tensor latent_attention(
     torch::Tensor q, torch::Tensor cache, torch::Tensor pos, torch::Tensor owner, torch::Tensor tables,

@@ -8,10 +8,10 @@
 // whole-span decode graph (the reference runs Mixtral experts densely inside
 // HF code with host-side routing: reference models/mixtral/block.py:73-81).
 //
-// Weight layouts match gemv.hip / nf4.hip exactly, stacked on a leading
-// expert axis:
+// Weight layouts match gemv.hip / nf4_tiles.hip, stacked on a leading expert axis:
 //   bf16: wt_all   [E, in, out]
-//   nf4:  packed   [E, in, out/2], absmax [E, in, out/64]
+//   nf4:  tiles    [E, out/64, in/128, 4, 64, 16], scales [E, out/64, in]; its GEMV is
+//         nf4_tiles.hip's
 // The per-row inner loop is the same x-broadcast split-K structure as the
 // dense kernels (each selected expert's weights are read exactly once per
 // token).
@@ -25,7 +25,6 @@
 #ifndef GEMV_OUT_PER_WAVE
 #define GEMV_OUT_PER_WAVE 512
 #endif
-#define NF4_OUT_PER_WAVE 1024
 
 using bf16x8_moe = __attribute__((ext_vector_type(8))) short;
 using f32x4_moe = __attribute__((ext_vector_type(4))) float;
@@ -114,113 +113,6 @@ __global__ __launch_bounds__(WAVE) void gemv_bf16_moe_kernel(
   }
 }
 
-// ------------------------------------------------------------- nf4 indexed
-
-__global__ __launch_bounds__(WAVE) void gemv_nf4_moe_kernel(
-    const unsigned char* __restrict__ packed_all,   // [E, in, out/2]
-    const unsigned short* __restrict__ absmax_all,  // [E, in, out/64]
-    const float* __restrict__ x,                    // [B, in]
-    const int* __restrict__ sel,                    // [R]
-    float* __restrict__ partials,                   // [n_splits, R, out]
-    int in_dim,
-    int out_dim,
-    int i_per_split,
-    int rows,
-    int k_per_tok) {
-  __shared__ float2 lut2[256];
-  for (int i = threadIdx.x; i < 256; i += blockDim.x)
-    lut2[i] = make_float2(MOE_NF4_LUT[i & 0xF], MOE_NF4_LUT[i >> 4]);
-  __syncthreads();
-
-  const int row = blockIdx.z;
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int out0 = blockIdx.x * NF4_OUT_PER_WAVE + lane * 16;
-  if (out0 >= out_dim) return;
-  const int split = blockIdx.y;
-  const int i_begin = split * i_per_split;
-  const int i_end = min(i_begin + i_per_split, in_dim);
-  const bool full = (out0 + 16) <= out_dim;
-
-  const int e = sel[row];
-  const unsigned char* packed = packed_all + (size_t)e * in_dim * (out_dim >> 1);
-  const unsigned short* absmax = absmax_all + (size_t)e * in_dim * (out_dim >> 6);
-  const float* xr = x + (size_t)(row / k_per_tok) * in_dim;
-
-  float acc[16];
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-
-  if (full) {
-    constexpr int UNROLL = 16;
-    const int half_out = out_dim >> 1;
-    const unsigned char* pp = packed + (size_t)i_begin * half_out + (out0 >> 1);
-    int i = i_begin;
-    for (; i + UNROLL <= i_end; i += UNROLL) {
-      uint2 pk[UNROLL];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u)
-        pk[u] = *reinterpret_cast<const uint2*>(pp + (size_t)u * half_out);
-      float am[UNROLL];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u)
-        am[u] = bf16_to_f32(absmax[(size_t)(i + u) * (out_dim >> 6) + (out0 >> 6)]);
-      float xs[UNROLL];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) xs[u] = xr[i + u];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        const float xa = xs[u] * am[u];
-        const unsigned int wds2[2] = {pk[u].x, pk[u].y};
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-#pragma unroll
-          for (int p2 = 0; p2 < 4; ++p2) {
-            const float2 w2 = lut2[(wds2[d] >> (8 * p2)) & 0xFFu];
-            acc[8 * d + 2 * p2] = fmaf(w2.x, xa, acc[8 * d + 2 * p2]);
-            acc[8 * d + 2 * p2 + 1] = fmaf(w2.y, xa, acc[8 * d + 2 * p2 + 1]);
-          }
-      }
-      pp += (size_t)UNROLL * half_out;
-    }
-    for (; i < i_end; ++i) {
-      const uint2 pk = *reinterpret_cast<const uint2*>(packed + (size_t)i * half_out + (out0 >> 1));
-      const float xa = xr[i] * bf16_to_f32(absmax[(size_t)i * (out_dim >> 6) + (out0 >> 6)]);
-      const unsigned int twds[2] = {pk.x, pk.y};
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int p2 = 0; p2 < 4; ++p2) {
-          const float2 w2 = lut2[(twds[d] >> (8 * p2)) & 0xFFu];
-          acc[8 * d + 2 * p2] = fmaf(w2.x, xa, acc[8 * d + 2 * p2]);
-          acc[8 * d + 2 * p2 + 1] = fmaf(w2.y, xa, acc[8 * d + 2 * p2 + 1]);
-        }
-    }
-  } else {
-    for (int i = i_begin; i < i_end; ++i) {
-      const float xa = xr[i] * bf16_to_f32(absmax[(size_t)i * (out_dim >> 6) + (out0 >> 6)]);
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if (out0 + v < out_dim) {
-          const unsigned char byte = packed[(size_t)i * (out_dim >> 1) + ((out0 + v) >> 1)];
-          const float2 w2 = lut2[byte];
-          acc[v] = fmaf(((out0 + v) & 1) ? w2.y : w2.x, xa, acc[v]);
-        }
-    }
-  }
-
-  float* dst = partials + ((size_t)split * rows + row) * out_dim + out0;
-  if (full) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      reinterpret_cast<float4v*>(dst)[q] =
-          float4v{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-  } else {
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-      if (out0 + v < out_dim) dst[v] = acc[v];
-  }
-}
-
 // ------------------------------------------------- grouped GEMM (prefill)
 //
 // Grouped GEMM over expert-sorted (token, slot) pairs: the caller sorts the R = T*k
@@ -236,10 +128,11 @@ __global__ __launch_bounds__(WAVE) void gemv_nf4_moe_kernel(
 //
 // 8 waves of 64 x 64; K in steps of 64, staged in two LDS buffers while the next step's
 // loads are in flight. The product is W^T X^T, so that a lane ends with 4 neighbouring
-// columns of one row. Weights lie in LDS as in memory and are read by transposing loads;
-// NF4 weights are dequantized on the way, so that their packed form is what is read.
-// LDS rows are 128 (X) and 512 (W) bytes: their 16-byte groups are permuted by the row, so
-// that the 16 rows that a load touches lie in different banks.
+// columns of one row. Weights in bf16 lie in LDS as in memory and are read by transposing
+// loads. NF4 weights are dequantized on the way, so that their packed form is what is read:
+// a thread has 16 codes of one column, and its LDS rows are columns. The 16-byte groups of
+// an LDS row, of 128 or (W in bf16) 512 bytes, are permuted by the row, so that the 16 rows
+// that a load touches lie in different banks.
 //
 // Workgroups are dealt to the 8 chiplets in turn; a chiplet takes every eighth run of
 // columns and all row groups of it one after the other: they find its weights in its L2.
@@ -285,8 +178,8 @@ __device__ __forceinline__ int moe_group_tile(const int* __restrict__ tile_exper
 template <bool NF4>
 __global__ __launch_bounds__(512) void moe_gemm_kernel(
     const unsigned short* __restrict__ wt_all,      // [E, in, out] bf16 (NF4: null)
-    const unsigned char* __restrict__ packed_all,   // [E, in, out/2] u8 (bf16: null)
-    const unsigned short* __restrict__ absmax_all,  // [E, in, out/64] bf16 (bf16: null)
+    const uint4* __restrict__ nf4_all,              // NF4: tiles (bf16: null)
+    const unsigned short* __restrict__ scales_all,  // NF4: [E, out/64, n_kb * 128] bf16
     const unsigned short* __restrict__ x,           // [T, in] bf16
     const int* __restrict__ sorted_pairs,           // [Rp] pair id or -1 (padding)
     const int* __restrict__ tile_expert,            // [Rp/MT] expert id or -1
@@ -314,8 +207,9 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
   const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;  // this wave's rows and columns
   if (NF4 && tid < 256) lut2[tid] = make_float2(MOE_NF4_LUT[tid & 0xF], MOE_NF4_LUT[tid >> 4]);
 
-  // loads of a step: two 16-byte groups of X, and four of W or 32 packed weights, per thread
-  constexpr int XN = MOE_BM * MOE_BK / 8 / 512, WN = NF4 ? 1 : MOE_BK * MOE_BN / 8 / 512;
+  // loads of a step: two 16-byte groups of X, and four of W, or for two steps two of NF4
+  // codes (32 of a column) and for each step their 16 scales, per thread
+  constexpr int XN = MOE_BM * MOE_BK / 8 / 512, WN = MOE_BK * MOE_BN / 8 / 512;
   const unsigned short* xp[XN];
 #pragma unroll
   for (int i = 0; i < XN; ++i) {
@@ -323,53 +217,64 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
     const int pr = row < rows ? sorted_pairs[tile * MOE_MT + row] : -1;
     xp[i] = pr < 0 ? nullptr : x + (size_t)(pr / k_per_tok) * in_dim + (tid & 7) * 8;
   }
-  const size_t w_stride = (size_t)in_dim * out_dim;
-  const int wc = NF4 ? (tid & 7) * 32 : (tid & 31) * 8;  // first column and row of this thread's weights
-  const int wr = NF4 ? tid >> 3 : tid >> 5;
-  const bool w_live = n0 + wc < out_dim;  // out_dim is a multiple of 128
-  const unsigned short* wp = NF4 ? nullptr : wt_all + e * w_stride + (size_t)wr * out_dim + n0 + wc;
-  const unsigned char* pp = NF4 ? packed_all + (e * w_stride + (size_t)wr * out_dim + n0 + wc) / 2 : nullptr;
-  const unsigned short* sp = NF4 ? absmax_all + (e * w_stride + (size_t)wr * out_dim + n0 + wc) / 64 : nullptr;
+  const int wc = (tid & 31) * 8, wr = tid >> 5;  // first column and row of this thread's weights
+  const bool w_live = n0 + wc < out_dim;         // out_dim is a multiple of 128
+  const unsigned short* wp = NF4 ? nullptr : wt_all + (size_t)e * in_dim * out_dim + (size_t)wr * out_dim + n0 + wc;
+  const int n_kb = (in_dim + 127) / 128;
 
-  short8 xn[XN], wnext[WN];
-  uint4 pk = {0u, 0u, 0u, 0u};
-  unsigned short am = 0;
+  short8 xn[XN], wnext[NF4 ? 1 : WN];
+  uint4 codes[2];
+  short8 scale[2][2];
 #pragma unroll
   for (int i = 0; i < XN; ++i) xn[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-  for (int i = 0; i < WN; ++i) wnext[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+  for (int i = 0; i < (NF4 ? 1 : WN); ++i) wnext[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    codes[i] = uint4{0u, 0u, 0u, 0u};
+    scale[i][0] = scale[i][1] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
   auto fetch = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < XN; ++i)
       if (xp[i]) xn[i] = *reinterpret_cast<const short8*>(xp[i] + kt);
-    if (w_live) {
-      if constexpr (NF4) {
-        pk = *reinterpret_cast<const uint4*>(pp + (size_t)kt * out_dim / 2);
-        am = sp[(size_t)kt * out_dim / 64];
-      } else {
+    if constexpr (NF4) {
 #pragma unroll
-        for (int i = 0; i < WN; ++i)
-          wnext[i] = *reinterpret_cast<const short8*>(wp + (size_t)(kt + i * 16) * out_dim);
+      for (int i = 0; i < 2; ++i) {
+        const int nb = n0 / 64 + tid / 256 + 2 * i;
+        if (nb * 64 >= out_dim) continue;
+        const size_t at = ((size_t)e * (out_dim / 64) + nb) * n_kb + kt / 128;
+        if (kt % 128 == 0) codes[i] = nf4_all[at * 256 + tid % 256];
+        const short8* p = reinterpret_cast<const short8*>(scales_all + at * 128 + kt % 128 + lane / 16 * 16);
+        scale[i][0] = p[0];
+        scale[i][1] = p[1];
       }
+    } else if (w_live) {
+#pragma unroll
+      for (int i = 0; i < WN; ++i)
+        wnext[i] = *reinterpret_cast<const short8*>(wp + (size_t)(kt + i * 16) * out_dim);
     }
   };
-  auto stage = [&](unsigned char* buf) {
+  auto stage = [&](unsigned char* buf, int kt) {
 #pragma unroll
     for (int i = 0; i < XN; ++i) *reinterpret_cast<short8*>(buf + moe_x_at((tid + i * 512) / 8, tid & 7)) = xn[i];
     unsigned char* w = buf + MOE_X_BYTES;
     if constexpr (NF4) {
-      const float scale = bf16_to_f32(am);
-      const unsigned int words[4] = {pk.x, pk.y, pk.z, pk.w};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        short8 v;
+      for (int i = 0; i < 2; ++i) {
+        const unsigned words[2] = {kt & 64 ? codes[i].z : codes[i].x, kt & 64 ? codes[i].w : codes[i].y};
+        const int row = (tid / 256 + 2 * i) * 64 + tid % 256 / 64 * 16 + col;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float2 two = lut2[(words[q] >> (8 * b)) & 0xFFu];
-          v[2 * b] = (short)f32_to_bf16(two.x * scale);
-          v[2 * b + 1] = (short)f32_to_bf16(two.y * scale);
+        for (int q = 0; q < 2; ++q) {
+          short8 v;
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            const float2 two = lut2[(words[q] >> (8 * b)) & 0xFFu];
+            v[b] = (short)f32_to_bf16(two.x * bf16_to_f32((unsigned short)scale[i][q][b]));
+            v[b + 4] = (short)f32_to_bf16(two.y * bf16_to_f32((unsigned short)scale[i][q][b + 4]));
+          }
+          *reinterpret_cast<short8*>(w + moe_x_at(row, hi * 2 + q)) = v;
         }
-        *reinterpret_cast<short8*>(w + moe_w_at(wr, wc / 8 + q)) = v;
       }
     } else {
 #pragma unroll
@@ -385,7 +290,7 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
 
   fetch(0);
   if (NF4) __syncthreads();  // the table
-  stage(smem);
+  stage(smem, 0);
   __syncthreads();
   int which = 0;
   for (int kt = 0; kt < in_dim; kt += MOE_BK, which ^= 1) {
@@ -401,6 +306,10 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
         xf[j] = *reinterpret_cast<const bf16x8_moe*>(xb + moe_x_at(wm + j * 16 + col, kc * 4 + hi));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        if constexpr (NF4) {
+          wf[i] = *reinterpret_cast<const bf16x8_moe*>(wb + moe_x_at(wn + i * 16 + col, kc * 4 + hi));
+          continue;
+        }
         // rows hi*8 + col/4 and 4 below, which are permuted alike; 4 columns a lane
         const int row = kc * 32 + hi * 8 + col / 4, group = (wn + i * 16) / 8 + ((col >> 1) & 1);
         wf[i] = load_keys(reinterpret_cast<const unsigned short*>(wb + moe_w_at(row, group) + (col & 1) * 8), MOE_BN);
@@ -410,7 +319,7 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
     }
-    if (more) stage(smem + (which ^ 1) * (MOE_X_BYTES + MOE_W_BYTES));
+    if (more) stage(smem + (which ^ 1) * (MOE_X_BYTES + MOE_W_BYTES), kt + MOE_BK);
     __syncthreads();
   }
 
@@ -434,8 +343,8 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
 
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all,      // [E, in, out] bf16
-    c10::optional<torch::Tensor> packed_all,  // [E, in, out/2] u8
-    c10::optional<torch::Tensor> absmax_all,  // [E, in, out/64] bf16
+    c10::optional<torch::Tensor> nf4_all,     // NF4: [E, out/64, ceil(in/128), 4, 64, 16] u8
+    c10::optional<torch::Tensor> scales_all,  // NF4: [E, out/64, ceil(in/128) * 128] bf16
     torch::Tensor x,                          // [T, in] bf16
     torch::Tensor sorted_pairs,               // [Rp] i32 (expert-sorted, MT-padded, -1 = pad)
     torch::Tensor tile_expert,                // [Rp/MT] i32 (-1 = pure padding tile)
@@ -444,15 +353,20 @@ torch::Tensor moe_gemm(
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16 && x.dim() == 2 && x.is_contiguous());
   TORCH_CHECK(sorted_pairs.dtype() == torch::kInt32 && sorted_pairs.is_contiguous());
   TORCH_CHECK(tile_expert.dtype() == torch::kInt32 && tile_expert.is_contiguous());
-  const bool nf4 = packed_all.has_value();
+  const bool nf4 = nf4_all.has_value();
   int in_dim, out_dim;
   if (nf4) {
-    TORCH_CHECK(packed_all->dtype() == torch::kUInt8 && packed_all->dim() == 3 && packed_all->is_contiguous());
-    TORCH_CHECK(absmax_all.has_value() && absmax_all->dtype() == torch::kBFloat16);
-    in_dim = packed_all->size(1);
-    out_dim = packed_all->size(2) * 2;
+    TORCH_CHECK(nf4_all->dtype() == torch::kUInt8 && nf4_all->dim() == 6 && nf4_all->is_contiguous());
+    TORCH_CHECK(scales_all.has_value() && scales_all->dtype() == torch::kBFloat16 && scales_all->dim() == 3 &&
+                scales_all->is_contiguous());
+    in_dim = x.size(1);
+    out_dim = nf4_all->size(1) * 64;
+    TORCH_CHECK(nf4_all->size(2) == (in_dim + 127) / 128 && nf4_all->size(3) == 4 && nf4_all->size(4) == 64 &&
+                nf4_all->size(5) == 16);
+    TORCH_CHECK(scales_all->size(0) == nf4_all->size(0) && scales_all->size(1) == nf4_all->size(1) &&
+                scales_all->size(2) == nf4_all->size(2) * 128);
   } else {
-    TORCH_CHECK(wt_all.has_value() && wt_all->dtype() == torch::kBFloat16 && wt_all->dim() == 3);
+    TORCH_CHECK(wt_all.has_value() && wt_all->dtype() == torch::kBFloat16 && wt_all->dim() == 3 && wt_all->is_contiguous());
     in_dim = wt_all->size(1);
     out_dim = wt_all->size(2);
   }
@@ -465,7 +379,7 @@ torch::Tensor moe_gemm(
   TORCH_CHECK(Rp % MOE_MT == 0 && tile_expert.size(0) == Rp / MOE_MT);
 
   auto c = torch::empty({n_rows, (long)out_dim}, x.options());
-  const long n_tiles = Rp / MOE_MT, experts = nf4 ? packed_all->size(0) : wt_all->size(0);
+  const long n_tiles = Rp / MOE_MT, experts = nf4 ? nf4_all->size(0) : wt_all->size(0);
   // an expert's last group may have one tile
   const long groups = std::min(n_tiles, (n_tiles + 3 * experts) / 4);
   if (groups == 0) return c;
@@ -473,19 +387,19 @@ torch::Tensor moe_gemm(
   const long blocks = groups * ((columns + 7) / 8) * 8;
   TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
   auto stream = at::cuda::getCurrentCUDAStream();
-#define MOE_GEMM(NF4, W, P, S)                                                                              \
-  do {                                                                                                      \
-    static const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_kernel<NF4>), \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS); \
-    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                 \
-    moe_gemm_kernel<NF4><<<blocks, 512, MOE_LDS, stream>>>(                                                 \
-        W, P, S, reinterpret_cast<const unsigned short*>(x.data_ptr()), sorted_pairs.data_ptr<int>(),       \
-        tile_expert.data_ptr<int>(), reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim,      \
-        (int)k_per_tok, (int)n_tiles, (int)experts, (int)groups);                                           \
+#define MOE_GEMM(NF4, W, P, S)                                                                               \
+  do {                                                                                                       \
+    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_kernel<NF4>),        \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS);        \
+    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                  \
+    moe_gemm_kernel<NF4><<<blocks, 512, MOE_LDS, stream>>>(                                                  \
+        W, P, S, reinterpret_cast<const unsigned short*>(x.data_ptr()), sorted_pairs.data_ptr<int>(),        \
+        tile_expert.data_ptr<int>(), reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim,       \
+        (int)k_per_tok, (int)n_tiles, (int)experts, (int)groups);                                            \
   } while (0)
   if (nf4) {
-    MOE_GEMM(true, nullptr, packed_all->data_ptr<unsigned char>(),
-             reinterpret_cast<const unsigned short*>(absmax_all->data_ptr()));
+    MOE_GEMM(true, nullptr, reinterpret_cast<const uint4*>(nf4_all->data_ptr()),
+             reinterpret_cast<const unsigned short*>(scales_all->data_ptr()));
   } else {
     MOE_GEMM(false, reinterpret_cast<const unsigned short*>(wt_all->data_ptr()), nullptr, nullptr);
   }
@@ -535,48 +449,4 @@ torch::Tensor gemv_bf16_moe(
   return launch_gemv_reduce(
       partials, c10::nullopt, c10::nullopt, (int)splits, rows, out_dim, (int)epilogue,
       x.options(), wt_all.options(), c10::nullopt, ClampedGate{(float)limit, (float)alpha});
-}
-
-torch::Tensor gemv_nf4_moe(
-    torch::Tensor packed_all,  // [E, in, out/2] u8
-    torch::Tensor absmax_all,  // [E, in, out/64] bf16
-    torch::Tensor x,           // [B, in] f32
-    torch::Tensor sel,         // [R] int32
-    int64_t k_per_tok,
-    torch::Tensor workspace,
-    int64_t epilogue,
-    int64_t splits_override) {
-  TORCH_CHECK(packed_all.is_cuda() && packed_all.dtype() == torch::kUInt8 && packed_all.dim() == 3);
-  TORCH_CHECK(x.dtype() == torch::kFloat32 && x.dim() == 2);
-  TORCH_CHECK(sel.dtype() == torch::kInt32 && sel.is_contiguous());
-  const int in_dim = packed_all.size(1);
-  const int out_dim = packed_all.size(2) * 2;
-  const int rows = sel.size(0);
-  TORCH_CHECK(x.size(1) == in_dim && rows == x.size(0) * k_per_tok);
-  TORCH_CHECK(rows <= 16, "moe gemv supports batch*k <= 16");
-
-  const long out_waves = (out_dim + NF4_OUT_PER_WAVE - 1) / NF4_OUT_PER_WAVE;
-  long splits = splits_override > 0 ? splits_override : (1536 + out_waves * rows - 1) / (out_waves * rows);
-  long max_splits = (in_dim + 31) / 32;
-  if (splits > max_splits) splits = max_splits;
-  if (splits < 1) splits = 1;
-  const int i_per_split = (in_dim + (int)splits - 1) / (int)splits;
-
-  torch::Tensor partials;
-  if (workspace.numel() >= (int64_t)splits * rows * out_dim) {
-    partials = workspace;
-  } else {
-    partials = torch::empty({splits, (long)rows, (long)out_dim}, x.options());
-  }
-  dim3 grid(out_waves, splits, rows);
-  auto stream = at::cuda::getCurrentCUDAStream();
-  gemv_nf4_moe_kernel<<<grid, WAVE, 0, stream>>>(
-      packed_all.data_ptr<unsigned char>(),
-      reinterpret_cast<const unsigned short*>(absmax_all.data_ptr()),
-      x.data_ptr<float>(), sel.data_ptr<int>(), partials.data_ptr<float>(),
-      in_dim, out_dim, i_per_split, rows, (int)k_per_tok);
-  HIP_CHECK_LAST();
-  return launch_gemv_reduce(
-      partials, c10::nullopt, c10::nullopt, (int)splits, rows, out_dim, (int)epilogue,
-      x.options(), absmax_all.options());
 }

@@ -1,0 +1,492 @@
+// Products of few rows with NF4 weights on the matrix cores, in whole numbers.
+//
+// A 4-bit level times 7783094 is a whole number up to 2 units in 10^8 of the largest
+// level (no other factor below 127.4 * 2^16 fits all 16 levels as well), and a whole number
+// is three signed digits of base 256. So is an input times its block's scale, with four
+// digits, once the inputs of a run are scaled by one power of two so that their largest
+// reaches 2^30. Sums of products of digits are exact in 32 bits for runs of 512, and a
+// product of 16 columns with 64 inputs is one v_mfma_i32_16x16x64_i8 per digit of the
+// levels: the four digits of up to four rows are its other 16 columns.
+//
+// Digits come from v_perm_b32, which looks four codes up in eight bytes at once. Two
+// lookups make up the 16 levels: a code of the other half selects a sign or a constant (0
+// for 12, all ones above), which for given tables is known, and which the other table is
+// xored with below, so that the xor of both lookups is the digit. That costs the same for
+// one row as for four, and no LDS, where the kernel that it stands for gathers the two
+// levels of a byte from a table: there random indices collide, and every row more is
+// another operation a weight.
+//
+//   tiles   [out/64, ceil(in/128), 4, 64 lanes, 16 bytes]: 128 inputs x 64 columns, in the
+//           order of the operands: lane l of part c has column c*16 + l%16, and of each 64
+//           inputs the 16 from (l/16)*16 on: bytes 0-3 of a half have the first four in
+//           their low and the next four in their high nibbles, bytes 4-7 the rest
+//   scales  [out/64, ceil(in/128)*128] bf16, zero beyond `in`
+//
+// Four waves of a workgroup take 64 columns and 512 inputs each (256 at a time beyond four
+// rows, whose digits fill twice the columns), all of whose weights are on their way while
+// the inputs are cut into digits. Five to eight rows stay for up to 1024 inputs, as long
+// as that leaves 2048 waves: their sums are 96 registers to combine at the end.
+//
+// It is bound by vector instructions (half-rate lookups; the chip lowers its clock under
+// them), not by memory. llama-2-70b, us a product with its reduction, the kernel in
+// nf4.hip and this one, for 1, 4 and 8 rows:
+//   qkv   8192 x 10240   19, 29, 47     20, 22, 29
+//   o     8192 x 8192    22, 30, 49     17, 18, 23
+//   gate  8192 x 57344   64, 96, 160    64, 78, 112
+//   down  28672 x 8192   36, 51, 84     36, 41, 63
+// (Runs of 1024 for one row: 70 and 38 us for the last two; four waves a SIMD: 71, 39.)
+// Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.7e-7).
+
+#include "common.h"
+#include "gemv_reduce.h"
+#include <torch/extension.h>
+#include <ATen/cuda/CUDAContext.h>
+
+using i32x4 = __attribute__((ext_vector_type(4))) int;
+
+#define NF4_UNIT (1.0f / 7783094.0f)
+
+static __device__ __constant__ float NF4_TILE_LEVELS[16] = {
+    -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
+    -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
+    0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f,
+    0.33791524171829224f, 0.4407098293304443f, 0.5626170039176941f,
+    0.7229568362236023f, 1.0f};
+
+// digits of the levels, lowest first: bytes 0-3 and 4-7 of the tables of codes 0-7 and 8-15,
+// each xored with what the other one yields for a code that is not its own
+__device__ constexpr unsigned NF4_DIGITS[3][4] = {
+    {0x70a4dab5u, 0xff2a9c36u, 0x7584b78au, 0x4926eac6u},
+    {0x19a4ad3du, 0xffcff138u, 0xddc51d8cu, 0x3c232e57u},
+    {0x2e3d5289u, 0xff0a15deu, 0xd71d1309u, 0x88a9bc34u},
+};
+
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// largest value of a wave
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+#define STEP(ctrl, rows) v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false))
+  STEP(0xB1, 0xf);   // quads: neighbours
+  STEP(0x4E, 0xf);   // quads: pairs
+  STEP(0x141, 0xf);  // halves of a row mirrored
+  STEP(0x140, 0xf);  // rows of 16 mirrored
+  STEP(0x142, 0xa);  // row 0 to 1, 2 to 3
+  STEP(0x143, 0xc);  // rows 0 and 1 to 2 and 3
+#undef STEP
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ float quad_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
+}
+
+// the 4 x 4 bytes of w transposed
+__device__ __forceinline__ void transpose_bytes(unsigned* w) {
+  const unsigned a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), b = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+  const unsigned c = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u), d = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+  w[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+  w[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+  w[2] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+  w[3] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+}
+
+// B rows; a wave takes KB tiles of 128 inputs and 64 columns at a time, `steps` times if LONG.
+// Grid: (out/64, runs of 4 KB `steps` tiles, rows of sel). With sel, B is 1 and row
+// blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z].
+template <int B, int KB, bool LONG>
+__global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
+    const uint4* __restrict__ tiles, const unsigned short* __restrict__ scales,
+    const float* __restrict__ x,      // [rows, in]
+    const int* __restrict__ sel,      // [rows * k_per_tok] or null
+    float* __restrict__ partials,     // [splits, B or gridDim.z, out]
+    int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4) {
+  const int steps = LONG ? n_steps : 1;
+  constexpr int NS = (B + 3) / 4, NCOL = 4 * B, PER = KB * 2;
+  __shared__ __align__(16) unsigned char digits[4][KB * 128 * NCOL];
+  __shared__ __align__(16) float red[4 * B * 64];  // [waves, rows, columns]
+
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
+  const int col = lane & 15, hi = lane >> 4;
+  const int nb = blockIdx.x, kb0 = (blockIdx.y * 4 + wave) * KB * steps;
+  const int live_kb = min(KB * steps, n_kb - kb0);  // may be negative
+  if (sel) {
+    const int e = sel[blockIdx.z];
+    if (e < 0 || e >= experts) return;  // uniform over the workgroup
+    tiles += (size_t)e * (out_dim / 64) * n_kb * 256;
+    scales += (size_t)e * (out_dim / 64) * n_kb * 128;
+    x += (size_t)(blockIdx.z / k_per_tok) * in_dim;
+  }
+
+  // inputs of a step: PER of this lane
+  auto fetch_x = [&](int step, int b, float* v) {
+    const int k = (kb0 + step * KB) * 128 + lane * PER;
+    const float* p = x + (size_t)b * in_dim + k;
+    if (by4 && k + PER <= in_dim) {
+#pragma unroll
+      for (int i = 0; i < PER; i += 4) *reinterpret_cast<float4v*>(v + i) = *reinterpret_cast<const float4v*>(p + i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) v[i] = k + i < in_dim ? p[i] : 0.f;
+    }
+  };
+  auto fetch_scales = [&](int step, unsigned* v) {
+    const int at = step * KB * 128 + lane * PER;
+#pragma unroll
+    for (int i = 0; i < PER / 2; ++i) v[i] = 0u;
+    if (at < live_kb * 128) {
+      const unsigned* p = reinterpret_cast<const unsigned*>(scales + ((size_t)nb * n_kb + kb0) * 128 + at);
+#pragma unroll
+      for (int i = 0; i < PER / 2; ++i) v[i] = p[i];
+    }
+  };
+  const uint4* wp = tiles + ((size_t)nb * n_kb + kb0) * 256 + lane;
+  uint4 w[KB][4];
+  auto fetch_w = [&](int step, int j) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      w[j][c] = uint4{0u, 0u, 0u, 0u};
+      if (step * KB + j < live_kb) w[j][c] = wp[((step * KB + j) * 4 + c) * 64];
+    }
+  };
+
+  // the first step's inputs, then its weights, which are awaited last
+  float xs[B][PER];
+  unsigned sc[PER / 2];
+  fetch_scales(0, sc);
+#pragma unroll
+  for (int b = 0; b < B; ++b) fetch_x(0, b, xs[b]);
+#pragma unroll
+  for (int j = 0; j < KB; ++j) fetch_w(0, j);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // largest input of each row and largest scale of the run bound the scaled inputs
+  unsigned top[B], top_scale = 0;
+#pragma unroll
+  for (int i = 0; i < PER / 2; ++i) top_scale = max(top_scale, max(sc[i] & 0xFFFF0000u, sc[i] << 16));
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    top[b] = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) top[b] = max(top[b], __float_as_uint(xs[b][i]) & 0x7FFFFFFFu);
+  }
+  for (int step = 1; step < steps; ++step) {
+    unsigned s[PER / 2];
+    fetch_scales(step, s);
+#pragma unroll
+    for (int i = 0; i < PER / 2; ++i) top_scale = max(top_scale, max(s[i] & 0xFFFF0000u, s[i] << 16));
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      float v[PER];
+      fetch_x(step, b, v);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) top[b] = max(top[b], __float_as_uint(v[i]) & 0x7FFFFFFFu);
+    }
+  }
+  float unit[B], factor[B];  // the scaled inputs' last place, and one over it
+  bool odd = false;
+  top_scale = wave_max_u32(top_scale);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const unsigned m = __float_as_uint(__uint_as_float(wave_max_u32(top[b])) * __uint_as_float(top_scale)) & 0x7FFFFFFFu;
+    odd |= m >= 0x7F800000u;
+    // below 2^(e - 126), times 2^(156 - e)
+    const unsigned up = min(283u - (m >> 23), 253u);
+    factor[b] = __uint_as_float(up << 23);
+    unit[b] = __uint_as_float((254u - up) << 23);
+  }
+
+  i32x4 acc[NS][4][3];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) acc[s][c][p] = i32x4{0, 0, 0, 0};
+
+  for (int step = 0; step < steps && !odd; ++step) {
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+      for (int i = 0; i < PER; i += 4) {
+        unsigned q[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const unsigned s = (i + j) & 1 ? sc[(i + j) / 2] & 0xFFFF0000u : sc[(i + j) / 2] << 16;
+          q[j] = ((unsigned)(int)(xs[b][i + j] * __uint_as_float(s) * factor[b]) + 0x00808080u) ^ 0x00808080u;
+        }
+        transpose_bytes(q);
+        const int at = lane * PER + i;  // of the step: group of 16, then column, then place
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          *reinterpret_cast<unsigned*>(&digits[wave][((at / 16) * NCOL + b * 4 + d) * 16 + at % 16]) = q[d];
+      }
+    wave_fence();
+    const bool more = step + 1 < steps;
+    if (more) {
+      fetch_scales(step + 1, sc);
+#pragma unroll
+      for (int b = 0; b < B; ++b) fetch_x(step + 1, b, xs[b]);
+    }
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        i32x4 xd[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          // columns without a row are zero, which takes less power than repeating others
+          const int n = s * 16 + col, live = n < NCOL ? -1 : 0;
+          xd[s] = *reinterpret_cast<const i32x4*>(&digits[wave][((j * 8 + half * 4 + hi) * NCOL + n % NCOL) * 16]);
+          if (NCOL % 16) xd[s] &= live;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const unsigned w0 = half ? w[j][c].z : w[j][c].x, w1 = half ? w[j][c].w : w[j][c].y;
+          unsigned lo[4], up[4];  // codes 0-7 select below 8; the others do with bit 3 turned
+          lo[0] = w0 & 0x0F0F0F0Fu;
+          lo[1] = (w0 >> 4) & 0x0F0F0F0Fu;
+          lo[2] = w1 & 0x0F0F0F0Fu;
+          lo[3] = (w1 >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) up[i] = lo[i] ^ 0x08080808u;
+#pragma unroll
+          for (int p = 0; p < 3; ++p) {
+            i32x4 a;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              a[i] = (int)(__builtin_amdgcn_perm(NF4_DIGITS[p][1], NF4_DIGITS[p][0], lo[i]) ^
+                           __builtin_amdgcn_perm(NF4_DIGITS[p][3], NF4_DIGITS[p][2], up[i]));
+#pragma unroll
+            for (int s = 0; s < NS; ++s) acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xd[s], acc[s][c][p], 0, 0, 0);
+          }
+        }
+      }
+      if (more) fetch_w(step + 1, j);
+    }
+    wave_fence();
+  }
+
+  if (__builtin_expect(odd, 0)) {  // infinities and NaNs: in 32-bit floats, a column per lane
+    float sum[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) sum[b] = 0.f;
+    const unsigned char* bytes = reinterpret_cast<const unsigned char*>(tiles + ((size_t)nb * n_kb + kb0) * 256);
+    for (int i = 0; i < live_kb * 128 && kb0 * 128 + i < in_dim; ++i) {
+      const int at = i % 16, half = i % 128 / 64;
+      const int byte = (((i / 128) * 4 + lane / 16) * 64 + i % 64 / 16 * 16 + lane % 16) * 16 + half * 8 + at / 8 * 4 + at % 4;
+      const float level = NF4_TILE_LEVELS[at & 4 ? bytes[byte] >> 4 : bytes[byte] & 15];
+      const float s = bf16_to_f32(scales[(size_t)nb * n_kb * 128 + kb0 * 128 + i]);
+#pragma unroll
+      for (int b = 0; b < B; ++b) sum[b] = fmaf(level, x[(size_t)b * in_dim + kb0 * 128 + i] * s, sum[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) red[(wave * B + b) * 64 + lane] = sum[b];
+  } else {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int row = s * 4 + col / 4;  // this lane's row and, col % 4, digit of its inputs
+      float last = 0.f;
+#pragma unroll
+      for (int b = s * 4; b < B && b < s * 4 + 4; ++b) last = row == b ? unit[b] : last;
+      const float place = __uint_as_float((127u + 8u * (col & 3)) << 23) * NF4_UNIT;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float4v v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float sum = fmaf((float)acc[s][c][2][r], 65536.f, fmaf((float)acc[s][c][1][r], 256.f, (float)acc[s][c][0][r]));
+          v[r] = quad_sum(sum * place) * last;
+        }
+        if ((col & 3) == 0 && row < B) *reinterpret_cast<float4v*>(&red[(wave * B + row) * 64 + c * 16 + hi * 4]) = v;
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < B * 64; i += 256) {
+    const float sum = (red[i] + red[B * 64 + i]) + (red[2 * B * 64 + i] + red[3 * B * 64 + i]);
+    const size_t row = sel ? (size_t)blockIdx.y * gridDim.z + blockIdx.z : (size_t)blockIdx.y * B + i / 64;
+    partials[row * out_dim + nb * 64 + i % 64] = sum;
+  }
+}
+
+// ------------------------------------------------------------ packing
+
+// one thread per 16 bytes of a tile
+__global__ void nf4_tile_kernel(
+    const unsigned char* __restrict__ packed,   // [in, out/2]
+    const unsigned short* __restrict__ absmax,  // [in, out/64]
+    uint4* __restrict__ tiles, unsigned short* __restrict__ scales, int in_dim, int out_dim, int n_kb) {
+  const size_t at = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t n = (size_t)(out_dim / 64) * n_kb;
+  if (at < n * 256) {
+    const int lane = at % 64, c = at / 64 % 4, kb = at / 256 % n_kb;
+    const size_t nb = at / 256 / n_kb;
+    const size_t column = nb * 64 + c * 16 + lane % 16;
+    unsigned words[4] = {0u, 0u, 0u, 0u};
+    for (int i = 0; i < 32; ++i) {
+      const int k = kb * 128 + i / 16 * 64 + lane / 16 * 16 + i % 16;
+      unsigned code = 7u;  // 0
+      if (k < in_dim) {
+        const unsigned char byte = packed[((size_t)k * out_dim + column) / 2];
+        code = column & 1 ? byte >> 4 : byte & 15;
+      }
+      words[i / 8] |= code << ((i & 3) * 8 + (i & 4));
+    }
+    tiles[at] = uint4{words[0], words[1], words[2], words[3]};
+  }
+  if (at < n * 128) {
+    const int k = at % ((size_t)n_kb * 128);
+    const size_t nb = at / ((size_t)n_kb * 128);
+    scales[at] = k < in_dim ? absmax[(size_t)k * (out_dim / 64) + nb] : (unsigned short)0;
+  }
+}
+
+// A tile per workgroup: dense[k, n] = bf16(level * scale), 128 bytes of a row at a time
+__global__ __launch_bounds__(256) void nf4_untile_kernel(
+    const uint4* __restrict__ tiles, const unsigned short* __restrict__ scales, unsigned short* __restrict__ dense,
+    int in_dim, int out_dim, int n_kb) {
+  __shared__ float levels[16];
+  __shared__ unsigned short scale[128];
+  __shared__ unsigned short tile[128][64 + 2];
+  const int tid = threadIdx.x, lane = tid & 63, c = tid >> 6;
+  const int kb = blockIdx.x % n_kb, nb = blockIdx.x / n_kb;
+  if (tid < 16) levels[tid] = NF4_TILE_LEVELS[tid];
+  if (tid < 128) scale[tid] = scales[((size_t)nb * n_kb + kb) * 128 + tid];
+  const uint4 w = tiles[(size_t)blockIdx.x * 256 + tid];
+  const unsigned words[4] = {w.x, w.y, w.z, w.w};
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const int k = i / 16 * 64 + lane / 16 * 16 + i % 16;
+    const unsigned code = (words[i / 8] >> ((i & 3) * 8 + (i & 4))) & 15u;
+    tile[k][c * 16 + lane % 16] = f32_to_bf16(levels[code] * bf16_to_f32(scale[k]));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int k = i * 8 + tid / 32, n = tid % 32 * 2;
+    if (kb * 128 + k < in_dim)
+      *reinterpret_cast<unsigned*>(dense + (size_t)(kb * 128 + k) * out_dim + nb * 64 + n) =
+          *reinterpret_cast<const unsigned*>(&tile[k][n]);
+  }
+}
+
+// ------------------------------------------------------------------- host
+
+// packed [in, out/2], absmax [in, out/64] -> (tiles, scales); [E, ...] for stacked experts
+std::vector<torch::Tensor> nf4_tile(torch::Tensor packed, torch::Tensor absmax) {
+  TORCH_CHECK(packed.is_cuda() && packed.dtype() == torch::kUInt8 && packed.dim() == 2 && packed.is_contiguous());
+  TORCH_CHECK(absmax.is_cuda() && absmax.dtype() == torch::kBFloat16 && absmax.is_contiguous());
+  const long in_dim = packed.size(0), out_dim = packed.size(1) * 2;
+  TORCH_CHECK(in_dim > 0 && out_dim % 64 == 0 && absmax.dim() == 2 && absmax.size(0) == in_dim &&
+              absmax.size(1) == out_dim / 64);
+  const long n_kb = (in_dim + 127) / 128, nb = out_dim / 64;
+  auto tiles = torch::empty({nb, n_kb, 4, 64, 16}, packed.options());
+  auto scales = torch::empty({nb, n_kb * 128}, absmax.options());
+  const long threads = nb * n_kb * 256;
+  TORCH_CHECK(threads / 256 < (1L << 31));
+  nf4_tile_kernel<<<threads / 256, 256, 0, at::cuda::getCurrentCUDAStream()>>>(
+      packed.data_ptr<unsigned char>(), reinterpret_cast<const unsigned short*>(absmax.data_ptr()),
+      reinterpret_cast<uint4*>(tiles.data_ptr()), reinterpret_cast<unsigned short*>(scales.data_ptr()), (int)in_dim,
+      (int)out_dim, (int)n_kb);
+  HIP_CHECK_LAST();
+  return {tiles, scales};
+}
+
+static void check_tiles(const torch::Tensor& tiles, const torch::Tensor& scales, int64_t in_dim, int lead) {
+  TORCH_CHECK(tiles.is_cuda() && tiles.dtype() == torch::kUInt8 && tiles.dim() == 5 + lead && tiles.is_contiguous());
+  TORCH_CHECK(scales.is_cuda() && scales.dtype() == torch::kBFloat16 && scales.dim() == 2 + lead && scales.is_contiguous());
+  const long nb = tiles.size(lead), n_kb = tiles.size(lead + 1);
+  TORCH_CHECK(tiles.size(lead + 2) == 4 && tiles.size(lead + 3) == 64 && tiles.size(lead + 4) == 16);
+  TORCH_CHECK(scales.size(lead) == nb && scales.size(lead + 1) == n_kb * 128);
+  TORCH_CHECK(lead == 0 || scales.size(0) == tiles.size(0));
+  TORCH_CHECK(in_dim > 0 && (in_dim + 127) / 128 == n_kb, "tiles of other inputs");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(tiles.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(scales.data_ptr()) % 4 == 0);
+}
+
+torch::Tensor nf4_untile(torch::Tensor tiles, torch::Tensor scales, int64_t in_dim) {
+  check_tiles(tiles, scales, in_dim, 0);
+  const long nb = tiles.size(0), n_kb = tiles.size(1);
+  auto dense = torch::empty({in_dim, nb * 64}, scales.options());
+  nf4_untile_kernel<<<nb * n_kb, 256, 0, at::cuda::getCurrentCUDAStream()>>>(
+      reinterpret_cast<const uint4*>(tiles.data_ptr()), reinterpret_cast<const unsigned short*>(scales.data_ptr()),
+      reinterpret_cast<unsigned short*>(dense.data_ptr()), (int)in_dim, (int)(nb * 64), (int)n_kb);
+  HIP_CHECK_LAST();
+  return dense;
+}
+
+// sel: [rows] experts or null; returns [splits, rows, out]
+static torch::Tensor launch_nf4_tiles(
+    const torch::Tensor& tiles, const torch::Tensor& scales, int64_t in_dim, const torch::Tensor& x,
+    const torch::Tensor* sel, int64_t k_per_tok, torch::Tensor workspace) {
+  const int lead = sel ? 1 : 0;
+  const long nb = tiles.size(lead), n_kb = tiles.size(lead + 1), out_dim = nb * 64;
+  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.dim() == 2 && x.is_contiguous() && x.size(1) == in_dim);
+  const int batch = sel ? 1 : (int)x.size(0);
+  const long rows = sel ? sel->numel() : batch, z = sel ? rows : 1;
+  TORCH_CHECK(batch >= 1 && batch <= 8, "NF4 products of few rows take at most 8");
+  const int kb = batch <= 4 ? 4 : 2;
+  // longer runs combine their sums once, but only where enough waves remain
+  const long units = nb * z * ((n_kb + kb - 1) / kb);
+  long steps = 1;
+  while (batch > 4 && steps < 4 && units / (2 * steps) >= 2048) steps *= 2;
+  const long splits = (n_kb + 4 * kb * steps - 1) / (4 * kb * steps);
+  TORCH_CHECK(workspace.numel() == 0 || (workspace.is_cuda() && workspace.dtype() == torch::kFloat32));
+  torch::Tensor partials = workspace.numel() >= splits * rows * out_dim
+                               ? workspace.view(-1).narrow(0, 0, splits * rows * out_dim).view({splits, rows, out_dim})
+                               : torch::empty({splits, rows, out_dim}, x.options());
+  if (z == 0) return partials;
+  const bool by4 = in_dim % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+  const dim3 grid(nb, splits, z);
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define NF4_TILES(B, KB)                                                                                       \
+  gemv_nf4_tiles_kernel<B, KB, (B > 4)><<<grid, 256, 0, stream>>>(                                                      \
+      reinterpret_cast<const uint4*>(tiles.data_ptr()), reinterpret_cast<const unsigned short*>(scales.data_ptr()), \
+      x.data_ptr<float>(), sel ? sel->data_ptr<int>() : nullptr, partials.data_ptr<float>(), (int)in_dim,      \
+      (int)out_dim, (int)n_kb, (int)steps, (int)k_per_tok, sel ? (int)tiles.size(0) : 1, by4)
+  switch (batch) {
+    case 1: NF4_TILES(1, 4); break;
+    case 2: NF4_TILES(2, 4); break;
+    case 3: NF4_TILES(3, 4); break;
+    case 4: NF4_TILES(4, 4); break;
+    case 5: NF4_TILES(5, 2); break;
+    case 6: NF4_TILES(6, 2); break;
+    case 7: NF4_TILES(7, 2); break;
+    case 8: NF4_TILES(8, 2); break;
+  }
+#undef NF4_TILES
+  HIP_CHECK_LAST();
+  return partials;
+}
+
+torch::Tensor gemv_nf4_tiles(
+    torch::Tensor tiles, torch::Tensor scales, int64_t in_dim,
+    torch::Tensor x,  // [batch, in] f32
+    torch::Tensor workspace, c10::optional<torch::Tensor> residual, int64_t epilogue,
+    c10::optional<torch::Tensor> bias) {  // epilogue < 0: the partial sums [splits, batch, out]
+  check_tiles(tiles, scales, in_dim, 0);
+  auto partials = launch_nf4_tiles(tiles, scales, in_dim, x, nullptr, 1, workspace);
+  if (epilogue < 0) return partials;
+  return launch_gemv_reduce(partials, residual, bias, (int)partials.size(0), (int)partials.size(1),
+                            (int)partials.size(2), (int)epilogue, x.options(), scales.options());
+}
+
+torch::Tensor gemv_nf4_tiles_moe(
+    torch::Tensor tiles, torch::Tensor scales, int64_t in_dim,
+    torch::Tensor x,    // [B, in] f32
+    torch::Tensor sel,  // [R] int32, R = B * k_per_tok
+    int64_t k_per_tok, torch::Tensor workspace, int64_t epilogue) {
+  check_tiles(tiles, scales, in_dim, 1);
+  TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());
+  const long rows = sel.numel();
+  TORCH_CHECK(x.dim() == 2 && rows == x.size(0) * k_per_tok);
+  TORCH_CHECK(rows <= 16, "moe gemv supports batch*k <= 16");
+  auto partials = launch_nf4_tiles(tiles, scales, in_dim, x, &sel, k_per_tok, workspace);
+  return launch_gemv_reduce(partials, c10::nullopt, c10::nullopt, (int)partials.size(0), (int)rows,
+                            (int)partials.size(2), (int)epilogue, x.options(), scales.options());
+}

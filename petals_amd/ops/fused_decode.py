@@ -85,6 +85,11 @@ class DecodeContext:
 _split_autotune_cache: Dict[Tuple[str, int, int], int] = {}
 
 
+def _fold_norm_wanted() -> bool:
+    """Folded norms run on the NF4 kernel without matrix cores, which takes packed rows."""
+    return os.environ.get("PETALS_AMD_FOLD_NORM", "0") == "1"
+
+
 class _FastWeight:
     """A transposed [in, out] weight in bf16, NF4 or weight-only int8
     (quantize-on-load; int8 = per-out-column symmetric absmax, the MI355X
@@ -99,11 +104,16 @@ class _FastWeight:
         self.quant = quant
         self.in_dim, self.out_dim = t_bf16.shape
         self.t = self.packed = self.absmax = self.absmax_t = self.q8 = self.scale8 = None
+        self.tiles = self.scales = None
         if quant == "nf4":
-            self.packed, self.absmax = hip.nf4_quantize(t_bf16.contiguous())
-            # transposed absmax copy: one contiguous 32 B load per 16-row
-            # unroll block in the gemv instead of 16 strided 2 B gathers
-            self.absmax_t = self.absmax.t().contiguous()
+            packed, absmax = hip.nf4_quantize(t_bf16.contiguous())
+            if _fold_norm_wanted():
+                self.packed, self.absmax = packed, absmax
+                # transposed absmax copy: one contiguous 32 B load per 16-row
+                # unroll block in the gemv instead of 16 strided 2 B gathers
+                self.absmax_t = self.absmax.t().contiguous()
+            else:
+                self.tiles, self.scales = hip.nf4_tile(packed, absmax)
         elif quant == "int8":
             w = t_bf16.float()
             scale = w.abs().amax(dim=0).clamp_min(1e-8) / 127.0
@@ -111,7 +121,8 @@ class _FastWeight:
             self.scale8 = scale.to(torch.bfloat16).contiguous()
         else:
             self.t = t_bf16.contiguous()
-        self.splits = self._autotune(t_bf16.device)
+        # tiles are split by a rule of their own
+        self.splits = 0 if self.tiles is not None else self._autotune(t_bf16.device)
 
     def _autotune(self, device) -> int:
         key = (self.quant, self.in_dim, self.out_dim)
@@ -156,6 +167,8 @@ class _FastWeight:
 
     def _gemv_raw(self, x, ws, residual, epilogue, splits, bias=None, x_parts=None,
                   fold_eps=0.0, sumsq_out=None):
+        if self.tiles is not None and x_parts is None and sumsq_out is None:
+            return self.hip.gemv_nf4_tiles(self.tiles, self.scales, self.in_dim, x, ws, residual, epilogue, bias)
         if self.quant == "nf4":
             return self.hip.gemv_nf4(self.packed, self.absmax, x, ws, residual, epilogue, splits, bias,
                                      self.absmax_t, x_parts, fold_eps, sumsq_out)
@@ -174,6 +187,8 @@ class _FastWeight:
         PETALS_AMD_DEQUANT_CACHE_MB) so chunked prefills and back-to-back
         sessions stop paying the per-matmul dequant (~337 us/weight
         measured)."""
+        if self.tiles is not None:
+            return _dequant_cached(self, lambda: self.hip.nf4_untile(self.tiles, self.scales, self.in_dim))
         if self.quant == "nf4":
             return _dequant_cached(self, lambda: self.hip.nf4_dequantize(self.packed, self.absmax))
         if self.quant == "int8":
@@ -332,7 +347,7 @@ class LlamaFastPath(_TPFastPathMixin):
             and getattr(type(self), "supports_fold_norm", True)
             and cfg.hidden_size % 64 == 0
             and cfg.hidden_size // 64 <= 128  # XS gemv prefetches <= 128 partials
-            and os.environ.get("PETALS_AMD_FOLD_NORM", "0") == "1"
+            and _fold_norm_wanted()
         )
         self.ln1_w = block.input_layernorm.weight.detach().to(torch.bfloat16).contiguous()
         self.ln2_w = block.post_attention_layernorm.weight.detach().to(torch.bfloat16).contiguous()

@@ -74,13 +74,8 @@ class _StackedExperts:
         self.quant = quant
         self.in_dim, self.out_dim = t_list[0].shape
         if quant == "nf4":
-            packed, absmax = [], []
-            for t in t_list:
-                p, a = hip.nf4_quantize(t.contiguous())
-                packed.append(p)
-                absmax.append(a)
-            self.packed_all = torch.stack(packed).contiguous()
-            self.absmax_all = torch.stack(absmax).contiguous()
+            tiles, scales = zip(*(hip.nf4_tile(*hip.nf4_quantize(t.contiguous())) for t in t_list))
+            self.tiles_all, self.scales_all = torch.stack(tiles), torch.stack(scales)
         else:
             assert quant == "none"
             self.wt_all = torch.stack([t.contiguous() for t in t_list]).contiguous()
@@ -91,14 +86,16 @@ class _StackedExperts:
     def moe_gemv(self, x: torch.Tensor, sel: torch.Tensor, k_per_tok: int, ws: torch.Tensor,
                  epilogue: int) -> torch.Tensor:
         if self.quant == "nf4":
-            return self.hip.gemv_nf4_moe(self.packed_all, self.absmax_all, x, sel, k_per_tok, ws, epilogue)
+            return self.hip.gemv_nf4_tiles_moe(
+                self.tiles_all, self.scales_all, self.in_dim, x, sel, k_per_tok, ws, epilogue
+            )
         return self.hip.gemv_bf16_moe(self.wt_all, x, sel, k_per_tok, ws, epilogue)
 
     def moe_gemm(self, x: torch.Tensor, sorted_pairs: torch.Tensor, tile_expert: torch.Tensor,
                  k_per_tok: int, n_rows: int) -> torch.Tensor:
         """Grouped MFMA GEMM (prefill): C[pair] = x[pair // k] @ W[expert(pair)]."""
         if self.quant == "nf4":
-            return self.hip.moe_gemm(None, self.packed_all, self.absmax_all, x,
+            return self.hip.moe_gemm(None, self.tiles_all, self.scales_all, x,
                                      sorted_pairs, tile_expert, k_per_tok, n_rows)
         return self.hip.moe_gemm(self.wt_all, None, None, x, sorted_pairs, tile_expert,
                                  k_per_tok, n_rows)
@@ -113,7 +110,7 @@ class _StackedExperts:
         if self.quant == "nf4":
             return _dequant_cached(
                 self._cache_keys[e],
-                lambda: self.hip.nf4_dequantize(self.packed_all[e], self.absmax_all[e]),
+                lambda: self.hip.nf4_untile(self.tiles_all[e], self.scales_all[e], self.in_dim),
             )
         return self.wt_all[e]
 
