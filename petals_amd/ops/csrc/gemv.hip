@@ -1,9 +1,10 @@
 // Decode-path GEMV suite for CDNA4 (gfx950).
 //
-// Weights are stored TRANSPOSED: Wt[in, out] bf16 row-major (= W^T). A wave
-// owns a strip of 512 output columns (8 per lane, one short8 = 16 B/lane per
-// input row) and iterates over a chunk of the input dimension; x[i] is a
-// wave-uniform scalar load (s_load, L2-resident) broadcast into 8 FMAs.
+// Weights are stored TRANSPOSED: Wt[in, out] bf16 row-major (= W^T). Matrices whose rows
+// are aligned to 16 bytes take the kernel in gemv_mfma.h. The one here takes any other: a
+// wave owns a strip of 512 output columns (8 per lane) and iterates over a chunk of the
+// input dimension; x[i] is a wave-uniform scalar load (s_load, L2-resident) broadcast into
+// 8 FMAs.
 // The input dimension is split across gridDim.y workgroups so 256 CUs stay
 // busy even for a single-token GEMV; each split writes a partial fp32 strip,
 // and gemv_reduce sums splits deterministically while fusing the epilogue
@@ -13,6 +14,7 @@
 // torch/CUDA inside HF blocks (reference models/llama/block.py:44-127).
 
 #include "common.h"
+#include "gemv_mfma.h"
 #include "gemv_reduce.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
@@ -130,21 +132,10 @@ static int pick_splits(int in_dim, int out_dim) {
   return (int)splits;
 }
 
-torch::Tensor gemv_bf16(
-    torch::Tensor wt,        // [in, out] bf16
-    torch::Tensor x,         // [batch, in] f32
-    torch::Tensor workspace, // [n_splits_max, batch, out] f32 (preallocated, may be empty)
-    c10::optional<torch::Tensor> residual,  // [batch, out] bf16
-    int64_t epilogue,
-    int64_t splits_override,
-    c10::optional<torch::Tensor> bias) {  // [out] bf16, added pre-activation
-  TORCH_CHECK(wt.is_cuda() && wt.dtype() == torch::kBFloat16 && wt.dim() == 2);
-  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.dim() == 2);
-  const int in_dim = wt.size(0), out_dim = wt.size(1);
-  TORCH_CHECK(x.size(1) == in_dim, "x/in mismatch");
-  const int batch = x.size(0);
-  TORCH_CHECK(batch <= 8, "decode gemv supports batch <= 8");
-
+// any alignment; returns [splits, batch, out]
+static torch::Tensor launch_gemv_rows(
+    const torch::Tensor& wt, const torch::Tensor& x, torch::Tensor workspace, int64_t splits_override) {
+  const int in_dim = wt.size(0), out_dim = wt.size(1), batch = x.size(0);
   int splits = splits_override > 0 ? (int)splits_override : pick_splits(in_dim, out_dim);
   // UNROLL(16)-aligned chunks: unaligned splits push rows onto the slow
   // per-row tail path (same fix as the NF4 gemv)
@@ -153,7 +144,7 @@ torch::Tensor gemv_bf16(
 
   torch::Tensor partials;
   if (workspace.numel() >= (int64_t)splits * batch * out_dim) {
-    partials = workspace;
+    partials = workspace.view(-1).narrow(0, 0, (int64_t)splits * batch * out_dim).view({splits, batch, out_dim});
   } else {
     partials = torch::empty({(int64_t)splits, batch, out_dim}, x.options());
   }
@@ -182,13 +173,34 @@ torch::Tensor gemv_bf16(
   }
 #undef LAUNCH_GEMV
   HIP_CHECK_LAST();
+  return partials;
+}
+
+torch::Tensor gemv_bf16(
+    torch::Tensor wt,        // [in, out] bf16
+    torch::Tensor x,         // [batch, in] f32
+    torch::Tensor workspace, // [n_splits_max, batch, out] f32 (preallocated, may be empty)
+    c10::optional<torch::Tensor> residual,  // [batch, out] bf16
+    int64_t epilogue,
+    int64_t splits_override,
+    c10::optional<torch::Tensor> bias) {  // [out] bf16, added pre-activation
+  TORCH_CHECK(wt.is_cuda() && wt.dtype() == torch::kBFloat16 && wt.dim() == 2);
+  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.dim() == 2);
+  const int in_dim = wt.size(0), out_dim = wt.size(1);
+  TORCH_CHECK(x.size(1) == in_dim, "x/in mismatch");
+  const int batch = x.size(0);
+  TORCH_CHECK(batch <= 8, "decode gemv supports batch <= 8");
+
+  // the matrix cores wherever rows can be read 16 bytes at a time; they choose their splits
+  torch::Tensor partials = gemv_mfma_fits(wt, out_dim) ? launch_gemv_mfma(wt, x, nullptr, 1, workspace)
+                                                       : launch_gemv_rows(wt, x, workspace, splits_override);
+  const int splits = (int)partials.size(0);
 
   // epilogue (shared with the NF4 path)
   if (epilogue < 0) {
     // RAW mode: the caller fuses its own reduce+epilogue (e.g. the qkv
     // rope+cache-write reduce); the view's shape carries the split count
-    return partials.view(-1).narrow(0, 0, (int64_t)splits * batch * out_dim)
-        .view({(int64_t)splits, (int64_t)batch, (int64_t)out_dim});
+    return partials;
   }
   torch::Tensor y = launch_gemv_reduce(
       partials, residual, bias, splits, batch, out_dim, (int)epilogue, x.options(), wt.options());

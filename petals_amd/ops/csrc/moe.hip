@@ -14,9 +14,10 @@
 //         nf4_tiles.hip's
 // The per-row inner loop is the same x-broadcast split-K structure as the
 // dense kernels (each selected expert's weights are read exactly once per
-// token).
+// token); experts whose rows are aligned to 16 bytes take gemv_mfma.h's.
 
 #include "common.h"
+#include "gemv_mfma.h"
 #include "gemv_reduce.h"
 #include "paged.h"
 #include <torch/extension.h>
@@ -425,6 +426,12 @@ torch::Tensor gemv_bf16_moe(
   const int rows = sel.size(0);
   TORCH_CHECK(x.size(1) == in_dim && rows == x.size(0) * k_per_tok);
   TORCH_CHECK(rows <= 64, "moe gemv supports batch*k <= 64");
+  if (gemv_mfma_fits(wt_all, out_dim)) {
+    auto sums = launch_gemv_mfma(wt_all, x, &sel, k_per_tok, workspace);
+    return launch_gemv_reduce(
+        sums, c10::nullopt, c10::nullopt, (int)sums.size(0), rows, out_dim, (int)epilogue, x.options(), wt_all.options(),
+        c10::nullopt, ClampedGate{(float)limit, (float)alpha});
+  }
 
   const long out_waves = (out_dim + GEMV_OUT_PER_WAVE - 1) / GEMV_OUT_PER_WAVE;
   long splits = splits_override > 0 ? splits_override : (768 + out_waves * rows - 1) / (out_waves * rows);

@@ -43,6 +43,7 @@
 #include <ATen/cuda/CUDAContext.h>
 
 using i32x4 = __attribute__((ext_vector_type(4))) int;
+using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
 #define NF4_UNIT (1.0f / 7783094.0f)
 
@@ -144,13 +145,13 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
       for (int i = 0; i < PER / 2; ++i) v[i] = p[i];
     }
   };
-  const uint4* wp = tiles + ((size_t)nb * n_kb + kb0) * 256 + lane;
-  uint4 w[KB][4];
+  const u32x4* wp = reinterpret_cast<const u32x4*>(tiles) + ((size_t)nb * n_kb + kb0) * 256 + lane;
+  u32x4 w[KB][4];
   auto fetch_w = [&](int step, int j) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      w[j][c] = uint4{0u, 0u, 0u, 0u};
-      if (step * KB + j < live_kb) w[j][c] = wp[((step * KB + j) * 4 + c) * 64];
+      w[j][c] = u32x4{0u, 0u, 0u, 0u};
+      if (step * KB + j < live_kb) w[j][c] = __builtin_nontemporal_load(wp + ((step * KB + j) * 4 + c) * 64);
     }
   };
 

@@ -121,8 +121,9 @@ class _FastWeight:
             self.scale8 = scale.to(torch.bfloat16).contiguous()
         else:
             self.t = t_bf16.contiguous()
-        # tiles are split by a rule of their own
-        self.splits = 0 if self.tiles is not None else self._autotune(t_bf16.device)
+        # the matrix-core kernels split by rules of their own
+        by_rule = self.tiles is not None or (self.t is not None and self.out_dim % 8 == 0)
+        self.splits = 0 if by_rule else self._autotune(t_bf16.device)
 
     def _autotune(self, device) -> int:
         key = (self.quant, self.in_dim, self.out_dim)

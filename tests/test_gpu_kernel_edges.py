@@ -134,3 +134,53 @@ def test_nf4_tiles_of_experts(hip, experts, tokens, top, k_in, n_out):
         xd, w, scale = x[r // top].double(), made[e][1], made[e][2]
         bound = (xd.abs() @ scale) * 2.4e-8 + 2.0**-21 * (xd.abs() @ w.abs())
         assert bool(((y[r] - xd @ w).abs() <= bound + k_in * 2.0**-31 * xd.abs().max() * scale.amax()).all())
+
+
+def sum_bound(xd, w):
+    """Sums of exact products in 32 bits: three for each of 32 inputs, and a few at the end."""
+    return (3 * (xd.shape[-1] // 32 + 1) + 16) * 2.0**-24 * (xd.abs() @ w.abs())
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", [1, 2, 5, 8])
+@pytest.mark.parametrize(
+    "k_in,n_out",
+    [(1, 8), (7, 128), (32, 120), (33, 136), (127, 1000), (130, 129), (512, 8), (513, 264), (2048, 2560), (4544, 65024), (300, 12)],
+)
+def test_gemv_against_64_bits(hip, k_in, n_out, batch):
+    gen = torch.Generator(device="cuda").manual_seed(k_in * 8 + batch)
+    w = torch.randn(k_in, n_out, device="cuda", generator=gen).to(BF16)
+    x = torch.randn(batch, k_in, device="cuda", generator=gen)
+    x[:, :: max(1, k_in // 5)] *= 50.0
+    x[batch // 2] *= 1e-20
+    y = hip.gemv_bf16(w, x, torch.empty(0, device="cuda"), None, 0)
+    assert bool(((y.double() - x.double() @ w.double()).abs() <= sum_bound(x.double(), w.double())).all())
+    parts = hip.gemv_bf16(w, x, torch.empty(0, device="cuda"), None, -1)
+    assert bool(((parts.double().sum(0) - x.double() @ w.double()).abs() <= sum_bound(x.double(), w.double())).all())
+
+
+@requires_gpu
+def test_gemv_infinities(hip):
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randn(200, 136, device="cuda", generator=gen).to(BF16)
+    w[w.abs() < 0.05] = 0.0
+    x = torch.randn(3, 200, device="cuda", generator=gen)
+    x[0, 100], x[1, 5] = float("inf"), float("nan")
+    y = hip.gemv_bf16(w, x, torch.empty(0, device="cuda"), None, 0).cpu()
+    ref = torch.stack([(row[:, None] * w.float()).sum(0) for row in x]).cpu()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.isfinite(y[2]).all()
+    odd = torch.isinf(ref)
+    assert odd.any() and torch.equal(y[odd], ref[odd])
+
+
+@requires_gpu
+@pytest.mark.parametrize("tokens,top,k_in,n_out", [(1, 2, 96, 136), (8, 2, 2048, 4096), (16, 4, 40, 24), (2, 1, 64, 12)])
+def test_gemv_of_experts(hip, tokens, top, k_in, n_out):
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    w = torch.randn(5, k_in, n_out, device="cuda", generator=gen).to(BF16)
+    sel = torch.randint(0, 5, (tokens * top,), device="cuda", generator=gen, dtype=torch.int32)
+    x = torch.randn(tokens, k_in, device="cuda", generator=gen)
+    y = hip.gemv_bf16_moe(w, x, sel, top, torch.empty(0, device="cuda"), 0).double()
+    for r, e in enumerate(sel.tolist()):
+        xd, wd = x[r // top].double(), w[e].double()
+        assert bool(((y[r] - xd @ wd).abs() <= sum_bound(xd, wd)).all())
