@@ -32,6 +32,19 @@ torch::Tensor attn_prefill_fused(
     torch::Tensor q, torch::Tensor k, torch::Tensor v,
     int64_t kv_len, int64_t kv_offset, double scale, bool causal,
     c10::optional<torch::Tensor> alibi_slopes);
+torch::Tensor attn_prefill_rows(
+    torch::Tensor q, torch::Tensor k, torch::Tensor v, int64_t kv_len, int64_t kv_offset, double scale, bool causal,
+    c10::optional<torch::Tensor> alibi_slopes);
+void qkv_rows(
+    torch::Tensor qkv, c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> cos_t,
+    c10::optional<torch::Tensor> sin_t, c10::optional<torch::Tensor> k_cache, c10::optional<torch::Tensor> v_cache,
+    int64_t start, int64_t qh, int64_t kh, int64_t hd);
+std::vector<torch::Tensor> add_norm_rows(
+    torch::Tensor x, torch::Tensor y, c10::optional<torch::Tensor> y_bias, torch::Tensor w,
+    c10::optional<torch::Tensor> b, double eps);
+torch::Tensor add_rows(torch::Tensor x, torch::Tensor y, c10::optional<torch::Tensor> z, c10::optional<torch::Tensor> bias);
+torch::Tensor swiglu_rows(torch::Tensor gu);
+void bias_gelu_rows(torch::Tensor y, c10::optional<torch::Tensor> bias);
 std::vector<torch::Tensor> nf4_quantize(torch::Tensor w);
 torch::Tensor gemv_int8(
     torch::Tensor q, torch::Tensor scale, torch::Tensor x, torch::Tensor workspace,
@@ -103,6 +116,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("wt_all"), py::arg("x"), py::arg("sel"), py::arg("k_per_tok"),
         py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0);
+  m.def("attn_prefill_rows", &attn_prefill_rows, "prompt attention on strided heads; results as rows of tokens");
+  m.def("qkv_rows", &qkv_rows, "fused projection of a prompt -> rotated queries in place, keys and values to the cache");
+  m.def("add_norm_rows", &add_norm_rows, "(x + y + bias, its RMS or layer norm)",
+        py::arg("x"), py::arg("y"), py::arg("y_bias"), py::arg("w"), py::arg("b"), py::arg("eps"));
+  m.def("add_rows", &add_rows, "x + y (+ z) (+ bias)",
+        py::arg("x"), py::arg("y"), py::arg("z") = py::none(), py::arg("bias") = py::none());
+  m.def("swiglu_rows", &swiglu_rows, "[..., gate | up] -> silu(gate) * up");
+  m.def("bias_gelu_rows", &bias_gelu_rows, "gelu(y + bias), in place", py::arg("y"), py::arg("bias") = py::none());
   m.def("nf4_tile", &nf4_tile, "NF4 in the order of the matrix cores: (packed, absmax) -> (tiles, scales)");
   m.def("nf4_untile", &nf4_untile, "(tiles, scales) -> bf16 [in, out]");
   m.def("gemv_nf4_tiles", &gemv_nf4_tiles, "few rows times NF4 tiles, with epilogue",

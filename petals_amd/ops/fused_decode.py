@@ -11,9 +11,8 @@ layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
     (HBM-bound by design; see profiles/).
 
   prefill (q_len > 1): bf16 GEMMs via torch.matmul on the SAME transposed
-    weights (rocBLAS), HIP rms_norm / rope / swiglu kernels, fp32-softmax
-    attention (chunked by the backend; flash prefill kernel is the planned
-    upgrade).
+    weights (rocBLAS), one kernel for each gap between them
+    (ops/csrc/prefill_rows.hip) and flash attention (prefill_attn.hip).
 
 The original nn.Linear weights are FREED after repacking (a 70B span must not
 hold two copies).
@@ -272,6 +271,36 @@ def decode_step_auto(fast, hidden, k_cache, v_cache, prefix_length: int = -1, ct
     return torch.cat(outs, dim=0)
 
 
+def _rows_fit(width: int) -> bool:
+    """Rows that ops/csrc/prefill_rows.hip takes: 16 bytes at a time, kept in registers by a norm."""
+    return width % 8 == 0 and width <= 16384
+
+
+def _takes_rows(cache: torch.Tensor) -> bool:
+    return cache.stride(3) == 1 and cache.data_ptr() % 16 == 0 and all(cache.stride(i) % 8 == 0 for i in range(3))
+
+
+def prompt_attention(hip, qkv, kv_cache, prefix, qh, kh, hd, scale, bias=None, cos=None, sin=None, slopes=None):
+    """Causal attention of a prompt's fused projection [B, S, (qh + 2 kh) * hd], which is
+    overwritten; keys and values go to the cache, if there is one. -> [B, S, qh * hd]"""
+    B, S, _ = qkv.shape
+    heads = qkv.view(B, S, qh + 2 * kh, hd).transpose(1, 2)
+    k, v, length, offset = heads[:, qh : qh + kh], heads[:, qh + kh :], S, 0
+    if kv_cache is None:
+        hip.qkv_rows(qkv, bias, cos, sin, None, None, prefix, qh, kh, hd)
+    else:
+        k_cache, v_cache = (t[:B] for t in kv_cache)
+        length, offset = prefix + S, prefix
+        if _takes_rows(k_cache) and _takes_rows(v_cache) and k_cache.stride() == v_cache.stride():
+            hip.qkv_rows(qkv, bias, cos, sin, k_cache, v_cache, prefix, qh, kh, hd)
+        else:
+            hip.qkv_rows(qkv, bias, cos, sin, None, None, prefix, qh, kh, hd)
+            k_cache[:, :, prefix:length].copy_(k)
+            v_cache[:, :, prefix:length].copy_(v)
+        k, v = k_cache, v_cache
+    return hip.attn_prefill_rows(heads[:, :qh], k, v, length, offset, scale, True, slopes)
+
+
 class _TPFastPathMixin:
     """Tensor-parallel hooks shared by the per-family fast paths. The shard's
     row-parallel outputs (o/down/dense) skip the fused residual epilogue and
@@ -427,6 +456,8 @@ class LlamaFastPath(_TPFastPathMixin):
                 up = up + du
         if autograd:
             act = reference.swiglu(gate, up).to(xn2.dtype)
+        elif adapter is None and inter % 8 == 0 and gateup.dtype == torch.bfloat16:
+            act = self.hip.swiglu_rows(gateup)
         else:
             act = self.hip.swiglu(gate.contiguous(), up.contiguous())
         down = torch.matmul(act, self.wdown_t.dense())
@@ -627,40 +658,28 @@ class LlamaFastPath(_TPFastPathMixin):
         adapter=None,
     ) -> torch.Tensor:
         B, S, H = hidden.shape
-        hidden = hidden.to(torch.bfloat16)
-        end = prefix_length + S
-        self._ensure_rope(end)
+        hidden = hidden.to(torch.bfloat16).contiguous()
+        self._ensure_rope(prefix_length + S)
 
         xn = self.hip.rms_norm(hidden, self.ln1_w_post, self.eps)
         qkv = torch.matmul(xn, self.wqkv_t.dense())  # [B, S, qkv] bf16 (rocBLAS)
         if adapter is not None:
             xd = self.hip.rms_norm(hidden, self.ln1_w, self.eps) if self.fold_norm else xn
             qkv = qkv + self._qkv_adapter_delta(xd, adapter).to(qkv.dtype)
-        q = qkv[..., : self.qh * self.hd].view(B, S, self.qh, self.hd).transpose(1, 2)
-        k = qkv[..., self.qh * self.hd : (self.qh + self.kh) * self.hd].view(B, S, self.kh, self.hd).transpose(1, 2)
-        v = qkv[..., (self.qh + self.kh) * self.hd :].view(B, S, self.kh, self.hd).transpose(1, 2)
-        pos = torch.arange(prefix_length, end, device=self.device).unsqueeze(0).expand(B, S).contiguous()
-        q, k = self.hip.apply_rope(q.contiguous(), k.contiguous(), self.rope_cos, self.rope_sin, pos)
-        if kv_cache is not None:
-            k_cache, v_cache = kv_cache
-            k_cache[:B, :, prefix_length:end].copy_(k)
-            v_cache[:B, :, prefix_length:end].copy_(v)
-            attn = self.hip.attn_prefill_fused(
-                q.contiguous(), k_cache[:B].contiguous(), v_cache[:B].contiguous(),
-                end, prefix_length, self.scale, True,
-            )
-        else:
-            attn = self.hip.attn_prefill_fused(
-                q.contiguous(), k.contiguous(), v.contiguous(), S, 0, self.scale, True
-            )
-        attn = attn.transpose(1, 2).reshape(B, S, self.qh * self.hd).to(torch.bfloat16)
+        attn = prompt_attention(
+            self.hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale,
+            cos=self.rope_cos, sin=self.rope_sin,
+        )
         o = self._tp_reduce(torch.matmul(attn, self.wo_t.dense()))
         if adapter is not None:
             d = adapter.delta("o", attn)
             if d is not None:
                 o = o + d
-        h2 = hidden + o
-        xn2 = self.hip.rms_norm(h2, self.ln2_w_post, self.eps)
+        if _rows_fit(H) and o.dtype == torch.bfloat16:
+            h2, xn2 = self.hip.add_norm_rows(hidden, o.contiguous(), None, self.ln2_w_post, None, self.eps)
+        else:
+            h2 = hidden + o
+            xn2 = self.hip.rms_norm(h2, self.ln2_w_post, self.eps)
         xd2 = self.hip.rms_norm(h2, self.ln2_w, self.eps) if (self.fold_norm and adapter is not None) else None
         return h2 + self._tp_reduce(self._mlp_dense(xn2, adapter, autograd=False, x_delta=xd2)).to(h2.dtype)
 
@@ -849,6 +868,8 @@ class BloomFastPath(_TPFastPathMixin):
                 return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
             return self.hip.layer_norm(x, w, b, self.eps)
 
+        if not autograd and hidden.device.type == "cuda" and _rows_fit(H) and self.w_h4h.out_dim % 8 == 0:
+            return self._prompt(hidden.contiguous(), kv_cache, prefix_length, adapter)
         xn = ln(hidden, self.ln1_w, self.ln1_b)
         res1 = xn if self.post_ln_residual else hidden
         xn = self._tp_copy(xn)
@@ -897,6 +918,43 @@ class BloomFastPath(_TPFastPathMixin):
             if d4 is not None:
                 out = out + d4.to(out.dtype)
         return res2 + self._tp_reduce(out)
+
+    def _prompt(self, hidden, kv_cache, prefix_length, adapter):
+        """The same without gradients: one kernel for each gap between dense products."""
+        hip = self.hip
+        xn = hip.layer_norm(hidden, self.ln1_w, self.ln1_b, self.eps)
+        qkv = torch.matmul(xn, self.wqkv_t.dense())
+        if adapter is not None:
+            d = adapter.delta("qkv", xn)
+            if d is not None:
+                qkv = qkv + d.to(qkv.dtype)[..., self._qkv_perm]
+        attn = prompt_attention(
+            hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale, bias=self.qkv_bias, slopes=self.slopes
+        )
+        o = torch.matmul(attn, self.wo_t.dense())
+        if adapter is not None:
+            d = adapter.delta("dense", attn)
+            if d is not None:
+                o = o + d.to(o.dtype)
+        res1, o_bias = (xn if self.post_ln_residual else hidden), self.o_bias
+        if self.tp_world > 1:
+            o, o_bias = self._tp_reduce(o + o_bias), None
+        h2, xn2 = hip.add_norm_rows(res1, o, o_bias, self.ln2_w, self.ln2_b, self.eps)
+        res2 = xn2 if self.post_ln_residual else h2
+        inter = torch.matmul(xn2, self.w_h4h.dense())
+        if adapter is not None:
+            dh = adapter.delta("h4h", xn2)
+            if dh is not None:
+                inter = inter + dh.to(inter.dtype)
+        hip.bias_gelu_rows(inter, self.b_h4h)
+        out = torch.matmul(inter, self.w_4hh.dense())
+        if adapter is not None:
+            d4 = adapter.delta("4hh", inter)
+            if d4 is not None:
+                out = out + d4.to(out.dtype)
+        if self.tp_world > 1:
+            return res2 + self._tp_reduce(out + self.b_4hh)
+        return hip.add_rows(res2, out, None, self.b_4hh)
 
     def forward(self, hidden, kv_cache, prefix_length, adapter=None):
         assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
@@ -1088,6 +1146,9 @@ class FalconFastPath(_TPFastPathMixin):
                 return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
             return self.hip.layer_norm(x, w, b, self.eps)
 
+        rows_fit = _rows_fit(H) and self.w_h4h.out_dim % 8 == 0
+        if not autograd and hidden.device.type == "cuda" and self.tp_world == 1 and rows_fit:
+            return self._prompt(hidden.contiguous(), kv_cache, prefix_length, adapter)
         xn_attn = self._tp_copy(ln(hidden, self.ln_attn_w, self.ln_attn_b))
         xn_mlp = xn_attn if self.single_ln else self._tp_copy(ln(hidden, self.ln_mlp_w, self.ln_mlp_b))
         qkv = torch.matmul(xn_attn, self.wqkv_t.dense())
@@ -1132,6 +1193,36 @@ class FalconFastPath(_TPFastPathMixin):
             if d4 is not None:
                 mlp_out = mlp_out + d4.to(mlp_out.dtype)
         return hidden + self._tp_reduce(o + mlp_out)
+
+    def _prompt(self, hidden, kv_cache, prefix_length, adapter):
+        """The same without gradients: one kernel for each gap between dense products."""
+        hip = self.hip
+        xn_attn = hip.layer_norm(hidden, self.ln_attn_w, self.ln_attn_b, self.eps)
+        xn_mlp = xn_attn if self.single_ln else hip.layer_norm(hidden, self.ln_mlp_w, self.ln_mlp_b, self.eps)
+        qkv = torch.matmul(xn_attn, self.wqkv_t.dense())
+        if adapter is not None:
+            d = adapter.delta("qkv", xn_attn)
+            if d is not None:
+                qkv = qkv + d.to(qkv.dtype)[..., self._qkv_perm]
+        attn = prompt_attention(
+            hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale, cos=self.rope_cos, sin=self.rope_sin
+        )
+        o = torch.matmul(attn, self.wo_t.dense())
+        inter = torch.matmul(xn_mlp, self.w_h4h.dense())
+        if adapter is not None:
+            d = adapter.delta("dense", attn)
+            if d is not None:
+                o = o + d.to(o.dtype)
+            dh = adapter.delta("h4h", xn_mlp)
+            if dh is not None:
+                inter = inter + dh.to(inter.dtype)
+        hip.bias_gelu_rows(inter)
+        out = torch.matmul(inter, self.w_4hh.dense())
+        if adapter is not None:
+            d4 = adapter.delta("4hh", inter)
+            if d4 is not None:
+                out = out + d4.to(out.dtype)
+        return hip.add_rows(hidden, o, out)
 
     def forward(self, hidden, kv_cache, prefix_length, adapter=None):
         assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"

@@ -213,9 +213,8 @@ class MixtralFastPath(LlamaFastPath):
             sorted_pairs, tile_expert = sort_pairs_by_expert(selected, self.num_experts)
             xb = x.to(torch.bfloat16).contiguous()
             gateup = self.stacked_gu.moe_gemm(xb, sorted_pairs, tile_expert, K, T * K)
-            inter = gateup.shape[-1] // 2
-            act = self.hip.swiglu(gateup[:, :inter].contiguous(), gateup[:, inter:].contiguous())
-            down = self.stacked_down.moe_gemm(act.contiguous(), sorted_pairs, tile_expert, 1, T * K)
+            act = self.hip.swiglu_rows(gateup)
+            down = self.stacked_down.moe_gemm(act, sorted_pairs, tile_expert, 1, T * K)
             out = (down.view(T, K, -1).float() * weights.unsqueeze(-1)).sum(dim=1)
             return out.reshape(*shape[:-1], -1).to(xn2.dtype)
         out_dim = self.stacked_down.out_dim if self.stacked_down is not None else self.wdown_e[0].shape[1]

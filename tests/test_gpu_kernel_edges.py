@@ -184,3 +184,115 @@ def test_gemv_of_experts(hip, tokens, top, k_in, n_out):
     for r, e in enumerate(sel.tolist()):
         xd, wd = x[r // top].double(), w[e].double()
         assert bool(((y[r] - xd @ wd).abs() <= sum_bound(xd, wd)).all())
+
+
+def attention_64(q, k, v, offset, scale, causal, slopes):
+    """(result, weights @ |v|) of [B, H, S, hd] over [B, G, L, hd], 64 bits"""
+    group = q.shape[1] // k.shape[1]
+    q, k, v = q.double(), k.double().repeat_interleave(group, 1), v.double().repeat_interleave(group, 1)
+    at = torch.arange(k.shape[2], device="cuda")
+    score = torch.matmul(q, k.transpose(2, 3).contiguous()) * scale
+    if slopes is not None:
+        score = score + slopes.double()[:, None, None] * at
+    if causal:
+        score = score.masked_fill(at > torch.arange(offset, offset + q.shape[2], device="cuda")[:, None], float("-inf"))
+    p = torch.softmax(score, dim=-1)
+    return torch.matmul(p, v), torch.matmul(p, v.abs())
+
+
+@requires_gpu
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize(
+    "b,qh,kh,s,offset,causal,alibi",
+    [
+        (1, 1, 1, 1, 0, True, False), (1, 2, 1, 15, 0, True, True), (2, 4, 2, 64, 0, True, False),
+        (1, 8, 8, 65, 7, True, True), (3, 6, 1, 130, 63, True, False), (1, 4, 4, 17, 200, True, False),
+        (2, 3, 3, 33, 31, False, True), (4, 128, 8, 129, 0, True, False), (2, 71, 1, 300, 100, True, False),
+        (8, 64, 64, 127, 1, False, True),
+    ],
+)  # fmt: skip
+def test_prompt_attention_edges(hip, hd, b, qh, kh, s, offset, causal, alibi):
+    gen = torch.Generator(device="cuda").manual_seed(qh * s + hd)
+
+    def made(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).to(BF16)
+
+    length = offset + s
+    k, v = (made(b + 1, kh, length + 5, hd) for _ in range(2))
+    slopes = torch.rand(qh, device="cuda", generator=gen) * 0.1 if alibi else None
+    rows = made(b, s, qh + 2, hd)  # queries among other columns
+    q = rows.transpose(1, 2)[:, 1 : 1 + qh]
+    ref, bound = attention_64(q, k[:b, :, :length], v[:b, :, :length], offset, hd**-0.5, causal, slopes)
+    bound = 2.0**-7 * bound + 1e-5  # weights and results are rounded to bf16, by up to 2^-8 each
+    out = hip.attn_prefill_rows(q, k[:b], v[:b], length, offset, hd**-0.5, causal, slopes)
+    assert out.shape == (b, s, qh * hd)
+    assert bool(((out.view(b, s, qh, hd).transpose(1, 2).double() - ref).abs() <= bound).all())
+    fused = hip.attn_prefill_fused(
+        q.contiguous(), k[:b].contiguous(), v[:b].contiguous(), length, offset, hd**-0.5, causal, slopes
+    )
+    assert torch.equal(fused.transpose(1, 2).reshape(b, s, qh * hd), out)
+
+
+@requires_gpu
+@pytest.mark.parametrize("hd,qh,kh,s,start", [(64, 3, 1, 1, 0), (128, 4, 2, 33, 5), (64, 2, 2, 70, 130)])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("turns", [False, True])
+@pytest.mark.parametrize("cached", [False, True])
+def test_qkv_rows(hip, hd, qh, kh, s, start, bias, turns, cached):
+    from petals_amd.ops import reference
+
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    b, width = 2, (qh + 2 * kh) * hd
+    qkv = torch.randn(b, s, width, device="cuda", generator=gen).to(BF16)
+    c = torch.randn(width, device="cuda", generator=gen).to(BF16) if bias else None
+    cos, sin = (t.cuda() for t in reference.build_rope_cache(hd, start + s))
+    ref = (qkv.float() + (0.0 if c is None else c.float())).view(b, s, -1, hd).transpose(1, 2)
+    if turns:
+        pos = torch.arange(start, start + s, device="cuda")
+        q, k = reference.apply_rope(ref[:, :qh], ref[:, qh : qh + kh], cos, sin, pos)
+        ref = torch.cat([q, k, ref[:, qh + kh :]], dim=1)
+    ref = ref.to(BF16)
+    caches = [torch.zeros(b + 1, kh, start + s + 3, hd, device="cuda", dtype=BF16) for _ in range(2)]
+    args = caches if cached else (None, None)
+    hip.qkv_rows(qkv, c, *((cos, sin) if turns else (None, None)), *args, start, qh, kh, hd)
+    got = qkv.view(b, s, -1, hd).transpose(1, 2)
+
+    def same(a, r):  # products and sums may be contracted: one unit in the last place
+        assert bool(((a.float() - r.float()).abs() <= 2.0**-7 * r.float().abs() + 1e-6).all())
+
+    same(got[:, :qh], ref[:, :qh])
+    if cached:
+        for t, lo in zip(caches, (qh, qh + kh)):
+            same(t[:b, :, start : start + s], ref[:, lo : lo + kh])
+            assert not t[b].any() and not t[:, :, :start].any() and not t[:, :, start + s :].any()
+    else:
+        same(got, ref)
+
+
+@requires_gpu
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 2048), (5, 2056), (130, 4544), (2, 16384)])
+def test_rows_between_products(hip, rows, width):
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    x, y, z = (torch.randn(rows, width, device="cuda", generator=gen).to(BF16) for _ in range(3))
+    c, w, b = (torch.randn(width, device="cuda", generator=gen).to(BF16) for _ in range(3))
+    fn = torch.nn.functional
+
+    def close(a, r):
+        assert bool(((a.double() - r).abs() <= 2.0**-8 * r.abs() + 1e-4).all())
+
+    close(hip.add_rows(x, y), x.double() + y.double())
+    close(hip.add_rows(x, y, z, c), x.double() + y.double() + z.double() + c.double())
+    for bias, layer in ((None, False), (c, False), (c, True)):
+        h, n = hip.add_norm_rows(x, y, bias, w, b if layer else None, 1e-5)
+        close(h, x.double() + y.double() + (0.0 if bias is None else c.double()))
+        hd = h.double()
+        if layer:
+            close(n, fn.layer_norm(hd, (width,), w.double(), b.double(), 1e-5))
+        else:
+            close(n, hd * torch.rsqrt(hd.square().mean(-1, keepdim=True) + 1e-5) * w.double())
+    both = torch.cat([x, y], dim=-1)
+    close(hip.swiglu_rows(both), fn.silu(x.double()) * y.double())
+    for bias in (None, c):
+        t = x.clone()
+        hip.bias_gelu_rows(t, bias)
+        close(t, fn.gelu(x.double() + (0.0 if bias is None else c.double()), approximate="tanh"))
