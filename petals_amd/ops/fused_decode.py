@@ -309,6 +309,10 @@ class _TPFastPathMixin:
     tp_world = 1
     tp_group = None
 
+    def widest_row(self) -> int:
+        """Most values that a prompt's token has between two dense products."""
+        return self._max_gemv_out()
+
     def _tp_copy(self, x: torch.Tensor) -> torch.Tensor:
         """Column-parallel input boundary (identity fwd, grad all-reduce bwd)."""
         if self.tp_world <= 1:

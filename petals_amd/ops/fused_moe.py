@@ -154,6 +154,9 @@ class MixtralFastPath(LlamaFastPath):
         gu_out = self.stacked_gu.out_dim if self.stacked_gu is not None else self.wgateup_e[0].shape[1]
         return max(gu_out, self.wqkv_t.shape[1], self.wo_t.shape[1])
 
+    def widest_row(self) -> int:
+        return self.top_k * self._max_gemv_out()  # a row per chosen expert
+
     def _route(self, xn2: torch.Tensor):
         """Router on [tokens, H] f32/bf16 -> (weights [t, k], experts [t, k]).
         All-device: safe inside hipGraph capture."""

@@ -91,13 +91,19 @@ class TransformerBackend:
             return (out,)
 
     def _estimate_max_chunk_length(self, hidden_states: torch.Tensor, prefix_length: int) -> int:
-        """Bound prefill chunks so attention score matrices fit reserved memory
-        (parity: backend.py:146-152)."""
+        """Bound prefill chunks so that what a block holds beside its inputs fits reserved
+        memory (parity: backend.py:146-152): attention score matrices, or for blocks whose
+        attention keeps none (their fast path) the widest rows between dense products."""
         batch_size, seq_length, _ = hidden_states.shape
         worst_case_length = prefix_length + seq_length
         n_heads = getattr(self.config, "num_attention_heads", 32)
         attn_bytes_per_token = n_heads * batch_size * 4 * worst_case_length  # fp32 scores
-        return max(1, self.max_chunk_size_bytes // attn_bytes_per_token)
+        longest = self.max_chunk_size_bytes // attn_bytes_per_token
+        fast = getattr(self.block, "_fast", None)
+        if fast is not None and hidden_states.is_cuda:
+            row_bytes = 2 * fast.widest_row()
+            longest = max(longest, self.max_chunk_size_bytes // (batch_size * row_bytes))
+        return max(1, longest)
 
     # ----------------------------------------------------------- training
 

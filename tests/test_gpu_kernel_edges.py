@@ -296,3 +296,29 @@ def test_rows_between_products(hip, rows, width):
         t = x.clone()
         hip.bias_gelu_rows(t, bias)
         close(t, fn.gelu(x.double() + (0.0 if bias is None else c.double()), approximate="tanh"))
+
+
+@requires_gpu
+@pytest.mark.parametrize("tokens,limit", [(37, 1 << 28), (300, 1 << 18), (300, 1)])
+def test_prompt_chunks_are_one_prompt(hip, tokens, limit):
+    """However a prompt is cut, its outputs and its cache are the same."""
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.server.backend import TransformerBackend
+    from petals_amd.server.from_pretrained import load_pretrained_block
+
+    config = load_model_config("test-llama-hd128")
+    block = load_pretrained_block("test-llama-hd128", config, 0, torch_dtype=BF16, device=torch.device("cuda"))
+    backend = TransformerBackend("b", block, config=config, memory_cache=None, dtype=BF16, max_chunk_size_bytes=limit)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(2, tokens, config.hidden_size, device="cuda", generator=gen).to(BF16)
+    n = backend._estimate_max_chunk_length(x, 0)
+    widest = 2 * config.intermediate_size
+    assert n == max(1, limit // (config.num_attention_heads * 2 * 4 * tokens), limit // (2 * 2 * widest))
+    caches = [[torch.zeros(2, 2, tokens, 128, device="cuda", dtype=BF16) for _ in "kv"] for _ in "ab"]
+    with torch.inference_mode():
+        whole = block(x, kv_cache=caches[0], prefix_length=0)
+        parts = [block(x[:, i : i + n], kv_cache=caches[1], prefix_length=i) for i in range(0, tokens, n)]
+    tol = dict(atol=0.03, rtol=0.03)  # dense products of other row counts are summed in other orders
+    assert torch.allclose(torch.cat(parts, 1).float(), whole.float(), **tol)
+    for a, b in zip(*caches):
+        assert torch.allclose(a.float(), b.float(), **tol)
