@@ -69,6 +69,9 @@ torch::Tensor gemv_nf4_tiles(
 torch::Tensor gemv_nf4_tiles_moe(
     torch::Tensor tiles, torch::Tensor scales, int64_t in_dim, torch::Tensor x, torch::Tensor sel,
     int64_t k_per_tok, torch::Tensor workspace, int64_t epilogue);
+std::vector<torch::Tensor> moe_route(torch::Tensor x, torch::Tensor w, int64_t top);
+torch::Tensor moe_combine(torch::Tensor rows, torch::Tensor weights, torch::Tensor residual);
+std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t mt);
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> nf4_all,
     c10::optional<torch::Tensor> scales_all, torch::Tensor x, torch::Tensor sorted_pairs,
@@ -133,6 +136,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "device-routed MoE gemv: stacked NF4 tiles, expert ids from a device tensor",
         py::arg("tiles"), py::arg("scales"), py::arg("in_dim"), py::arg("x"), py::arg("sel"),
         py::arg("k_per_tok"), py::arg("workspace"), py::arg("epilogue"));
+  m.def("moe_route", &moe_route, "router, softmax, top-k, renormalized: (weights, experts)");
+  m.def("moe_combine", &moe_combine, "residual + weighted sum of a token's expert rows");
+  m.def("moe_group", &moe_group, "expert-sorted, tile-padded pairs");
   m.def("moe_gemm", &moe_gemm,
         "grouped MFMA GEMM over expert-sorted (token, slot) pairs (prefill; NF4 dequant fused "
         "into the LDS B-tile staging)",

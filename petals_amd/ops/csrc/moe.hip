@@ -114,6 +114,149 @@ __global__ __launch_bounds__(WAVE) void gemv_bf16_moe_kernel(
   }
 }
 
+// ------------------------------------------------------------- routing
+//
+// A token's router, softmax, choice and renormalization in one launch, its experts' sum
+// and the residual in another: as torch operations they were 12 and 5 launches of 4 to 20
+// us each (the selection alone 19), half of a decoding step of two Mixtral 8x7B blocks.
+
+#define ROUTE_EXPERTS 256  // at most
+#define ROUTE_TOP 16
+
+// One token per workgroup: 4 waves take every fourth expert.
+template <typename T>
+__global__ __launch_bounds__(256) void moe_route_kernel(
+    const T* __restrict__ x,                // [tokens, dim]
+    const unsigned short* __restrict__ w,   // [experts, dim] bf16
+    float* __restrict__ weights, int* __restrict__ sel, int dim, int experts, int top) {
+  __shared__ float logits[ROUTE_EXPERTS];
+  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
+  const T* row = x + (size_t)blockIdx.x * dim;
+  for (int e = wave; e < experts; e += 4) {
+    float sum = 0.f;
+    for (int c = lane * 8; c < dim; c += WAVE * 8) {
+      float a[8], b[8];
+      load8(row + c, a);
+      load8(w + (size_t)e * dim + c, b);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum = fmaf(a[i], b[i], sum);
+    }
+    sum = wave_reduce_sum(sum);
+    if (lane == 0) logits[e] = sum;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  float v[ROUTE_EXPERTS / WAVE];  // of this lane's experts; chosen ones drop out
+#pragma unroll
+  for (int i = 0; i < ROUTE_EXPERTS / WAVE; ++i) v[i] = lane + i * WAVE < experts ? logits[lane + i * WAVE] : NEG_SENTINEL;
+  float first = 0.f, total = 0.f, mine = 0.f;
+  int chosen = 0;
+  for (int j = 0; j < top; ++j) {
+    float best = v[0];
+    int at = lane;
+#pragma unroll
+    for (int i = 1; i < ROUTE_EXPERTS / WAVE; ++i)
+      if (v[i] > best) best = v[i], at = lane + i * WAVE;
+    if (at >= experts) at = 0;  // nothing left here
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const float other = __shfl_xor(best, off, WAVE);
+      const int where = __shfl_xor(at, off, WAVE);
+      if (other > best || (other == best && where < at)) best = other, at = where;
+    }
+#pragma unroll
+    for (int i = 0; i < ROUTE_EXPERTS / WAVE; ++i)
+      if (at == lane + i * WAVE) v[i] = NEG_SENTINEL;
+    if (j == 0) first = best;
+    const float p = __expf(best - first);  // of the softmax over all, up to the factor that cancels
+    total += p;
+    if (lane == j) mine = p, chosen = at;
+  }
+  if (lane < top) {
+    weights[(size_t)blockIdx.x * top + lane] = mine / total;
+    sel[(size_t)blockIdx.x * top + lane] = chosen;
+  }
+}
+
+// y[b] = residual[b] + sum_j weights[b, j] * (sum over splits of partials[:, b * top + j]);
+// 64 outputs by 16 groups of (split, slot) per workgroup
+__global__ __launch_bounds__(1024) void moe_reduce_kernel(
+    const float* __restrict__ partials,  // [splits, tokens * top, out]
+    const float* __restrict__ weights, const unsigned short* __restrict__ residual, unsigned short* __restrict__ y,
+    int splits, int tokens, int top, int out_dim) {
+  __shared__ float part[16][64];
+  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int o = blockIdx.x * 64 + c, b = blockIdx.y;
+  float sum = 0.f;
+  if (o < out_dim)
+    for (int i = g; i < splits * top; i += 16) {
+      const int s = i / top, j = i - s * top;
+      sum = fmaf(weights[b * top + j], partials[((size_t)s * tokens * top + b * top + j) * out_dim + o], sum);
+    }
+  part[g][c] = sum;
+  __syncthreads();
+  if (g != 0 || o >= out_dim) return;
+  sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sum += part[i][c];
+  y[(size_t)b * out_dim + o] = f32_to_bf16(bf16_to_f32(residual[(size_t)b * out_dim + o]) + sum);
+}
+
+// the same for rows [tokens * top, out] in bf16, 8 values per thread
+__global__ __launch_bounds__(256) void moe_combine_kernel(
+    const unsigned short* __restrict__ rows, const float* __restrict__ weights, const unsigned short* __restrict__ residual,
+    unsigned short* __restrict__ y, int top, int out_dim, long groups) {
+  const long g = (long)blockIdx.x * 256 + threadIdx.x;
+  if (g >= groups) return;
+  const long t = g * 8 / out_dim, c = g * 8 - t * out_dim;
+  float sum[8], v[8];
+  load8(residual + g * 8, sum);
+  for (int j = 0; j < top; ++j) {
+    load8(rows + (t * top + j) * out_dim + c, v);
+    const float w = weights[t * top + j];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum[i] = fmaf(w, v[i], sum[i]);
+  }
+  store8(y + g * 8, sum);
+}
+
+// One workgroup. counts -> padded offsets -> scatter; every sorted slot and
+// every tile is written. The order of an expert's pairs is not fixed, which no
+// result depends on (each pair is a row of its own).
+__global__ __launch_bounds__(1024) void moe_group_kernel(
+    const int* __restrict__ sel, int pairs, int experts, int mt, int slots,
+    int* __restrict__ sorted_pairs, int* __restrict__ tile_expert) {
+  extern __shared__ int cnt[];  // [experts] counts, then next free slot
+  int* end = cnt + experts;     // [experts] end of the padded segment
+  const int tid = threadIdx.x;
+  for (int e = tid; e < experts; e += blockDim.x) cnt[e] = 0;
+  for (int i = tid; i < slots; i += blockDim.x) sorted_pairs[i] = -1;
+  for (int i = tid; i < slots / mt; i += blockDim.x) tile_expert[i] = -1;
+  __syncthreads();
+  for (int i = tid; i < pairs; i += blockDim.x) {
+    const int e = sel[i];
+    if (e >= 0 && e < experts) atomicAdd(&cnt[e], 1);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int at = 0;
+    for (int e = 0; e < experts; ++e) {
+      const int padded = (cnt[e] + mt - 1) / mt * mt;
+      cnt[e] = at;
+      at += padded;
+      end[e] = at;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < experts; e += blockDim.x)
+    for (int i = cnt[e]; i < end[e]; i += mt) tile_expert[i / mt] = e;
+  __syncthreads();
+  for (int i = tid; i < pairs; i += blockDim.x) {
+    const int e = sel[i];
+    if (e >= 0 && e < experts) sorted_pairs[atomicAdd(&cnt[e], 1)] = i;
+  }
+}
+
 // ------------------------------------------------- grouped GEMM (prefill)
 //
 // Grouped GEMM over expert-sorted (token, slot) pairs: the caller sorts the R = T*k
@@ -342,6 +485,71 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
 
 // ------------------------------------------------------------------- host
 
+// x [T, dim] f32 or bf16, w [experts, dim] bf16 -> (weights [T, top] f32, experts [T, top] int32): the
+// `top` largest of a softmax over all experts, renormalized
+std::vector<torch::Tensor> moe_route(torch::Tensor x, torch::Tensor w, int64_t top) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && w.is_cuda() && w.dtype() == torch::kBFloat16 &&
+              w.dim() == 2 && w.is_contiguous() && w.size(1) == x.size(1));
+  const long t = x.size(0), dim = x.size(1), experts = w.size(0);
+  TORCH_CHECK(dim % 8 == 0 && top >= 1 && top <= experts && experts <= ROUTE_EXPERTS && top <= ROUTE_TOP);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
+  TORCH_CHECK(x.dtype() == torch::kFloat32 || x.dtype() == torch::kBFloat16);
+  auto weights = torch::empty({t, top}, x.options().dtype(torch::kFloat32));
+  auto sel = torch::empty({t, top}, x.options().dtype(torch::kInt32));
+  if (t == 0) return {weights, sel};
+  auto stream = at::cuda::getCurrentCUDAStream();
+  if (x.dtype() == torch::kFloat32)
+    moe_route_kernel<<<t, 256, 0, stream>>>(x.data_ptr<float>(), BF16P(w), weights.data_ptr<float>(),
+                                            sel.data_ptr<int>(), (int)dim, (int)experts, (int)top);
+  else
+    moe_route_kernel<<<t, 256, 0, stream>>>((const unsigned short*)BF16P(x), BF16P(w), weights.data_ptr<float>(),
+                                            sel.data_ptr<int>(), (int)dim, (int)experts, (int)top);
+  HIP_CHECK_LAST();
+  return {weights, sel};
+}
+
+// rows: partial sums [splits, T * top, out] f32, or [T * top, out] bf16 -> residual [T, out] + their weighted sum, bf16
+torch::Tensor moe_combine(torch::Tensor rows, torch::Tensor weights, torch::Tensor residual) {
+  TORCH_CHECK(weights.is_cuda() && weights.dtype() == torch::kFloat32 && weights.dim() == 2 && weights.is_contiguous());
+  TORCH_CHECK(residual.is_cuda() && residual.dtype() == torch::kBFloat16 && residual.dim() == 2 && residual.is_contiguous());
+  TORCH_CHECK(rows.is_cuda() && rows.is_contiguous());
+  const long t = weights.size(0), top = weights.size(1), out_dim = residual.size(1);
+  TORCH_CHECK(residual.size(0) == t && rows.size(-1) == out_dim && rows.size(-2) == t * top);
+  auto y = torch::empty_like(residual);
+  if (y.numel() == 0) return y;
+  auto stream = at::cuda::getCurrentCUDAStream();
+  if (rows.dim() == 3) {
+    TORCH_CHECK(rows.dtype() == torch::kFloat32 && t <= 65535);
+    moe_reduce_kernel<<<dim3((out_dim + 63) / 64, t), 1024, 0, stream>>>(
+        rows.data_ptr<float>(), weights.data_ptr<float>(), BF16P(residual), BF16P(y), (int)rows.size(0), (int)t, (int)top,
+        (int)out_dim);
+  } else {
+    TORCH_CHECK(rows.dim() == 2 && rows.dtype() == torch::kBFloat16 && out_dim % 8 == 0);
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(rows.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0);
+    const long groups = t * out_dim / 8, blocks = (groups + 255) / 256;
+    TORCH_CHECK(blocks < (1L << 31));
+    moe_combine_kernel<<<blocks, 256, 0, stream>>>(BF16P(rows), weights.data_ptr<float>(), BF16P(residual), BF16P(y),
+                                                   (int)top, (int)out_dim, groups);
+  }
+  HIP_CHECK_LAST();
+  return y;
+}
+
+std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t mt) {
+  TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());
+  TORCH_CHECK(experts >= 1 && experts <= 4096 && mt >= 1);
+  const long r = sel.numel();
+  // at most min(r, experts) segments end in a partly filled tile
+  const long slots = (r + std::min(r, (long)experts) * (mt - 1) + mt - 1) / mt * mt;
+  auto pairs = torch::empty({slots}, sel.options());
+  auto tiles = torch::empty({slots / mt}, sel.options());
+  moe_group_kernel<<<1, 1024, experts * 8, at::cuda::getCurrentCUDAStream()>>>(
+      sel.data_ptr<int>(), r, experts, mt, slots, pairs.data_ptr<int>(), tiles.data_ptr<int>());
+  HIP_CHECK_LAST();
+  return {pairs, tiles};
+}
+
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all,      // [E, in, out] bf16
     c10::optional<torch::Tensor> nf4_all,     // NF4: [E, out/64, ceil(in/128), 4, 64, 16] u8
@@ -428,6 +636,7 @@ torch::Tensor gemv_bf16_moe(
   TORCH_CHECK(rows <= 64, "moe gemv supports batch*k <= 64");
   if (gemv_mfma_fits(wt_all, out_dim)) {
     auto sums = launch_gemv_mfma(wt_all, x, &sel, k_per_tok, workspace);
+    if (epilogue < 0) return sums;  // [splits, rows, out]
     return launch_gemv_reduce(
         sums, c10::nullopt, c10::nullopt, (int)sums.size(0), rows, out_dim, (int)epilogue, x.options(), wt_all.options(),
         c10::nullopt, ClampedGate{(float)limit, (float)alpha});
@@ -453,6 +662,7 @@ torch::Tensor gemv_bf16_moe(
       sel.data_ptr<int>(), partials.data_ptr<float>(), in_dim, out_dim, i_per_split,
       rows, (int)k_per_tok);
   HIP_CHECK_LAST();
+  if (epilogue < 0) return partials.view(-1).narrow(0, 0, splits * rows * out_dim).view({splits, rows, out_dim});
   return launch_gemv_reduce(
       partials, c10::nullopt, c10::nullopt, (int)splits, rows, out_dim, (int)epilogue,
       x.options(), wt_all.options(), c10::nullopt, ClampedGate{(float)limit, (float)alpha});

@@ -488,6 +488,7 @@ torch::Tensor gemv_nf4_tiles_moe(
   TORCH_CHECK(x.dim() == 2 && rows == x.size(0) * k_per_tok);
   TORCH_CHECK(rows <= 16, "moe gemv supports batch*k <= 16");
   auto partials = launch_nf4_tiles(tiles, scales, in_dim, x, &sel, k_per_tok, workspace);
+  if (epilogue < 0) return partials;
   return launch_gemv_reduce(partials, c10::nullopt, c10::nullopt, (int)partials.size(0), (int)rows,
                             (int)partials.size(2), (int)epilogue, x.options(), scales.options());
 }

@@ -8,7 +8,6 @@
 //   batched_linear    out[t, h, n] = sum_k a[t, h, k] w[h, n, k]: the per-head
 //                     projections of latent attention, MFMA for bf16 weights
 //   clamped_swiglu    g * sigmoid(alpha g) * (u + 1), g and u clamped
-//   moe_group         expert-sorted, tile-padded (token, slot) pairs for moe_gemm
 //   moe_linear_f32    expert products in 32-bit
 
 #include "common.h"
@@ -345,43 +344,6 @@ __global__ __launch_bounds__(256) void clamped_swiglu_kernel(
 
 // ------------------------------------------------------------ expert groups
 
-// One workgroup. counts -> padded offsets -> scatter; every sorted slot and
-// every tile is written. The order of an expert's pairs is not fixed, which no
-// result depends on (each pair is a row of its own).
-__global__ __launch_bounds__(1024) void moe_group_kernel(
-    const int* __restrict__ sel, int pairs, int experts, int mt, int slots,
-    int* __restrict__ sorted_pairs, int* __restrict__ tile_expert) {
-  extern __shared__ int cnt[];  // [experts] counts, then next free slot
-  int* end = cnt + experts;     // [experts] end of the padded segment
-  const int tid = threadIdx.x;
-  for (int e = tid; e < experts; e += blockDim.x) cnt[e] = 0;
-  for (int i = tid; i < slots; i += blockDim.x) sorted_pairs[i] = -1;
-  for (int i = tid; i < slots / mt; i += blockDim.x) tile_expert[i] = -1;
-  __syncthreads();
-  for (int i = tid; i < pairs; i += blockDim.x) {
-    const int e = sel[i];
-    if (e >= 0 && e < experts) atomicAdd(&cnt[e], 1);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int at = 0;
-    for (int e = 0; e < experts; ++e) {
-      const int padded = (cnt[e] + mt - 1) / mt * mt;
-      cnt[e] = at;
-      at += padded;
-      end[e] = at;
-    }
-  }
-  __syncthreads();
-  for (int e = tid; e < experts; e += blockDim.x)
-    for (int i = cnt[e]; i < end[e]; i += mt) tile_expert[i / mt] = e;
-  __syncthreads();
-  for (int i = tid; i < pairs; i += blockDim.x) {
-    const int e = sel[i];
-    if (e >= 0 && e < experts) sorted_pairs[atomicAdd(&cnt[e], 1)] = i;
-  }
-}
-
 __global__ __launch_bounds__(64) void moe_linear_f32_kernel(
     const float* __restrict__ w,  // [E, in, out]
     const float* __restrict__ x,  // [rows / k, in]
@@ -545,20 +507,6 @@ torch::Tensor clamped_swiglu(torch::Tensor gu, double limit, double alpha) {
 }
 
 // sel [R] expert of each (token, slot) pair -> (sorted_pairs, tile_expert), see moe.hip
-std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t mt) {
-  TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());
-  TORCH_CHECK(experts >= 1 && experts <= 4096 && mt >= 1);
-  const long r = sel.numel();
-  // at most min(r, experts) segments end in a partly filled tile
-  const long slots = (r + std::min(r, (long)experts) * (mt - 1) + mt - 1) / mt * mt;
-  auto pairs = torch::empty({slots}, sel.options());
-  auto tiles = torch::empty({slots / mt}, sel.options());
-  moe_group_kernel<<<1, 1024, experts * 8, at::cuda::getCurrentCUDAStream()>>>(
-      sel.data_ptr<int>(), r, experts, mt, slots, pairs.data_ptr<int>(), tiles.data_ptr<int>());
-  HIP_CHECK_LAST();
-  return {pairs, tiles};
-}
-
 torch::Tensor moe_linear_f32(torch::Tensor w, torch::Tensor x, torch::Tensor sel, int64_t k) {
   TORCH_CHECK(is_f32(w) && is_f32(x) && w.dim() == 3 && x.dim() == 2 && w.is_contiguous() && x.is_contiguous());
   TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());

@@ -685,7 +685,11 @@ class LlamaFastPath(_TPFastPathMixin):
             h2 = hidden + o
             xn2 = self.hip.rms_norm(h2, self.ln2_w_post, self.eps)
         xd2 = self.hip.rms_norm(h2, self.ln2_w, self.eps) if (self.fold_norm and adapter is not None) else None
-        return h2 + self._tp_reduce(self._mlp_dense(xn2, adapter, autograd=False, x_delta=xd2)).to(h2.dtype)
+        return self._mlp_prompt(h2, xn2, adapter, xd2)
+
+    def _mlp_prompt(self, h2, xn2, adapter, x_delta):
+        """h2 + MLP(xn2) of a prompt's rows."""
+        return h2 + self._tp_reduce(self._mlp_dense(xn2, adapter, autograd=False, x_delta=x_delta)).to(h2.dtype)
 
 
 # ---------------------------------------------------------------------------

@@ -24,6 +24,7 @@ import torch.nn.functional as F
 
 from petals_amd.ops.fused_decode import (
     _EPI_PLAIN_F32,
+    _EPI_RAW,
     _EPI_SWIGLU_F32,
     LlamaFastPath,
     _FastWeight,
@@ -127,7 +128,8 @@ class MixtralFastPath(LlamaFastPath):
         moe = block.block_sparse_moe
         self.top_k = moe.top_k
         self.num_experts = moe.num_experts
-        self.w_router_t = t(moe.gate.weight)  # [H, E]
+        self.w_router = moe.gate.weight.detach().to(torch.bfloat16).contiguous()  # [E, H]
+        self.w_router_t = self.w_router.t()
         self.stacked_gu: Optional[_StackedExperts] = None
         self.stacked_down: Optional[_StackedExperts] = None
         self.wgateup_e: List[_FastWeight] = []
@@ -166,16 +168,24 @@ class MixtralFastPath(LlamaFastPath):
         weights = weights / weights.sum(dim=-1, keepdim=True)
         return weights, selected
 
+    def _route_rows(self, x: torch.Tensor):
+        """Router on [tokens, H]: (weights [t, k] f32, experts [t, k] int32), one launch
+        for as many experts as the kernel takes."""
+        if x.shape[1] % 8 == 0 and self.num_experts <= 256 and self.top_k <= 16:
+            return self.hip.moe_route(x, self.w_router, self.top_k)
+        weights, selected = self._route(x)
+        return weights.contiguous(), selected.to(torch.int32).contiguous()
+
     def _mlp_decode(self, xn2, h2, ws, adapter):
         """xn2 f32 [B, H]; returns h3 bf16 [B, H]."""
         B = xn2.shape[0]
-        weights, selected = self._route(xn2)
         if self.stacked_gu is not None:
-            sel = selected.to(torch.int32).reshape(-1).contiguous()  # [B*k]
+            weights, sel = self._route_rows(xn2.contiguous())
+            sel = sel.view(-1)  # [B*k]
             act = self.stacked_gu.moe_gemv(xn2.contiguous(), sel, self.top_k, ws, _EPI_SWIGLU_F32)
-            down = self.stacked_down.moe_gemv(act.contiguous(), sel, 1, ws, _EPI_PLAIN_F32)
-            moe_out = (down.view(B, self.top_k, -1) * weights.unsqueeze(-1)).sum(dim=1)
-            return (h2.float() + moe_out).to(torch.bfloat16)
+            parts = self.stacked_down.moe_gemv(act, sel, 1, ws, _EPI_RAW)
+            return self.hip.moe_combine(parts, weights, h2)
+        weights, selected = self._route(xn2)
 
         # int8: host-synced routing (~10 us, amortized against MBs of expert reads)
         sel_l = selected.tolist()
@@ -196,30 +206,25 @@ class MixtralFastPath(LlamaFastPath):
     def _expert_down_dense(self, e: int) -> torch.Tensor:
         return self.stacked_down.dense(e) if self.stacked_down is not None else self.wdown_e[e].dense()
 
+    def _mlp_prompt(self, h2, xn2, adapter, x_delta):
+        """Prompts run the grouped MFMA GEMM (ops/csrc/moe.hip moe_gemm: NF4 dequant fused
+        into the staging, so packed weights are what crosses HBM)."""
+        stacked = self.stacked_gu is not None and self.stacked_gu.gemm_ok and self.stacked_down.gemm_ok
+        if not stacked or xn2.device.type != "cuda" or self.tp_world > 1:
+            return super()._mlp_prompt(h2, xn2, adapter, x_delta)
+        x = xn2.reshape(-1, xn2.shape[-1]).contiguous()
+        weights, sel = self._route_rows(x)
+        order, tile_expert = self.hip.moe_group(sel.view(-1), self.num_experts, MOE_GEMM_MT)
+        gateup = self.stacked_gu.moe_gemm(x, order, tile_expert, self.top_k, sel.numel())
+        down = self.stacked_down.moe_gemm(self.hip.swiglu_rows(gateup), order, tile_expert, 1, sel.numel())
+        return self.hip.moe_combine(down, weights, h2.reshape(x.shape[0], -1)).view(h2.shape)
+
     def _mlp_dense(self, xn2, adapter, autograd: bool, x_delta=None):
-        """Prefill / training MLP over the routed experts. Inference prefill
-        runs the grouped MFMA GEMM (ops/csrc/moe.hip moe_gemm: NF4 dequant
-        fused into the LDS B-tile staging — packed weights are what cross
-        HBM, read ceil(rows_e/32) times per expert instead of once per
-        token); training/CPU fall back to token-grouped dense matmuls."""
+        """MLP over the routed experts by token-grouped dense matmuls: training, CPU, and
+        geometries or quantizations that the grouped GEMM does not take."""
         shape = xn2.shape
         x = xn2.reshape(-1, shape[-1])
         weights, selected = self._route(x)
-        if (
-            not autograd
-            and x.device.type == "cuda"
-            and self.stacked_gu is not None
-            and self.stacked_gu.gemm_ok
-            and self.stacked_down.gemm_ok
-        ):
-            T, K = x.shape[0], self.top_k
-            sorted_pairs, tile_expert = sort_pairs_by_expert(selected, self.num_experts)
-            xb = x.to(torch.bfloat16).contiguous()
-            gateup = self.stacked_gu.moe_gemm(xb, sorted_pairs, tile_expert, K, T * K)
-            act = self.hip.swiglu_rows(gateup)
-            down = self.stacked_down.moe_gemm(act, sorted_pairs, tile_expert, 1, T * K)
-            out = (down.view(T, K, -1).float() * weights.unsqueeze(-1)).sum(dim=1)
-            return out.reshape(*shape[:-1], -1).to(xn2.dtype)
         out_dim = self.stacked_down.out_dim if self.stacked_down is not None else self.wdown_e[0].shape[1]
         out = torch.zeros(x.shape[0], out_dim, dtype=torch.float32, device=x.device)
         expert_mask = F.one_hot(selected, num_classes=self.num_experts).permute(2, 1, 0)

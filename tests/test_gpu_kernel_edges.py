@@ -322,3 +322,36 @@ def test_prompt_chunks_are_one_prompt(hip, tokens, limit):
     assert torch.allclose(torch.cat(parts, 1).float(), whole.float(), **tol)
     for a, b in zip(*caches):
         assert torch.allclose(a.float(), b.float(), **tol)
+
+
+@requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, BF16])
+@pytest.mark.parametrize("tokens,dim,experts,top", [(1, 8, 1, 1), (3, 64, 4, 2), (5, 4096, 8, 2), (2, 520, 64, 16), (7, 128, 65, 3), (1, 2048, 256, 8)])
+def test_router(hip, dtype, tokens, dim, experts, top):
+    gen = torch.Generator(device="cuda").manual_seed(experts)
+    x = torch.randn(tokens, dim, device="cuda", generator=gen).to(dtype)
+    w = torch.randn(experts, dim, device="cuda", generator=gen).to(BF16)
+    weights, sel = hip.moe_route(x, w, top)
+    logits = x.double() @ w.double().t()
+    best, chosen = torch.topk(logits, top, dim=-1)
+    assert torch.equal(sel.long(), chosen)  # no ties among random values
+    # 32-bit logits: sums of dim terms; exponentials and a division
+    err = 2.0**-24 * (dim / 64 + 16) * (x.double().abs() @ w.double().abs().t()).amax() + 2.0**-20
+    assert bool(((weights.double() - torch.softmax(best, -1)).abs() <= err).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("tokens,top,splits,width", [(1, 1, 1, 8), (3, 2, 5, 72), (2, 3, 7, 4096), (130, 2, 1, 128)])
+def test_expert_sums(hip, tokens, top, splits, width):
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    parts = torch.randn(splits, tokens * top, width, device="cuda", generator=gen)
+    weights = torch.rand(tokens, top, device="cuda", generator=gen)
+    residual = torch.randn(tokens, width, device="cuda", generator=gen).to(BF16)
+
+    def check(y, rows):
+        ref = residual.double() + (rows.view(tokens, top, width) * weights.double()[..., None]).sum(1)
+        assert bool(((y.double() - ref).abs() <= 2.0**-8 * ref.abs() + 1e-4).all())
+
+    check(hip.moe_combine(parts, weights, residual), parts.double().sum(0))
+    rows = parts[0].to(BF16)
+    check(hip.moe_combine(rows, weights, residual), rows.double())
