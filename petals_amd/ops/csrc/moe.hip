@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     const unsigned short* __restrict__ w,   // [experts, dim] bf16
     float* __restrict__ weights, int* __restrict__ sel, int dim, int experts, int top) {
   __shared__ float logits[ROUTE_EXPERTS];
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const T* row = x + (size_t)blockIdx.x * dim;
   for (int e = wave; e < experts; e += 4) {
     float sum = 0.f;
@@ -268,26 +268,36 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
 // With a tile of 32 rows and 128 columns each, weights crossed the caches four times as
 // often and every product waited for a transposing store of its weights. Both products of
 // a layer of 8 experts, width 4096 and inner size 14336: with 290 rows an expert from 6.06
-// to 1.73 ms (135 to 472 TFLOP/s), with 71 from 2.09 to 0.80 ms (weights at 3.5 TB/s).
+// to 1.20 ms (135 to 680 TFLOP/s), with 71 from 2.09 to 0.57 ms (weights at 5.0 TB/s).
 //
-// 8 waves of 64 x 64; K in steps of 64, staged in two LDS buffers while the next step's
-// loads are in flight. The product is W^T X^T, so that a lane ends with 4 neighbouring
-// columns of one row. Weights in bf16 lie in LDS as in memory and are read by transposing
-// loads. NF4 weights are dequantized on the way, so that their packed form is what is read:
-// a thread has 16 codes of one column, and its LDS rows are columns. The 16-byte groups of
-// an LDS row, of 128 or (W in bf16) 512 bytes, are permuted by the row, so that the 16 rows
-// that a load touches lie in different banks.
+// 8 waves of 64 x 64, two on a SIMD; K in steps of 64 through two LDS buffers. The two
+// waves of a SIMD take turns, half a step apart: while one moves (fragments out of LDS, the
+// next step's tile into it), the other keeps the matrix cores busy and asks for the tile
+// after next but one. All in step, with both halves of a step's fragments read ahead:
+// 1.33 and 0.61 ms; fragments read as they were needed and loads one step ahead: 1.73 and
+// 0.80 ms, 58% of all wave time spent waiting (with NF4 weights 2.31 to 2.02 ms with 290
+// rows, 0.96 to 0.86 ms with 71). Loads have no conditions, rows and columns
+// beyond the end repeat the last: with a condition on one of them the compiler can't tell
+// how many are in flight and waits for all. Tiles of 256 rows, of 128 columns with two
+// workgroups on a CU, and steps of 32 were all slower.
+//
+// The product is W^T X^T, so that a lane ends with 4 neighbouring columns of one row.
+// Weights in bf16 lie in LDS as in memory and are read by transposing loads. NF4 weights
+// are dequantized on the way, so that their packed form is what is read: a thread has 16
+// codes of one column, and its LDS rows are columns. The 16-byte groups of an LDS row, of
+// 128 or (W in bf16) 512 bytes, are permuted by the row, so that the 16 rows that a load
+// touches lie in different banks.
 //
 // Workgroups are dealt to the 8 chiplets in turn; a chiplet takes every eighth run of
-// columns and all row groups of it one after the other: they find its weights in its L2.
+// columns. Up to MOE_SHARE row groups of an expert follow each other with the same run:
+// they find its weights in the chiplet's L2, and the next run finds their rows there
+// (2 to 5% over all groups of all experts with one run).
 
-#define MOE_MT 32   // rows of a tile of one expert
-#define MOE_BM 128  // rows of a workgroup
-#define MOE_BN 256  // columns of a workgroup
-#define MOE_BK 64   // k step
-#define MOE_X_BYTES (MOE_BM * MOE_BK * 2)
-#define MOE_W_BYTES (MOE_BK * MOE_BN * 2)
-#define MOE_LDS (2 * (MOE_X_BYTES + MOE_W_BYTES))
+#define MOE_MT 32    // rows of a tile of one expert
+#define MOE_BM 128   // rows of a workgroup
+#define MOE_BN 256   // columns of a workgroup
+#define MOE_BK 64    // k step
+#define MOE_SHARE 8  // row groups that share a run of columns
 
 // where 16-byte group c of a row lies
 __device__ __forceinline__ int moe_x_at(int row, int c) { return row * (MOE_BK * 2) + ((c ^ ((row >> 1) & 7)) << 4); }
@@ -295,10 +305,15 @@ __device__ __forceinline__ int moe_w_at(int row, int c) {
   return row * (MOE_BN * 2) + ((c ^ (((row & 3) | ((row >> 1) & 4)) << 1)) << 4);
 }
 
-// The first tile of the which-th group: tiles come in runs of one expert, a run's groups
-// have four tiles, its last one maybe fewer. -1: there are not so many. Uniform over a wave.
-__device__ __forceinline__ int moe_group_tile(const int* __restrict__ tile_expert, int n_tiles, int which) {
-  const int lane = threadIdx.x & (WAVE - 1);
+// A chiplet's slot-th workgroup: the first tile of its group of rows (-1: it has none) and its
+// run of columns, of `columns`. Tiles come in runs of one expert, a run's groups have four
+// tiles, its last one maybe fewer. Uniform over a wave.
+struct MoeSpot {
+  int tile, column;
+};
+__device__ __forceinline__ MoeSpot moe_spot(const int* __restrict__ tile_expert, int n_tiles, int slot, int columns) {
+  constexpr int PER = MOE_BM / MOE_MT;
+  const int lane = threadIdx.x & (WAVE - 1), which = slot / columns;
   int seen = 0, run = 0;  // groups so far; first tile of the run that reaches into this chunk
   for (int base = 0; base < n_tiles; base += WAVE) {
     const int i = base + lane;
@@ -307,20 +322,28 @@ __device__ __forceinline__ int moe_group_tile(const int* __restrict__ tile_exper
     const unsigned long long starts = __ballot(e != before || i == 0);
     const unsigned long long upto = starts & (~0ull >> (WAVE - 1 - lane));
     const int first = upto ? base + WAVE - 1 - __clzll((long long)upto) : run;
-    const unsigned long long leads = __ballot(e >= 0 && ((i - first) & 3) == 0);
+    const unsigned long long leads = __ballot(e >= 0 && ((i - first) & (PER - 1)) == 0);
     const int n = __popcll(leads);
     if (which < seen + n) {
       const bool mine = ((leads >> lane) & 1) && __popcll(leads & ((1ull << lane) - 1)) == which - seen;
-      return base + __ffsll((long long)__ballot(mine)) - 1;
+      const int at = __ffsll((long long)__ballot(mine)) - 1;
+      const int begin = __shfl(first, at), expert = __shfl(e, at);
+      int end = base + at;
+      for (unsigned long long same = ~0ull; same == ~0ull; end += same == ~0ull ? WAVE : __ffsll((long long)~same) - 1)
+        same = __ballot(end + lane < n_tiles && tile_expert[min(end + lane, n_tiles - 1)] == expert);
+      const int mid = (base + at - begin) / PER, chunk = mid & ~(MOE_SHARE - 1);
+      const int share = min(MOE_SHARE, (end - begin + PER - 1) / PER - chunk);
+      const int r = slot - columns * (which - mid + chunk);
+      return {begin + PER * (chunk + r % share), r / share};
     }
     seen += n;
     if (starts) run = base + WAVE - 1 - __clzll((long long)starts);
   }
-  return -1;
+  return {-1, 0};
 }
 
 template <bool NF4>
-__global__ __launch_bounds__(512) void moe_gemm_kernel(
+__global__ __launch_bounds__(512, 2) void moe_gemm_kernel(
     const unsigned short* __restrict__ wt_all,      // [E, in, out] bf16 (NF4: null)
     const uint4* __restrict__ nf4_all,              // NF4: tiles (bf16: null)
     const unsigned short* __restrict__ scales_all,  // NF4: [E, out/64, n_kb * 128] bf16
@@ -333,81 +356,74 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
     int k_per_tok,
     int n_tiles,
     int experts,
-    int groups) {
+    int columns) {
+  constexpr int BN = MOE_BN, BK = MOE_BK, T = 512;
+  constexpr int AHEAD = NF4 ? 1 : 2;  // steps whose loads are in registers (NF4: codes last for two)
+  constexpr int X_BYTES = MOE_BM * BK * 2, STAGE = X_BYTES + BN * BK * 2;
   extern __shared__ unsigned char smem[];
   __shared__ float2 lut2[NF4 ? 256 : 1];
-  const int slot = blockIdx.x >> 3;
-  const int n0 = ((slot / groups) * 8 + (blockIdx.x & 7)) * MOE_BN;
-  if (n0 >= out_dim) return;
-  const int tile = moe_group_tile(tile_expert, n_tiles, slot % groups);
-  if (tile < 0) return;
+  const MoeSpot spot = moe_spot(tile_expert, n_tiles, blockIdx.x >> 3, columns);
+  const int tile = spot.tile, n0 = (spot.column * 8 + (blockIdx.x & 7)) * BN;
+  if (tile < 0 || n0 >= out_dim) return;
   const int e = tile_expert[tile];
   if (e >= experts) return;
   int rows = MOE_MT;  // of this group
   while (rows < MOE_BM && tile + rows / MOE_MT < n_tiles && tile_expert[tile + rows / MOE_MT] == e) rows += MOE_MT;
 
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 15, hi = lane >> 4;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;  // this wave's rows and columns
+  const int wm = ((wave ^ (wave >> 2)) & 1) * 64, wn = wave / 2 * 64;  // this wave's rows and columns
+  const bool idle = wm >= rows;                              // uniform over the wave
   if (NF4 && tid < 256) lut2[tid] = make_float2(MOE_NF4_LUT[tid & 0xF], MOE_NF4_LUT[tid >> 4]);
 
   // loads of a step: two 16-byte groups of X, and four of W, or for two steps two of NF4
   // codes (32 of a column) and for each step their 16 scales, per thread
-  constexpr int XN = MOE_BM * MOE_BK / 8 / 512, WN = MOE_BK * MOE_BN / 8 / 512;
+  constexpr int X8 = BK / 8, XN = MOE_BM * X8 / T, WN = BK * BN / 8 / T;
   const unsigned short* xp[XN];
 #pragma unroll
   for (int i = 0; i < XN; ++i) {
-    const int row = (tid + i * 512) / 8;
-    const int pr = row < rows ? sorted_pairs[tile * MOE_MT + row] : -1;
-    xp[i] = pr < 0 ? nullptr : x + (size_t)(pr / k_per_tok) * in_dim + (tid & 7) * 8;
+    const int row = (tid + i * T) / X8;
+    const int pr = max(sorted_pairs[tile * MOE_MT + min(row, rows - 1)], 0);
+    xp[i] = x + (size_t)(pr / k_per_tok) * in_dim + tid % X8 * 8;
   }
-  const int wc = (tid & 31) * 8, wr = tid >> 5;  // first column and row of this thread's weights
-  const bool w_live = n0 + wc < out_dim;         // out_dim is a multiple of 128
-  const unsigned short* wp = NF4 ? nullptr : wt_all + (size_t)e * in_dim * out_dim + (size_t)wr * out_dim + n0 + wc;
+  const int wc = tid % (BN / 8) * 8, wr = tid / (BN / 8);  // first column and row of this thread's weights
+  const unsigned short* wp =
+      NF4 ? nullptr : wt_all + (size_t)e * in_dim * out_dim + (size_t)wr * out_dim + min(n0 + wc, out_dim - 8);
   const int n_kb = (in_dim + 127) / 128;
 
-  short8 xn[XN], wnext[NF4 ? 1 : WN];
+  short8 xn_all[AHEAD][XN], wn_all[AHEAD][NF4 ? 1 : WN];
   uint4 codes[2];
   short8 scale[2][2];
-#pragma unroll
-  for (int i = 0; i < XN; ++i) xn[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < (NF4 ? 1 : WN); ++i) wnext[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    codes[i] = uint4{0u, 0u, 0u, 0u};
-    scale[i][0] = scale[i][1] = short8{0, 0, 0, 0, 0, 0, 0, 0};
-  }
-  auto fetch = [&](int kt) {
+  auto fetch = [&](int step, short8* xn, short8* wnext) {
+    const int kt = min(step, in_dim - BK);
 #pragma unroll
     for (int i = 0; i < XN; ++i)
-      if (xp[i]) xn[i] = *reinterpret_cast<const short8*>(xp[i] + kt);
+      xn[i] = *reinterpret_cast<const short8*>(xp[i] + kt);
     if constexpr (NF4) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const int nb = n0 / 64 + tid / 256 + 2 * i;
-        if (nb * 64 >= out_dim) continue;
+        const int nb = min(n0 / 64 + tid / 256 + T / 256 * i, out_dim / 64 - 1);
         const size_t at = ((size_t)e * (out_dim / 64) + nb) * n_kb + kt / 128;
-        if (kt % 128 == 0) codes[i] = nf4_all[at * 256 + tid % 256];
+        if (step % 128 == 0) codes[i] = nf4_all[at * 256 + tid % 256];
         const short8* p = reinterpret_cast<const short8*>(scales_all + at * 128 + kt % 128 + lane / 16 * 16);
         scale[i][0] = p[0];
         scale[i][1] = p[1];
       }
-    } else if (w_live) {
+    } else {
 #pragma unroll
       for (int i = 0; i < WN; ++i)
         wnext[i] = *reinterpret_cast<const short8*>(wp + (size_t)(kt + i * 16) * out_dim);
     }
   };
-  auto stage = [&](unsigned char* buf, int kt) {
+  auto stage = [&](unsigned char* buf, int kt, const short8* xn, const short8* wnext) {
 #pragma unroll
-    for (int i = 0; i < XN; ++i) *reinterpret_cast<short8*>(buf + moe_x_at((tid + i * 512) / 8, tid & 7)) = xn[i];
-    unsigned char* w = buf + MOE_X_BYTES;
+    for (int i = 0; i < XN; ++i) *reinterpret_cast<short8*>(buf + moe_x_at((tid + i * T) / X8, tid % X8)) = xn[i];
+    unsigned char* w = buf + X_BYTES;
     if constexpr (NF4) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const unsigned words[2] = {kt & 64 ? codes[i].z : codes[i].x, kt & 64 ? codes[i].w : codes[i].y};
-        const int row = (tid / 256 + 2 * i) * 64 + tid % 256 / 64 * 16 + col;
+        const int row = (tid / 256 + T / 256 * i) * 64 + tid % 256 / 64 * 16 + col;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
           short8 v;
@@ -431,41 +447,72 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_moe{0.f, 0.f, 0.f, 0.f};
-
-  fetch(0);
-  if (NF4) __syncthreads();  // the table
-  stage(smem, 0);
-  __syncthreads();
-  int which = 0;
-  for (int kt = 0; kt < in_dim; kt += MOE_BK, which ^= 1) {
-    const bool more = kt + MOE_BK < in_dim;
-    if (more) fetch(kt + MOE_BK);
-    const unsigned char* xb = smem + which * (MOE_X_BYTES + MOE_W_BYTES);
-    const unsigned char* wb = xb + MOE_X_BYTES;
+  static_assert(BK == 64);  // two halves of a step
+  bf16x8_moe xf[2][4], wf[2][4];
+  auto read = [&](const unsigned char* xb, int kc) {
+    if (idle) return;
+    const unsigned char* wb = xb + X_BYTES;
 #pragma unroll
-    for (int kc = 0; kc < MOE_BK / 32; ++kc) {
-      bf16x8_moe xf[4], wf[4];
+    for (int j = 0; j < 4; ++j)
+      xf[kc][j] = *reinterpret_cast<const bf16x8_moe*>(xb + moe_x_at(wm + j * 16 + col, kc * 4 + hi));
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        xf[j] = *reinterpret_cast<const bf16x8_moe*>(xb + moe_x_at(wm + j * 16 + col, kc * 4 + hi));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (NF4) {
-          wf[i] = *reinterpret_cast<const bf16x8_moe*>(wb + moe_x_at(wn + i * 16 + col, kc * 4 + hi));
-          continue;
-        }
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (NF4) {
+        wf[kc][i] = *reinterpret_cast<const bf16x8_moe*>(wb + moe_x_at(wn + i * 16 + col, kc * 4 + hi));
+      } else {
         // rows hi*8 + col/4 and 4 below, which are permuted alike; 4 columns a lane
         const int row = kc * 32 + hi * 8 + col / 4, group = (wn + i * 16) / 8 + ((col >> 1) & 1);
-        wf[i] = load_keys(reinterpret_cast<const unsigned short*>(wb + moe_w_at(row, group) + (col & 1) * 8), MOE_BN);
+        wf[kc][i] = load_keys(reinterpret_cast<const unsigned short*>(wb + moe_w_at(row, group) + (col & 1) * 8), BN);
       }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
     }
-    if (more) stage(smem + (which ^ 1) * (MOE_X_BYTES + MOE_W_BYTES), kt + MOE_BK);
+  };
+  auto multiply = [&](int kc) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (idle) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kc][i], xf[kc][j], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Step t lies in buffer t % 2; its loads are in registers t % AHEAD. A wave's step is two
+  // intervals between barriers; waves 4 to 7, which have the same SIMDs as 0 to 3, are one
+  // interval late. What an early wave writes in interval 2t, and a late one in 2t + 1, is
+  // step t + 1's tile, read from 2t + 2 on; the buffer was last read in 2t - 1.
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) fetch(s * BK, xn_all[s], wn_all[s]);
+  if (NF4) __syncthreads();  // the table
+  stage(smem, 0, xn_all[0], wn_all[0]);
+  __syncthreads();
+  auto step = [&](int kt, int half) {
+    constexpr int last = AHEAD - 1;
+    read(smem + half * STAGE, 0);
+    read(smem + half * STAGE, 1);
+    stage(smem + (half ^ 1) * STAGE, kt + BK, xn_all[(half + 1) & last], wn_all[(half + 1) & last]);
     __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(kt + (AHEAD + 1) * BK, xn_all[(half + 1) & last], wn_all[(half + 1) & last]);
+    multiply(0);
+    multiply(1);
+    __syncthreads();
+  };
+  fetch(AHEAD * BK, xn_all[0], wn_all[0]);
+  const bool late = wave >= 4;
+  if (late) __syncthreads();
+  int kt = 0;
+  for (; kt + BK < in_dim; kt += 2 * BK) {
+    step(kt, 0);
+    step(kt + BK, 1);
   }
+  if (kt < in_dim) {
+    read(smem, 0);
+    read(smem, 1);
+    multiply(0);
+    multiply(1);
+  }
+  if (!late) __syncthreads();
 
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -583,35 +630,36 @@ torch::Tensor moe_gemm(
   // staging loads are 16B/32-value vectors: callers fall back to the dense
   // path for geometries outside these alignments (fused_moe.py)
   TORCH_CHECK(out_dim % 128 == 0, "moe_gemm needs out_dim % 128 == 0");
-  TORCH_CHECK(in_dim % MOE_BK == 0, "moe_gemm needs in_dim % 64 == 0");
+  TORCH_CHECK(in_dim % 64 == 0, "moe_gemm needs in_dim % 64 == 0");
   const long Rp = sorted_pairs.size(0);
   TORCH_CHECK(Rp % MOE_MT == 0 && tile_expert.size(0) == Rp / MOE_MT);
 
   auto c = torch::empty({n_rows, (long)out_dim}, x.options());
   const long n_tiles = Rp / MOE_MT, experts = nf4 ? nf4_all->size(0) : wt_all->size(0);
   // an expert's last group may have one tile
-  const long groups = std::min(n_tiles, (n_tiles + 3 * experts) / 4);
-  if (groups == 0) return c;
-  const long columns = (out_dim + MOE_BN - 1) / MOE_BN;
-  const long blocks = groups * ((columns + 7) / 8) * 8;
+  constexpr long per = MOE_BM / MOE_MT;
+  const long groups = std::min(n_tiles, (n_tiles + (per - 1) * experts) / per);
+  if (groups == 0 || x.size(0) == 0) return c;
+  const long columns = (out_dim + 8 * MOE_BN - 1) / (8 * MOE_BN);  // runs of a chiplet
+  const long blocks = groups * columns * 8;
   TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
   auto stream = at::cuda::getCurrentCUDAStream();
-#define MOE_GEMM(NF4, W, P, S)                                                                               \
-  do {                                                                                                       \
-    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_kernel<NF4>),        \
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, MOE_LDS);        \
-    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                  \
-    moe_gemm_kernel<NF4><<<blocks, 512, MOE_LDS, stream>>>(                                                  \
-        W, P, S, reinterpret_cast<const unsigned short*>(x.data_ptr()), sorted_pairs.data_ptr<int>(),        \
-        tile_expert.data_ptr<int>(), reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim,       \
-        (int)k_per_tok, (int)n_tiles, (int)experts, (int)groups);                                            \
+  const int lds = 2 * (MOE_BM + MOE_BN) * MOE_BK * 2;
+#define MOE_GEMM(NF4, W, P, S)                                                                                   \
+  do {                                                                                                           \
+    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_kernel<NF4>),            \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);                \
+    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                      \
+    moe_gemm_kernel<NF4><<<blocks, 512, lds, stream>>>(                                                          \
+        W, P, S, reinterpret_cast<const unsigned short*>(x.data_ptr()), sorted_pairs.data_ptr<int>(),            \
+        tile_expert.data_ptr<int>(), reinterpret_cast<unsigned short*>(c.data_ptr()), in_dim, out_dim,           \
+        (int)k_per_tok, (int)n_tiles, (int)experts, (int)columns);                                               \
   } while (0)
-  if (nf4) {
+  if (nf4)
     MOE_GEMM(true, nullptr, reinterpret_cast<const uint4*>(nf4_all->data_ptr()),
              reinterpret_cast<const unsigned short*>(scales_all->data_ptr()));
-  } else {
+  else
     MOE_GEMM(false, reinterpret_cast<const unsigned short*>(wt_all->data_ptr()), nullptr, nullptr);
-  }
 #undef MOE_GEMM
   HIP_CHECK_LAST();
   return c;

@@ -40,6 +40,7 @@ def test_swiglu_writes_every_value(hip, n):
         ([300, 0, 1, 256], 64, 640),  # several groups of one expert
         ([3] * 70, 64, 128),  # more tiles than lanes of a wave
         ([2050, 40], 64, 128),  # a run of one expert longer than a wave's lanes
+        ([1100, 40], 192, 2304),  # more groups than share a run of columns, several runs
     ],
 )
 def test_expert_gemm_group_edges(hip, quant, counts, k_in, n_out):
