@@ -32,6 +32,15 @@ torch::Tensor attn_prefill_fused(
     torch::Tensor q, torch::Tensor k, torch::Tensor v,
     int64_t kv_len, int64_t kv_offset, double scale, bool causal,
     c10::optional<torch::Tensor> alibi_slopes);
+std::vector<torch::Tensor> attn_prefill_sums(torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale);
+torch::Tensor attn_prompt_grad(
+    torch::Tensor qkv, torch::Tensor out, torch::Tensor grad_out, torch::Tensor lse, torch::Tensor cos_t,
+    torch::Tensor sin_t, int64_t start, int64_t qh, int64_t kh, int64_t hd, double scale);
+torch::Tensor rotate_rows(
+    torch::Tensor qkv, torch::Tensor cos_t, torch::Tensor sin_t, int64_t start, int64_t qh, int64_t kh, int64_t hd);
+torch::Tensor norm_rows_grad(
+    torch::Tensor x, torch::Tensor w, torch::Tensor g, c10::optional<torch::Tensor> residual, double eps);
+torch::Tensor swiglu_rows_grad(torch::Tensor gu, torch::Tensor g);
 torch::Tensor attn_prefill_rows(
     torch::Tensor q, torch::Tensor k, torch::Tensor v, int64_t kv_len, int64_t kv_offset, double scale, bool causal,
     c10::optional<torch::Tensor> alibi_slopes);
@@ -120,6 +129,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0);
   m.def("attn_prefill_rows", &attn_prefill_rows, "prompt attention on strided heads; results as rows of tokens");
+  m.def("attn_prefill_sums", &attn_prefill_sums, "causal prompt attention with log2 of its rows' sums of weights");
+  m.def("attn_prompt_grad", &attn_prompt_grad, "gradient of a fused projection through rotation and causal attention");
+  m.def("rotate_rows", &rotate_rows, "fused projection with queries and keys rotated");
+  m.def("norm_rows_grad", &norm_rows_grad, "gradient of an RMS norm's rows (+ residual)");
+  m.def("swiglu_rows_grad", &swiglu_rows_grad, "gradient of [gate | up] rows");
   m.def("qkv_rows", &qkv_rows, "fused projection of a prompt -> rotated queries in place, keys and values to the cache");
   m.def("add_norm_rows", &add_norm_rows, "(x + y + bias, its RMS or layer norm)",
         py::arg("x"), py::arg("y"), py::arg("y_bias"), py::arg("w"), py::arg("b"), py::arg("eps"));

@@ -45,6 +45,7 @@ struct Rows4 {
 template <int HD, int QB>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     Rows4 q, Rows4 k, Rows4 v, unsigned short* __restrict__ out, long out_batch, long out_head, long out_row,
+    float* __restrict__ lse,  // [B, QH, S]: log2 of each row's sum of weights, or null
     AttnShape a, int runs, int sequences, int s_q, int kv_len, int kv_offset, bool causal) {
   constexpr int KT = PF_KEYS, NB = KT / 16, RC = HD / 32, VB = HD / 16;
   constexpr int ROW = HD + TPAD;        // of keys and of values in LDS
@@ -164,6 +165,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     const int row = r0 + i * 16 + col;
     const float sum = row_sum(l[i]), inv = sum > 0.f ? 1.f / sum : 0.f;
     if (row >= s_q) continue;
+    if (lse && hi == 0) lse[(size_t)own.y * s_q + row] = m[i] + log2f(sum);
     unsigned short* dst = out + b * out_batch + head * out_head + row * out_row + hi * 4;
 #pragma unroll
     for (int d = 0; d < VB; ++d)
@@ -187,7 +189,7 @@ static Rows4 rows4(const torch::Tensor& t) {
 // q [B, QH, S, HD], k and v [B, KVH, Lmax, HD] of any strides; out likewise, rows aligned to 8 bytes
 static void run_prefill(
     torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor out, int64_t kv_len, int64_t kv_offset, double scale,
-    bool causal, const c10::optional<torch::Tensor>& alibi_slopes) {
+    bool causal, const c10::optional<torch::Tensor>& alibi_slopes, float* lse = nullptr) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16 && q.dim() == 4);
   TORCH_CHECK(k.dtype() == torch::kBFloat16 && k.dim() == 4 && v.dtype() == torch::kBFloat16 && v.dim() == 4);
   const int B = q.size(0), QH = q.size(1), S = q.size(2), HD = q.size(3);
@@ -221,7 +223,7 @@ static void run_prefill(
     allow_lds(&attn_prefill_kernel<HDV, QB>, lds);                                                                    \
     attn_prefill_kernel<HDV, QB><<<runs * sequences, 256, lds, stream>>>(                                                         \
         rows4(q), rows4(k), rows4(v), reinterpret_cast<unsigned short*>(out.data_ptr()), out.stride(0), out.stride(1), \
-        out.stride(2), a, (int)runs, (int)sequences, S, (int)kv_len, (int)kv_offset, causal);                         \
+        out.stride(2), lse, a, (int)runs, (int)sequences, S, (int)kv_len, (int)kv_offset, causal);                         \
   } while (0)
   if (HD == 128) {
     if (wide) PREFILL(128, 2);
@@ -258,4 +260,14 @@ torch::Tensor attn_prefill_rows(
   run_prefill(q, k, v, out.view({q.size(0), q.size(2), q.size(1), q.size(3)}).transpose(1, 2), kv_len, kv_offset, scale,
               causal, alibi_slopes);
   return out;
+}
+
+// what training keeps: a prompt's causal attention over itself, and [B, QH, S] log2 of the sums of its rows' weights
+std::vector<torch::Tensor> attn_prefill_sums(torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale) {
+  TORCH_CHECK(q.dim() == 4);
+  auto out = torch::empty({q.size(0), q.size(2), q.size(1) * q.size(3)}, q.options());
+  auto lse = torch::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(torch::kFloat32));
+  run_prefill(q, k, v, out.view({q.size(0), q.size(2), q.size(1), q.size(3)}).transpose(1, 2), q.size(2), 0, scale, true,
+              c10::nullopt, lse.data_ptr<float>());
+  return {out, lse};
 }

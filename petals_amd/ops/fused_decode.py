@@ -26,7 +26,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
-from petals_amd.ops import reference
+from petals_amd.ops import prompt_grad, reference
 
 _EPI_RAW = -1  # return split partials; caller fuses its own reduce+epilogue
 _EPI_PLAIN_F32 = 0
@@ -458,7 +458,9 @@ class LlamaFastPath(_TPFastPathMixin):
                 gate = gate + dg
             if du is not None:
                 up = up + du
-        if autograd:
+        if autograd and adapter is None and inter % 8 == 0 and prompt_grad.fused_training(gateup):
+            act = prompt_grad.swiglu(gateup, self.hip)
+        elif autograd:
             act = reference.swiglu(gate, up).to(xn2.dtype)
         elif adapter is None and inter % 8 == 0 and gateup.dtype == torch.bfloat16:
             act = self.hip.swiglu_rows(gateup)
@@ -623,32 +625,36 @@ class LlamaFastPath(_TPFastPathMixin):
                 qkv[:, lo:hi] += d.float()
 
     def forward_autograd(self, hidden: torch.Tensor, prefix_length: int = 0, adapter=None) -> torch.Tensor:
-        """Differentiable forward on the transposed weights (torch primitives
-        only — the HIP kernels are inference-only). Used by rpc_backward on GPU
+        """Differentiable forward on the transposed weights. Used by rpc_backward on GPU
         servers; weights are frozen, grads flow to inputs/prompts."""
         B, S, H = hidden.shape
         end = prefix_length + S
         self._ensure_rope(end)
-        xn = reference.rms_norm(hidden, self.ln1_w_post, self.eps)
+        fused = _rows_fit(H) and prompt_grad.fused_training(hidden)
+        if fused:
+            xn = prompt_grad.norm(hidden, self.ln1_w_post, self.eps, self.hip)
+        else:
+            xn = reference.rms_norm(hidden, self.ln1_w_post, self.eps)
         xn = self._tp_copy(xn)  # backward: all-reduce the shard-partial grads
         qkv = torch.matmul(xn, self.wqkv_t.dense())
         if adapter is not None:
             xd = reference.rms_norm(hidden, self.ln1_w, self.eps) if self.fold_norm else xn
             qkv = qkv + self._qkv_adapter_delta(xd, adapter)
-        q = qkv[..., : self.qh * self.hd].view(B, S, self.qh, self.hd).transpose(1, 2)
-        k = qkv[..., self.qh * self.hd : (self.qh + self.kh) * self.hd].view(B, S, self.kh, self.hd).transpose(1, 2)
-        v = qkv[..., (self.qh + self.kh) * self.hd :].view(B, S, self.kh, self.hd).transpose(1, 2)
-        pos = torch.arange(prefix_length, end, device=hidden.device)
-        q, k = reference.apply_rope(q, k, self.rope_cos, self.rope_sin, pos)
-        attn = reference.attention(q, k, v, causal=True)
-        attn = attn.transpose(1, 2).reshape(B, S, self.qh * self.hd).to(hidden.dtype)
+        shape = (prefix_length, self.qh, self.kh, self.hd)
+        if fused and qkv.dtype == torch.bfloat16 and self.hd in (64, 128):
+            attn = prompt_grad.attention(qkv, self.rope_cos, self.rope_sin, *shape, self.scale, self.hip)
+        else:
+            attn = prompt_grad.torch_attention(qkv, self.rope_cos, self.rope_sin, *shape).to(hidden.dtype)
         o = self._tp_reduce(torch.matmul(attn, self.wo_t.dense()))
         if adapter is not None:
             d = adapter.delta("o", attn)
             if d is not None:
                 o = o + d
-        h2 = hidden + o
-        xn2 = reference.rms_norm(h2, self.ln2_w_post, self.eps)
+        if fused and o.dtype == torch.bfloat16:
+            h2, xn2 = prompt_grad.add_norm(hidden, o, self.ln2_w_post, self.eps, self.hip)
+        else:
+            h2 = hidden + o
+            xn2 = reference.rms_norm(h2, self.ln2_w_post, self.eps)
         xd2 = reference.rms_norm(h2, self.ln2_w, self.eps) if (self.fold_norm and adapter is not None) else None
         return h2 + self._tp_reduce(self._mlp_dense(xn2, adapter, autograd=True, x_delta=xd2)).to(h2.dtype)
 

@@ -1,0 +1,147 @@
+"""Differentiable pieces of a prompt's pass: what stands between its dense products, by
+the HIP kernels in either direction (csrc/prefill_rows.hip, csrc/attn_grad.hip).
+
+As torch operations, a llama block's forward and backward was 133 launches besides its
+products, 1.1 of its 2.0 ms at 2 x 379 tokens, width 4096; now it is 11, 0.15 ms. Kept for the backward: rows, and
+one number per attention row, where torch kept several [heads, rows, rows] matrices.
+
+Ordinary reverse mode only (`fused_training`); what traces or transforms torch operations
+sees those of `ops.reference`. Gradients of gradients are taken through them, too.
+"""
+
+from __future__ import annotations
+
+import torch
+from torch.autograd import forward_ad
+
+from petals_amd.ops import reference
+
+
+def fused_training(*rows: torch.Tensor) -> bool:
+    """Whether these bf16 rows go through the kernels."""
+    return (
+        all(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0 for t in rows)
+        and getattr(forward_ad, "_current_level", -1) < 0
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and not torch.jit.is_tracing()
+        and not torch.compiler.is_compiling()
+    )
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous rows that 16-byte loads can read."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
+def _through_torch(function, inputs, grads):
+    """Gradients that have gradients themselves (create_graph)."""
+    with torch.enable_grad():
+        outputs = function(*inputs)
+        outputs = outputs if isinstance(outputs, tuple) else (outputs,)
+        kept = [(o, g) for o, g in zip(outputs, grads) if g is not None]
+        return torch.autograd.grad([o for o, _ in kept], inputs, [g for _, g in kept], create_graph=True, allow_unused=True)
+
+
+class _Norm(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w, eps, hip):
+        ctx.save_for_backward(x)
+        ctx.w, ctx.eps, ctx.hip = w, eps, hip
+        return hip.rms_norm(_aligned(x), w, eps)
+
+    @staticmethod
+    def backward(ctx, g):
+        (x,), w = ctx.saved_tensors, ctx.w
+        if torch.is_grad_enabled():
+            return (*_through_torch(lambda t: reference.rms_norm(t, w, ctx.eps), (x,), (g,)), None, None, None)
+        return ctx.hip.norm_rows_grad(_aligned(x), w, _aligned(g), None, ctx.eps), None, None, None
+
+
+class _AddNorm(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, y, w, eps, hip):
+        h, n = hip.add_norm_rows(_aligned(x), _aligned(y), None, w, None, eps)
+        ctx.save_for_backward(x, y, h)
+        ctx.set_materialize_grads(False)
+        ctx.w, ctx.eps, ctx.hip = w, eps, hip
+        return h, n
+
+    @staticmethod
+    def backward(ctx, gh, gn):
+        (x, y, h), w = ctx.saved_tensors, ctx.w
+        if gh is None and gn is None:
+            return None, None, None, None, None
+        if torch.is_grad_enabled():
+
+            def composed(a, b):
+                s = a + b
+                return s, reference.rms_norm(s, w, ctx.eps)
+
+            return (*_through_torch(composed, (x, y), (gh, gn)), None, None, None)
+        if gn is not None:
+            gh = ctx.hip.norm_rows_grad(_aligned(h), w, _aligned(gn), None if gh is None else _aligned(gh), ctx.eps)
+        return gh, gh, None, None, None
+
+
+class _SwiGLU(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, gateup, hip):
+        ctx.save_for_backward(gateup)
+        ctx.hip = hip
+        return hip.swiglu_rows(_aligned(gateup))
+
+    @staticmethod
+    def backward(ctx, g):
+        (gateup,) = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*_through_torch(lambda t: reference.swiglu(*t.chunk(2, dim=-1)), (gateup,), (g,)), None)
+        return ctx.hip.swiglu_rows_grad(_aligned(gateup), _aligned(g)), None
+
+
+def torch_attention(qkv, cos, sin, start, qh, kh, hd):
+    """Causal attention of a fused projection [B, S, (qh + 2 kh) * hd], by torch operations."""
+    B, S, _ = qkv.shape
+    heads = qkv.view(B, S, qh + 2 * kh, hd).transpose(1, 2)
+    pos = torch.arange(start, start + S, device=qkv.device)
+    q, k = reference.apply_rope(heads[:, :qh], heads[:, qh : qh + kh], cos, sin, pos)
+    attn = reference.attention(q, k, heads[:, qh + kh :], causal=True)
+    return attn.transpose(1, 2).reshape(B, S, qh * hd)
+
+
+class _Attention(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, qkv, cos, sin, start, qh, kh, hd, scale, hip):
+        rows = hip.rotate_rows(_aligned(qkv), cos, sin, start, qh, kh, hd)
+        heads = rows.view(*rows.shape[:2], qh + 2 * kh, hd).transpose(1, 2)
+        out, sums = hip.attn_prefill_sums(heads[:, :qh], heads[:, qh : qh + kh], heads[:, qh + kh :], scale)
+        ctx.save_for_backward(qkv, rows, out, sums)
+        ctx.tables = cos, sin  # constants, maybe made in inference mode: such tensors can't be saved
+        ctx.shape, ctx.scale, ctx.hip = (start, qh, kh, hd), scale, hip
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        (qkv, rows, out, sums), (cos, sin) = ctx.saved_tensors, ctx.tables
+        none = (None,) * 8
+        if torch.is_grad_enabled():
+            return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
+        return (ctx.hip.attn_prompt_grad(rows, out, _aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
+
+
+def norm(x, w, eps, hip):
+    return _Norm.apply(x, w, eps, hip)
+
+
+def add_norm(x, y, w, eps, hip):
+    """(x + y, its RMS norm)"""
+    return _AddNorm.apply(x, y, w, eps, hip)
+
+
+def swiglu(gateup, hip):
+    """[..., gate | up] -> silu(gate) * up"""
+    return _SwiGLU.apply(gateup, hip)
+
+
+def attention(qkv, cos, sin, start, qh, kh, hd, scale, hip):
+    return _Attention.apply(qkv, cos, sin, start, qh, kh, hd, scale, hip)

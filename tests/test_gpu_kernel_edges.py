@@ -356,3 +356,145 @@ def test_expert_sums(hip, tokens, top, splits, width):
     check(hip.moe_combine(parts, weights, residual), parts.double().sum(0))
     rows = parts[0].to(BF16)
     check(hip.moe_combine(rows, weights, residual), rows.double())
+
+
+# ------------------------------------------------- gradients of a prompt's rows
+
+
+def _bf16_leaf(gen, *shape, scale=1.0):
+    return (torch.randn(*shape, device="cuda", generator=gen) * scale).to(BF16).requires_grad_(True)
+
+
+def _gradients(outputs, inputs, grads, **kw):
+    return torch.autograd.grad(outputs, inputs, grads, **kw)
+
+
+@requires_gpu
+@pytest.mark.parametrize("rows,dim", [(1, 8), (3, 2048), (5, 2056), (7, 16384)])
+def test_norm_gradients(hip, rows, dim):
+    from petals_amd.ops import prompt_grad
+
+    gen = torch.Generator(device="cuda").manual_seed(dim)
+    x, y = _bf16_leaf(gen, rows, dim), _bf16_leaf(gen, rows, dim)
+    w = torch.randn(dim, device="cuda", generator=gen).to(BF16)
+    gh, gn = (torch.randn(rows, dim, device="cuda", generator=gen).to(BF16) for _ in range(2))
+    h, n = prompt_grad.add_norm(x, y, w, 1e-5, hip)
+    got = _gradients([h, n], [x, y], [gh, gn])
+    s = h.detach().double().requires_grad_(True)
+    normed = s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    (want,) = _gradients([s, normed], [s], [gh.double(), gn.double()])
+    # one rounding to bf16 of a sum in 32 bits; terms of the sum may cancel
+    inv = torch.rsqrt(s.detach().pow(2).mean(-1, keepdim=True) + 1e-5)
+    terms = gh.double().abs() + inv * (gn.double() * w.double()).abs() * 2 + want.abs()
+    for t in got:
+        assert bool(((t.double() - want).abs() <= 2.0**-8 * want.abs() + 2.0**-18 * (terms + terms.mean(-1, keepdim=True))).all())
+    only = _gradients([prompt_grad.norm(x, w, 1e-5, hip)], [x], [gn])[0]
+    z = x.detach().double().requires_grad_(True)
+    (want,) = _gradients([z * torch.rsqrt(z.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()], [z], [gn.double()])
+    inv = torch.rsqrt(z.detach().pow(2).mean(-1, keepdim=True) + 1e-5)
+    terms = inv * (gn.double() * w.double()).abs() * 2 + want.abs()
+    assert bool(((only.double() - want).abs() <= 2.0**-8 * want.abs() + 2.0**-18 * (terms + terms.mean(-1, keepdim=True))).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("rows,inner", [(1, 8), (3, 72), (130, 2048)])
+def test_swiglu_gradients(hip, rows, inner):
+    from petals_amd.ops import prompt_grad
+
+    gen = torch.Generator(device="cuda").manual_seed(inner)
+    gu = _bf16_leaf(gen, rows, 2 * inner, scale=3.0)
+    g = torch.randn(rows, inner, device="cuda", generator=gen).to(BF16)
+    (got,) = _gradients([prompt_grad.swiglu(gu, hip)], [gu], [g])
+    z = gu.detach().double().requires_grad_(True)
+    (want,) = _gradients([torch.nn.functional.silu(z[:, :inner]) * z[:, inner:]], [z], [g.double()])
+    # a rounding to bf16; 1 + a (1 - gate) may cancel, with terms up to |a|
+    size = (g.double() * gu.detach().double()[:, inner:]).abs() * (1 + gu.detach().double()[:, :inner].abs())
+    slack = torch.cat([size, (g.double() * gu.detach().double()[:, :inner]).abs()], dim=-1)
+    assert bool(((got.double() - want).abs() <= 2.0**-8 * want.abs() + 2.0**-20 * slack).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize(
+    "b,s,qh,kh,start",
+    [
+        (1, 1, 1, 1, 0),  # a row that sees itself
+        (2, 63, 2, 2, 0),  # a tile, not filled
+        (1, 65, 4, 1, 3),  # one row more than a tile; heads that share keys
+        (3, 128, 6, 2, 0),
+        (1, 200, 8, 8, 11),  # several tiles; heads a multiple of the chiplets
+    ],
+)
+def test_prompt_attention_gradients(hip, hd, b, s, qh, kh, start):
+    from petals_amd.ops import prompt_grad, reference
+
+    gen = torch.Generator(device="cuda").manual_seed(s + hd)
+    cos, sin = (t.to("cuda") for t in reference.build_rope_cache(hd, start + s + 2))
+    qkv = _bf16_leaf(gen, b, s, (qh + 2 * kh) * hd)
+    g = torch.randn(b, s, qh * hd, device="cuda", generator=gen).to(BF16)
+    out = prompt_grad.attention(qkv, cos, sin, start, qh, kh, hd, hd**-0.5, hip)
+    (got,) = _gradients([out], [qkv], [g])
+
+    z = qkv.detach().cpu().double().requires_grad_(True)
+    want_out = prompt_grad.torch_attention(z.float(), cos.cpu(), sin.cpu(), start, qh, kh, hd)
+    heads = z.view(b, s, qh + 2 * kh, hd).transpose(1, 2)
+    c, n = (t.cpu().double()[start : start + s] for t in (cos, sin))
+
+    def turn(t):
+        return t * c + torch.cat([-t[..., hd // 2 :], t[..., : hd // 2]], -1) * n
+
+    q, k, v = turn(heads[:, :qh]), turn(heads[:, qh : qh + kh]), heads[:, qh + kh :]
+    k, v = (t.repeat_interleave(qh // kh, 1) for t in (k, v))
+    scores = (q @ k.transpose(-1, -2) * hd**-0.5).masked_fill(torch.ones(s, s).triu(1).bool(), float("-inf"))
+    exact = (torch.softmax(scores, -1) @ v).transpose(1, 2).reshape(b, s, qh * hd)
+    (want,) = _gradients([exact], [z], [g.cpu().double()])
+    assert bool((want_out.double() - exact).abs().max() < 1e-3)  # the composition is the same function
+    # Turned queries and keys are rounded to bf16, 2^-9 each: scores off by delta at most, weights
+    # by a factor of exp(2 delta). Results, weights and rows enter products rounded, four times at
+    # most. Errors of a sum are bounded by its terms' sizes, of which turning back adds two.
+    with torch.no_grad():
+        go = g.cpu().double().view(b, s, qh, hd).transpose(1, 2)
+        delta = hd**-0.5 * (q.abs() @ k.abs().transpose(-1, -2)).max() * 2.0**-8
+        share = torch.expm1(2 * delta) + 2.0**-7
+        weights = torch.softmax(scores, -1)
+        dots = (go.abs() * (weights @ v).abs()).sum(-1, keepdim=True)
+        ds = weights * ((go @ v.transpose(-1, -2)).abs() + dots) * hd**-0.5
+        parts = [ds @ k.abs(), ds.transpose(-1, -2) @ q.abs(), weights.transpose(-1, -2) @ go.abs()]
+        parts[:2] = [t + t.roll(hd // 2, -1) for t in parts[:2]]
+        parts[1:] = [t.view(b, kh, qh // kh, s, hd).sum(2) for t in parts[1:]]
+        terms = torch.cat(parts, 1)
+    err = (got.cpu().double() - want).view(b, s, -1, hd).transpose(1, 2)
+    assert bool((err.abs() <= share * terms).all())
+    assert bool(err.norm() <= 2.0**-7 * want.norm())  # and roundings don't all add up
+
+
+@requires_gpu
+def test_prompt_gradients_have_gradients(hip):
+    from petals_amd.ops import prompt_grad, reference
+
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    cos, sin = (t.to("cuda") for t in reference.build_rope_cache(64, 8))
+    w = torch.ones(64, device="cuda", dtype=BF16)
+    for function, width in [
+        (lambda t: prompt_grad.norm(t, w, 1e-5, hip), 64),
+        (lambda t: prompt_grad.add_norm(t, t, w, 1e-5, hip)[1], 64),
+        (lambda t: prompt_grad.swiglu(t, hip), 64),
+        (lambda t: prompt_grad.attention(t, cos, sin, 0, 1, 1, 64, 0.125, hip), 192),
+    ]:
+        x = _bf16_leaf(gen, 2, 5, width)
+        (g,) = _gradients([function(x).float().square().sum()], [x], [None], create_graph=True)
+        (gg,) = _gradients([g.float().square().sum()], [x], [None])
+        assert bool(torch.isfinite(gg).all()) and float(gg.float().abs().sum()) > 0
+
+
+@requires_gpu
+def test_prompt_gradients_by_transforms(hip):
+    from petals_amd.ops import prompt_grad
+
+    x = torch.randn(2, 64, device="cuda").to(BF16)
+    assert prompt_grad.fused_training(x)
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(prompt_grad.fused_training(t)), t)[1])(x)
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(prompt_grad.fused_training(x))
+    assert seen == [False, False]
