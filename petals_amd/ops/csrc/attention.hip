@@ -1,14 +1,24 @@
 // GQA decode attention for CDNA4 (gfx950), flash-decoding style.
 //
-// Default path (mfma_decode_kernel): the GQ query heads of one kv head form
-// the rows of an mfma_f32_16x16x32_bf16 A-fragment (padded to 16), so 32
-// cache keys cost 4 QK MFMAs + 8 PV MFMAs per wave instead of 32*GQ
-// shuffle-reduced dot products. K is consumed directly from global as
-// B-fragments (16 B/lane); V goes through the XOR-swizzled LDS transpose
-// (same as the prefill kernel); 4 waves take interleaved 32-key tiles of the
-// workgroup's split range and combine through LDS; attn_decode_combine merges
-// splits. Measured (scripts/decode_mfma.hip, llama-2-70b shape): 1039 GB/s at
-// kv=4k -> 3509 GB/s at kv=131k, 2.2-2.4x the VALU kernel at every length.
+// Default path (mfma_decode_kernel): scores as K Q^T and results as V^T P^T, the GQ query
+// heads of one kv head (16 at a time) being the columns of both products, as in paged_attn.h:
+// a lane has one head, its maximum takes two exchanges between lanes, and its weights are
+// the second product's operand as they are. No tile passes through LDS: keys are read as
+// operands, and of values a lane reads 8 (HD 64: 4) dims of the 8 keys whose weights it has
+// and transposes them by byte permutes. Four waves take every fourth tile of 32 keys of
+// their workgroup's part, with the next tile's loads in flight, and meet in LDS at the end;
+// attn_decode_combine merges the parts.
+//
+// Bound by memory for long contexts, by two trips to it for short ones. MI355X, us with the
+// combination, before (values through LDS, transposed one by one; every load waited for;
+// weights through LDS) and now:
+//   kv heads x queries each, head size, keys: 8 x 8, 128, 154           12.9 ->  6.2
+//   8 x 8, 128, 2004                                                    18.8 -> 11.3
+//   64 x 8, 128, 2004                                                   41.4 -> 20.6   3.2 TB/s
+//   16 x 4, 128, 7901                                                   44.0 -> 22.4   2.9 TB/s
+//   8 x 4, 128, 32000                                                   73.3 -> 37.9   3.5 TB/s
+//   256 x 1, 128, 1000                                                  44.6 -> 27.1   4.8 TB/s
+//   1 x 71, 64, 1000 (in cache)                                         39.8 -> 20.3
 //
 // The original VALU kernel (attn_decode_kernel: 16-lane-group dot products,
 // online softmax in registers) is kept behind PETALS_DECODE_KERNEL=valu.
@@ -19,20 +29,14 @@
 // (reference models/llama/block.py:108-127) on the MI355X fast path.
 
 #include "common.h"
+#include "paged_attn.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 
 #include <cstdlib>
 
-using bf16x8 = __attribute__((ext_vector_type(8))) short;
-using f32x4 = __attribute__((ext_vector_type(4))) float;
-
 #define DKVT 32    // keys per wave-tile (MFMA path)
 #define DWAVES 4   // waves per workgroup (MFMA path)
-#define DKPAD 8
-
-#define DVT_BYTE(dim, key_byte) \
-  ((((unsigned)(dim)) * ((DKVT + DKPAD) * 2) + (unsigned)(key_byte)) ^ ((((unsigned)(dim) >> 3) & 7u) << 4))
 
 // Arbitrary GQ: heads are processed in ceil(GQ/16) groups of <=16 (one
 // A-fragment each). The group loop sits OUTSIDE the kv loop so live registers
@@ -41,7 +45,7 @@ using f32x4 = __attribute__((ext_vector_type(4))) float;
 // GQ > 16 (falcon-7b MQA gq=71, falcon-180b gq=29 — reference
 // models/falcon/block.py:100-110).
 template <int HD, int GQ>
-__global__ __launch_bounds__(DWAVES * 64) void mfma_decode_kernel(
+__global__ __launch_bounds__(DWAVES * 64, GQ > 16 ? 1 : 2) void mfma_decode_kernel(
     const float* __restrict__ q,            // [B, KV, GQ, HD]
     const unsigned short* __restrict__ k_cache,  // [B, KV, lmax, HD]
     const unsigned short* __restrict__ v_cache,
@@ -55,201 +59,176 @@ __global__ __launch_bounds__(DWAVES * 64) void mfma_decode_kernel(
     float scale,
     float* __restrict__ out_direct) {  // n_splits==1: normalized out [B, KV*GQ*HD]
                                        // written here; the combine kernel is skipped
+  constexpr int KC = HD / 32;
+  constexpr int NV = HD / 16;                  // dims of a lane's values
+  constexpr int GA = (GQ + 15) / 16;           // head groups of <=16
+  constexpr int GN = GQ < 16 ? GQ : 16;
+  constexpr int OROW = HD + 4;
+  using values = __attribute__((ext_vector_type(NV / 2))) unsigned;
+  using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
+  __shared__ float c_o[DWAVES][GN][OROW];
+  __shared__ float c_ml[DWAVES][16][2];
+
   const int bkv = blockIdx.x;
   const int kvh = bkv % kv_heads;
   const int split = blockIdx.y;
   const int kv_len = *kv_len_ptr;
-
   const int rows_per_split = (kv_len + n_splits - 1) / n_splits;
   const int j_begin = split * rows_per_split;
   const int j_end = min(j_begin + rows_per_split, kv_len);
 
-  const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
-  const int lane = tid & (WAVE - 1);
-  const int col = lane & 15;
-  const int hi = lane >> 4;
-
-  constexpr int KCH = HD / 32;
-  constexpr int GA = (GQ + 15) / 16;  // head groups of <=16
-
-  // per-wave LDS: swizzled V^T tile + P scratch; the cross-wave combine
-  // overlays the V^T storage after the main loop (one <=16-head group at a
-  // time, so the overlay always fits)
-  __shared__ unsigned char vt_raw[DWAVES][HD * (DKVT + DKPAD) * 2];
-  __shared__ unsigned short p_lds[DWAVES][16][DKVT + DKPAD];
-  __shared__ float c_ml[DWAVES][16][2];
-  static_assert(16 * HD * 4 <= HD * (DKVT + DKPAD) * 2, "combine O overlay too big");
-
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
+  const int col = lane & 15, hi = lane >> 4;
   const size_t kv_base = (size_t)bkv * lmax * HD;
-  const unsigned short* kb = k_cache + kv_base;
-  const unsigned short* vb = v_cache + kv_base;
-  const size_t q_base = (size_t)bkv * GQ * HD;
+  const unsigned short* kb = k_cache + kv_base + hi * 8;
+  const unsigned short* vb = v_cache + kv_base + col * NV;
+
+  struct Tile {
+    bf16x8 k[2][KC];  // keys col and 16 + col
+    values v[8];      // keys hi*4 to +3 and 16 + hi*4 to +3
+  };
+  auto fetch = [&](Tile& t, int j0) {  // rows beyond the end repeat the last
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const unsigned short* row = kb + (size_t)min(j0 + nb * 16 + col, j_end - 1) * HD;
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) t.k[nb][kc] = *reinterpret_cast<const bf16x8*>(row + kc * 32);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      t.v[e] = *reinterpret_cast<const values*>(vb + (size_t)min(j0 + (e / 4) * 16 + hi * 4 + e % 4, j_end - 1) * HD);
+  };
 
   for (int a = 0; a < GA; ++a) {
     const int g0 = a * 16;  // first head of this group
-    if (a > 0) __syncthreads();  // wave0's combine reads of vt_raw are done
-
-    // ---- q tile: A-fragment rows = q heads of this group (zero-padded), pre-scaled
-    bf16x8 q_frag[KCH];
+    bf16x8 qf[KC];
 #pragma unroll
-    for (int kc = 0; kc < KCH; ++kc) {
+    for (int kc = 0; kc < KC; ++kc) {
+      qf[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
       if (g0 + col < GQ) {
-        const float* src = q + q_base + (size_t)(g0 + col) * HD + kc * 32 + hi * 8;
-        short v[8];
+        const float* src = q + ((size_t)bkv * GQ + g0 + col) * HD + kc * 32 + hi * 8;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (short)f32_to_bf16(src[e] * scale);
-        q_frag[kc] = bf16x8{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-      } else {
-        q_frag[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        for (int e = 0; e < 8; ++e) qf[kc][e] = (short)f32_to_bf16(src[e] * scale);
+      }
+    }
+    const float slope = alibi && g0 + col < GQ ? alibi[kvh * GQ + g0 + col] : 0.f;
+
+    f32x4 acc[NV];  // [dim % NV][r]: dim (hi*4 + r) * NV + j of head g0 + col
+#pragma unroll
+    for (int j = 0; j < NV; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = NEG_SENTINEL, l = 0.f;  // l: this lane's share
+
+    auto weigh = [&](Tile& t, int j0) {
+      f32x4 s[2];
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        s[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) s[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t.k[nb][kc], qf[kc], s[nb], 0, 0, 0);
+      }
+      const int first = j0 + hi * 4;  // key of register 0 in block 0
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[nb][r] += slope * (first + nb * 16 + r);
+      // masking and the maximum stay in separate loops (see prefill_attn.hip)
+      if (j0 + DKVT > j_end) {
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (first + nb * 16 + r >= j_end) {
+              s[nb][r] = NEG_SENTINEL;
+              t.v[nb * 4 + r] = values{};
+            }
+      }
+      float mx = m;
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[nb][r]);
+      const float m_new = row_max(mx);
+      if (__any(m_new > m)) {
+        const float corr = m <= NEG_THRESHOLD ? 0.f : __expf(m - m_new);
+        l *= corr;
+        m = m_new;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[j] *= corr;
+      }
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[nb][r] = s[nb][r] <= NEG_THRESHOLD ? 0.f : __expf(s[nb][r] - m);
+          l += s[nb][r];
+        }
+      const bf16x8 p = weight_operand(s[0], s[1]);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        u32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = __builtin_amdgcn_perm(t.v[2 * i + 1][j / 2], t.v[2 * i][j / 2], j & 1 ? 0x07060302u : 0x05040100u);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), p, acc[j], 0, 0, 0);
+      }
+    };
+
+    constexpr int STEP = DWAVES * DKVT;
+    int j0 = j_begin + wave * DKVT;
+    if (j0 < j_end) {  // uniform over the wave
+      Tile one, two;
+      fetch(one, j0);
+      for (;; j0 += 2 * STEP) {
+        fetch(two, j0 + STEP);
+        weigh(one, j0);
+        if (j0 + STEP >= j_end) break;
+        fetch(one, j0 + 2 * STEP);
+        weigh(two, j0 + STEP);
+        if (j0 + 2 * STEP >= j_end) break;
       }
     }
 
-    // per-lane-row ALiBi slopes (rows = heads g0 + hi*4 + r)
-    float sl[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int g = g0 + hi * 4 + r;
-      sl[r] = (alibi && g < GQ) ? alibi[kvh * GQ + g] : 0.f;
-    }
-
-    f32x4 acc_o[HD / 16];
-#pragma unroll
-    for (int d = 0; d < HD / 16; ++d) acc_o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_row[4], l_row[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      m_row[r] = NEG_SENTINEL;
-      l_row[r] = 0.f;
-    }
-
-    // wave w handles tiles j_begin + (t*DWAVES + w)*DKVT
-    for (int j0 = j_begin + wave * DKVT; j0 < j_end; j0 += DWAVES * DKVT) {
-      const int tile_n = min(DKVT, j_end - j0);
-      const bool full = tile_n == DKVT;
-
-      // ---- stage V^T (this wave only: no block barrier; the waitcnt orders
-      // this wave's LDS writes before its reads)
-      for (int idx = lane; idx < DKVT * (HD / 8); idx += WAVE) {
-        const int row = idx / (HD / 8);
-        const int c8 = (idx - row * (HD / 8)) * 8;
-        bf16x8 vv8 = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (j0 + row < j_end) vv8 = *reinterpret_cast<const bf16x8*>(vb + (size_t)(j0 + row) * HD + c8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          *reinterpret_cast<unsigned short*>(&vt_raw[wave][DVT_BYTE(c8 + e, row * 2)]) = (unsigned short)vv8[e];
-      }
-      __builtin_amdgcn_s_waitcnt(0);
-
-      // ---- S = Q K^T, K direct from global: B[k = kdim][n = key]
-      f32x4 s_acc[DKVT / 16];
-#pragma unroll
-      for (int nb = 0; nb < DKVT / 16; ++nb) {
-        s_acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const int key = j0 + nb * 16 + col;
-        const unsigned short* krow = kb + (size_t)min(key, j_end - 1) * HD + hi * 8;
-#pragma unroll
-        for (int kc = 0; kc < KCH; ++kc) {
-          const bf16x8 kt = *reinterpret_cast<const bf16x8*>(krow + kc * 32);
-          s_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q_frag[kc], kt, s_acc[nb], 0, 0, 0);
-        }
-      }
-
-      // ---- online softmax over this tile (rows = heads g0 + hi*4+r)
-      float p[DKVT / 16][4];
-      float corr[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float s[DKVT / 16];
-#pragma unroll
-        for (int nb = 0; nb < DKVT / 16; ++nb) {
-          const int key = j0 + nb * 16 + col;
-          s[nb] = s_acc[nb][r] + sl[r] * key;
-          if (!full && key >= j_end) s[nb] = NEG_SENTINEL;
-        }
-        float mx = NEG_SENTINEL;
-#pragma unroll
-        for (int nb = 0; nb < DKVT / 16; ++nb) mx = fmaxf(mx, s[nb]);
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, WAVE));
-        const float m_new = fmaxf(m_row[r], mx);
-        corr[r] = (m_row[r] <= NEG_THRESHOLD) ? 0.f : __expf(m_row[r] - m_new);
-        float lsum = 0.f;
-#pragma unroll
-        for (int nb = 0; nb < DKVT / 16; ++nb) {
-          p[nb][r] = (s[nb] <= NEG_THRESHOLD) ? 0.f : __expf(s[nb] - m_new);
-          lsum += p[nb][r];
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, WAVE);
-        l_row[r] = l_row[r] * corr[r] + lsum;
-        m_row[r] = m_new;
-      }
-
+    // ---- cross-wave combine for this head group
+    l = row_sum(l);
+    if (a > 0) __syncthreads();  // the last group's sums have been read
+    if (g0 + col < GQ) {
+      float* dst = &c_o[wave][col][hi * 4 * NV];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int nb = 0; nb < DKVT / 16; ++nb)
-          p_lds[wave][hi * 4 + r][nb * 16 + col] = f32_to_bf16(p[nb][r]);
-      __builtin_amdgcn_s_waitcnt(0);
-
-      const bf16x8 p_frag = *reinterpret_cast<const bf16x8*>(&p_lds[wave][col][hi * 8]);
-
-#pragma unroll
-      for (int d = 0; d < HD / 16; ++d)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc_o[d][r] *= corr[r];
-#pragma unroll
-      for (int d = 0; d < HD / 16; ++d) {
-        const bf16x8 vfrag = *reinterpret_cast<const bf16x8*>(&vt_raw[wave][DVT_BYTE(d * 16 + col, hi * 16)]);
-        acc_o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p_frag, vfrag, acc_o[d], 0, 0, 0);
-      }
-    }
-
-    // ---- cross-wave combine for this head group (overlay V^T LDS with O rows)
-    __syncthreads();
-    float* c_o = reinterpret_cast<float*>(vt_raw[wave]);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gl = hi * 4 + r;
-      if (g0 + gl < GQ) {
-#pragma unroll
-        for (int d = 0; d < HD / 16; ++d) c_o[gl * HD + d * 16 + col] = acc_o[d][r];
-        if (col == 0) {
-          c_ml[wave][gl][0] = m_row[r];
-          c_ml[wave][gl][1] = l_row[r];
-        }
+        for (int j = 0; j < NV; j += 4)
+          *reinterpret_cast<f32x4*>(dst + r * NV + j) = f32x4{acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r]};
+      if (hi == 0) {
+        c_ml[wave][col][0] = m;
+        c_ml[wave][col][1] = l;
       }
     }
     __syncthreads();
 
-    if (wave == 0) {
-      const int gn = min(16, GQ - g0);  // heads in this group
-      float* po = part_o + (((size_t)bkv * n_splits + split) * GQ + g0) * HD;
-      float* pml = part_ml + (((size_t)bkv * n_splits + split) * GQ + g0) * 2;
-      for (int idx = lane; idx < gn * HD; idx += WAVE) {
-        const int gl = idx / HD, d = idx - gl * HD;
-        float m_star = c_ml[0][gl][0];
+    const int gn = min(16, GQ - g0);  // heads in this group
+    float* po = part_o + (((size_t)bkv * n_splits + split) * GQ + g0) * HD;
+    float* pml = part_ml + (((size_t)bkv * n_splits + split) * GQ + g0) * 2;
+    for (int idx = tid; idx < gn * HD; idx += DWAVES * WAVE) {
+      const int gl = idx / HD, d = idx - gl * HD;
+      float m_star = c_ml[0][gl][0];
 #pragma unroll
-        for (int w = 1; w < DWAVES; ++w) m_star = fmaxf(m_star, c_ml[w][gl][0]);
-        float osum = 0.f, lsum = 0.f;
+      for (int w = 1; w < DWAVES; ++w) m_star = fmaxf(m_star, c_ml[w][gl][0]);
+      float osum = 0.f, lsum = 0.f;
 #pragma unroll
-        for (int w = 0; w < DWAVES; ++w) {
-          const float wgt = (c_ml[w][gl][0] <= NEG_THRESHOLD) ? 0.f : __expf(c_ml[w][gl][0] - m_star);
-          osum += wgt * reinterpret_cast<const float*>(vt_raw[w])[gl * HD + d];
-          lsum += wgt * c_ml[w][gl][1];
-        }
-        if (out_direct) {
-          // single split: normalize here (matches the combine kernel's
-          // n_splits==1 output exactly) and skip that kernel entirely —
-          // at short kv both kernels are pure launch latency
-          out_direct[((size_t)bkv * GQ + g0 + gl) * HD + d] = osum / fmaxf(lsum, 1e-20f);
-        } else {
-          po[idx] = osum;
-          if (d == 0) {
-            pml[gl * 2 + 0] = m_star;
-            pml[gl * 2 + 1] = lsum;
-          }
+      for (int w = 0; w < DWAVES; ++w) {
+        const float wgt = (c_ml[w][gl][0] <= NEG_THRESHOLD) ? 0.f : __expf(c_ml[w][gl][0] - m_star);
+        osum += wgt * c_o[w][gl][d];
+        lsum += wgt * c_ml[w][gl][1];
+      }
+      if (out_direct) {
+        // single split: normalize here (matches the combine kernel's
+        // n_splits==1 output exactly) and skip that kernel entirely
+        out_direct[((size_t)bkv * GQ + g0 + gl) * HD + d] = osum / fmaxf(lsum, 1e-20f);
+      } else {
+        po[idx] = osum;
+        if (d == 0) {
+          pml[gl * 2 + 0] = m_star;
+          pml[gl * 2 + 1] = lsum;
         }
       }
     }
@@ -394,28 +373,41 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(
   }
 }
 
+// One workgroup per (batch and kv head, query head), of hd threads. The parts' weights are
+// made once, then every thread's loads are independent.
+#define COMBINE_CHUNK 64
 __global__ void attn_decode_combine_kernel(
     const float* __restrict__ part_o,   // [B*KV, splits, GQ, HD]
     const float* __restrict__ part_ml,  // [B*KV, splits, GQ, 2]
     float* __restrict__ out,            // [B, KV*GQ*HD]
     int n_splits, int gq, int hd) {
+  __shared__ float weight[COMBINE_CHUNK];
   const int bkv = blockIdx.x;
   const int g = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+  const float* ml = part_ml + ((size_t)bkv * n_splits * gq + g) * 2;
+  const float* o = part_o + ((size_t)bkv * n_splits * gq + g) * hd;
   float m_star = NEG_SENTINEL;
-  for (int s = 0; s < n_splits; ++s)
-    m_star = fmaxf(m_star, part_ml[(((size_t)bkv * n_splits + s) * gq + g) * 2]);
-  for (int d = threadIdx.x; d < hd; d += blockDim.x) {
-    float osum = 0.f, lsum = 0.f;
-    for (int s = 0; s < n_splits; ++s) {
-      const float ms = part_ml[(((size_t)bkv * n_splits + s) * gq + g) * 2];
-      const float ls = part_ml[(((size_t)bkv * n_splits + s) * gq + g) * 2 + 1];
-      if (ms <= NEG_THRESHOLD) continue;
-      const float w = __expf(ms - m_star);
-      osum += w * part_o[(((size_t)bkv * n_splits + s) * gq + g) * hd + d];
-      lsum += w * ls;
+  for (int s = lane; s < n_splits; s += WAVE) m_star = fmaxf(m_star, ml[(size_t)s * gq * 2]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m_star = fmaxf(m_star, __shfl_xor(m_star, off, WAVE));
+  float osum = 0.f, lsum = 0.f;
+  for (int s0 = 0; s0 < n_splits; s0 += COMBINE_CHUNK) {
+    const int s = s0 + lane;
+    const float ms = s < n_splits ? ml[(size_t)s * gq * 2] : NEG_SENTINEL;
+    const float w = ms <= NEG_THRESHOLD ? 0.f : __expf(ms - m_star);
+    lsum += wave_reduce_sum(w != 0.f ? w * ml[(size_t)s * gq * 2 + 1] : 0.f);
+    if (s0 > 0) __syncthreads();  // the last chunk's weights have been read
+    if (tid < WAVE) weight[lane] = w;
+    __syncthreads();
+    const int n = min(COMBINE_CHUNK, n_splits - s0);
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) {
+      const float part = o[(size_t)(s0 + i) * gq * hd + tid];
+      osum += weight[i] == 0.f ? 0.f : weight[i] * part;
     }
-    out[(size_t)bkv * gq * hd + (size_t)g * hd + d] = osum / fmaxf(lsum, 1e-20f);
   }
+  out[((size_t)bkv * gq + g) * hd + tid] = osum / fmaxf(lsum, 1e-20f);
 }
 
 // ---------------------------------------------------------------- host API
@@ -449,22 +441,16 @@ torch::Tensor attn_decode_fused(
       // VALU kernel: target ~1024 single-wave workgroups, chunks >= 64 rows
       n_splits = std::max(1, std::min(1024 / bkv, (lmax + 63) / 64));
     } else {
-      // MFMA kernel: 4-wave workgroups; fill ~256 CUs (chunks >= 128 rows) and
-      // go up to 3 wgs/CU only when chunks stay >= 512 rows (measured knees,
-      // profiles/decode_longctx_sweep.log + scripts/decode_mfma.hip)
-      const int by_occ = std::min(768 / bkv, lmax / 512);
-      const int by_min = std::min(256 / bkv, (lmax + 127) / 128);
-      n_splits = std::max(1, std::max(by_occ, by_min));
-      // measured dead end (profiles/attn_direct_ab.log): forcing one split
-      // + in-kernel normalization (combine kernel skipped) at short caches
-      // LOST 1.4 tok/s end to end — halving the split occupancy costs more
-      // than the removed launch. Off by default; the env knob keeps the
-      // single-split direct-out path selectable for re-evaluation.
+      // One workgroup for each of the 256 compute units, parts of 128 rows or more: two or
+      // three per unit were slower (32000 keys of 8 heads: 16 parts 37.5 us, 32 parts 37.9,
+      // 62 parts 48.3; 256 heads: 1 part 27.1, 2 parts 30.6). Below 384 rows one part, as the
+      // second launch costs more than the longer chain (300 keys of 8 heads: 8.0 us, 8.6 with
+      // 4 parts; 500 of 32 heads: 9.7, 9.2).
       static const int short_max = [] {
         const char* e = std::getenv("PETALS_AMD_DECODE_SHORT_LMAX");
-        return e ? std::atoi(e) : 0;
+        return e ? std::atoi(e) : 384;
       }();
-      if (lmax <= short_max) n_splits = 1;
+      n_splits = lmax <= short_max ? 1 : std::max(1, std::min(256 / bkv, (lmax + 127) / 128));
     }
   }
   auto opts = q.options();

@@ -498,3 +498,42 @@ def test_prompt_gradients_by_transforms(hip):
     with torch.autograd.forward_ad.dual_level():
         seen.append(prompt_grad.fused_training(x))
     assert seen == [False, False]
+
+
+# ------------------------------------------------------ decode attention
+
+
+@requires_gpu
+@pytest.mark.parametrize("hd,gq,kv,alibi", [(128, 1, 3, True), (128, 8, 2, False), (64, 16, 1, True), (64, 71, 1, False), (128, 32, 1, False)])
+@pytest.mark.parametrize(
+    "kv_len,lmax",
+    [
+        (1, 64),
+        (31, 32),
+        (33, 200),  # a tile and one key more
+        (161, 384),  # one part, second round of the first wave
+        (3, 4096),  # parts without keys
+        (385, 385),  # parts that end within a tile
+        (4000, 8300),  # more parts than a wave has lanes, of few heads
+    ],
+)
+def test_decode_attention_edges(hip, hd, gq, kv, alibi, kv_len, lmax):
+    b = 2
+    gen = torch.Generator(device="cuda").manual_seed(kv_len + gq)
+    q = torch.randn(b, kv * gq * hd, device="cuda", generator=gen)
+    k, v = (torch.full((b, kv, lmax, hd), float("nan"), device="cuda", dtype=BF16) for _ in range(2))
+    for t in (k, v):  # nothing from kv_len on is used
+        t[:, :, :kv_len] = torch.randn(b, kv, kv_len, hd, device="cuda", generator=gen).to(BF16)
+    slopes = torch.rand(kv * gq, device="cuda", generator=gen) * 0.1 if alibi else None
+    empty = torch.empty(0, device="cuda")
+    length = torch.tensor([kv_len], dtype=torch.int32, device="cuda")
+    got = hip.attn_decode_fused(q, k, v, length, gq, 0, empty, empty, hd**-0.5, slopes).view(b, kv, gq, hd).double()
+    qd, kd, vd = q.view(b, kv, gq, hd).double(), k[:, :, :kv_len].double(), v[:, :, :kv_len].double()
+    scores = qd @ kd.transpose(-1, -2) * hd**-0.5
+    if alibi:
+        scores = scores + slopes.double().view(kv, gq, 1) * torch.arange(kv_len, device="cuda")
+    weights = torch.softmax(scores, -1)
+    # scaled queries are rounded to bf16 (2^-9 each), weights too (2^-9), scores with slopes to 24 bits
+    delta = (qd.abs() @ kd.abs().transpose(-1, -2) * hd**-0.5).max() * 2.0**-9 + scores.abs().max() * 2.0**-22
+    bound = (torch.expm1(2 * delta) + 2.0**-8) * (weights @ vd.abs())
+    assert bool(((got - weights @ vd).abs() <= bound).all())
