@@ -925,8 +925,14 @@ static void run_attention(const torch::Tensor& q, const torch::Tensor& cache, co
   dim3 grid(tiles.size(0), a.kv_heads * (decode ? 1 : row_groups), 1);
   int n_splits = (int)splits;
   if (n_splits <= 0) {
-    // enough workgroups for the chip; a decoding workgroup reads 4 tiles at once
-    const long tiles_per = decode ? 4 : 1, wanted = decode ? 512 : 256;
+    // Enough workgroups for the chip; a decoding workgroup reads 4 tiles at once. Two a compute
+    // unit, where registers hold two: keys and values of large heads don't leave them, and the
+    // second 256 only lengthen the sum. us with 512 and with 256 wanted: two maps of 128, values
+    // of 256, 16 heads, 8 x 2049 keys 70.5, 62.0; 4 x 2049 50.1, 40.6; 1 x 2049 23.5, 19.7;
+    // 8 x 300 23.2, 19.2; one of 256, 8 heads, 8 x 2049 41.0, 35.9; 2 x 2049 20.9, 18.2. Heads
+    // of 128, 8 x 2049 of 8: 22.9, 25.0; 1 x 2049: 10.6, 11.4.
+    const bool large = MAPS * a.dk > 128 && a.dv > 128;
+    const long tiles_per = decode ? 4 : 1, wanted = decode && !large ? 512 : 256;
     const long wgs = (long)grid.x * grid.y;
     n_splits = (int)std::max(
         1L, std::min({(long)((max_keys + KVT * tiles_per - 1) / (KVT * tiles_per)), wanted / std::max(1L, wgs), 64L}));
