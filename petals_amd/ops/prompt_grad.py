@@ -35,8 +35,10 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 
 
 def _through_torch(function, inputs, grads):
-    """Gradients that have gradients themselves (create_graph)."""
+    """Gradients that have gradients themselves (create_graph). They are taken at aliases of the
+    inputs: one input may depend on another, and that path is the caller's graph's to follow."""
     with torch.enable_grad():
+        inputs = tuple(t.view_as(t) for t in inputs)
         outputs = function(*inputs)
         outputs = outputs if isinstance(outputs, tuple) else (outputs,)
         kept = [(o, g) for o, g in zip(outputs, grads) if g is not None]

@@ -1,0 +1,112 @@
+"""Gradients of what stands between a prompt's products (ops/prompt_grad.py), without a GPU:
+the kernels are stood for by torch operations that autograd does not see."""
+
+import pytest
+import torch
+
+from petals_amd.ops import prompt_grad, reference
+
+QH, KH, HD, START = 2, 1, 8, 3
+COS, SIN = reference.build_rope_cache(HD, 16)
+
+
+class Kernels:
+    """The kernels' results on plain tensors; like them, it reads memory by its address."""
+
+    @staticmethod
+    def _plain(*tensors):
+        for t in tensors:
+            t.data_ptr()
+        return [t.detach().clone() for t in tensors]
+
+    def _pull(self, function, t, g):
+        t, g = self._plain(t, g)
+        with torch.enable_grad():
+            t.requires_grad_(True)
+            return torch.autograd.grad(function(t), t, g)[0]
+
+    def rms_norm(self, x, w, eps):
+        return reference.rms_norm(*self._plain(x), w, eps)
+
+    def add_norm_rows(self, x, y, y_bias, w, b, eps):
+        x, y = self._plain(x, y)
+        return x + y, reference.rms_norm(x + y, w, eps)
+
+    def norm_rows_grad(self, x, w, g, residual, eps):
+        d = self._pull(lambda t: reference.rms_norm(t, w, eps), x, g)
+        return d if residual is None else d + self._plain(residual)[0]
+
+    def swiglu_rows(self, gateup):
+        return reference.swiglu(*self._plain(gateup)[0].chunk(2, dim=-1))
+
+    def swiglu_rows_grad(self, gateup, g):
+        return self._pull(lambda t: reference.swiglu(*t.chunk(2, dim=-1)), gateup, g)
+
+    def rotate_rows(self, qkv, cos, sin, start, qh, kh, hd):
+        (qkv,) = self._plain(qkv)
+        self.projection = qkv  # what attn_prompt_grad turns its rows back to
+        return qkv.clone()
+
+    def attn_prefill_sums(self, q, k, v, scale):
+        shape = (START, QH, KH, HD)
+        return prompt_grad.torch_attention(self.projection, COS, SIN, *shape).detach(), torch.zeros(1)
+
+    def attn_prompt_grad(self, rows, out, g, sums, cos, sin, start, qh, kh, hd, scale):
+        return self._pull(lambda t: prompt_grad.torch_attention(t, cos, sin, start, qh, kh, hd), rows, g)
+
+
+HIP = Kernels()
+W = torch.rand(16, generator=torch.Generator().manual_seed(0)) + 0.5
+
+
+def through_kernels(x, a, b, c, d):
+    """A llama block without its quantization: what `forward_autograd` composes."""
+    n = prompt_grad.norm(x, W, 1e-5, HIP)
+    attn = prompt_grad.attention(n @ a, COS, SIN, START, QH, KH, HD, HD**-0.5, HIP)
+    h, n = prompt_grad.add_norm(x, attn @ b, W, 1e-5, HIP)
+    return h + prompt_grad.swiglu(n @ c, HIP) @ d
+
+
+def through_torch(x, a, b, c, d):
+    attn = prompt_grad.torch_attention(reference.rms_norm(x, W, 1e-5) @ a, COS, SIN, START, QH, KH, HD)
+    h = x + attn @ b
+    return h + reference.swiglu(*(reference.rms_norm(h, W, 1e-5) @ c).chunk(2, dim=-1)) @ d
+
+
+def drawn(*shapes):
+    gen = torch.Generator().manual_seed(1)
+    return [torch.randn(s, generator=gen) * 0.3 for s in shapes]
+
+
+def block_inputs():
+    x, *weights = drawn((2, 5, 16), (16, (QH + 2 * KH) * HD), (QH * HD, 16), (16, 24), (12, 16))
+    return x.requires_grad_(True), weights
+
+
+def close(got, want):
+    assert (got - want).norm() <= 1e-5 * want.norm()  # 32-bit sums
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_block_gradients(create_graph):
+    """Gradients that will have gradients themselves are the same as those that will not."""
+    x, weights = block_inputs()
+    (want,) = torch.autograd.grad(through_torch(x, *weights).pow(3).sum(), x, create_graph=create_graph)
+    (got,) = torch.autograd.grad(through_kernels(x, *weights).pow(3).sum(), x, create_graph=create_graph)
+    close(got, want)
+    if create_graph:
+        close(*(torch.autograd.grad(g.square().sum(), x)[0] for g in (got, want)))
+
+
+@pytest.mark.parametrize("same", [False, True])
+def test_sum_and_norm_of_dependent_rows(same):
+    """The second operand is made of the first, or is the first."""
+    x, a = drawn((3, 16), (16, 16))
+    x.requires_grad_(True)
+    y = x if same else x @ a
+    got, want = (
+        torch.autograd.grad(h.square().sum() + n.pow(3).sum(), x, create_graph=True)[0]
+        for h, n in (prompt_grad.add_norm(x, y, W, 1e-5, HIP), (x + y, reference.rms_norm(x + y, W, 1e-5)))
+    )
+    close(got, want)
+    close(*(torch.autograd.grad(g.square().sum(), x)[0] for g in (got, want)))
