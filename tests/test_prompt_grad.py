@@ -73,6 +73,14 @@ def through_torch(x, a, b, c, d):
     return h + reference.swiglu(*(reference.rms_norm(h, W, 1e-5) @ c).chunk(2, dim=-1)) @ d
 
 
+def kernel_add_norm(x, y):
+    return prompt_grad.add_norm(x, y, W, 1e-5, HIP)
+
+
+def torch_add_norm(x, y):
+    return x + y, reference.rms_norm(x + y, W, 1e-5)
+
+
 def drawn(*shapes):
     gen = torch.Generator().manual_seed(1)
     return [torch.randn(s, generator=gen) * 0.3 for s in shapes]
@@ -103,10 +111,9 @@ def test_sum_and_norm_of_dependent_rows(same):
     """The second operand is made of the first, or is the first."""
     x, a = drawn((3, 16), (16, 16))
     x.requires_grad_(True)
-    y = x if same else x @ a
     got, want = (
         torch.autograd.grad(h.square().sum() + n.pow(3).sum(), x, create_graph=True)[0]
-        for h, n in (prompt_grad.add_norm(x, y, W, 1e-5, HIP), (x + y, reference.rms_norm(x + y, W, 1e-5)))
+        for h, n in (function(x, x if same else x @ a) for function in (kernel_add_norm, torch_add_norm))
     )
     close(got, want)
     close(*(torch.autograd.grad(g.square().sum(), x)[0] for g in (got, want)))
