@@ -34,7 +34,7 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
-def _through_torch(function, inputs, grads):
+def _through_torch(function, inputs, grads, needed=(True,)):
     """Gradients that have gradients themselves (create_graph). They are taken at aliases of the
     inputs: one input may depend on another, and that path is the caller's graph's to follow."""
     with torch.enable_grad():
@@ -42,7 +42,9 @@ def _through_torch(function, inputs, grads):
         outputs = function(*inputs)
         outputs = outputs if isinstance(outputs, tuple) else (outputs,)
         kept = [(o, g) for o, g in zip(outputs, grads) if g is not None]
-        return torch.autograd.grad([o for o, _ in kept], inputs, [g for _, g in kept], create_graph=True, allow_unused=True)
+        wanted = [t for t, need in zip(inputs, needed) if need]
+        found = iter(torch.autograd.grad([o for o, _ in kept], wanted, [g for _, g in kept], create_graph=True, allow_unused=True))
+        return tuple(next(found) if need else None for need in needed)
 
 
 class _Norm(torch.autograd.Function):
@@ -80,7 +82,7 @@ class _AddNorm(torch.autograd.Function):
                 s = a + b
                 return s, reference.rms_norm(s, w, ctx.eps)
 
-            return (*_through_torch(composed, (x, y), (gh, gn)), None, None, None)
+            return (*_through_torch(composed, (x, y), (gh, gn), ctx.needs_input_grad[:2]), None, None, None)
         if gn is not None:
             gh = ctx.hip.norm_rows_grad(_aligned(h), w, _aligned(gn), None if gh is None else _aligned(gh), ctx.eps)
         return gh, gh, None, None, None

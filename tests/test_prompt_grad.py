@@ -117,3 +117,16 @@ def test_sum_and_norm_of_dependent_rows(same):
     )
     close(got, want)
     close(*(torch.autograd.grad(g.square().sum(), x)[0] for g in (got, want)))
+
+
+@pytest.mark.parametrize("first", [False, True])
+def test_one_operand_needs_gradients(first):
+    """Rows that are frozen beside rows that an adapter, say, has had a part in."""
+    x, y = drawn((3, 16), (3, 16))
+    leaf = (x if first else y).requires_grad_(True)
+    got, want = (
+        torch.autograd.grad(sum(t.pow(3).sum() for t in function(x, y)), leaf, create_graph=True)[0]
+        for function in (kernel_add_norm, torch_add_norm)
+    )
+    close(got, want)
+    close(*(torch.autograd.grad(g.square().sum(), leaf)[0] for g in (got, want)))
