@@ -6,7 +6,8 @@ products, 1.1 of its 2.0 ms at 2 x 379 tokens, width 4096; now it is 11, 0.15 ms
 one number per attention row, where torch kept several [heads, rows, rows] matrices.
 
 Ordinary reverse mode only (`fused_training`); what traces or transforms torch operations
-sees those of `ops.reference`. Gradients of gradients are taken through them, too.
+sees those of `ops.reference`. Gradients of gradients and
+batches of gradients are taken through them, too.
 """
 
 from __future__ import annotations
@@ -34,16 +35,30 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
+def _by_torch(*grads) -> bool:
+    """Whether these gradients are taken through torch operations: those that are to have gradients
+    themselves, and batches of them that look like one."""
+    batched = torch._C._functorch
+    return torch.is_grad_enabled() or any(
+        g is not None and (batched.is_functorch_wrapped_tensor(g) or batched.is_legacy_batchedtensor(g)) for g in grads
+    )
+
+
 def _through_torch(function, inputs, grads, needed=(True,)):
-    """Gradients that have gradients themselves (create_graph). They are taken at aliases of the
-    inputs: one input may depend on another, and that path is the caller's graph's to follow."""
+    """Gradients by torch operations. They are taken at aliases of the inputs: one input may
+    depend on another, and that path is the caller's graph's to follow."""
+    create_graph = torch.is_grad_enabled()
     with torch.enable_grad():
         inputs = tuple(t.view_as(t) for t in inputs)
         outputs = function(*inputs)
         outputs = outputs if isinstance(outputs, tuple) else (outputs,)
         kept = [(o, g) for o, g in zip(outputs, grads) if g is not None]
         wanted = [t for t, need in zip(inputs, needed) if need]
-        found = iter(torch.autograd.grad([o for o, _ in kept], wanted, [g for _, g in kept], create_graph=True, allow_unused=True))
+        found = iter(
+            torch.autograd.grad(
+                [o for o, _ in kept], wanted, [g for _, g in kept], create_graph=create_graph, allow_unused=True
+            )
+        )
         return tuple(next(found) if need else None for need in needed)
 
 
@@ -57,7 +72,7 @@ class _Norm(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         (x,), w = ctx.saved_tensors, ctx.w
-        if torch.is_grad_enabled():
+        if _by_torch(g):
             return (*_through_torch(lambda t: reference.rms_norm(t, w, ctx.eps), (x,), (g,)), None, None, None)
         return ctx.hip.norm_rows_grad(_aligned(x), w, _aligned(g), None, ctx.eps), None, None, None
 
@@ -76,7 +91,7 @@ class _AddNorm(torch.autograd.Function):
         (x, y, h), w = ctx.saved_tensors, ctx.w
         if gh is None and gn is None:
             return None, None, None, None, None
-        if torch.is_grad_enabled():
+        if _by_torch(gh, gn):
 
             def composed(a, b):
                 s = a + b
@@ -98,7 +113,7 @@ class _SwiGLU(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         (gateup,) = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if _by_torch(g):
             return (*_through_torch(lambda t: reference.swiglu(*t.chunk(2, dim=-1)), (gateup,), (g,)), None)
         return ctx.hip.swiglu_rows_grad(_aligned(gateup), _aligned(g)), None
 
@@ -128,7 +143,7 @@ class _Attention(torch.autograd.Function):
     def backward(ctx, g):
         (qkv, rows, out, sums), (cos, sin) = ctx.saved_tensors, ctx.tables
         none = (None,) * 8
-        if torch.is_grad_enabled():
+        if _by_torch(g):
             return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
         return (ctx.hip.attn_prompt_grad(rows, out, _aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 

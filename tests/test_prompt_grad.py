@@ -130,3 +130,14 @@ def test_one_operand_needs_gradients(first):
     )
     close(got, want)
     close(*(torch.autograd.grad(g.square().sum(), leaf)[0] for g in (got, want)))
+
+
+def test_batched_gradients():
+    """Several gradients of the result at once (is_grads_batched), as they are one by one."""
+    x, weights = block_inputs()
+    (grads,) = drawn((3, *x.shape))
+    (got,) = torch.autograd.grad(through_kernels(x, *weights), x, grads, is_grads_batched=True)
+    (want,) = torch.autograd.grad(through_torch(x, *weights), x, grads, is_grads_batched=True)
+    close(got, want)
+    by_one = [torch.autograd.grad(through_kernels(x, *weights), x, g)[0] for g in grads]
+    close(got, torch.stack(by_one))
