@@ -5,9 +5,9 @@ As torch operations, a llama block's forward and backward was 133 launches besid
 products, 1.1 of its 2.0 ms at 2 x 379 tokens, width 4096; now it is 11, 0.15 ms. Kept for the backward: rows, and
 one number per attention row, where torch kept several [heads, rows, rows] matrices.
 
-Ordinary reverse mode only (`fused_training`); what traces or transforms torch operations
-sees those of `ops.reference`. Gradients of gradients and
-batches of gradients are taken through them, too.
+Ordinary reverse mode only (`fused_training`): the kernels read and write memory by its address,
+which what traces, transforms or counts torch operations does not see. Under any of these, and
+for gradients of gradients and batches of gradients, the operations of `ops.reference` are run.
 """
 
 from __future__ import annotations
@@ -18,15 +18,28 @@ from torch.autograd import forward_ad
 from petals_amd.ops import reference
 
 
+def _watched(*tensors) -> bool:
+    """Whether something stands between torch operations and memory: a trace, a transform or a
+    mode, in force or wrapped around one of these tensors."""
+    wrapped = torch._C._functorch
+    return (
+        getattr(forward_ad, "_current_level", -1) >= 0
+        or wrapped.peek_interpreter_stack() is not None
+        or torch._C._len_torch_dispatch_stack() > 0
+        or torch.jit.is_tracing()
+        or torch.compiler.is_compiling()
+        or any(
+            type(t) not in (torch.Tensor, torch.nn.Parameter)
+            or wrapped.is_functorch_wrapped_tensor(t)
+            or wrapped.is_legacy_batchedtensor(t)
+            for t in tensors
+        )
+    )
+
+
 def fused_training(*rows: torch.Tensor) -> bool:
     """Whether these bf16 rows go through the kernels."""
-    return (
-        all(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0 for t in rows)
-        and getattr(forward_ad, "_current_level", -1) < 0
-        and torch._C._functorch.peek_interpreter_stack() is None
-        and not torch.jit.is_tracing()
-        and not torch.compiler.is_compiling()
-    )
+    return all(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0 for t in rows) and not _watched(*rows)
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
@@ -37,11 +50,8 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 
 def _by_torch(*grads) -> bool:
     """Whether these gradients are taken through torch operations: those that are to have gradients
-    themselves, and batches of them that look like one."""
-    batched = torch._C._functorch
-    return torch.is_grad_enabled() or any(
-        g is not None and (batched.is_functorch_wrapped_tensor(g) or batched.is_legacy_batchedtensor(g)) for g in grads
-    )
+    themselves, and those that are watched, which the forward pass need not have been."""
+    return torch.is_grad_enabled() or _watched(*(g for g in grads if g is not None))
 
 
 def _through_torch(function, inputs, grads, needed=(True,)):

@@ -3,6 +3,10 @@ the kernels are stood for by torch operations that autograd does not see."""
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils._python_dispatch import _disable_current_modes
+from torch.utils.flop_counter import FlopCounterMode
 
 from petals_amd.ops import prompt_grad, reference
 
@@ -11,7 +15,19 @@ COS, SIN = reference.build_rope_cache(HD, 16)
 
 
 class Kernels:
-    """The kernels' results on plain tensors; like them, it reads memory by its address."""
+    """The kernels' results on plain tensors; like them, it reads memory by its address, and no
+    mode sees what it does."""
+
+    def __getattribute__(self, name):
+        found = object.__getattribute__(self, name)
+        if name.startswith("_") or not callable(found):
+            return found
+
+        def unseen(*args):
+            with _disable_current_modes():
+                return found(*args)
+
+        return unseen
 
     @staticmethod
     def _plain(*tensors):
@@ -141,3 +157,51 @@ def test_batched_gradients():
     close(got, want)
     by_one = [torch.autograd.grad(through_kernels(x, *weights), x, g)[0] for g in grads]
     close(got, torch.stack(by_one))
+
+
+def test_traced_gradients():
+    """A trace of the backward pass holds operations, not what the kernels once returned."""
+    x, weights = block_inputs()
+    first, second = drawn((2, *x.shape))[0]
+    out = through_kernels(x, *weights)
+
+    def pull(g):
+        return torch.autograd.grad(out, x, g, retain_graph=True)[0]
+
+    close(make_fx(pull)(first)(second), pull(second))
+
+
+def test_what_watches_torch_operations():
+    assert not prompt_grad._watched()
+    seen = []
+
+    def look(t):
+        seen.append(prompt_grad._watched())
+        return t * 2
+
+    t = torch.ones(2, 3)
+    make_fx(look)(t)
+    with FlopCounterMode(display=False):
+        look(t)
+    torch.func.vmap(look)(t)
+    torch.func.grad(lambda u: look(u).sum())(t)
+    torch.jit.trace(look, t, check_trace=False)
+    with torch.autograd.forward_ad.dual_level():
+        look(t)
+    assert seen == [True] * 6 and not prompt_grad._watched()
+    with FakeTensorMode() as mode:
+        fake = mode.from_tensor(t)
+    assert prompt_grad._watched(fake) and not prompt_grad._watched(t, torch.nn.Parameter(t))
+
+
+def test_gradients_of_dual_numbers():
+    """The backward pass is linear in the result's gradient: so are the tangents it carries."""
+    x, weights = block_inputs()
+    g, tangent = drawn((2, *x.shape))[0]
+    out = through_kernels(x, *weights)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(g, tangent)
+        (got,) = torch.autograd.grad(out, x, dual, retain_graph=True)
+        value, moved = torch.autograd.forward_ad.unpack_dual(got)
+    close(value, torch.autograd.grad(out, x, g, retain_graph=True)[0])
+    close(moved, torch.autograd.grad(out, x, tangent)[0])
