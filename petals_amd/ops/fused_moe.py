@@ -22,6 +22,7 @@ from typing import List, Optional
 import torch
 import torch.nn.functional as F
 
+from petals_amd.ops import prompt_grad
 from petals_amd.ops.fused_decode import (
     _EPI_PLAIN_F32,
     _EPI_RAW,
@@ -159,20 +160,28 @@ class MixtralFastPath(LlamaFastPath):
     def widest_row(self) -> int:
         return self.top_k * self._max_gemv_out()  # a row per chosen expert
 
+    def _takes_router(self, x: torch.Tensor) -> bool:
+        """Rows and experts that the router's kernel takes."""
+        return x.is_cuda and x.shape[1] % 8 == 0 and self.num_experts <= 256 and self.top_k <= 16
+
     def _route(self, xn2: torch.Tensor):
-        """Router on [tokens, H] f32/bf16 -> (weights [t, k], experts [t, k]).
+        """Router on [tokens, H] f32/bf16 -> (weights [t, k] f32, experts [t, k]), differentiable.
+        Logits in 32 bits as in the kernel, and the kernel's choice where it can be asked, so that
+        gradients go through the experts that the forward pass runs.
         All-device: safe inside hipGraph capture."""
-        logits = xn2.to(self.w_router_t.dtype) @ self.w_router_t
-        probs = F.softmax(logits.float(), dim=-1)
-        weights, selected = torch.topk(probs, self.top_k, dim=-1)
-        weights = weights / weights.sum(dim=-1, keepdim=True)
-        return weights, selected
+        logits = xn2.float() @ self.w_router_t.float()
+        if self._takes_router(xn2) and not prompt_grad.watched(xn2):
+            selected = self._route_rows(xn2.detach())[1].long()
+        else:
+            selected = torch.topk(logits, self.top_k, dim=-1)[1]
+        # a softmax over all, renormalized over the chosen
+        return F.softmax(logits.gather(1, selected), dim=-1), selected
 
     def _route_rows(self, x: torch.Tensor):
         """Router on [tokens, H]: (weights [t, k] f32, experts [t, k] int32), one launch
         for as many experts as the kernel takes."""
-        if x.shape[1] % 8 == 0 and self.num_experts <= 256 and self.top_k <= 16:
-            return self.hip.moe_route(x, self.w_router, self.top_k)
+        if self._takes_router(x):
+            return self.hip.moe_route(prompt_grad.aligned(x), self.w_router, self.top_k)
         weights, selected = self._route(x)
         return weights.contiguous(), selected.to(torch.int32).contiguous()
 

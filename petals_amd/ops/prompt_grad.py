@@ -18,7 +18,7 @@ from torch.autograd import forward_ad
 from petals_amd.ops import reference
 
 
-def _watched(*tensors) -> bool:
+def watched(*tensors) -> bool:
     """Whether something stands between torch operations and memory: a trace, a transform or a
     mode, in force or wrapped around one of these tensors."""
     wrapped = torch._C._functorch
@@ -39,10 +39,10 @@ def _watched(*tensors) -> bool:
 
 def fused_training(*rows: torch.Tensor) -> bool:
     """Whether these bf16 rows go through the kernels."""
-    return all(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0 for t in rows) and not _watched(*rows)
+    return all(t.is_cuda and t.dtype == torch.bfloat16 and t.shape[-1] % 8 == 0 for t in rows) and not watched(*rows)
 
 
-def _aligned(t: torch.Tensor) -> torch.Tensor:
+def aligned(t: torch.Tensor) -> torch.Tensor:
     """Contiguous rows that 16-byte loads can read."""
     t = t.contiguous()
     return t.clone() if t.data_ptr() % 16 else t
@@ -51,7 +51,7 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 def _by_torch(*grads) -> bool:
     """Whether these gradients are taken through torch operations: those that are to have gradients
     themselves, and those that are watched, which the forward pass need not have been."""
-    return torch.is_grad_enabled() or _watched(*(g for g in grads if g is not None))
+    return torch.is_grad_enabled() or watched(*(g for g in grads if g is not None))
 
 
 def _through_torch(function, inputs, grads, needed=(True,)):
@@ -77,20 +77,20 @@ class _Norm(torch.autograd.Function):
     def forward(ctx, x, w, eps, hip):
         ctx.save_for_backward(x)
         ctx.w, ctx.eps, ctx.hip = w, eps, hip
-        return hip.rms_norm(_aligned(x), w, eps)
+        return hip.rms_norm(aligned(x), w, eps)
 
     @staticmethod
     def backward(ctx, g):
         (x,), w = ctx.saved_tensors, ctx.w
         if _by_torch(g):
             return (*_through_torch(lambda t: reference.rms_norm(t, w, ctx.eps), (x,), (g,)), None, None, None)
-        return ctx.hip.norm_rows_grad(_aligned(x), w, _aligned(g), None, ctx.eps), None, None, None
+        return ctx.hip.norm_rows_grad(aligned(x), w, aligned(g), None, ctx.eps), None, None, None
 
 
 class _AddNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, y, w, eps, hip):
-        h, n = hip.add_norm_rows(_aligned(x), _aligned(y), None, w, None, eps)
+        h, n = hip.add_norm_rows(aligned(x), aligned(y), None, w, None, eps)
         ctx.save_for_backward(x, y, h)
         ctx.set_materialize_grads(False)
         ctx.w, ctx.eps, ctx.hip = w, eps, hip
@@ -109,7 +109,7 @@ class _AddNorm(torch.autograd.Function):
 
             return (*_through_torch(composed, (x, y), (gh, gn), ctx.needs_input_grad[:2]), None, None, None)
         if gn is not None:
-            gh = ctx.hip.norm_rows_grad(_aligned(h), w, _aligned(gn), None if gh is None else _aligned(gh), ctx.eps)
+            gh = ctx.hip.norm_rows_grad(aligned(h), w, aligned(gn), None if gh is None else aligned(gh), ctx.eps)
         return gh, gh, None, None, None
 
 
@@ -118,14 +118,14 @@ class _SwiGLU(torch.autograd.Function):
     def forward(ctx, gateup, hip):
         ctx.save_for_backward(gateup)
         ctx.hip = hip
-        return hip.swiglu_rows(_aligned(gateup))
+        return hip.swiglu_rows(aligned(gateup))
 
     @staticmethod
     def backward(ctx, g):
         (gateup,) = ctx.saved_tensors
         if _by_torch(g):
             return (*_through_torch(lambda t: reference.swiglu(*t.chunk(2, dim=-1)), (gateup,), (g,)), None)
-        return ctx.hip.swiglu_rows_grad(_aligned(gateup), _aligned(g)), None
+        return ctx.hip.swiglu_rows_grad(aligned(gateup), aligned(g)), None
 
 
 def torch_attention(qkv, cos, sin, start, qh, kh, hd):
@@ -141,7 +141,7 @@ def torch_attention(qkv, cos, sin, start, qh, kh, hd):
 class _Attention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, qkv, cos, sin, start, qh, kh, hd, scale, hip):
-        rows = hip.rotate_rows(_aligned(qkv), cos, sin, start, qh, kh, hd)
+        rows = hip.rotate_rows(aligned(qkv), cos, sin, start, qh, kh, hd)
         heads = rows.view(*rows.shape[:2], qh + 2 * kh, hd).transpose(1, 2)
         out, sums = hip.attn_prefill_sums(heads[:, :qh], heads[:, qh : qh + kh], heads[:, qh + kh :], scale)
         ctx.save_for_backward(qkv, rows, out, sums)
@@ -155,7 +155,7 @@ class _Attention(torch.autograd.Function):
         none = (None,) * 8
         if _by_torch(g):
             return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
-        return (ctx.hip.attn_prompt_grad(rows, out, _aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
+        return (ctx.hip.attn_prompt_grad(rows, out, aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 
 
 def norm(x, w, eps, hip):

@@ -172,11 +172,11 @@ def test_traced_gradients():
 
 
 def test_what_watches_torch_operations():
-    assert not prompt_grad._watched()
+    assert not prompt_grad.watched()
     seen = []
 
     def look(t):
-        seen.append(prompt_grad._watched())
+        seen.append(prompt_grad.watched())
         return t * 2
 
     t = torch.ones(2, 3)
@@ -188,10 +188,10 @@ def test_what_watches_torch_operations():
     torch.jit.trace(look, t, check_trace=False)
     with torch.autograd.forward_ad.dual_level():
         look(t)
-    assert seen == [True] * 6 and not prompt_grad._watched()
+    assert seen == [True] * 6 and not prompt_grad.watched()
     with FakeTensorMode() as mode:
         fake = mode.from_tensor(t)
-    assert prompt_grad._watched(fake) and not prompt_grad._watched(t, torch.nn.Parameter(t))
+    assert prompt_grad.watched(fake) and not prompt_grad.watched(t, torch.nn.Parameter(t))
 
 
 def test_gradients_of_dual_numbers():
