@@ -468,23 +468,47 @@ def test_prompt_attention_gradients(hip, hd, b, s, qh, kh, start):
     assert bool(err.norm() <= 2.0**-7 * want.norm())  # and roundings don't all add up
 
 
+def near(got, want, rel):
+    assert (got.double() - want.double()).norm() <= rel * want.double().norm()
+
+
 @requires_gpu
-def test_prompt_gradients_have_gradients(hip):
+@pytest.mark.parametrize("which", ["norm", "add_norm", "swiglu", "attention"])
+def test_prompt_gradients_have_gradients(hip, which):
+    """First gradients with create_graph are the kernels', second ones those of the function."""
     from petals_amd.ops import prompt_grad, reference
 
     gen = torch.Generator(device="cuda").manual_seed(0)
     cos, sin = (t.to("cuda") for t in reference.build_rope_cache(64, 8))
-    w = torch.ones(64, device="cuda", dtype=BF16)
-    for function, width in [
-        (lambda t: prompt_grad.norm(t, w, 1e-5, hip), 64),
-        (lambda t: prompt_grad.add_norm(t, t, w, 1e-5, hip)[1], 64),
-        (lambda t: prompt_grad.swiglu(t, hip), 64),
-        (lambda t: prompt_grad.attention(t, cos, sin, 0, 1, 1, 64, 0.125, hip), 192),
-    ]:
-        x = _bf16_leaf(gen, 2, 5, width)
-        (g,) = _gradients([function(x).float().square().sum()], [x], [None], create_graph=True)
-        (gg,) = _gradients([g.float().square().sum()], [x], [None])
-        assert bool(torch.isfinite(gg).all()) and float(gg.float().abs().sum()) > 0
+    w = torch.rand(64, device="cuda", generator=gen).to(BF16) + 0.5
+    a = (torch.randn(64, 64, device="cuda", generator=gen) * 0.125).to(BF16)
+
+    def composed(t):  # 32-bit
+        if which == "norm":
+            return reference.rms_norm(t, w, 1e-5)
+        if which == "add_norm":
+            return reference.rms_norm(t + t @ a.float(), w, 1e-5)
+        if which == "swiglu":
+            return reference.swiglu(*t.chunk(2, dim=-1))
+        return prompt_grad.torch_attention(t, cos, sin, 0, 1, 1, 64)
+
+    kernels = {
+        "norm": lambda t: prompt_grad.norm(t, w, 1e-5, hip),
+        "add_norm": lambda t: prompt_grad.add_norm(t, t @ a, w, 1e-5, hip)[1],
+        "swiglu": lambda t: prompt_grad.swiglu(t, hip),
+        "attention": lambda t: prompt_grad.attention(t, cos, sin, 0, 1, 1, 64, 0.125, hip),
+    }[which]
+    x = _bf16_leaf(gen, 2, 5, 192 if which == "attention" else 64)
+    z = x.detach().float().requires_grad_(True)
+    (plain,) = _gradients([kernels(x).float().pow(3).sum()], [x], [None])
+    found = []
+    for function, leaf in ((kernels, x), (composed, z)):
+        (g,) = _gradients([function(leaf).float().pow(3).sum()], [leaf], [None], create_graph=True)
+        found.append((g.detach(), *_gradients([g.float().square().sum()], [leaf], [None])))
+    # a dozen roundings to bf16 of 2^-9 on the way, of which a gradient's gradient has twice as many
+    near(found[0][0], plain, 12 * 2.0**-9)
+    near(found[0][0], found[1][0], 12 * 2.0**-9)
+    near(found[0][1], found[1][1], 24 * 2.0**-9)
 
 
 @requires_gpu
@@ -498,6 +522,36 @@ def test_prompt_gradients_by_transforms(hip):
     with torch.autograd.forward_ad.dual_level():
         seen.append(prompt_grad.fused_training(x))
     assert seen == [False, False]
+
+
+@requires_gpu
+def test_block_gradients_by_transforms(hip):
+    """What traces or transforms a block's training pass gets the gradients that the kernels give."""
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.ops import prompt_grad
+    from petals_amd.server.from_pretrained import load_pretrained_block
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    config = load_model_config("test-llama-hd128")
+    block = load_pretrained_block("test-llama-hd128", config, 0, torch_dtype=BF16, device=torch.device("cuda"))
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    x, other = (_bf16_leaf(gen, 2, 9, config.hidden_size) for _ in range(2))
+    grads = torch.randn(3, 2, 9, config.hidden_size, device="cuda", generator=gen).to(BF16)
+    assert prompt_grad.fused_training(x)
+
+    def pull(t, g, **kw):
+        t = t.detach().requires_grad_(True)
+        return _gradients([block(t)], [t], [g], **kw)[0]
+
+    want = [pull(x, g) for g in grads]
+    rel = 24 * 2.0**-9  # roundings to bf16 of rows between products, at most so many on the way and back
+    near(pull(x, grads[0], create_graph=True).detach(), want[0], rel)
+    near(pull(x, grads, is_grads_batched=True), torch.stack(want), rel)
+    near(make_fx(lambda t, g: pull(t, g))(other.detach(), grads[1])(x.detach(), grads[0]), want[0], rel)
+    out = block(x)
+    back = make_fx(lambda g: _gradients([out], [x], [g], retain_graph=True)[0])(grads[1])
+    near(back(grads[0]), want[0], rel)
+    assert torch.equal(_gradients([out], [x], [grads[0]])[0], want[0])
 
 
 # ------------------------------------------------------ decode attention
