@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
 static torch::Tensor readable_rows(const torch::Tensor& t) {
   bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   for (int i = 0; i < 3; ++i) ok = ok && (t.size(i) == 1 || t.stride(i) % 8 == 0);
-  return ok ? t : t.contiguous();
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 static Rows4 rows4(const torch::Tensor& t) {

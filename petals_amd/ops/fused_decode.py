@@ -276,6 +276,11 @@ def _rows_fit(width: int) -> bool:
     return width % 8 == 0 and width <= 16384
 
 
+def _vector(t: torch.Tensor) -> torch.Tensor:
+    """A norm's weight or a bias, as the kernels read it."""
+    return prompt_grad.aligned(t.detach().to(torch.bfloat16))
+
+
 def _takes_rows(cache: torch.Tensor) -> bool:
     return cache.stride(3) == 1 and cache.data_ptr() % 16 == 0 and all(cache.stride(i) % 8 == 0 for i in range(3))
 
@@ -383,8 +388,8 @@ class LlamaFastPath(_TPFastPathMixin):
             and cfg.hidden_size // 64 <= 128  # XS gemv prefetches <= 128 partials
             and _fold_norm_wanted()
         )
-        self.ln1_w = block.input_layernorm.weight.detach().to(torch.bfloat16).contiguous()
-        self.ln2_w = block.post_attention_layernorm.weight.detach().to(torch.bfloat16).contiguous()
+        self.ln1_w = _vector(block.input_layernorm.weight)
+        self.ln2_w = _vector(block.post_attention_layernorm.weight)
         if self.fold_norm:
             ln1f = block.input_layernorm.weight.detach().float().to(device)
 
@@ -668,7 +673,7 @@ class LlamaFastPath(_TPFastPathMixin):
         adapter=None,
     ) -> torch.Tensor:
         B, S, H = hidden.shape
-        hidden = hidden.to(torch.bfloat16).contiguous()
+        hidden = prompt_grad.aligned(hidden.to(torch.bfloat16))
         self._ensure_rope(prefix_length + S)
 
         xn = self.hip.rms_norm(hidden, self.ln1_w_post, self.eps)
@@ -752,7 +757,7 @@ class BloomFastPath(_TPFastPathMixin):
             return w.detach().to(torch.bfloat16).t().contiguous()
 
         def bias(lin):
-            return lin.bias.detach().to(torch.bfloat16).contiguous()
+            return _vector(lin.bias)
 
         perm = _bloom_qkv_perm(self.qh, self.hd).to(device)
         self._qkv_perm = perm  # HF->flat [q|k|v] column map (LoRA deltas reuse it)
@@ -765,10 +770,10 @@ class BloomFastPath(_TPFastPathMixin):
         self.b_h4h = bias(mlp.dense_h_to_4h)
         self.w_4hh = _FastWeight(t(mlp.dense_4h_to_h.weight), hip_ops, quant)
         self.b_4hh = bias(mlp.dense_4h_to_h)
-        self.ln1_w = block.input_layernorm.weight.detach().to(torch.bfloat16).contiguous()
-        self.ln1_b = block.input_layernorm.bias.detach().to(torch.bfloat16).contiguous()
-        self.ln2_w = block.post_attention_layernorm.weight.detach().to(torch.bfloat16).contiguous()
-        self.ln2_b = block.post_attention_layernorm.bias.detach().to(torch.bfloat16).contiguous()
+        self.ln1_w = _vector(block.input_layernorm.weight)
+        self.ln1_b = _vector(block.input_layernorm.bias)
+        self.ln2_w = _vector(block.post_attention_layernorm.weight)
+        self.ln2_b = _vector(block.post_attention_layernorm.bias)
         self._empty_bf16 = torch.empty(0, device=device, dtype=torch.bfloat16)
         for lin in (attn.query_key_value, attn.dense, mlp.dense_h_to_4h, mlp.dense_4h_to_h):
             lin.weight.data = self._empty_bf16
@@ -883,7 +888,7 @@ class BloomFastPath(_TPFastPathMixin):
             return self.hip.layer_norm(x, w, b, self.eps)
 
         if not autograd and hidden.device.type == "cuda" and _rows_fit(H) and self.w_h4h.out_dim % 8 == 0:
-            return self._prompt(hidden.contiguous(), kv_cache, prefix_length, adapter)
+            return self._prompt(prompt_grad.aligned(hidden), kv_cache, prefix_length, adapter)
         xn = ln(hidden, self.ln1_w, self.ln1_b)
         res1 = xn if self.post_ln_residual else hidden
         xn = self._tp_copy(xn)
@@ -1045,10 +1050,10 @@ class FalconFastPath(_TPFastPathMixin):
         self.w_4hh = _FastWeight(t(mlp.dense_4h_to_h.weight), hip_ops, quant)
         ln_attn = block.input_layernorm if self.single_ln else block.ln_attn
         ln_mlp = block.input_layernorm if self.single_ln else block.ln_mlp
-        self.ln_attn_w = ln_attn.weight.detach().to(torch.bfloat16).contiguous()
-        self.ln_attn_b = ln_attn.bias.detach().to(torch.bfloat16).contiguous()
-        self.ln_mlp_w = ln_mlp.weight.detach().to(torch.bfloat16).contiguous()
-        self.ln_mlp_b = ln_mlp.bias.detach().to(torch.bfloat16).contiguous()
+        self.ln_attn_w = _vector(ln_attn.weight)
+        self.ln_attn_b = _vector(ln_attn.bias)
+        self.ln_mlp_w = _vector(ln_mlp.weight)
+        self.ln_mlp_b = _vector(ln_mlp.bias)
         self._empty_bf16 = torch.empty(0, device=device, dtype=torch.bfloat16)
         for lin in (attn.query_key_value, attn.dense, mlp.dense_h_to_4h, mlp.dense_4h_to_h):
             lin.weight.data = self._empty_bf16
@@ -1162,7 +1167,7 @@ class FalconFastPath(_TPFastPathMixin):
 
         rows_fit = _rows_fit(H) and self.w_h4h.out_dim % 8 == 0
         if not autograd and hidden.device.type == "cuda" and self.tp_world == 1 and rows_fit:
-            return self._prompt(hidden.contiguous(), kv_cache, prefix_length, adapter)
+            return self._prompt(prompt_grad.aligned(hidden), kv_cache, prefix_length, adapter)
         xn_attn = self._tp_copy(ln(hidden, self.ln_attn_w, self.ln_attn_b))
         xn_mlp = xn_attn if self.single_ln else self._tp_copy(ln(hidden, self.ln_mlp_w, self.ln_mlp_b))
         qkv = torch.matmul(xn_attn, self.wqkv_t.dense())

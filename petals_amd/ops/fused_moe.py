@@ -29,6 +29,7 @@ from petals_amd.ops.fused_decode import (
     _EPI_SWIGLU_F32,
     LlamaFastPath,
     _FastWeight,
+    _vector,
     _dequant_cached,
 )
 
@@ -129,7 +130,7 @@ class MixtralFastPath(LlamaFastPath):
         moe = block.block_sparse_moe
         self.top_k = moe.top_k
         self.num_experts = moe.num_experts
-        self.w_router = moe.gate.weight.detach().to(torch.bfloat16).contiguous()  # [E, H]
+        self.w_router = _vector(moe.gate.weight)  # [E, H]
         self.w_router_t = self.w_router.t()
         self.stacked_gu: Optional[_StackedExperts] = None
         self.stacked_down: Optional[_StackedExperts] = None

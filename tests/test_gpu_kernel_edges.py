@@ -325,6 +325,42 @@ def test_prompt_chunks_are_one_prompt(hip, tokens, limit):
         assert torch.allclose(a.float(), b.float(), **tol)
 
 
+def off_by_one_value(t):
+    """The same values, contiguous, on an address that is no multiple of 16 bytes."""
+    moved = torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape)
+    assert moved.is_contiguous() and moved.data_ptr() % 16
+    return moved.copy_(t)
+
+
+@requires_gpu
+@pytest.mark.parametrize("preset", ["test-llama-hd128", "test-bloom-hd64", "test-falcon-hd64"])
+def test_prompts_at_any_address(hip, preset):
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.server.from_pretrained import build_empty_block, init_random_block_, load_pretrained_block
+
+    config = load_model_config(preset)
+    block = load_pretrained_block(preset, config, 0, torch_dtype=BF16, device=torch.device("cuda"))
+    assert block._fast is not None
+    moved = build_empty_block(config, 0, torch.device("cuda"), BF16)
+    init_random_block_(moved, config, 0)
+    for p in moved.parameters():
+        p.data = off_by_one_value(p.data)
+    moved = moved.eval().optimize_for_inference()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(2, 19, config.hidden_size, device="cuda", generator=gen).to(BF16)
+    empty = [torch.zeros(shape, device="cuda", dtype=BF16) for shape in block.kv_cache_shape(2, 32)]
+    with torch.inference_mode():
+        assert torch.equal(block(off_by_one_value(x)), block(x))
+        want = [t.clone() for t in empty]
+        out = block(x, kv_cache=want, prefix_length=3)
+        for caches in ([t.clone() for t in empty], [off_by_one_value(t) for t in empty]):
+            assert torch.equal(block(off_by_one_value(x), kv_cache=caches, prefix_length=3), out)
+            assert all(torch.equal(a, b) for a, b in zip(caches, want))
+        assert torch.isfinite(moved(x).float()).all()
+    moved(x.requires_grad_(True)).sum().backward()
+    assert torch.isfinite(x.grad.float()).all()
+
+
 @requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, BF16])
 @pytest.mark.parametrize("tokens,dim,experts,top", [(1, 8, 1, 1), (3, 64, 4, 2), (5, 4096, 8, 2), (2, 520, 64, 16), (7, 128, 65, 3), (1, 2048, 256, 8)])
