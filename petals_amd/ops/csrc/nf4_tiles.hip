@@ -1,12 +1,15 @@
 // Products of few rows with NF4 weights on the matrix cores, in whole numbers.
 //
-// A 4-bit level times 7783094 is a whole number up to 2 units in 10^8 of the largest
-// level (no other factor below 127.4 * 2^16 fits all 16 levels as well), and a whole number
-// is three signed digits of base 256. So is an input times its block's scale, with four
-// digits, once the inputs of a run are scaled by one power of two so that their largest
-// reaches 2^30. Sums of products of digits are exact in 32 bits for runs of 512, and a
-// product of 16 columns with 64 inputs is one v_mfma_i32_16x16x64_i8 per digit of the
-// levels: the four digits of up to four rows are its other 16 columns.
+// A 4-bit level times 7783094 is a whole number up to 9.4e-8 of itself (no other factor below
+// 127.4 * 2^16 fits all 16 levels as well; a 32-bit product of level, scale and input is
+// rounded twice by up to 6e-8), and a whole number is three signed digits of base 256. So is
+// an input times its block's scale, with four digits, once the inputs of a run are scaled by
+// one power of two so that 64 times their mean size reaches 2^29: a last place is 2^-23 of the
+// mean. Inputs that are larger would leave the others fewer places; they are left out and
+// multiplied in 32-bit floats, one by one (see `strip`). Sums of products of digits are exact
+// in 32 bits for runs of 512, and a product of 16 columns with 64 inputs is one
+// v_mfma_i32_16x16x64_i8 per digit of the levels: the four digits of up to four rows are its
+// other 16 columns.
 //
 // Digits come from v_perm_b32, which looks four codes up in eight bytes at once. Two
 // lookups make up the 16 levels: a code of the other half selects a sign or a constant (0
@@ -35,7 +38,10 @@
 //   gate  8192 x 57344   64, 96, 160    64, 78, 112
 //   down  28672 x 8192   36, 51, 84     36, 41, 63
 // (Runs of 1024 for one row: 70 and 38 us for the last two; four waves a SIMD: 71, 39.)
-// Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.7e-7).
+// With the largest input of a run at 2^30 whatever the others are, 0 to 4% less (8192 x 57344:
+// 61.0, 69.4, 98.2 us for 1, 4, 8 rows beside 62.5, 71.8, 102.0). A run with inputs beyond 64
+// times its mean takes longer: two inputs of 8192 a thousand times the rest, 59.3, 72.0, 126.6.
+// Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.6e-7).
 
 #include "common.h"
 #include "gemv_reduce.h"
@@ -46,6 +52,10 @@ using i32x4 = __attribute__((ext_vector_type(4))) int;
 using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
 #define NF4_UNIT (1.0f / 7783094.0f)
+// times a run's mean size. Channels ten times as loud as the rest stay below it; with 16 they
+// didn't, and 8 rows of 8192 x 57344 took 197 us (the loud ones then in loops of their own)
+#define NF4_GATE 64.f
+#define NF4_FINITE 0x7F7FFFFFu  // bits of the largest number
 
 static __device__ __constant__ float NF4_TILE_LEVELS[16] = {
     -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
@@ -68,9 +78,10 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// largest value of a wave
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
-#define STEP(ctrl, rows) v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false))
+// sum of a wave, the same for all lanes
+__device__ __forceinline__ float wave_sum(float v) {
+#define STEP(ctrl, rows) \
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, false))
   STEP(0xB1, 0xf);   // quads: neighbours
   STEP(0x4E, 0xf);   // quads: pairs
   STEP(0x141, 0xf);  // halves of a row mirrored
@@ -78,7 +89,7 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
   STEP(0x142, 0xa);  // row 0 to 1, 2 to 3
   STEP(0x143, 0xc);  // rows 0 and 1 to 2 and 3
 #undef STEP
-  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 __device__ __forceinline__ float quad_sum(float v) {
@@ -100,7 +111,7 @@ __device__ __forceinline__ void transpose_bytes(unsigned* w) {
 // Grid: (out/64, runs of 4 KB `steps` tiles, rows of sel). With sel, B is 1 and row
 // blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z].
 template <int B, int KB, bool LONG>
-__global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
+__global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     const uint4* __restrict__ tiles, const unsigned short* __restrict__ scales,
     const float* __restrict__ x,      // [rows, in]
     const int* __restrict__ sel,      // [rows * k_per_tok] or null
@@ -165,38 +176,105 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
   for (int j = 0; j < KB; ++j) fetch_w(0, j);
   __builtin_amdgcn_sched_barrier(0);
 
-  // largest input of each row and largest scale of the run bound the scaled inputs
-  unsigned top[B], top_scale = 0;
+  // Digits hold sizes up to NF4_GATE times the run's mean, if there are none beyond. If there
+  // are, they hold up to 128 times a mean of sizes clipped at itself (twice the mean, clipped,
+  // again and again while that at least halves it), which a few sizes can't move however large.
+  const float share = 1.f / (KB * 128 * steps);
+  float mean[B], top[B], next[B];
+  auto add_sizes = [&](const unsigned* s, int b, const float* v, bool clip) {
 #pragma unroll
-  for (int i = 0; i < PER / 2; ++i) top_scale = max(top_scale, max(sc[i] & 0xFFFF0000u, sc[i] << 16));
+    for (int i = 0; i < PER; ++i) {
+      const float size = fabsf(v[i] * __uint_as_float(i & 1 ? s[i / 2] & 0xFFFF0000u : s[i / 2] << 16));
+      if (clip) {
+        next[b] += __float_as_uint(size) > NF4_FINITE ? 0.f : fminf(size, mean[b]) * share;
+      } else {
+        mean[b] += size;
+        top[b] = fmaxf(top[b], size);
+      }
+    }
+  };
+  auto add_all = [&](bool clip) {
+#pragma unroll
+    for (int b = 0; b < B; ++b) add_sizes(sc, b, xs[b], clip);
+    for (int step = 1; step < steps; ++step) {
+      unsigned s[PER / 2];
+      fetch_scales(step, s);
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        float v[PER];
+        fetch_x(step, b, v);
+        add_sizes(s, b, v, clip);
+      }
+    }
+  };
+#pragma unroll
+  for (int b = 0; b < B; ++b) mean[b] = top[b] = 0.f;
+  add_all(false);
+  unsigned most[B];  // bits of the largest size that digits hold
+  bool loud = false;
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    top[b] = 0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) top[b] = max(top[b], __float_as_uint(xs[b][i]) & 0x7FFFFFFFu);
+    mean[b] = wave_sum(mean[b]) * share;
+    most[b] = __float_as_uint(mean[b] * NF4_GATE) & 0x7FFFFFFFu;
+    loud |= __float_as_uint(top[b]) > most[b] || most[b] > NF4_FINITE;  // the latter: infinities, NaNs
   }
-  for (int step = 1; step < steps; ++step) {
-    unsigned s[PER / 2];
-    fetch_scales(step, s);
-#pragma unroll
-    for (int i = 0; i < PER / 2; ++i) top_scale = max(top_scale, max(s[i] & 0xFFFF0000u, s[i] << 16));
+  loud = __any(loud);
+  if (__builtin_expect(loud, 0)) {
 #pragma unroll
     for (int b = 0; b < B; ++b) {
-      float v[PER];
-      fetch_x(step, b, v);
-#pragma unroll
-      for (int i = 0; i < PER; ++i) top[b] = max(top[b], __float_as_uint(v[i]) & 0x7FFFFFFFu);
+      if (most[b] > NF4_FINITE) mean[b] = __uint_as_float(NF4_FINITE);
+      red[(wave * B + b) * 64 + lane] = 0.f;
     }
+    for (bool more = true; more;) {
+#pragma unroll
+      for (int b = 0; b < B; ++b) next[b] = 0.f;
+      add_all(true);
+      more = false;
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        next[b] = wave_sum(next[b]) * 2.f;
+        if (next[b] < mean[b] * 0.5f) {  // uniform
+          mean[b] = next[b];
+          more = true;
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) most[b] = min(__float_as_uint(mean[b] * 128.f), NF4_FINITE);
+    wave_fence();
   }
+  // takes what digits don't hold out of a step's inputs: in 32-bit floats, a column per lane
+  auto strip = [&](int step) {
+    unsigned over = 0;
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const float v = xs[b][i] * __uint_as_float(i & 1 ? sc[i / 2] & 0xFFFF0000u : sc[i / 2] << 16);
+        if ((__float_as_uint(v) & 0x7FFFFFFFu) > most[b]) {
+          xs[b][i] = 0.f;
+          over |= 1u << (b * PER + i);
+        }
+      }
+    const unsigned char* bytes = reinterpret_cast<const unsigned char*>(tiles + ((size_t)nb * n_kb + kb0) * 256);
+    for (unsigned long long lanes = __ballot(over != 0); lanes; lanes &= lanes - 1) {
+      const int from = __ffsll((long long)lanes) - 1;
+      for (unsigned left = __builtin_amdgcn_readlane((int)over, from); left; left &= left - 1) {
+        const int bit = __ffs((int)left) - 1, b = bit / PER, i = step * KB * 128 + from * PER + bit % PER;
+        const int at = i % 16, half = i % 128 / 64;
+        const int byte = (((i / 128) * 4 + lane / 16) * 64 + i % 64 / 16 * 16 + lane % 16) * 16 + half * 8 + at / 8 * 4 + at % 4;
+        const float level = NF4_TILE_LEVELS[at & 4 ? bytes[byte] >> 4 : bytes[byte] & 15];
+        const float v = x[(size_t)b * in_dim + kb0 * 128 + i] * bf16_to_f32(scales[((size_t)nb * n_kb + kb0) * 128 + i]);
+        float* sum = &red[(wave * B + b) * 64 + lane];
+        *sum = fmaf(level, v, *sum);
+      }
+    }
+  };
   float unit[B], factor[B];  // the scaled inputs' last place, and one over it
-  bool odd = false;
-  top_scale = wave_max_u32(top_scale);
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    const unsigned m = __float_as_uint(__uint_as_float(wave_max_u32(top[b])) * __uint_as_float(top_scale)) & 0x7FFFFFFFu;
-    odd |= m >= 0x7F800000u;
     // below 2^(e - 126), times 2^(156 - e)
-    const unsigned up = min(283u - (m >> 23), 253u);
+    const unsigned up = min(283u - (most[b] >> 23), 253u);
     factor[b] = __uint_as_float(up << 23);
     unit[b] = __uint_as_float((254u - up) << 23);
   }
@@ -209,7 +287,8 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
 #pragma unroll
       for (int p = 0; p < 3; ++p) acc[s][c][p] = i32x4{0, 0, 0, 0};
 
-  for (int step = 0; step < steps && !odd; ++step) {
+  for (int step = 0; step < steps; ++step) {
+    if (__builtin_expect(loud, 0)) strip(step);
 #pragma unroll
     for (int b = 0; b < B; ++b)
 #pragma unroll
@@ -218,7 +297,8 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const unsigned s = (i + j) & 1 ? sc[(i + j) / 2] & 0xFFFF0000u : sc[(i + j) / 2] << 16;
-          q[j] = ((unsigned)(int)(xs[b][i + j] * __uint_as_float(s) * factor[b]) + 0x00808080u) ^ 0x00808080u;
+          const float v = xs[b][i + j] * __uint_as_float(s);
+          q[j] = ((unsigned)(int)(v * factor[b]) + 0x00808080u) ^ 0x00808080u;
         }
         transpose_bytes(q);
         const int at = lane * PER + i;  // of the step: group of 16, then column, then place
@@ -227,8 +307,8 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
           *reinterpret_cast<unsigned*>(&digits[wave][((at / 16) * NCOL + b * 4 + d) * 16 + at % 16]) = q[d];
       }
     wave_fence();
-    const bool more = step + 1 < steps;
-    if (more) {
+    const bool next = step + 1 < steps;
+    if (next) {
       fetch_scales(step + 1, sc);
 #pragma unroll
       for (int b = 0; b < B; ++b) fetch_x(step + 1, b, xs[b]);
@@ -267,43 +347,29 @@ __global__ __launch_bounds__(256, B <= 2 ? 3 : 2) void gemv_nf4_tiles_kernel(
           }
         }
       }
-      if (more) fetch_w(step + 1, j);
+      if (next) fetch_w(step + 1, j);
     }
     wave_fence();
   }
 
-  if (__builtin_expect(odd, 0)) {  // infinities and NaNs: in 32-bit floats, a column per lane
-    float sum[B];
 #pragma unroll
-    for (int b = 0; b < B; ++b) sum[b] = 0.f;
-    const unsigned char* bytes = reinterpret_cast<const unsigned char*>(tiles + ((size_t)nb * n_kb + kb0) * 256);
-    for (int i = 0; i < live_kb * 128 && kb0 * 128 + i < in_dim; ++i) {
-      const int at = i % 16, half = i % 128 / 64;
-      const int byte = (((i / 128) * 4 + lane / 16) * 64 + i % 64 / 16 * 16 + lane % 16) * 16 + half * 8 + at / 8 * 4 + at % 4;
-      const float level = NF4_TILE_LEVELS[at & 4 ? bytes[byte] >> 4 : bytes[byte] & 15];
-      const float s = bf16_to_f32(scales[(size_t)nb * n_kb * 128 + kb0 * 128 + i]);
+  for (int s = 0; s < NS; ++s) {
+    const int row = s * 4 + col / 4;  // this lane's row and, col % 4, digit of its inputs
+    float last = 0.f;
 #pragma unroll
-      for (int b = 0; b < B; ++b) sum[b] = fmaf(level, x[(size_t)b * in_dim + kb0 * 128 + i] * s, sum[b]);
-    }
+    for (int b = s * 4; b < B && b < s * 4 + 4; ++b) last = row == b ? unit[b] : last;
+    const float place = __uint_as_float((127u + 8u * (col & 3)) << 23) * NF4_UNIT;
 #pragma unroll
-    for (int b = 0; b < B; ++b) red[(wave * B + b) * 64 + lane] = sum[b];
-  } else {
+    for (int c = 0; c < 4; ++c) {
+      float4v v;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int row = s * 4 + col / 4;  // this lane's row and, col % 4, digit of its inputs
-      float last = 0.f;
-#pragma unroll
-      for (int b = s * 4; b < B && b < s * 4 + 4; ++b) last = row == b ? unit[b] : last;
-      const float place = __uint_as_float((127u + 8u * (col & 3)) << 23) * NF4_UNIT;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        float4v v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float sum = fmaf((float)acc[s][c][2][r], 65536.f, fmaf((float)acc[s][c][1][r], 256.f, (float)acc[s][c][0][r]));
-          v[r] = quad_sum(sum * place) * last;
-        }
-        if ((col & 3) == 0 && row < B) *reinterpret_cast<float4v*>(&red[(wave * B + row) * 64 + c * 16 + hi * 4]) = v;
+      for (int r = 0; r < 4; ++r) {
+        const float sum = fmaf((float)acc[s][c][2][r], 65536.f, fmaf((float)acc[s][c][1][r], 256.f, (float)acc[s][c][0][r]));
+        v[r] = quad_sum(sum * place) * last;
+      }
+      if ((col & 3) == 0 && row < B) {
+        float4v* sum = reinterpret_cast<float4v*>(&red[(wave * B + row) * 64 + c * 16 + hi * 4]);
+        *sum = loud ? *sum + v : v;
       }
     }
   }

@@ -100,11 +100,44 @@ def test_nf4_tiles_against_64_bits(hip, k_in, n_out, batch):
         x[2] *= 1e30
     y = hip.gemv_nf4_tiles(tiles, scales, k_in, x, torch.empty(0, device="cuda"), None, 0).double()
     xd = x.double()
-    # levels are off by 2.4e-8 at most, inputs by 2^-31 of the largest (but not by less than
-    # 2^-127), and 2^3 roundings follow
-    bound = (xd.abs() @ scale) * 2.4e-8 + 2.0**-21 * (xd.abs() @ w.abs())
-    bound += k_in * (2.0**-31 * xd.abs().amax(1, keepdim=True) * scale.amax() + 2.0**-127)
-    assert bool(((y - xd @ w).abs() <= bound + 1e-38).all())
+    assert bool(((y - xd @ w).abs() <= nf4_bound(xd, w, scale)).all())
+
+
+def nf4_bound(xd, w, scale):
+    """Scaled inputs are cut off below 2^-20 of their run's mean, large ones clipped (but not below
+    2^-126), levels are off by 9.4e-8 of themselves, and 2^3 roundings follow."""
+    return 2.0**-20 * (xd.abs() @ scale) + 2.0**-20 * (xd.abs() @ w.abs()) + xd.shape[-1] * 2.0**-126
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", range(1, 9))
+@pytest.mark.parametrize("loud", [[30.0], [1e4], [1e10], [1e20], [1e3, 1e6, 1e9], [1e2, 1e15, 1e30]])
+def test_nf4_tiles_of_a_wide_range(hip, batch, loud):
+    """A few inputs that dwarf the rest cost it nothing where they meet a weight of zero."""
+    k_in, n_out = 1030, 128
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    w = (torch.randn(k_in, n_out, device="cuda", generator=gen) * 0.05).to(BF16)
+    at = torch.tensor([0, 127, 128, 300, 400, 500, 511, 512, 600, 700, 1029], device="cuda")
+    w[at, ::2] = 0.0
+    packed, absmax = hip.nf4_quantize(w)
+    codes = torch.stack([packed & 15, packed >> 4], dim=-1).view(k_in, n_out).long()
+    scale = absmax.double().repeat_interleave(64, dim=1)
+    held = NF4_LEVELS.cuda().double()[codes] * scale
+    assert not held[at, ::2].any()
+    x = torch.randn(batch, k_in, device="cuda", generator=gen)
+    for b in range(batch):
+        for i, k in enumerate(at.tolist()):
+            if (i + b) % 4 or b == batch // 2:  # all of one row
+                x[b, k] = loud[i % len(loud)]
+    if batch > 3:
+        x[0, ::2] = 0.0
+        x[3, 5:-5] = 0.0
+    y = hip.gemv_nf4_tiles(*hip.nf4_tile(packed, absmax), k_in, x, torch.empty(0, device="cuda"), None, 0).double()
+    xd, quiet = x.double(), x.double()
+    quiet[:, at] = 0.0
+    error = (y - xd @ held).abs()
+    assert bool((error[:, ::2] <= nf4_bound(quiet, held, scale)[:, ::2]).all())
+    assert bool((error <= nf4_bound(xd, held, scale)).all())
 
 
 @requires_gpu
@@ -133,8 +166,7 @@ def test_nf4_tiles_of_experts(hip, experts, tokens, top, k_in, n_out):
     y = hip.gemv_nf4_tiles_moe(tiles, scales, k_in, x, sel, top, torch.empty(0, device="cuda"), 0).double()
     for r, e in enumerate(sel.tolist()):
         xd, w, scale = x[r // top].double(), made[e][1], made[e][2]
-        bound = (xd.abs() @ scale) * 2.4e-8 + 2.0**-21 * (xd.abs() @ w.abs())
-        assert bool(((y[r] - xd @ w).abs() <= bound + k_in * 2.0**-31 * xd.abs().max() * scale.amax()).all())
+        assert bool(((y[r] - xd @ w).abs() <= nf4_bound(xd, w, scale)).all())
 
 
 def sum_bound(xd, w):
