@@ -3,10 +3,11 @@
 // A 4-bit level times 7783094 is a whole number up to 9.4e-8 of itself (no other factor below
 // 127.4 * 2^16 fits all 16 levels as well; a 32-bit product of level, scale and input is
 // rounded twice by up to 6e-8), and a whole number is three signed digits of base 256. So is
-// an input times its block's scale, with four digits, once the inputs of a run are scaled by
-// one power of two so that 64 times their mean size reaches 2^29: a last place is 2^-23 of the
-// mean. Inputs that are larger would leave the others fewer places; they are left out and
-// multiplied in 32-bit floats, one by one (see `strip`). Sums of products of digits are exact
+// an input times its block's scale, rounded to four digits, once the inputs of a run are
+// scaled by one power of two so that their largest reaches 2^29. Inputs beyond 64 times the
+// run's mean size would leave the others few places; those runs leave out what is too large
+// and multiply it in 32-bit floats, one by one (see `strip`), so that a last place is at most
+// 2^-22 of a mean that they have no part in. Sums of products of digits are exact
 // in 32 bits for runs of 512, and a product of 16 columns with 64 inputs is one
 // v_mfma_i32_16x16x64_i8 per digit of the levels: the four digits of up to four rows are its
 // other 16 columns.
@@ -38,9 +39,10 @@
 //   gate  8192 x 57344   64, 96, 160    64, 78, 112
 //   down  28672 x 8192   36, 51, 84     36, 41, 63
 // (Runs of 1024 for one row: 70 and 38 us for the last two; four waves a SIMD: 71, 39.)
-// With the largest input of a run at 2^30 whatever the others are, 0 to 4% less (8192 x 57344:
-// 61.0, 69.4, 98.2 us for 1, 4, 8 rows beside 62.5, 71.8, 102.0). A run with inputs beyond 64
-// times its mean takes longer: two inputs of 8192 a thousand times the rest, 59.3, 72.0, 126.6.
+// Cut off instead of rounded, and with the largest input of a run at 2^30 whatever the others
+// are, it took 0 to 5% less (8192 x 8192: 14.7, 16.1, 18.5 us without the reduction for 1, 4,
+// 8 rows beside 14.8, 16.6, 19.5). Runs with inputs beyond 64 times their mean take longer: two
+// of 8192 inputs a thousand times the rest, 15.2, 18.2, 23.6.
 // Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.6e-7).
 
 #include "common.h"
@@ -78,10 +80,15 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// sum of a wave, the same for all lanes
-__device__ __forceinline__ float wave_sum(float v) {
-#define STEP(ctrl, rows) \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, false))
+// sum, or largest of numbers from zero on, over a wave, the same for all lanes. Bits, as the
+// compiler takes what comes out of float arithmetic for finite.
+template <bool MAX>
+__device__ __forceinline__ unsigned wave_all(float v) {
+#define STEP(ctrl, rows)                                                                                   \
+  do {                                                                                                     \
+    const float other = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, false)); \
+    v = MAX ? fmaxf(v, other) : v + other;                                                                 \
+  } while (0)
   STEP(0xB1, 0xf);   // quads: neighbours
   STEP(0x4E, 0xf);   // quads: pairs
   STEP(0x141, 0xf);  // halves of a row mirrored
@@ -89,7 +96,7 @@ __device__ __forceinline__ float wave_sum(float v) {
   STEP(0x142, 0xa);  // row 0 to 1, 2 to 3
   STEP(0x143, 0xc);  // rows 0 and 1 to 2 and 3
 #undef STEP
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+  return (unsigned)__builtin_amdgcn_readlane(__float_as_int(v), 63);
 }
 
 __device__ __forceinline__ float quad_sum(float v) {
@@ -176,9 +183,9 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   for (int j = 0; j < KB; ++j) fetch_w(0, j);
   __builtin_amdgcn_sched_barrier(0);
 
-  // Digits hold sizes up to NF4_GATE times the run's mean, if there are none beyond. If there
-  // are, they hold up to 128 times a mean of sizes clipped at itself (twice the mean, clipped,
-  // again and again while that at least halves it), which a few sizes can't move however large.
+  // Digits hold all sizes, if none is beyond NF4_GATE times the run's mean. Else they hold up to
+  // 128 times a mean of sizes clipped at itself (twice the mean, clipped, again and again while
+  // that at least halves it), which a few sizes can't move however large.
   const float share = 1.f / (KB * 128 * steps);
   float mean[B], top[B], next[B];
   auto add_sizes = [&](const unsigned* s, int b, const float* v, bool clip) {
@@ -186,7 +193,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     for (int i = 0; i < PER; ++i) {
       const float size = fabsf(v[i] * __uint_as_float(i & 1 ? s[i / 2] & 0xFFFF0000u : s[i / 2] << 16));
       if (clip) {
-        next[b] += __float_as_uint(size) > NF4_FINITE ? 0.f : fminf(size, mean[b]) * share;
+        next[b] += fminf(size, mean[b]) * share;  // NaNs are clipped, too
       } else {
         mean[b] += size;
         top[b] = fmaxf(top[b], size);
@@ -214,17 +221,14 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   bool loud = false;
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    mean[b] = wave_sum(mean[b]) * share;
-    most[b] = __float_as_uint(mean[b] * NF4_GATE) & 0x7FFFFFFFu;
-    loud |= __float_as_uint(top[b]) > most[b] || most[b] > NF4_FINITE;  // the latter: infinities, NaNs
+    const unsigned sum = wave_all<false>(mean[b]) & 0x7FFFFFFFu;
+    mean[b] = __uint_as_float(min(sum, NF4_FINITE)) * share;
+    most[b] = wave_all<true>(top[b]);
+    loud |= most[b] > __float_as_uint(mean[b] * NF4_GATE) || sum > NF4_FINITE;  // the latter: infinities, NaNs
   }
-  loud = __any(loud);
   if (__builtin_expect(loud, 0)) {
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-      if (most[b] > NF4_FINITE) mean[b] = __uint_as_float(NF4_FINITE);
-      red[(wave * B + b) * 64 + lane] = 0.f;
-    }
+    for (int b = 0; b < B; ++b) red[(wave * B + b) * 64 + lane] = 0.f;
     for (bool more = true; more;) {
 #pragma unroll
       for (int b = 0; b < B; ++b) next[b] = 0.f;
@@ -232,7 +236,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
       more = false;
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        next[b] = wave_sum(next[b]) * 2.f;
+        next[b] = __uint_as_float(wave_all<false>(next[b])) * 2.f;
         if (next[b] < mean[b] * 0.5f) {  // uniform
           mean[b] = next[b];
           more = true;
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
         for (int j = 0; j < 4; ++j) {
           const unsigned s = (i + j) & 1 ? sc[(i + j) / 2] & 0xFFFF0000u : sc[(i + j) / 2] << 16;
           const float v = xs[b][i + j] * __uint_as_float(s);
-          q[j] = ((unsigned)(int)(v * factor[b]) + 0x00808080u) ^ 0x00808080u;
+          q[j] = ((unsigned)(int)rintf(v * factor[b]) + 0x00808080u) ^ 0x00808080u;
         }
         transpose_bytes(q);
         const int at = lane * PER + i;  // of the step: group of 16, then column, then place

@@ -104,9 +104,9 @@ def test_nf4_tiles_against_64_bits(hip, k_in, n_out, batch):
 
 
 def nf4_bound(xd, w, scale):
-    """Scaled inputs are cut off below 2^-20 of their run's mean, large ones clipped (but not below
-    2^-126), levels are off by 9.4e-8 of themselves, and 2^3 roundings follow."""
-    return 2.0**-20 * (xd.abs() @ scale) + 2.0**-20 * (xd.abs() @ w.abs()) + xd.shape[-1] * 2.0**-126
+    """Scaled inputs are rounded to 2^-20 of their run's mean, large ones clipped, or finer (but not
+    below 2^-126), levels are off by 9.4e-8 of themselves, and 2^3 roundings follow."""
+    return 2.0**-21 * (xd.abs() @ scale) + 2.0**-20 * (xd.abs() @ w.abs()) + xd.shape[-1] * 2.0**-126
 
 
 @requires_gpu
@@ -138,6 +138,23 @@ def test_nf4_tiles_of_a_wide_range(hip, batch, loud):
     error = (y - xd @ held).abs()
     assert bool((error[:, ::2] <= nf4_bound(quiet, held, scale)[:, ::2]).all())
     assert bool((error <= nf4_bound(xd, held, scale)).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", [4, 8])
+def test_nf4_tiles_round_inputs(hip, batch):
+    """Errors of a sum of like terms cancel: scaled inputs are rounded, not cut off."""
+    k_in = 8192
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    w = torch.ones(k_in, 64, device="cuda", dtype=BF16)
+    w[::256, ::2] = 0.0
+    x = torch.rand(batch, k_in, device="cuda", generator=gen) + 1.0
+    x[:, ::256] = 1e6  # in every run: the others are then held to 2^-21 or 2^-20
+    made = hip.nf4_tile(*hip.nf4_quantize(w))
+    y = hip.gemv_nf4_tiles(*made, k_in, x, torch.empty(0, device="cuda"), None, 0).double()
+    error = (y - x.double() @ w.double())[:, ::2]  # without the large ones
+    # cut off, 2^-22 an input or more; rounded, the 32-bit sums' errors of 2^-11 now and then
+    assert abs(float(error.mean())) <= 0.5 * k_in * 2.0**-22
 
 
 @requires_gpu
