@@ -43,6 +43,9 @@
 // are, it took 0 to 5% less (8192 x 8192: 14.7, 16.1, 18.5 us without the reduction for 1, 4,
 // 8 rows beside 14.8, 16.6, 19.5). Runs with inputs beyond 64 times their mean take longer: two
 // of 8192 inputs a thousand times the rest, 15.2, 18.2, 23.6.
+// Weights are read once and marked so (non-temporal): a decoding step of four blocks of width
+// 8192 takes 589 us instead of 601 with one row, 1059 instead of 1071 with eight, one of two
+// blocks of 8 experts 301 instead of 312.
 // Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.6e-7).
 
 #include "common.h"
