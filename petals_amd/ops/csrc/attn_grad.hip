@@ -106,12 +106,14 @@ __device__ __forceinline__ void store_rotated(
   }
 }
 
-// Gradients of queries, and `dots`: each row's result times its gradient.
+// Gradients of queries, and `dots`: the mean by weight of each row's gradients of weights. It
+// is what is taken off every one of them, so a walk of its own finds it in 32 bits first: the
+// result times its gradient is the same number, but of a result that was rounded to bf16, and
+// where keys are alike its error does not cancel (up to 0.5 of the terms that should have).
 // Grid: runs of 64 rows x (batch, head) pairs.
 template <int HD>
 __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
     const unsigned short* __restrict__ qkv,  // [B, S, (QH + 2 KH) HD], rotated
-    const unsigned short* __restrict__ out,  // [B, S, QH HD]
     const unsigned short* __restrict__ go,   // [B, S, QH HD]
     const float* __restrict__ lse,           // [B, QH, S], log2
     const float* __restrict__ cos_t, const float* __restrict__ sin_t,  // [positions, HD]
@@ -131,48 +133,62 @@ __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
   const bool live = row < a.s;
 
   bf16x8 qf[RC], gf[RC];
-  float dot = 0.f, sum = 0.f;
 #pragma unroll
   for (int kc = 0; kc < RC; ++kc) {
     qf[kc] = gf[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     if (!live) continue;
     qf[kc] = *reinterpret_cast<const bf16x8*>(base + row * width + head * HD + kc * 32 + hi * 8);
     gf[kc] = *reinterpret_cast<const bf16x8*>(go + at + kc * 32 + hi * 8);
-    const bf16x8 of = *reinterpret_cast<const bf16x8*>(out + at + kc * 32 + hi * 8);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) dot = fmaf(bf16_to_f32((unsigned short)gf[kc][e]), bf16_to_f32((unsigned short)of[e]), dot);
   }
-  dot = row_sum(dot);
-  if (live) {
-    sum = lse[stat];
-    if (hi == 0) dots[stat] = dot;
-  }
+  const float sum = live ? lse[stat] : 0.f;
   f32x4 acc[VB];
 #pragma unroll
   for (int d = 0; d < VB; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int key_end = min(a.s, first + 64);
+  const int key_end = min(a.s, first + 64), tiles = (key_end + AG_TILE - 1) / AG_TILE;
   const float in = a.scale * LOG2E;
   TilePair<HD> tile;
-  tile.fetch(kp, width, vp, width, 0, key_end);
+  auto fetch = [&](int step) { tile.fetch(kp, width, vp, width, step % tiles * AG_TILE, key_end); };
+  fetch(0);
   tile.stage(smem);
   __syncthreads();
-  int which = 0;
-  for (int j0 = 0; j0 < key_end; j0 += AG_TILE, which ^= 1) {
-    const unsigned short* k_lds = smem + which * BUF;
-    const bool more = j0 + AG_TILE < key_end;
-    if (more) tile.fetch(kp, width, vp, width, j0 + AG_TILE, key_end);
-    f32x4 s[NB], ds[NB];
-    tile_product<HD>(k_lds, qf, col, hi, s);
-    tile_product<HD>(k_lds + AG_TILE * ROW, gf, col, hi, ds);
+  auto walk = [&](int from, auto&& use) {  // over all tiles, the from-th step on
+    for (int step = from; step < from + tiles; ++step) {
+      const unsigned short* k_lds = smem + (step & 1) * BUF;
+      const bool more = step + 1 < 2 * tiles;
+      if (more) fetch(step + 1);
+      f32x4 s[NB], ds[NB];
+      tile_product<HD>(k_lds, qf, col, hi, s);
+      tile_product<HD>(k_lds + AG_TILE * ROW, gf, col, hi, ds);
+      const int j0 = (step - from) * AG_TILE + hi * 4;  // key of register 0 in block 0
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[nb][r] = live && j0 + nb * 16 + r <= row ? __builtin_amdgcn_exp2f(fmaf(s[nb][r], in, -sum)) : 0.f;
+      use(k_lds, s, ds);
+      if (more) tile.stage(smem + ((step + 1) & 1) * BUF);
+      __syncthreads();
+    }
+  };
+  float dot = 0.f, weight = 0.f;
+  walk(0, [&](const unsigned short*, f32x4* s, f32x4* ds) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool seen = live && j0 + nb * 16 + hi * 4 + r <= row;
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[nb][r], in, -sum));
-        ds[nb][r] = seen ? p * (ds[nb][r] - dot) : 0.f;
+        weight += s[nb][r];
+        dot = fmaf(s[nb][r], ds[nb][r], dot);
       }
+  });
+  weight = row_sum(weight);
+  dot = row_sum(dot) / (live ? weight : 1.f);
+  if (live && hi == 0) dots[stat] = dot;
+  walk(tiles, [&](const unsigned short* k_lds, f32x4* s, f32x4* ds) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ds[nb][r] = s[nb][r] * (ds[nb][r] - dot);
 #pragma unroll
     for (int ks = 0; ks < NB / 2; ++ks) {
       bf16x8 high, low;
@@ -185,9 +201,7 @@ __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
         acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, low, acc[d], 0, 0, 0);
       }
     }
-    if (more) tile.stage(smem + (which ^ 1) * BUF);
-    __syncthreads();
-  }
+  });
   if (live)
     store_rotated<HD>(grad + ((size_t)b * a.s + row) * width + head * HD, acc, a.scale, cos_t + (size_t)(a.start + row) * HD,
                       sin_t + (size_t)(a.start + row) * HD, hi);
@@ -282,8 +296,7 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
 // -> the gradient of the projection before its rotation
 torch::Tensor attn_prompt_grad(
     torch::Tensor qkv,  // [B, S, (qh + 2 kh) * hd] bf16, rotated
-    torch::Tensor out,  // [B, S, qh * hd] bf16
-    torch::Tensor grad_out,
+    torch::Tensor grad_out,  // [B, S, qh * hd] bf16
     torch::Tensor lse,  // [B, qh, S] f32
     torch::Tensor cos_t, torch::Tensor sin_t,  // [>= start + S, hd] f32
     int64_t start, int64_t qh, int64_t kh, int64_t hd, double scale) {
@@ -291,11 +304,10 @@ torch::Tensor attn_prompt_grad(
   TORCH_CHECK(qkv.is_cuda() && qkv.dim() == 3 && kh > 0 && qh > 0 && qh % kh == 0 && start >= 0);
   const long b = qkv.size(0), s = qkv.size(1);
   TORCH_CHECK(qkv.size(2) == (qh + 2 * kh) * hd);
-  for (const auto* t : {&qkv, &out, &grad_out})
+  for (const auto* t : {&qkv, &grad_out})
     TORCH_CHECK(t->is_cuda() && t->dtype() == torch::kBFloat16 && t->is_contiguous() &&
                 reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "contiguous bf16 rows, aligned to 16 bytes, expected");
-  for (const auto* t : {&out, &grad_out})
-    TORCH_CHECK(t->dim() == 3 && t->size(0) == b && t->size(1) == s && t->size(2) == qh * hd);
+  TORCH_CHECK(grad_out.dim() == 3 && grad_out.size(0) == b && grad_out.size(1) == s && grad_out.size(2) == qh * hd);
   TORCH_CHECK(lse.is_cuda() && lse.dtype() == torch::kFloat32 && lse.is_contiguous() && lse.numel() == b * qh * s);
   for (const auto* t : {&cos_t, &sin_t})
     TORCH_CHECK(t->is_cuda() && t->dtype() == torch::kFloat32 && t->is_contiguous() && t->dim() == 2 && t->size(1) == hd &&
@@ -314,7 +326,7 @@ torch::Tensor attn_prompt_grad(
     allow_lds(&attn_grad_q_kernel<HD>, lds);                                                                        \
     allow_lds(&attn_grad_kv_kernel<HD>, lds);                                                                       \
     attn_grad_q_kernel<HD><<<runs * b * qh, 256, lds, stream>>>(                                                    \
-        bf(qkv), bf(out), bf(grad_out), lse.data_ptr<float>(), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),    \
+        bf(qkv), bf(grad_out), lse.data_ptr<float>(), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(),    \
         bf(grad), dots.data_ptr<float>(), a);                                                                       \
     attn_grad_kv_kernel<HD><<<runs * b * kh, 256, lds, stream>>>(                                                   \
         bf(qkv), bf(grad_out), lse.data_ptr<float>(), dots.data_ptr<float>(), cos_t.data_ptr<float>(),              \

@@ -34,7 +34,7 @@ torch::Tensor attn_prefill_fused(
     c10::optional<torch::Tensor> alibi_slopes);
 std::vector<torch::Tensor> attn_prefill_sums(torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale);
 torch::Tensor attn_prompt_grad(
-    torch::Tensor qkv, torch::Tensor out, torch::Tensor grad_out, torch::Tensor lse, torch::Tensor cos_t,
+    torch::Tensor qkv, torch::Tensor grad_out, torch::Tensor lse, torch::Tensor cos_t,
     torch::Tensor sin_t, int64_t start, int64_t qh, int64_t kh, int64_t hd, double scale);
 torch::Tensor rotate_rows(
     torch::Tensor qkv, torch::Tensor cos_t, torch::Tensor sin_t, int64_t start, int64_t qh, int64_t kh, int64_t hd);

@@ -144,18 +144,18 @@ class _Attention(torch.autograd.Function):
         rows = hip.rotate_rows(aligned(qkv), cos, sin, start, qh, kh, hd)
         heads = rows.view(*rows.shape[:2], qh + 2 * kh, hd).transpose(1, 2)
         out, sums = hip.attn_prefill_sums(heads[:, :qh], heads[:, qh : qh + kh], heads[:, qh + kh :], scale)
-        ctx.save_for_backward(qkv, rows, out, sums)
+        ctx.save_for_backward(qkv, rows, sums)
         ctx.tables = cos, sin  # constants, maybe made in inference mode: such tensors can't be saved
         ctx.shape, ctx.scale, ctx.hip = (start, qh, kh, hd), scale, hip
         return out
 
     @staticmethod
     def backward(ctx, g):
-        (qkv, rows, out, sums), (cos, sin) = ctx.saved_tensors, ctx.tables
+        (qkv, rows, sums), (cos, sin) = ctx.saved_tensors, ctx.tables
         none = (None,) * 8
         if _by_torch(g):
             return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
-        return (ctx.hip.attn_prompt_grad(rows, out, aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
+        return (ctx.hip.attn_prompt_grad(rows, aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 
 
 def norm(x, w, eps, hip):

@@ -553,6 +553,39 @@ def test_prompt_attention_gradients(hip, hd, b, s, qh, kh, start):
     assert bool(err.norm() <= 2.0**-7 * want.norm())  # and roundings don't all add up
 
 
+def cancelling_gradient(hip, hd, s, spread):
+    """Gradients of queries whose keys are all alike, so that nothing is left of them, beside what
+    they are sums of: [b, qh, s] sums of p (|dP| + |dot|), of p |dP - dot|, and of the gradient."""
+    from petals_amd.ops import prompt_grad
+
+    gen = torch.Generator(device="cuda").manual_seed(s + hd)
+    b, qh, kh = 2, 4, 2
+    cos, sin = torch.ones(s, hd, device="cuda"), torch.zeros(s, hd, device="cuda")
+    heads = torch.randn(b, s, qh + 2 * kh, hd, device="cuda", generator=gen)
+    heads[:, :, qh : qh + kh] = heads[:, :1, qh : qh + kh]
+    heads[:, :, qh + kh :] = heads[:, :1, qh + kh :] + spread * heads[:, :, qh + kh :]
+    qkv = heads.view(b, s, -1).to(BF16).requires_grad_(True)
+    g = torch.randn(b, s, qh * hd, device="cuda", generator=gen).to(BF16)
+    (got,) = _gradients([prompt_grad.attention(qkv, cos, sin, 0, qh, kh, hd, hd**-0.5, hip)], [qkv], [g])
+    heads = qkv.detach().double().view(b, s, -1, hd).transpose(1, 2)
+    k, v = (t.repeat_interleave(qh // kh, 1) for t in (heads[:, qh : qh + kh], heads[:, qh + kh :]))
+    dp = torch.matmul(g.double().view(b, s, qh, hd).transpose(1, 2), v.transpose(2, 3).contiguous())
+    p = torch.ones(s, s, device="cuda", dtype=torch.float64).tril()
+    p = p / p.sum(-1, keepdim=True)  # scores are alike, too
+    dot = (p * dp).sum(-1, keepdim=True)
+    left = got.double().view(b, s, -1, hd)[:, :, :qh].transpose(1, 2) / k * hd**0.5
+    return (p * (dp.abs() + dot.abs())).sum(-1), left.abs().amax(-1)
+
+
+@requires_gpu
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("s", [8, 70, 200])
+def test_score_gradients_add_up_to_nothing(hip, hd, s):
+    """With values far from zero: the mean that is taken off is that of the same 32-bit terms."""
+    sums, left = cancelling_gradient(hip, hd, s, 0.01)
+    assert bool((left <= 2.0**-18 * sums).all())
+
+
 def near(got, want, rel):
     assert (got.double() - want.double()).norm() <= rel * want.double().norm()
 

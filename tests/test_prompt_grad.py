@@ -67,7 +67,7 @@ class Kernels:
         shape = (START, QH, KH, HD)
         return prompt_grad.torch_attention(self.projection, COS, SIN, *shape).detach(), torch.zeros(1)
 
-    def attn_prompt_grad(self, rows, out, g, sums, cos, sin, start, qh, kh, hd, scale):
+    def attn_prompt_grad(self, rows, g, sums, cos, sin, start, qh, kh, hd, scale):
         return self._pull(lambda t: prompt_grad.torch_attention(t, cos, sin, start, qh, kh, hd), rows, g)
 
 
