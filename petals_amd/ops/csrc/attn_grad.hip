@@ -8,13 +8,14 @@
 // the others, which four waves share in LDS, the next tile's loads in flight. Weights are
 // made again from the scores, nothing of size rows x keys is ever in memory; weights and
 // score gradients are the next product's operand without leaving their registers, as in
-// paged_attn.h. Score gradients enter their products as two bf16 values, high and low (16
-// bits of mantissa): products with 32-bit score gradients are what the results are to
-// match. A workgroup of keys goes over all heads that share them.
+// paged_attn.h. Score gradients enter their products as three bf16 values, which hold all 24
+// bits: products with 32-bit score gradients are what the results are to match. A workgroup
+// of keys goes over all heads that share them.
 //
 // 32 heads of 128, 2 x 379 tokens: from the result's gradient back to the projection's it was
 // 42 launches of torch operations over [heads, rows, keys] in 32 bits and over copies of
-// rows, 419 us; the two kernels take 21 and 44 us. At this size they are bound by the chain
+// rows, 419 us; the two kernels take 71 us (61 with the mean of a row's gradients taken from
+// its rounded result, and score gradients of 16 bits). At this size they are bound by the chain
 // of a workgroup's tiles (six, and six times the heads that share keys): 384 workgroups for
 // 256 compute units, 1.3 GFLOP of products.
 
@@ -73,16 +74,18 @@ __device__ __forceinline__ void tile_product(const unsigned short* lds, const bf
   }
 }
 
-// v = high + low to 16 bits
-__device__ __forceinline__ void split_operand(const f32x4& a, const f32x4& b, bf16x8& high, bf16x8& low) {
-  high = weight_operand(a, b);
-  f32x4 ra, rb;
+// v = p[0] + p[1] + p[2], all its 24 bits
+__device__ __forceinline__ void split_operand(const f32x4& a, const f32x4& b, bf16x8* p) {
+  f32x4 ra = a, rb = b;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    ra[r] = a[r] - bf16_to_f32((unsigned short)high[r]);
-    rb[r] = b[r] - bf16_to_f32((unsigned short)high[r + 4]);
+  for (int i = 0; i < 3; ++i) {
+    p[i] = weight_operand(ra, rb);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      ra[r] -= bf16_to_f32((unsigned short)p[i][r]);
+      rb[r] -= bf16_to_f32((unsigned short)p[i][r + 4]);
+    }
   }
-  low = weight_operand(ra, rb);
 }
 
 // sums over a head's dims x 16 columns: a lane has one column and 4 neighbouring dims a block
@@ -191,14 +194,14 @@ __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
       for (int r = 0; r < 4; ++r) ds[nb][r] = s[nb][r] * (ds[nb][r] - dot);
 #pragma unroll
     for (int ks = 0; ks < NB / 2; ++ks) {
-      bf16x8 high, low;
-      split_operand(ds[2 * ks], ds[2 * ks + 1], high, low);
+      bf16x8 parts[3];
+      split_operand(ds[2 * ks], ds[2 * ks + 1], parts);
       const unsigned short* t = k_lds + (ks * 32 + hi * 4 + col / 4) * ROW + (col & 3) * 4;
 #pragma unroll
       for (int d = 0; d < VB; ++d) {
         const bf16x8 kt = load_values(t + d * 16, ROW);
-        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, high, acc[d], 0, 0, 0);
-        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, low, acc[d], 0, 0, 0);
+#pragma unroll
+        for (int i = 2; i >= 0; --i) acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, parts[i], acc[d], 0, 0, 0);
       }
     }
   });
@@ -270,15 +273,15 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
 #pragma unroll
     for (int ks = 0; ks < NB / 2; ++ks) {
       const bf16x8 pf = weight_operand(s[2 * ks], s[2 * ks + 1]);
-      bf16x8 high, low;
-      split_operand(ds[2 * ks], ds[2 * ks + 1], high, low);
+      bf16x8 parts[3];
+      split_operand(ds[2 * ks], ds[2 * ks + 1], parts);
       const int t = (ks * 32 + hi * 4 + col / 4) * ROW + (col & 3) * 4;
 #pragma unroll
       for (int d = 0; d < VB; ++d) {
         dv[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_values(g_lds + t + d * 16, ROW), pf, dv[d], 0, 0, 0);
         const bf16x8 qt = load_values(q_lds + t + d * 16, ROW);
-        dk[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qt, high, dk[d], 0, 0, 0);
-        dk[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qt, low, dk[d], 0, 0, 0);
+#pragma unroll
+        for (int i = 2; i >= 0; --i) dk[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qt, parts[i], dk[d], 0, 0, 0);
       }
     }
     if (more) tile.stage(smem + ((step + 1) & 1) * BUF);

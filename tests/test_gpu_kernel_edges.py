@@ -586,6 +586,14 @@ def test_score_gradients_add_up_to_nothing(hip, hd, s):
     assert bool((left <= 2.0**-18 * sums).all())
 
 
+@requires_gpu
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("s", [8, 70, 200])
+def test_score_gradients_keep_32_bits(hip, hd, s):
+    sums, left = cancelling_gradient(hip, hd, s, 1.0)
+    assert bool((left <= 2.0**-21 * sums).all())
+
+
 def near(got, want, rel):
     assert (got.double() - want.double()).norm() <= rel * want.double().norm()
 
