@@ -1,7 +1,8 @@
 // Decode-path GEMV suite for CDNA4 (gfx950).
 //
 // Weights are stored TRANSPOSED: Wt[in, out] bf16 row-major (= W^T). Matrices whose rows
-// are aligned to 16 bytes take the kernel in gemv_mfma.h. The one here takes any other: a
+// are aligned to 16 bytes take the kernel in gemv_mfma.h. The one here takes any other, and
+// any number of parts that a caller asks for: a
 // wave owns a strip of 512 output columns (8 per lane) and iterates over a chunk of the
 // input dimension; x[i] is a wave-uniform scalar load (s_load, L2-resident) broadcast into
 // 8 FMAs.
@@ -191,9 +192,11 @@ torch::Tensor gemv_bf16(
   const int batch = x.size(0);
   TORCH_CHECK(batch <= 8, "decode gemv supports batch <= 8");
 
-  // the matrix cores wherever rows can be read 16 bytes at a time; they choose their splits
-  torch::Tensor partials = gemv_mfma_fits(wt, out_dim) ? launch_gemv_mfma(wt, x, nullptr, 1, workspace)
-                                                       : launch_gemv_rows(wt, x, workspace, splits_override);
+  // the matrix cores wherever rows can be read 16 bytes at a time and the number of parts is
+  // theirs to choose
+  const bool mfma = splits_override <= 0 && gemv_mfma_fits(wt, out_dim);
+  torch::Tensor partials = mfma ? launch_gemv_mfma(wt, x, nullptr, 1, workspace)
+                                : launch_gemv_rows(wt, x, workspace, splits_override);
   const int splits = (int)partials.size(0);
 
   // epilogue (shared with the NF4 path)

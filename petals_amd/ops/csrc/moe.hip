@@ -682,7 +682,7 @@ torch::Tensor gemv_bf16_moe(
   const int rows = sel.size(0);
   TORCH_CHECK(x.size(1) == in_dim && rows == x.size(0) * k_per_tok);
   TORCH_CHECK(rows <= 64, "moe gemv supports batch*k <= 64");
-  if (gemv_mfma_fits(wt_all, out_dim)) {
+  if (splits_override <= 0 && gemv_mfma_fits(wt_all, out_dim)) {
     auto sums = launch_gemv_mfma(wt_all, x, &sel, k_per_tok, workspace);
     if (epilogue < 0) return sums;  // [splits, rows, out]
     return launch_gemv_reduce(

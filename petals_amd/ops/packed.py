@@ -118,14 +118,10 @@ class PackedBlock:
 
     # ---------------------------------------------------------------- products
 
-    def _splits(self, w: torch.Tensor) -> int:
-        # 64 input rows a wave keeps the loads of a short gemv in flight
-        return max(1, min(w.shape[0] // 64, 1024 // (-(-w.shape[1] // 512))))
-
     def _dense(self, x, w, few: bool, epilogue: int = _EPI_PLAIN_F32, bias=None):
         """x [T, in] (32-bit if few rows or float32, else the weight dtype) @ w [in, out]."""
         if few:
-            return self.hip.gemv_bf16(w, x, self._no_ws, None, epilogue, self._splits(w), bias)
+            return self.hip.gemv_bf16(w, x, self._no_ws, None, epilogue, 0, bias)
         return x @ w
 
     def _parts(self, x, w):

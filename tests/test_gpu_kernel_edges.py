@@ -210,6 +210,23 @@ def test_gemv_against_64_bits(hip, k_in, n_out, batch):
 
 
 @requires_gpu
+@pytest.mark.parametrize("splits", [1, 3, 8])
+def test_gemv_in_as_many_parts_as_asked_for(hip, splits):
+    gen = torch.Generator(device="cuda").manual_seed(splits)
+    k_in, n_out = 768, 256
+    w = torch.randn(2, k_in, n_out, device="cuda", generator=gen).to(BF16)
+    x = torch.randn(3, k_in, device="cuda", generator=gen)
+    empty, sel = torch.empty(0, device="cuda"), torch.tensor([1, 0, 1], dtype=torch.int32, device="cuda")
+    parts = hip.gemv_bf16(w[0], x, empty, None, -1, splits)
+    assert parts.shape == (splits, 3, n_out)
+    ref = x.double() @ w[0].double()
+    bound = k_in * 2.0**-24 * (x.double().abs() @ w[0].double().abs())  # 32-bit sums in any order
+    assert bool(((parts.double().sum(0) - ref).abs() <= bound).all())
+    # experts' parts have 256 inputs or more
+    assert hip.gemv_bf16_moe(w, x, sel, 1, empty, -1, splits).shape == (min(splits, 3), 3, n_out)
+
+
+@requires_gpu
 def test_gemv_infinities(hip):
     gen = torch.Generator(device="cuda").manual_seed(3)
     w = torch.randn(200, 136, device="cuda", generator=gen).to(BF16)
