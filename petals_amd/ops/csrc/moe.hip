@@ -146,9 +146,21 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
   }
   __syncthreads();
   if (wave != 0) return;
-  float v[ROUTE_EXPERTS / WAVE];  // of this lane's experts; chosen ones drop out
+  // Of this lane's experts; chosen ones drop out. A softmax of infinities or NaNs has NaNs for
+  // all, but for logits below every number among others: those count as just above the sentinel.
+  float v[ROUTE_EXPERTS / WAVE];
+  bool odd = false, some = false;
 #pragma unroll
-  for (int i = 0; i < ROUTE_EXPERTS / WAVE; ++i) v[i] = lane + i * WAVE < experts ? logits[lane + i * WAVE] : NEG_SENTINEL;
+  for (int i = 0; i < ROUTE_EXPERTS / WAVE; ++i) {
+    v[i] = NEG_SENTINEL;
+    if (lane + i * WAVE >= experts) continue;
+    const unsigned bits = __float_as_uint(logits[lane + i * WAVE]);
+    const bool finite = (bits & 0x7FFFFFFFu) < 0x7F800000u;
+    odd |= !finite && bits != 0xFF800000u;
+    some |= finite;
+    v[i] = finite ? fmaxf(__uint_as_float(bits), NEG_THRESHOLD) : NEG_THRESHOLD;
+  }
+  odd = __any(odd) || !__any(some);
   float first = 0.f, total = 0.f, mine = 0.f;
   int chosen = 0;
   for (int j = 0; j < top; ++j) {
@@ -173,7 +185,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     if (lane == j) mine = p, chosen = at;
   }
   if (lane < top) {
-    weights[(size_t)blockIdx.x * top + lane] = mine / total;
+    weights[(size_t)blockIdx.x * top + lane] = odd ? __uint_as_float(0x7FC00000u) : mine / total;
     sel[(size_t)blockIdx.x * top + lane] = chosen;
   }
 }

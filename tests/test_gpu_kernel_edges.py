@@ -444,6 +444,30 @@ def test_router(hip, dtype, tokens, dim, experts, top):
 
 
 @requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, BF16])
+def test_router_of_infinities(hip, dtype):
+    """Weights that a softmax has no numbers for are NaNs, and experts are always some."""
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    w = torch.randn(70, 64, device="cuda", generator=gen).to(BF16)
+    x = torch.randn(6, 64, device="cuda", generator=gen).to(dtype)
+    x[1, 3], x[2, 5], x[3, 7] = float("nan"), float("inf"), float("-inf")
+    x[4, 9], w[:, 9] = float("inf"), -w[:, 9].abs()  # all logits below every number
+    for spoilt in (False, True):
+        if spoilt:
+            w[66, 0] = float("nan")  # one expert's logits
+        weights, sel = (t.cpu() for t in hip.moe_route(x, w, 3))
+        logits = (x.double() @ w.double().t()).cpu()
+        best, chosen = torch.topk(torch.softmax(logits, -1), 3, dim=-1)
+        want = best / best.sum(-1, keepdim=True)
+        assert torch.equal(torch.isnan(weights), torch.isnan(want))
+        assert bool(((sel >= 0) & (sel < 70)).all()) and all(len(set(row.tolist())) == 3 for row in sel)
+        fine = ~torch.isnan(want)
+        assert torch.allclose(weights[fine].double(), want[fine], atol=1e-3)
+        assert torch.equal(sel[fine].long(), chosen[fine])
+        assert fine.any() != spoilt
+
+
+@requires_gpu
 @pytest.mark.parametrize("tokens,top,splits,width", [(1, 1, 1, 8), (3, 2, 5, 72), (2, 3, 7, 4096), (130, 2, 1, 128)])
 def test_expert_sums(hip, tokens, top, splits, width):
     gen = torch.Generator(device="cuda").manual_seed(width)
