@@ -285,6 +285,22 @@ def _takes_rows(cache: torch.Tensor) -> bool:
     return cache.stride(3) == 1 and cache.data_ptr() % 16 == 0 and all(cache.stride(i) % 8 == 0 for i in range(3))
 
 
+def add_norm(hip, x, y, y_bias, w, b, eps):
+    """(x + y + y_bias, its layer norm, or RMS norm without b) of a prompt's rows"""
+    if _rows_fit(x.shape[-1]):
+        return hip.add_norm_rows(x, y, y_bias, w, b, eps)
+    h = x + y if y_bias is None else x + (y + y_bias)
+    return h, hip.rms_norm(h, w, eps) if b is None else hip.layer_norm(h, w, b, eps)
+
+
+def bias_gelu(hip, y, bias=None):
+    """gelu(y + bias) of a prompt's rows, maybe in their place"""
+    if y.shape[-1] % 8 == 0:
+        hip.bias_gelu_rows(y, bias)
+        return y
+    return reference.gelu((y if bias is None else y + bias).float()).to(torch.bfloat16)
+
+
 def prompt_attention(hip, qkv, kv_cache, prefix, qh, kh, hd, scale, bias=None, cos=None, sin=None, slopes=None):
     """Causal attention of a prompt's fused projection [B, S, (qh + 2 kh) * hd], which is
     overwritten; keys and values go to the cache, if there is one. -> [B, S, qh * hd]"""
@@ -876,19 +892,17 @@ class BloomFastPath(_TPFastPathMixin):
         v = qkv[..., 2 * qd :].view(B, S, self.kh, self.hd).transpose(1, 2)
         return q, k, v
 
-    def _body(self, hidden, kv_cache, prefix_length, autograd: bool, adapter=None):
+    def forward_autograd(self, hidden, prefix_length: int = 0, adapter=None):
+        """Differentiable forward on the transposed weights, by torch operations."""
+        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
         B, S, H = hidden.shape
         hidden = hidden.to(torch.bfloat16)
         end = prefix_length + S
         fln = torch.nn.functional.layer_norm
 
         def ln(x, w, b):
-            if autograd or x.device.type != "cuda":
-                return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
-            return self.hip.layer_norm(x, w, b, self.eps)
+            return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
 
-        if not autograd and hidden.device.type == "cuda" and _rows_fit(H) and self.w_h4h.out_dim % 8 == 0:
-            return self._prompt(prompt_grad.aligned(hidden), kv_cache, prefix_length, adapter)
         xn = ln(hidden, self.ln1_w, self.ln1_b)
         res1 = xn if self.post_ln_residual else hidden
         xn = self._tp_copy(xn)
@@ -898,23 +912,10 @@ class BloomFastPath(_TPFastPathMixin):
             if d is not None:
                 qkv = qkv + d.to(qkv.dtype)[..., self._qkv_perm]
         q, k, v = self._split_heads(qkv, B, S)
-        if kv_cache is not None and not autograd:
-            k_cache, v_cache = kv_cache
-            k_cache[:B, :, prefix_length:end].copy_(k)
-            v_cache[:B, :, prefix_length:end].copy_(v)
-            attn = self.hip.attn_prefill_fused(
-                q.contiguous(), k_cache[:B].contiguous(), v_cache[:B].contiguous(),
-                end, prefix_length, self.scale, True, self.slopes,
-            )
-        elif not autograd and hidden.device.type == "cuda":
-            attn = self.hip.attn_prefill_fused(
-                q.contiguous(), k.contiguous(), v.contiguous(), S, 0, self.scale, True, self.slopes
-            )
-        else:
-            k_pos = torch.arange(end, device=hidden.device, dtype=torch.float32)
-            bias = (self.slopes.to(hidden.device)[:, None, None] * k_pos[None, None, :]).unsqueeze(0)
-            attn = reference.attention(q.float(), k.float(), v.float(), causal=True,
-                                       kv_offset=prefix_length, attn_bias=bias.float())
+        k_pos = torch.arange(end, device=hidden.device, dtype=torch.float32)
+        bias = (self.slopes.to(hidden.device)[:, None, None] * k_pos[None, None, :]).unsqueeze(0)
+        attn = reference.attention(q.float(), k.float(), v.float(), causal=True,
+                                   kv_offset=prefix_length, attn_bias=bias.float())
         attn = attn.transpose(1, 2).reshape(B, S, self.qh * self.hd).to(torch.bfloat16)
         o = torch.matmul(attn, self.wo_t.dense()) + self.o_bias
         if adapter is not None:
@@ -938,9 +939,10 @@ class BloomFastPath(_TPFastPathMixin):
                 out = out + d4.to(out.dtype)
         return res2 + self._tp_reduce(out)
 
-    def _prompt(self, hidden, kv_cache, prefix_length, adapter):
+    def forward(self, hidden, kv_cache, prefix_length, adapter=None):
         """The same without gradients: one kernel for each gap between dense products."""
-        hip = self.hip
+        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
+        hip, hidden = self.hip, prompt_grad.aligned(hidden.to(torch.bfloat16))
         xn = hip.layer_norm(hidden, self.ln1_w, self.ln1_b, self.eps)
         qkv = torch.matmul(xn, self.wqkv_t.dense())
         if adapter is not None:
@@ -958,30 +960,22 @@ class BloomFastPath(_TPFastPathMixin):
         res1, o_bias = (xn if self.post_ln_residual else hidden), self.o_bias
         if self.tp_world > 1:
             o, o_bias = self._tp_reduce(o + o_bias), None
-        h2, xn2 = hip.add_norm_rows(res1, o, o_bias, self.ln2_w, self.ln2_b, self.eps)
+        h2, xn2 = add_norm(hip, res1, o, o_bias, self.ln2_w, self.ln2_b, self.eps)
         res2 = xn2 if self.post_ln_residual else h2
         inter = torch.matmul(xn2, self.w_h4h.dense())
         if adapter is not None:
             dh = adapter.delta("h4h", xn2)
             if dh is not None:
                 inter = inter + dh.to(inter.dtype)
-        hip.bias_gelu_rows(inter, self.b_h4h)
-        out = torch.matmul(inter, self.w_4hh.dense())
+        act = bias_gelu(hip, inter, self.b_h4h)
+        out = torch.matmul(act, self.w_4hh.dense())
         if adapter is not None:
-            d4 = adapter.delta("4hh", inter)
+            d4 = adapter.delta("4hh", act)
             if d4 is not None:
                 out = out + d4.to(out.dtype)
         if self.tp_world > 1:
             return res2 + self._tp_reduce(out + self.b_4hh)
         return hip.add_rows(res2, out, None, self.b_4hh)
-
-    def forward(self, hidden, kv_cache, prefix_length, adapter=None):
-        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
-        return self._body(hidden, kv_cache, prefix_length, autograd=False, adapter=adapter)
-
-    def forward_autograd(self, hidden, prefix_length: int = 0, adapter=None):
-        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
-        return self._body(hidden, None, prefix_length, autograd=True, adapter=adapter)
 
 
 # ---------------------------------------------------------------------------
@@ -1153,7 +1147,9 @@ class FalconFastPath(_TPFastPathMixin):
         v = qkv[..., qd + kd :].view(B, S, self.kh, self.hd).transpose(1, 2)
         return q, k, v
 
-    def _body(self, hidden, kv_cache, prefix_length, autograd: bool, adapter=None):
+    def forward_autograd(self, hidden, prefix_length: int = 0, adapter=None):
+        """Differentiable forward on the transposed weights, by torch operations."""
+        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
         B, S, H = hidden.shape
         hidden = hidden.to(torch.bfloat16)
         end = prefix_length + S
@@ -1161,13 +1157,8 @@ class FalconFastPath(_TPFastPathMixin):
         fln = torch.nn.functional.layer_norm
 
         def ln(x, w, b):
-            if autograd or x.device.type != "cuda":
-                return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
-            return self.hip.layer_norm(x, w, b, self.eps)
+            return fln(x.float(), (H,), w.float(), b.float(), self.eps).to(torch.bfloat16)
 
-        rows_fit = _rows_fit(H) and self.w_h4h.out_dim % 8 == 0
-        if not autograd and hidden.device.type == "cuda" and self.tp_world == 1 and rows_fit:
-            return self._prompt(prompt_grad.aligned(hidden), kv_cache, prefix_length, adapter)
         xn_attn = self._tp_copy(ln(hidden, self.ln_attn_w, self.ln_attn_b))
         xn_mlp = xn_attn if self.single_ln else self._tp_copy(ln(hidden, self.ln_mlp_w, self.ln_mlp_b))
         qkv = torch.matmul(xn_attn, self.wqkv_t.dense())
@@ -1177,24 +1168,8 @@ class FalconFastPath(_TPFastPathMixin):
                 qkv = qkv + d.to(qkv.dtype)[..., self._qkv_perm]
         q, k, v = self._split_heads(qkv, B, S)
         pos = torch.arange(prefix_length, end, device=hidden.device)
-        if autograd:
-            q, k = reference.apply_rope(q, k, self.rope_cos, self.rope_sin, pos)
-            attn = reference.attention(q.float(), k.float(), v.float(), causal=True, kv_offset=prefix_length)
-        else:
-            posb = pos.unsqueeze(0).expand(B, S).contiguous()
-            q, k = self.hip.apply_rope(q.contiguous(), k.contiguous(), self.rope_cos, self.rope_sin, posb)
-            if kv_cache is not None:
-                k_cache, v_cache = kv_cache
-                k_cache[:B, :, prefix_length:end].copy_(k)
-                v_cache[:B, :, prefix_length:end].copy_(v)
-                attn = self.hip.attn_prefill_fused(
-                    q.contiguous(), k_cache[:B].contiguous(), v_cache[:B].contiguous(),
-                    end, prefix_length, self.scale, True,
-                )
-            else:
-                attn = self.hip.attn_prefill_fused(
-                    q.contiguous(), k.contiguous(), v.contiguous(), S, 0, self.scale, True
-                )
+        q, k = reference.apply_rope(q, k, self.rope_cos, self.rope_sin, pos)
+        attn = reference.attention(q.float(), k.float(), v.float(), causal=True, kv_offset=prefix_length)
         attn = attn.transpose(1, 2).reshape(B, S, self.qh * self.hd).to(torch.bfloat16)
         o = torch.matmul(attn, self.wo_t.dense())
         inter = torch.matmul(xn_mlp, self.w_h4h.dense())
@@ -1213,9 +1188,11 @@ class FalconFastPath(_TPFastPathMixin):
                 mlp_out = mlp_out + d4.to(mlp_out.dtype)
         return hidden + self._tp_reduce(o + mlp_out)
 
-    def _prompt(self, hidden, kv_cache, prefix_length, adapter):
+    def forward(self, hidden, kv_cache, prefix_length, adapter=None):
         """The same without gradients: one kernel for each gap between dense products."""
-        hip = self.hip
+        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
+        hip, hidden = self.hip, prompt_grad.aligned(hidden.to(torch.bfloat16))
+        self._ensure_rope(prefix_length + hidden.shape[1])
         xn_attn = hip.layer_norm(hidden, self.ln_attn_w, self.ln_attn_b, self.eps)
         xn_mlp = xn_attn if self.single_ln else hip.layer_norm(hidden, self.ln_mlp_w, self.ln_mlp_b, self.eps)
         qkv = torch.matmul(xn_attn, self.wqkv_t.dense())
@@ -1235,18 +1212,12 @@ class FalconFastPath(_TPFastPathMixin):
             dh = adapter.delta("h4h", xn_mlp)
             if dh is not None:
                 inter = inter + dh.to(inter.dtype)
-        hip.bias_gelu_rows(inter)
-        out = torch.matmul(inter, self.w_4hh.dense())
+        act = bias_gelu(hip, inter)
+        out = torch.matmul(act, self.w_4hh.dense())
         if adapter is not None:
-            d4 = adapter.delta("4hh", inter)
+            d4 = adapter.delta("4hh", act)
             if d4 is not None:
                 out = out + d4.to(out.dtype)
+        if self.tp_world > 1:  # parallel residual: one all-reduce for both partial sums
+            return hidden + self._tp_reduce(o + out)
         return hip.add_rows(hidden, o, out)
-
-    def forward(self, hidden, kv_cache, prefix_length, adapter=None):
-        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
-        return self._body(hidden, kv_cache, prefix_length, autograd=False, adapter=adapter)
-
-    def forward_autograd(self, hidden, prefix_length: int = 0, adapter=None):
-        assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
-        return self._body(hidden, None, prefix_length, autograd=True, adapter=adapter)
