@@ -595,6 +595,7 @@ torch::Tensor moe_combine(torch::Tensor rows, torch::Tensor weights, torch::Tens
   return y;
 }
 
+// sel [R] expert of each (token, slot) pair -> (sorted_pairs, tile_expert) as moe_gemm takes them
 std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t mt) {
   TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());
   TORCH_CHECK(experts >= 1 && experts <= 4096 && mt >= 1);

@@ -506,7 +506,6 @@ torch::Tensor clamped_swiglu(torch::Tensor gu, double limit, double alpha) {
   return out;
 }
 
-// sel [R] expert of each (token, slot) pair -> (sorted_pairs, tile_expert), see moe.hip
 torch::Tensor moe_linear_f32(torch::Tensor w, torch::Tensor x, torch::Tensor sel, int64_t k) {
   TORCH_CHECK(is_f32(w) && is_f32(x) && w.dim() == 3 && x.dim() == 2 && w.is_contiguous() && x.is_contiguous());
   TORCH_CHECK(sel.is_cuda() && sel.dtype() == torch::kInt32 && sel.is_contiguous());

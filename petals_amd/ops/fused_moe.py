@@ -29,36 +29,12 @@ from petals_amd.ops.fused_decode import (
     _EPI_SWIGLU_F32,
     LlamaFastPath,
     _FastWeight,
-    _vector,
     _dequant_cached,
+    _vector,
 )
 
 
 MOE_GEMM_MT = 32  # rows of a tile of one expert (ops/csrc/moe.hip MOE_MT)
-
-
-def sort_pairs_by_expert(selected: torch.Tensor, num_experts: int):
-    """Expert-sorted (token, slot) pair ids with each expert's segment padded
-    to MT rows, so every MT-row GEMM tile belongs to one expert (all device
-    ops — no host sync; the pad buffer is sized by the static upper bound).
-    Returns (sorted_pairs [Rp] i32 with -1 padding, tile_expert [Rp/MT] i32)."""
-    MT = MOE_GEMM_MT
-    dev = selected.device
-    sel = selected.reshape(-1)  # [R] expert per pair
-    R = sel.shape[0]
-    order = torch.argsort(sel, stable=True)
-    sel_sorted = sel[order]
-    counts = torch.bincount(sel, minlength=num_experts)
-    padded = (counts + MT - 1) // MT * MT
-    pad_off = torch.cumsum(padded, 0) - padded       # padded segment starts
-    unpad_off = torch.cumsum(counts, 0) - counts     # unpadded segment starts
-    slot = pad_off[sel_sorted] + (torch.arange(R, device=dev) - unpad_off[sel_sorted])
-    rp = (R + num_experts * (MT - 1) + MT - 1) // MT * MT  # static upper bound
-    sorted_pairs = torch.full((rp,), -1, dtype=torch.int32, device=dev)
-    sorted_pairs[slot] = order.to(torch.int32)
-    tile_expert = torch.full((rp // MT,), -1, dtype=torch.int32, device=dev)
-    tile_expert[slot // MT] = sel_sorted.to(torch.int32)
-    return sorted_pairs, tile_expert
 
 
 class _CacheKey:

@@ -4,6 +4,8 @@ against plain 32-bit or 64-bit references."""
 import pytest
 import torch
 
+from expert_pairs import sort_pairs_by_expert
+
 pytestmark = pytest.mark.gpu
 
 requires_gpu = pytest.mark.skipif(not torch.cuda.is_available(), reason="needs MI355X")
@@ -44,7 +46,7 @@ def test_swiglu_writes_every_value(hip, n):
     ],
 )
 def test_expert_gemm_group_edges(hip, quant, counts, k_in, n_out):
-    from petals_amd.ops.fused_moe import _StackedExperts, sort_pairs_by_expert
+    from petals_amd.ops.fused_moe import MOE_GEMM_MT, _StackedExperts
 
     gen = torch.Generator(device="cuda").manual_seed(sum(counts) + n_out)
     experts = len(counts)
@@ -55,8 +57,12 @@ def test_expert_gemm_group_edges(hip, quant, counts, k_in, n_out):
     sel = torch.cat([torch.full((n,), e, device="cuda") for e, n in enumerate(counts)])
     sel = sel[torch.randperm(len(sel), device="cuda", generator=gen)].view(-1, 1)
     x = torch.randn(len(sel), k_in, device="cuda", generator=gen).to(BF16)
-    order, tiles = sort_pairs_by_expert(sel, experts)
-    out = st.moe_gemm(x, order, tiles, 1, len(sel)).double()
+    order, tiles = sort_pairs_by_expert(sel, experts, MOE_GEMM_MT)
+    out = st.moe_gemm(x, order, tiles, 1, len(sel))
+    # by the kernel that prompts use, which leaves fewer unused tiles
+    order, tiles = hip.moe_group(sel.view(-1).to(torch.int32), experts, MOE_GEMM_MT)
+    assert torch.equal(st.moe_gemm(x, order, tiles, 1, len(sel)), out)
+    out = out.double()
     for e in range(experts):
         rows = torch.where(sel[:, 0] == e)[0]
         if len(rows):
@@ -363,6 +369,33 @@ def test_rows_between_products(hip, rows, width):
         t = x.clone()
         hip.bias_gelu_rows(t, bias)
         close(t, fn.gelu(x.double() + (0.0 if bias is None else c.double()), approximate="tanh"))
+
+
+@requires_gpu
+@pytest.mark.parametrize("width", [20, 4100, 16384, 16392])
+@pytest.mark.parametrize("biased", [False, True])
+def test_rows_of_any_width(hip, width, biased):
+    """Shards of uneven sizes, and rows that are too long for a norm's registers."""
+    from petals_amd.ops.fused_decode import add_norm, bias_gelu
+
+    gen = torch.Generator(device="cuda").manual_seed(width)
+    x, y = (torch.randn(3, width, device="cuda", generator=gen).to(BF16) for _ in range(2))
+    c, w, b = (torch.randn(width, device="cuda", generator=gen).to(BF16) for _ in range(3))
+    fn, c = torch.nn.functional, c if biased else None
+    total = y.double() + (0.0 if c is None else c.double())
+    got = bias_gelu(hip, y.clone(), c)
+    want = fn.gelu(total, approximate="tanh")
+    # a sum and a result rounded to bf16; the function's slope is 1.13 at most
+    assert bool(((got.double() - want).abs() <= 2.0**-8 * (want.abs() + 1.2 * total.abs()) + 1e-4).all())
+    for layer in (None, b):
+        h, n = add_norm(hip, x, y, c, w, layer, 1e-5)
+        assert bool(((h.double() - x.double() - total).abs() <= 2.0**-8 * (h.double().abs() + total.abs())).all())
+        hd = h.double()
+        if layer is None:
+            want = hd * torch.rsqrt(hd.square().mean(-1, keepdim=True) + 1e-5) * w.double()
+        else:
+            want = fn.layer_norm(hd, (width,), w.double(), b.double(), 1e-5)
+        assert bool(((n.double() - want).abs() <= 2.0**-8 * want.abs() + 1e-4).all())
 
 
 @requires_gpu

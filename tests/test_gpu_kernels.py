@@ -381,7 +381,8 @@ def test_mixtral_block_fast_decode_matches_cpu(hip):
 def test_moe_grouped_gemm_matches_dense(hip, quant):
     """Prefill grouped MFMA GEMM (expert-sorted padded tiles, NF4 dequant
     fused into the LDS B staging) vs per-expert dense matmuls."""
-    from petals_amd.ops.fused_moe import _StackedExperts, sort_pairs_by_expert
+    from expert_pairs import sort_pairs_by_expert
+    from petals_amd.ops.fused_moe import MOE_GEMM_MT, _StackedExperts
 
     torch.manual_seed(11)
     E, IN, OUT, T, K = 8, 512, 1152, 96, 2  # IN % 64 == 0, OUT % 128 == 0
@@ -394,7 +395,7 @@ def test_moe_grouped_gemm_matches_dense(hip, quant):
     sel[:40, 0] = 3
     sel[sel == 7] = 1
 
-    sorted_pairs, tile_expert = sort_pairs_by_expert(sel, E)
+    sorted_pairs, tile_expert = sort_pairs_by_expert(sel, E, MOE_GEMM_MT)
     out = st.moe_gemm(x, sorted_pairs, tile_expert, K, T * K)
     assert out.shape == (T * K, OUT)
 
