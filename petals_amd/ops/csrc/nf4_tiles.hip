@@ -271,9 +271,9 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
         const int at = i % 16, half = i % 128 / 64;
         const int byte = (((i / 128) * 4 + lane / 16) * 64 + i % 64 / 16 * 16 + lane % 16) * 16 + half * 8 + at / 8 * 4 + at % 4;
         const float level = NF4_TILE_LEVELS[at & 4 ? bytes[byte] >> 4 : bytes[byte] & 15];
-        const float v = x[(size_t)b * in_dim + kb0 * 128 + i] * bf16_to_f32(scales[((size_t)nb * n_kb + kb0) * 128 + i]);
+        const float weight = level * bf16_to_f32(scales[((size_t)nb * n_kb + kb0) * 128 + i]);
         float* sum = &red[(wave * B + b) * 64 + lane];
-        *sum = fmaf(level, v, *sum);
+        *sum = fmaf(weight, x[(size_t)b * in_dim + kb0 * 128 + i], *sum);
       }
     }
   };

@@ -147,6 +147,28 @@ def test_nf4_tiles_of_a_wide_range(hip, batch, loud):
 
 
 @requires_gpu
+@pytest.mark.parametrize("batch", [1, 5])
+def test_nf4_tiles_of_the_largest_numbers(hip, batch):
+    """An input that overflows with its block's scale is multiplied by its weight, which may be zero."""
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    w = torch.randn(300, 64, device="cuda", generator=gen).to(BF16)
+    w[7] = torch.tensor([0.0, 0.08 * 64, 64.0, 0.0] * 16, device="cuda").to(BF16)
+    packed, absmax = hip.nf4_quantize(w)
+    held = NF4_LEVELS.cuda().double()[torch.stack([packed & 15, packed >> 4], dim=-1).view(300, 64).long()]
+    held = held * absmax.double().repeat_interleave(64, dim=1)
+    x = torch.randn(batch, 300, device="cuda", generator=gen)
+    x[0, 7] = 2e37  # times 64, beyond 32-bit floats; times 5, not
+    y = hip.gemv_nf4_tiles(*hip.nf4_tile(packed, absmax), 300, x, torch.empty(0, device="cuda"), None, 0)
+    ref = x.double() @ held
+    assert bool(torch.isinf(y[0, 2::4]).all())
+    y[0, 2::4] = ref[0, 2::4] = 0.0
+    quiet = x.double()
+    quiet[0, 7] = 0.0
+    bound = nf4_bound(quiet, held, absmax.double().repeat_interleave(64, dim=1)) + 2.0**-20 * (x.double() * 64).abs().amax(1, keepdim=True) * (held[7] != 0)
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+@requires_gpu
 @pytest.mark.parametrize("batch", [4, 8])
 def test_nf4_tiles_round_inputs(hip, batch):
     """Errors of a sum of like terms cancel: scaled inputs are rounded, not cut off."""
