@@ -155,7 +155,7 @@ class _Attention(torch.autograd.Function):
         none = (None,) * 8
         if _by_torch(g):
             return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
-        return (ctx.hip.attn_prompt_grad(rows, aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
+        return (ctx.hip.attn_prompt_grad(aligned(rows), aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 
 
 def norm(x, w, eps, hip):

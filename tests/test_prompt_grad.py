@@ -32,7 +32,7 @@ class Kernels:
     @staticmethod
     def _plain(*tensors):
         for t in tensors:
-            t.data_ptr()
+            assert t.data_ptr() % 16 == 0 and t.is_contiguous()
         return [t.detach().clone() for t in tensors]
 
     def _pull(self, function, t, g):
@@ -207,3 +207,17 @@ def test_gradients_of_dual_numbers():
         value, moved = torch.autograd.forward_ad.unpack_dual(got)
     close(value, torch.autograd.grad(out, x, g, retain_graph=True)[0])
     close(moved, torch.autograd.grad(out, x, tangent)[0])
+
+
+def test_saved_tensors_from_hooks():
+    """Hooks may give back what they were given at another address, as copies from a buffer do."""
+
+    def unpack(t):
+        moved = torch.empty(t.numel() + 1, dtype=t.dtype)[1:].view(t.shape)
+        return moved.copy_(t)
+
+    x, weights = block_inputs()
+    (want,) = torch.autograd.grad(through_kernels(x, *weights).sum(), x)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        out = through_kernels(x, *weights)
+    close(torch.autograd.grad(out.sum(), x)[0], want)
