@@ -441,11 +441,13 @@ torch::Tensor attn_decode_fused(
       // VALU kernel: target ~1024 single-wave workgroups, chunks >= 64 rows
       n_splits = std::max(1, std::min(1024 / bkv, (lmax + 63) / 64));
     } else {
-      // One workgroup for each of the 256 compute units, parts of 128 rows or more: two or
-      // three per unit were slower (32000 keys of 8 heads: 16 parts 37.5 us, 32 parts 37.9,
-      // 62 parts 48.3; 256 heads: 1 part 27.1, 2 parts 30.6). Below 384 rows one part, as the
-      // second launch costs more than the longer chain (300 keys of 8 heads: 8.0 us, 8.6 with
-      // 4 parts; 500 of 32 heads: 9.7, 9.2).
+      // One workgroup for each of the 256 compute units, parts of 128 rows or more of a full
+      // cache: two or three per unit were slower (32000 keys of 8 heads: 16 parts 37.5 us, 32
+      // parts 37.9, 62 parts 48.3; 256 heads: 1 part 27.1, 2 parts 30.6). Up to 384 rows one
+      // part, as the second launch costs more than the longer chain (300 keys of 8 heads: 8.0
+      // us, 8.6 with 4 parts; 500 of 32 heads: 9.7, 9.2). Rows are those that the cache can
+      // hold, as a captured launch stays while it fills; a short text in a long cache is read
+      // in as many parts, of few rows each.
       static const int short_max = [] {
         const char* e = std::getenv("PETALS_AMD_DECODE_SHORT_LMAX");
         return e ? std::atoi(e) : 384;

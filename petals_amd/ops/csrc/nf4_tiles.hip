@@ -34,10 +34,10 @@
 // It is bound by vector instructions (half-rate lookups; the chip lowers its clock under
 // them), not by memory. llama-2-70b, us a product with its reduction, the kernel in
 // nf4.hip and this one, for 1, 4 and 8 rows:
-//   qkv   8192 x 10240   19, 29, 47     20, 22, 29
-//   o     8192 x 8192    22, 30, 49     17, 18, 23
-//   gate  8192 x 57344   64, 96, 160    64, 78, 112
-//   down  28672 x 8192   36, 51, 84     36, 41, 63
+//   qkv   8192 x 10240   19, 29, 47     20, 23, 31
+//   o     8192 x 8192    22, 30, 49     17, 19, 23
+//   gate  8192 x 57344   64, 96, 160    65, 79, 112
+//   down  28672 x 8192   36, 51, 84     34, 40, 61
 // (Runs of 1024 for one row: 70 and 38 us for the last two; four waves a SIMD: 71, 39.)
 // Cut off instead of rounded, and with the largest input of a run at 2^30 whatever the others
 // are, it took 0 to 5% less (8192 x 8192: 14.7, 16.1, 18.5 us without the reduction for 1, 4,

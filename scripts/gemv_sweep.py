@@ -1,4 +1,5 @@
-"""Sweep gemv split counts per decode shape to find the bandwidth knee."""
+"""Sweep split counts of the row kernel (gemv.hip) per decode shape to find the bandwidth knee;
+s0 is the matrix-core kernel (gemv_mfma.h) with the splits that it chooses."""
 
 import os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

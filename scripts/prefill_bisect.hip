@@ -2,7 +2,8 @@
 // (dead keys leak into C-layout rows with reg index r=0).
 //
 // Variants, all KVT-templated:
-//   0 = exact copy of the current ops/csrc/prefill_attn.hip kernel
+//   0 = the kernel that ops/csrc/prefill_attn.hip had when the failure was seen (values
+//       transposed into LDS, weights through LDS), before it took the form of paged_attn.h
 //   1 = exact copy of the OLD (pre-KVT) kernel, hardwired NB=2 scalar softmax
 //   2 = new kernel, but mask+mx split into two loops
 //   3 = new kernel, but p[][] written in the same loop that computes expf
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(WAVES * 64) void kern(
         l_row[r] = l_row[r] * corr[r] + lsum;
         m_row[r] = m_new;
       } else {
-        // VAR == 0: exact current kernel
+        // VAR == 0: the kernel as it was
         float s[NB];
         float mx = NEG_SENTINEL;
 #pragma unroll
