@@ -146,10 +146,14 @@ class MixtralFastPath(LlamaFastPath):
         Logits in 32 bits as in the kernel, and the kernel's choice where it can be asked, so that
         gradients go through the experts that the forward pass runs.
         All-device: safe inside hipGraph capture."""
-        logits = xn2.float() @ self.w_router_t.float()
+        selected = None
         if self._takes_router(xn2) and not prompt_grad.watched(xn2):
-            selected = self._route_rows(xn2.detach())[1].long()
-        else:
+            weights, selected = self._route_rows(xn2.detach())
+            selected = selected.long()
+            if not (torch.is_grad_enabled() and xn2.requires_grad):
+                return weights, selected
+        logits = xn2.float() @ self.w_router_t.float()
+        if selected is None:
             selected = torch.topk(logits, self.top_k, dim=-1)[1]
         # a softmax over all, renormalized over the chosen
         return F.softmax(logits.gather(1, selected), dim=-1), selected
