@@ -85,6 +85,7 @@ torch::Tensor rms_norm(torch::Tensor x, torch::Tensor w, double eps) {
   auto x2 = x.contiguous().view({-1, dim});
   const int rows = x2.size(0);
   auto y = torch::empty_like(x2);
+  if (rows == 0) return y.view(shape);
   auto stream = at::cuda::getCurrentCUDAStream();
   if (rows <= 4)
     rms_norm_kernel<false, 1024><<<rows, 1024, 0, stream>>>(

@@ -747,6 +747,19 @@ def test_prompt_gradients_by_transforms(hip):
 
 
 @requires_gpu
+@pytest.mark.parametrize("shape", [(0, 5), (2, 0)])
+def test_gradients_of_no_rows(hip, shape):
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.server.from_pretrained import load_pretrained_block
+
+    config = load_model_config("test-llama-hd128")
+    block = load_pretrained_block("test-llama-hd128", config, 0, torch_dtype=BF16, device=torch.device("cuda"))
+    x = torch.zeros(*shape, config.hidden_size, device="cuda", dtype=BF16, requires_grad=True)
+    block(x).sum().backward()
+    assert x.grad.shape == x.shape
+
+
+@requires_gpu
 def test_block_gradients_by_transforms(hip):
     """What traces or transforms a block's training pass gets the gradients that the kernels give."""
     from petals_amd.models.config_base import load_model_config
