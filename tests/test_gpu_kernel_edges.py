@@ -483,6 +483,28 @@ def test_prompts_at_any_address(hip, preset):
 
 
 @requires_gpu
+@pytest.mark.parametrize("preset", ["test-llama-hd128", "test-bloom-hd64", "test-falcon-hd64"])
+def test_prompts_with_sums_over_ranks(hip, preset, monkeypatch):
+    """A shard that holds everything, whose sums over ranks have one term, is the block."""
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.server.from_pretrained import load_pretrained_block
+
+    config = load_model_config(preset)
+    block = load_pretrained_block(preset, config, 0, torch_dtype=BF16, device=torch.device("cuda"))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(2, 19, config.hidden_size, device="cuda", generator=gen).to(BF16)
+    caches = [[torch.zeros(shape, device="cuda", dtype=BF16) for shape in block.kv_cache_shape(2, 32)] for _ in "ab"]
+    with torch.inference_mode():
+        want = block(x, kv_cache=caches[0], prefix_length=3)
+        monkeypatch.setattr(type(block._fast), "_tp_reduce", lambda self, t: t)
+        block._fast.tp_world = 2
+        got = block(x, kv_cache=caches[1], prefix_length=3)
+    # sums are rounded to bf16 once or twice more on the way
+    assert (got.double() - want.double()).norm() <= 2.0**-6 * want.double().norm()
+    assert all(torch.equal(a, b) for a, b in zip(*caches))
+
+
+@requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, BF16])
 @pytest.mark.parametrize("tokens,dim,experts,top", [(1, 8, 1, 1), (3, 64, 4, 2), (5, 4096, 8, 2), (2, 520, 64, 16), (7, 128, 65, 3), (1, 2048, 256, 8)])
 def test_router(hip, dtype, tokens, dim, experts, top):
