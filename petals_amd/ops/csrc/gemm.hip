@@ -1,0 +1,425 @@
+// Products of a prompt's rows with a bf16 matrix for CDNA4 (gfx950): X [M, K] times W [K, N],
+// or W [N, K] transposed (a backward pass), and what follows them: a bias and GELU, a
+// residual, or the SwiGLU of a fused gate and up projection.
+//
+// For tens to some hundreds of rows: there the library's kernels leave many compute units
+// without a tile (758 x 4096 has 48 tiles of 256 x 256) or one with twice the others' work,
+// and read weights at 2 TB/s where a prompt of 128 tokens is bound by reading them.
+//
+// A workgroup of 8 waves has a tile of BM x BN and K in steps of 64, through ST buffers of LDS
+// that are filled straight from memory (buffer_load ... lds: no registers, no stores, and
+// what lies beyond the rows or columns repeats the last ones). A step is two phases of 32 of K;
+// in each, the matrix cores work on one set of fragments while the next set is read from LDS
+// and some of the loads of the step ST - 1 ahead are issued. All loads of a step issued at
+// once, behind the barrier, block the waves until the caches' queues have taken them: 512 x
+// 4096 x 16384 took 70.3 instead of 60.5 us then. The barrier leaves the loads of later steps
+// in flight.
+//
+// Tiles that fill all compute units are summed over all of K; those left over in the last wave
+// of workgroups are split along K, so that it is as full as the others, and a second
+// kernel adds their parts up. Each chiplet has its own consecutive run of tiles, rows first: they find
+// a run of columns' weights in its L2.
+//
+// The product is W^T X^T, so that a lane ends with 4 neighbouring columns of one row. 16-byte groups of
+// LDS rows are permuted by the row, so that the rows that a load touches lie in different
+// banks; W [K, N] is read by transposing loads.
+//
+// Bound by reading weights for up to 128 rows (28672 x 8192: 4.9 TB/s), beyond that by the
+// matrix cores waiting for fragments (1.0 to 1.1 PFLOP/s where tiles fill all compute units; without
+// loads 1.3, without loads and fragments 1.7). MI355X, us, the library's kernels and this one with its sum of
+// parts, weights from memory:
+//   rows                 16          128          512          758
+//   4096 x 4096        19, 14      33, 18       34, 28       39, 36
+//   8192 x 10240       48, 37      76, 45      112, 110     134, 121
+//   16384 x 4096       79, 34     139, 38      139, 74      149, 119
+//   28672 x 8192      134, 86     199, 96      352, 216     301, 389
+//   8192 x 57344      161, 161    173, 175     413, 459     602, 651
+//   22016, transposed, to 4096:   114, 52      233, 102     232, 162
+// Which of the two a product takes is ops/prompt_grad.py's rule.
+
+#include "common.h"
+#include "gemv_reduce.h"
+#include "paged.h"
+#include <torch/extension.h>
+#include <ATen/cuda/CUDAContext.h>
+
+#define GEMM_THREADS 512
+#define GEMM_BK 64
+#define GEMM_CUS 256
+
+enum GemmEpilogue : int {
+  GEMM_PLAIN = 0,     // y
+  GEMM_RESIDUAL = 1,  // residual + y + bias
+  GEMM_GELU = 2,      // gelu(y + bias)
+  GEMM_SWIGLU = 3,    // silu(y[:N/2]) * y[N/2:]
+};
+
+struct GemmShape {
+  int m, n, k;
+  int row_tiles;  // of a run of columns
+  int whole;      // tiles summed over all of K
+  int rest;       // tiles split along K
+  int splits, per;  // parts of these, and steps of each
+};
+
+struct GemmOut {
+  unsigned short* y;               // [M, N], or [M, N/2] for GEMM_SWIGLU
+  const unsigned short* residual;  // [M, N] or null
+  const unsigned short* bias;      // [N] or null
+  float* parts;                    // [splits, rest, BM, BN]
+  int epilogue;
+};
+
+using gemm_rsrc = __attribute__((ext_vector_type(4))) int;
+
+// where a tile's column comes from: with GEMM_SWIGLU, half of a wave's columns are gates, and
+// the other half the same columns of up
+template <int FN>
+__device__ __forceinline__ int gemm_source_column(int tile, int c, int bn, int n, bool pairs) {
+  if (!pairs) return tile * bn + c;
+  constexpr int HALF = FN * 8;
+  const int in = c % (2 * HALF);
+  return tile * (bn / 2) + c / (2 * HALF) * HALF + in % HALF + (in >= HALF ? n / 2 : 0);
+}
+
+// four neighbouring values of a row, at column c of y's
+__device__ __forceinline__ void gemm_store(const GemmShape& s, const GemmOut& o, int m, int c, f32x4 v) {
+  if (m >= s.m || c >= s.n) return;
+  if (o.bias) {
+    const v4s b = *reinterpret_cast<const v4s*>(o.bias + c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += bf16_to_f32((unsigned short)b[i]);
+  }
+  const size_t at = (size_t)m * s.n + c;
+  if (o.residual) {
+    const v4s r = *reinterpret_cast<const v4s*>(o.residual + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += bf16_to_f32((unsigned short)r[i]);
+  }
+  v4s y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = (short)f32_to_bf16(o.epilogue == GEMM_GELU ? gelu_tanh_f32(v[i]) : v[i]);
+  *reinterpret_cast<v4s*>(o.y + at) = y;
+}
+
+__device__ __forceinline__ void gemm_store_pair(const GemmShape& s, const GemmOut& o, int m, int c, f32x4 g, f32x4 u) {
+  if (m >= s.m || c >= s.n / 2) return;
+  v4s y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = (short)f32_to_bf16(g[i] / (1.f + __expf(-g[i])) * u[i]);
+  *reinterpret_cast<v4s*>(o.y + (size_t)m * (s.n / 2) + c) = y;
+}
+
+// byte offset of 16-byte group c in a row of 128 bytes, and of one in a row of W [K, N]
+__device__ __forceinline__ int gemm_row_group(int row, int c) { return row * (GEMM_BK * 2) + ((c ^ (row & 7)) << 4); }
+template <int BN>
+__device__ __forceinline__ int gemm_w_swizzle(int row) {
+  constexpr int GROUPS = BN / 8;  // a power of two, at least 16
+  return (((row & 3) | ((row >> 1) & 4)) << 1) & (GROUPS - 1);
+}
+
+// WT: W is [N, K]. WR x WC waves of 16 FM rows and 16 FN columns.
+template <bool WT, int WR, int WC, int FM, int FN, int ST>
+__global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, GemmShape s, GemmOut o) {
+  constexpr int BK = GEMM_BK, BM = WR * FM * 16, BN = WC * FN * 16;
+  constexpr int XB = BM * BK * 2, STAGE = XB + BK * BN * 2;
+  // loads of 1 KB: of X; of a step; per wave (what is left over repeats the last); in the first phase
+  constexpr int XI = XB / 1024, ALL = STAGE / 1024, L = (ALL + 7) / 8, H = (L + 1) / 2;
+  static_assert(WR * WC == 8 && ST >= 3);
+  extern __shared__ __align__(1024) unsigned char gemm_lds[];
+
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
+  const int col = lane & 15, hi = lane >> 4;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  int tile, first = 0, steps = s.k / BK, part = -1;
+  if (local < s.whole / 8) {  // `whole` is a multiple of 8
+    tile = xcd * (s.whole / 8) + local;
+  } else {
+    const int units = s.rest * s.splits, share = (units + 7) / 8, unit = xcd * share + local - s.whole / 8;
+    if (local - s.whole / 8 >= share || unit >= units) return;  // uniform over the workgroup
+    tile = s.whole + unit % s.rest;
+    part = s.splits > 1 ? unit / s.rest : -1;
+    first = unit / s.rest * s.per;
+    steps = min(s.per, steps - first);
+  }
+  const bool pairs = o.epilogue == GEMM_SWIGLU;
+  const int m0 = tile % s.row_tiles * BM, column_tile = tile / s.row_tiles;
+  const int wm = wave / WC * FM * 16, wn = wave % WC * FN * 16;
+
+  // this wave's loads: byte offsets of each lane, of the step, and what a step adds
+  unsigned lane_at[L], step_at[L], step_size[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int load = min(wave * L + i, ALL - 1);
+    if (load < XI) {
+      const int p = load * 64 + lane, row = p / 8, c = p % 8 ^ (row & 7);
+      lane_at[i] = ((unsigned)min(m0 + row, s.m - 1) * s.k + c * 8) * 2;
+      step_size[i] = BK * 2;
+    } else if (WT) {
+      const int p = (load - XI) * 64 + lane, row = p / 8, c = p % 8 ^ (row & 7);
+      const int n = gemm_source_column<FN>(column_tile, row, BN, s.n, pairs);
+      lane_at[i] = ((unsigned)min(n, s.n - 1) * s.k + c * 8) * 2;
+      step_size[i] = BK * 2;
+    } else {
+      const int p = (load - XI) * 64 + lane, row = p / (BN / 8), c = p % (BN / 8) ^ gemm_w_swizzle<BN>(row);
+      const int n = gemm_source_column<FN>(column_tile, c * 8, BN, s.n, pairs);
+      lane_at[i] = ((unsigned)row * s.n + min(n, s.n - 8)) * 2;
+      step_size[i] = (unsigned)BK * s.n * 2;
+    }
+    step_at[i] = first * step_size[i];
+  }
+  auto resource = [](const void* p, unsigned bytes) {
+    const size_t at = (size_t)p;
+    return gemm_rsrc{__builtin_amdgcn_readfirstlane((int)at), __builtin_amdgcn_readfirstlane((int)(at >> 32) & 0xFFFF),
+                     (int)bytes, 0x00020000};
+  };
+  const gemm_rsrc xr = resource(x, (unsigned)s.m * s.k * 2), wr = resource(w, (unsigned)s.k * s.n * 2);
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)gemm_lds;
+  auto load = [&](unsigned to, int i) {
+    const int n = min(wave * L + i, ALL - 1);
+    const gemm_rsrc r = n < XI ? xr : wr;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(to + n * 1024), "v"(lane_at[i]), "s"(r), "s"(step_at[i])
+                 : "memory", "m0");
+    step_at[i] += step_size[i];
+  };
+
+  unsigned xa[2], wa[WT ? 2 : FN];  // addresses of this lane's fragments
+#pragma unroll
+  for (int kc = 0; kc < 2; ++kc) {
+    xa[kc] = base + gemm_row_group(wm + col, kc * 4 + hi);
+    if (WT) wa[kc] = base + XB + gemm_row_group(wn + col, kc * 4 + hi);
+  }
+  if (!WT)
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      const int row = hi * 8 + col / 4, c = (wn + i * 16) / 8 + ((col >> 1) & 1);
+      wa[i] = base + XB + row * (BN * 2) + ((c ^ gemm_w_swizzle<BN>(row)) << 4) + (col & 1) * 8;
+    }
+  using lds_v4s = __attribute__((address_space(3))) v4s;
+  using lds_frag = const __attribute__((address_space(3))) bf16x8;
+  f32x4 acc[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 xf[2][FM] = {}, wf[2][FN] = {};
+  auto read = [&](int set, unsigned buf, int n) {  // the n-th fragment, of the step's half `set`
+    if (n < FM) {
+      xf[set][n] = *(lds_frag*)(size_t)(xa[set] + buf + n * 16 * BK * 2);
+    } else if (n < FM + FN) {
+      const int i = n - FM;
+      if (WT) {
+        wf[set][i] = *(lds_frag*)(size_t)(wa[set] + buf + i * 16 * BK * 2);
+      } else {
+        // rows hi*8 + col/4 and 4 below, which are permuted alike; 4 columns a lane
+        const unsigned p = wa[i] + buf + set * 32 * BN * 2;
+        const v4s a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(size_t)p);
+        const v4s b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(size_t)(p + 4 * BN * 2));
+        wf[set][i] = bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      }
+    }
+  };
+  // products of one set; meanwhile the other set is read (half of a step later), and loads
+  // [l0, l1) of a later step are issued
+  auto phase = [&](bool multiply, int set, bool reads, unsigned buf, bool loads, unsigned to, int l0, int l1) {
+    constexpr int EARLY = FN > 1 ? (FM + FN + FN / 2 - 1) / (FN / 2) : FM + FN;  // reads are over half way through
+#pragma unroll
+    for (int i = 0; i < FN; ++i) {
+      if (reads)
+#pragma unroll
+        for (int e = 0; e < EARLY; ++e) read(set ^ 1, buf, i * EARLY + e);
+      if (loads)
+#pragma unroll
+        for (int l = 0; l < L; ++l)
+          if (l >= l0 && l < l1 && (l - l0) * FN / (l1 - l0) == i) load(to, l);
+      if (multiply)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][i], xf[set][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // Step t is whole in LDS, and all waves have read step t - 1, whose buffer is the next to be filled.
+  // Loads come back in order: those of the ST - 2 steps after t may be out.
+  auto arrive = [&](bool more) {
+    if (more)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((ST - 2) * L) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+#pragma unroll
+  for (int t = 0; t < ST - 1; ++t)
+    if (t < steps)
+#pragma unroll
+      for (int l = 0; l < L; ++l) load(base + t * STAGE, l);
+  unsigned from = 0, to = base + (ST - 1) * STAGE;
+  const bool longer = steps >= ST;
+  arrive(longer);
+  phase(false, 1, true, from, longer, to, 0, H);
+  phase(true, 0, true, from, longer, to, H, L);
+  int t = 1;
+  for (; t + ST - 1 < steps; ++t) {
+    from = from + STAGE == ST * STAGE ? 0 : from + STAGE;
+    to = to + STAGE == base + ST * STAGE ? base : to + STAGE;
+    arrive(true);
+    phase(true, 1, true, from, true, to, 0, H);
+    phase(true, 0, true, from, true, to, H, L);
+  }
+  for (; t < steps; ++t) {
+    from = from + STAGE == ST * STAGE ? 0 : from + STAGE;
+    arrive(false);
+    phase(true, 1, true, from, false, to, 0, H);
+    phase(true, 0, true, from, false, to, H, L);
+  }
+  phase(true, 1, false, from, false, to, 0, H);
+
+  if (part >= 0) {
+    float* to_part = o.parts + ((size_t)part * s.rest + tile - s.whole) * (BM * BN);
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+        *reinterpret_cast<f32x4*>(to_part + (wm + j * 16 + col) * BN + wn + i * 16 + hi * 4) = acc[i][j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int m = m0 + wm + j * 16 + col;
+    if (pairs) {
+#pragma unroll
+      for (int i = 0; i < FN / 2; ++i)
+        gemm_store_pair(s, o, m, gemm_source_column<FN>(column_tile, wn + i * 16 + hi * 4, BN, s.n, true), acc[i][j],
+                        acc[i + FN / 2][j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < FN; ++i) gemm_store(s, o, m, column_tile * BN + wn + i * 16 + hi * 4, acc[i][j]);
+    }
+  }
+}
+
+// four values of a tile per thread
+template <int BM, int BN, int FN>
+__global__ __launch_bounds__(256) void gemm_parts_kernel(GemmShape s, GemmOut o) {
+  const bool pairs = o.epilogue == GEMM_SWIGLU;
+  const int at = blockIdx.x * 256 + threadIdx.x, columns = pairs ? BN / 2 : BN;
+  const int tile = at / (BM * columns / 4), in = at % (BM * columns / 4) * 4;
+  if (tile >= s.rest) return;
+  const int row = in / columns;
+  int c = in % columns;
+  if (pairs) c = c / (FN * 8) * (FN * 16) + c % (FN * 8);
+  const int m = (s.whole + tile) % s.row_tiles * BM + row, column_tile = (s.whole + tile) / s.row_tiles;
+  if (m >= s.m) return;
+  const float* p = o.parts + (size_t)tile * (BM * BN) + row * BN + c;
+  const size_t stride = (size_t)s.rest * (BM * BN);
+  f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f}, up = sum;
+  for (int i = 0; i < s.splits; ++i) {
+    sum += *reinterpret_cast<const f32x4*>(p + i * stride);
+    if (pairs) up += *reinterpret_cast<const f32x4*>(p + i * stride + FN * 8);
+  }
+  const int n = gemm_source_column<FN>(column_tile, c, BN, s.n, pairs);
+  if (pairs) gemm_store_pair(s, o, m, n, sum, up);
+  else gemm_store(s, o, m, n, sum);
+}
+
+// ------------------------------------------------------------------- host
+
+struct GemmTile {
+  int bm, bn;
+  float step;  // us of 64 of K, a tile on every compute unit
+};
+static const GemmTile GEMM_TILES[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
+
+static GemmShape gemm_plan(long m, long n, long k, const GemmTile& t, float* us) {
+  const long row_tiles = (m + t.bm - 1) / t.bm, tiles = row_tiles * ((n + t.bn - 1) / t.bn), steps = k / GEMM_BK;
+  long whole = tiles / GEMM_CUS * GEMM_CUS, rest = tiles - whole, splits = 1;
+  // parts of at least 8 steps
+  if (rest) splits = std::max(1L, std::min(GEMM_CUS / rest, steps / 8));
+  long per = (steps + splits - 1) / splits;
+  splits = (steps + per - 1) / per;
+  *us = t.step * (tiles / GEMM_CUS * steps + (rest ? per : 0));
+  if (splits > 1) *us += 5.f + rest * splits * t.bm * t.bn * 4 * 2 / 8e6f;
+  return GemmShape{(int)m, (int)n, (int)k, (int)row_tiles, (int)whole, (int)rest, (int)splits, (int)per};
+}
+
+// x [M, K] bf16, w [K, N] (or [N, K], transposed) bf16 -> [M, N] bf16 (swiglu: [M, N/2])
+torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
+                        c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile) {
+  for (const auto& t : {x, w})
+    TORCH_CHECK(t.is_cuda() && t.dtype() == torch::kBFloat16 && t.dim() == 2 && t.is_contiguous() &&
+                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "gemm_rows takes aligned bf16 matrices");
+  TORCH_CHECK(w.device() == x.device());
+  const long m = x.size(0), k = x.size(1), n = w.size(transposed ? 0 : 1);
+  TORCH_CHECK(w.size(transposed ? 1 : 0) == k, "gemm_rows: shapes differ");
+  const bool pairs = epilogue == GEMM_SWIGLU;
+  TORCH_CHECK(epilogue >= 0 && epilogue <= 3 && k >= GEMM_BK && k % GEMM_BK == 0 && n >= 8 && n % (pairs ? 16 : 8) == 0,
+              "gemm_rows: sizes out of range");
+  // offsets into either are 32-bit
+  TORCH_CHECK(m * k < (1L << 31) && k * n < (1L << 31) && m < (1L << 24), "gemm_rows: too large");
+  TORCH_CHECK((epilogue == GEMM_RESIDUAL) == residual.has_value(), "a residual belongs to its epilogue");
+  auto y = torch::empty({m, pairs ? n / 2 : n}, x.options());
+  if (m == 0) return y;
+  GemmOut o{BF16P(y), nullptr, nullptr, nullptr, (int)epilogue};
+  if (residual.has_value()) {
+    TORCH_CHECK(residual->is_cuda() && residual->dtype() == torch::kBFloat16 && residual->is_contiguous() &&
+                residual->numel() == m * n && reinterpret_cast<uintptr_t>(residual->data_ptr()) % 8 == 0);
+    o.residual = BF16P(*residual);
+  }
+  if (bias.has_value()) {
+    TORCH_CHECK(!pairs && epilogue != GEMM_PLAIN && bias->is_cuda() && bias->dtype() == torch::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == n && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 8 == 0);
+    o.bias = BF16P(*bias);
+  }
+  int best = 0;
+  float least = 0.f;
+  GemmShape s{};
+  for (int i = 0; i < 4; ++i) {
+    if (tile >= 0 && tile != i) continue;
+    float us;
+    const GemmShape p = gemm_plan(m, n, k, GEMM_TILES[i], &us);
+    if (s.m == 0 || us < least) best = i, least = us, s = p;
+  }
+  const GemmTile& t = GEMM_TILES[best];
+  torch::Tensor parts;
+  if (s.splits > 1) {
+    parts = torch::empty({(long)s.splits * s.rest * t.bm * t.bn}, x.options().dtype(torch::kFloat32));
+    o.parts = parts.data_ptr<float>();
+  }
+  const long blocks = s.whole + ((long)s.rest * s.splits + 7) / 8 * 8;
+  TORCH_CHECK(blocks < (1L << 31));
+  auto stream = at::cuda::getCurrentCUDAStream();
+#define GEMM(WT, WR, WC, FM, FN, ST)                                                                                \
+  do {                                                                                                              \
+    constexpr int BM = WR * FM * 16, BN = WC * FN * 16, LDS = ST * (BM + BN) * GEMM_BK * 2;                         \
+    TORCH_CHECK(BM == t.bm && BN == t.bn);                                                                          \
+    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<WT, WR, WC, FM, FN, ST>), \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                   \
+    TORCH_CHECK(fits == hipSuccess, "gemm_rows: ", hipGetErrorString(fits));                                        \
+    gemm_kernel<WT, WR, WC, FM, FN, ST><<<blocks, GEMM_THREADS, LDS, stream>>>(BF16P(x), BF16P(w), s, o);           \
+    HIP_CHECK_LAST();                                                                                               \
+    if (s.splits > 1) {                                                                                             \
+      const long threads = (long)s.rest * BM * (pairs ? BN / 2 : BN) / 4;                                           \
+      gemm_parts_kernel<BM, BN, FN><<<(threads + 255) / 256, 256, 0, stream>>>(s, o);                               \
+      HIP_CHECK_LAST();                                                                                             \
+    }                                                                                                               \
+  } while (0)
+#define GEMM_EITHER(...)                       \
+  do {                                         \
+    if (transposed) GEMM(true, __VA_ARGS__);   \
+    else GEMM(false, __VA_ARGS__);             \
+  } while (0)
+  switch (best) {
+    case 0: GEMM_EITHER(2, 4, 4, 4, 3); break;
+    case 1: GEMM_EITHER(2, 4, 4, 2, 4); break;
+    case 2: GEMM_EITHER(2, 4, 2, 4, 4); break;
+    case 3: GEMM_EITHER(1, 8, 2, 2, 4); break;
+  }
+#undef GEMM_EITHER
+#undef GEMM
+  return y;
+}

@@ -10,8 +10,8 @@ layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
     ... 8 kernel launches per block, every byte of weights read exactly once
     (HBM-bound by design; see profiles/).
 
-  prefill (q_len > 1): bf16 GEMMs via torch.matmul on the SAME transposed
-    weights (rocBLAS), one kernel for each gap between them
+  prefill (q_len > 1): bf16 GEMMs on the SAME transposed weights (ops/csrc/gemm.hip up to
+    some hundreds of rows, the library beyond), one kernel for each gap between them
     (ops/csrc/prefill_rows.hip) and flash attention (prefill_attn.hip).
 
 The original nn.Linear weights are FREED after repacking (a 70B span must not
@@ -285,6 +285,38 @@ def _takes_rows(cache: torch.Tensor) -> bool:
     return cache.stride(3) == 1 and cache.data_ptr() % 16 == 0 and all(cache.stride(i) % 8 == 0 for i in range(3))
 
 
+_GEMM_PLAIN = 0
+_GEMM_RESIDUAL = 1
+_GEMM_GELU = 2
+_GEMM_SWIGLU = 3
+
+
+def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=None):
+    """A prompt's rows [..., K] times a _FastWeight, without gradients, and what follows: residual +
+    y + bias, gelu(y + bias), or the SwiGLU of [gate | up]."""
+    w = weight.dense()
+    fused = epilogue in (_GEMM_GELU, _GEMM_SWIGLU)
+    if (
+        x.is_cuda and x.dtype == torch.bfloat16 and prompt_grad.gemm_matrix(w)
+        and prompt_grad.takes_gemm(x.numel() // w.shape[0], *w.shape, fused=fused)
+    ):
+        rows = prompt_grad.aligned(x).view(-1, w.shape[0])
+        if residual is not None:
+            residual = prompt_grad.aligned(residual).view(rows.shape[0], -1)
+        return hip.gemm_rows(rows, w, False, epilogue, residual, bias).view(*x.shape[:-1], -1)
+    y = torch.matmul(x, w)
+    if epilogue == _GEMM_RESIDUAL:
+        return residual + y if bias is None else hip.add_rows(residual, y, None, bias)
+    if epilogue == _GEMM_GELU:
+        return bias_gelu(hip, y, bias)
+    if epilogue == _GEMM_SWIGLU:
+        inter = y.shape[-1] // 2
+        if inter % 8 == 0 and y.dtype == torch.bfloat16:
+            return hip.swiglu_rows(y)
+        return hip.swiglu(y[..., :inter].contiguous(), y[..., inter:].contiguous())
+    return y
+
+
 def add_norm(hip, x, y, y_bias, w, b, eps):
     """(x + y + y_bias, its layer norm, or RMS norm without b) of a prompt's rows"""
     if _rows_fit(x.shape[-1]):
@@ -359,6 +391,7 @@ class _TPFastPathMixin:
 
 class LlamaFastPath(_TPFastPathMixin):
     graph_safe = True  # whole-span hipGraph capture is valid for this block
+    dense_mlp = True  # one gated MLP for all tokens
 
     def __init__(self, block, hip_ops, quant: str = "none", tp_world: int = 1, tp_group=None):
         cfg = block.config
@@ -464,13 +497,16 @@ class LlamaFastPath(_TPFastPathMixin):
             lin.weight.data = self._empty_bf16
 
     def _mlp_dense(self, xn2, adapter, autograd: bool, x_delta=None):
-        """MLP on [B, S, H] inputs via rocBLAS matmuls on the transposed
-        (possibly NF4-dequantized) weights; differentiable when autograd.
+        """MLP on [B, S, H] inputs with the transposed (possibly dequantized) weights;
+        differentiable when autograd.
         `x_delta`: adapter-delta input when it differs from the matmul input
         (folded-norm weights take the scale-only normed x)."""
         xn2 = self._tp_copy(xn2)
+        if adapter is None and not autograd:
+            act = prompt_product(self.hip, xn2, self.wgateup_t, _GEMM_SWIGLU)
+            return prompt_product(self.hip, act, self.wdown_t)
         xd = xn2 if x_delta is None else x_delta
-        gateup = torch.matmul(xn2, self.wgateup_t.dense())
+        gateup = self._matmul(xn2, self.wgateup_t, autograd)
         inter = self.wgateup_t.shape[1] // 2
         gate, up = gateup[..., :inter], gateup[..., inter:]
         if adapter is not None:
@@ -483,16 +519,18 @@ class LlamaFastPath(_TPFastPathMixin):
             act = prompt_grad.swiglu(gateup, self.hip)
         elif autograd:
             act = reference.swiglu(gate, up).to(xn2.dtype)
-        elif adapter is None and inter % 8 == 0 and gateup.dtype == torch.bfloat16:
-            act = self.hip.swiglu_rows(gateup)
         else:
             act = self.hip.swiglu(gate.contiguous(), up.contiguous())
-        down = torch.matmul(act, self.wdown_t.dense())
+        down = self._matmul(act, self.wdown_t, autograd)
         if adapter is not None:
             dd = adapter.delta("down", act)
             if dd is not None:
                 down = down + dd
         return down
+
+    def _matmul(self, x, weight, autograd: bool):
+        """x times a weight, differentiable when autograd."""
+        return prompt_grad.product(x, weight.dense(), self.hip) if autograd else prompt_product(self.hip, x, weight)
 
     def _ensure_rope(self, needed: int):
         if self.rope_cos is None or self.rope_cos.shape[0] < needed:
@@ -657,7 +695,7 @@ class LlamaFastPath(_TPFastPathMixin):
         else:
             xn = reference.rms_norm(hidden, self.ln1_w_post, self.eps)
         xn = self._tp_copy(xn)  # backward: all-reduce the shard-partial grads
-        qkv = torch.matmul(xn, self.wqkv_t.dense())
+        qkv = self._matmul(xn, self.wqkv_t, True)
         if adapter is not None:
             xd = reference.rms_norm(hidden, self.ln1_w, self.eps) if self.fold_norm else xn
             qkv = qkv + self._qkv_adapter_delta(xd, adapter)
@@ -666,7 +704,7 @@ class LlamaFastPath(_TPFastPathMixin):
             attn = prompt_grad.attention(qkv, self.rope_cos, self.rope_sin, *shape, self.scale, self.hip)
         else:
             attn = prompt_grad.torch_attention(qkv, self.rope_cos, self.rope_sin, *shape).to(hidden.dtype)
-        o = self._tp_reduce(torch.matmul(attn, self.wo_t.dense()))
+        o = self._tp_reduce(self._matmul(attn, self.wo_t, True))
         if adapter is not None:
             d = adapter.delta("o", attn)
             if d is not None:
@@ -693,7 +731,7 @@ class LlamaFastPath(_TPFastPathMixin):
         self._ensure_rope(prefix_length + S)
 
         xn = self.hip.rms_norm(hidden, self.ln1_w_post, self.eps)
-        qkv = torch.matmul(xn, self.wqkv_t.dense())  # [B, S, qkv] bf16 (rocBLAS)
+        qkv = self._matmul(xn, self.wqkv_t, False)  # [B, S, qkv] bf16
         if adapter is not None:
             xd = self.hip.rms_norm(hidden, self.ln1_w, self.eps) if self.fold_norm else xn
             qkv = qkv + self._qkv_adapter_delta(xd, adapter).to(qkv.dtype)
@@ -701,7 +739,7 @@ class LlamaFastPath(_TPFastPathMixin):
             self.hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale,
             cos=self.rope_cos, sin=self.rope_sin,
         )
-        o = self._tp_reduce(torch.matmul(attn, self.wo_t.dense()))
+        o = self._tp_reduce(self._matmul(attn, self.wo_t, False))
         if adapter is not None:
             d = adapter.delta("o", attn)
             if d is not None:
@@ -716,6 +754,9 @@ class LlamaFastPath(_TPFastPathMixin):
 
     def _mlp_prompt(self, h2, xn2, adapter, x_delta):
         """h2 + MLP(xn2) of a prompt's rows."""
+        if adapter is None and self.tp_world == 1 and self.dense_mlp:
+            act = prompt_product(self.hip, xn2, self.wgateup_t, _GEMM_SWIGLU)
+            return prompt_product(self.hip, act, self.wdown_t, _GEMM_RESIDUAL, residual=h2)
         return h2 + self._tp_reduce(self._mlp_dense(xn2, adapter, autograd=False, x_delta=x_delta)).to(h2.dtype)
 
 
@@ -944,7 +985,7 @@ class BloomFastPath(_TPFastPathMixin):
         assert adapter is None or self.tp_world == 1, "LoRA on TP shards is served via the generic path"
         hip, hidden = self.hip, prompt_grad.aligned(hidden.to(torch.bfloat16))
         xn = hip.layer_norm(hidden, self.ln1_w, self.ln1_b, self.eps)
-        qkv = torch.matmul(xn, self.wqkv_t.dense())
+        qkv = prompt_product(hip, xn, self.wqkv_t)
         if adapter is not None:
             d = adapter.delta("qkv", xn)
             if d is not None:
@@ -952,7 +993,7 @@ class BloomFastPath(_TPFastPathMixin):
         attn = prompt_attention(
             hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale, bias=self.qkv_bias, slopes=self.slopes
         )
-        o = torch.matmul(attn, self.wo_t.dense())
+        o = prompt_product(hip, attn, self.wo_t)
         if adapter is not None:
             d = adapter.delta("dense", attn)
             if d is not None:
@@ -962,13 +1003,16 @@ class BloomFastPath(_TPFastPathMixin):
             o, o_bias = self._tp_reduce(o + o_bias), None
         h2, xn2 = add_norm(hip, res1, o, o_bias, self.ln2_w, self.ln2_b, self.eps)
         res2 = xn2 if self.post_ln_residual else h2
-        inter = torch.matmul(xn2, self.w_h4h.dense())
+        if adapter is None and self.tp_world == 1:
+            act = prompt_product(hip, xn2, self.w_h4h, _GEMM_GELU, bias=self.b_h4h)
+            return prompt_product(hip, act, self.w_4hh, _GEMM_RESIDUAL, residual=res2, bias=self.b_4hh)
+        inter = prompt_product(hip, xn2, self.w_h4h)
         if adapter is not None:
             dh = adapter.delta("h4h", xn2)
             if dh is not None:
                 inter = inter + dh.to(inter.dtype)
         act = bias_gelu(hip, inter, self.b_h4h)
-        out = torch.matmul(act, self.w_4hh.dense())
+        out = prompt_product(hip, act, self.w_4hh)
         if adapter is not None:
             d4 = adapter.delta("4hh", act)
             if d4 is not None:
@@ -1195,7 +1239,7 @@ class FalconFastPath(_TPFastPathMixin):
         self._ensure_rope(prefix_length + hidden.shape[1])
         xn_attn = hip.layer_norm(hidden, self.ln_attn_w, self.ln_attn_b, self.eps)
         xn_mlp = xn_attn if self.single_ln else hip.layer_norm(hidden, self.ln_mlp_w, self.ln_mlp_b, self.eps)
-        qkv = torch.matmul(xn_attn, self.wqkv_t.dense())
+        qkv = prompt_product(hip, xn_attn, self.wqkv_t)
         if adapter is not None:
             d = adapter.delta("qkv", xn_attn)
             if d is not None:
@@ -1203,8 +1247,8 @@ class FalconFastPath(_TPFastPathMixin):
         attn = prompt_attention(
             hip, qkv, kv_cache, prefix_length, self.qh, self.kh, self.hd, self.scale, cos=self.rope_cos, sin=self.rope_sin
         )
-        o = torch.matmul(attn, self.wo_t.dense())
-        inter = torch.matmul(xn_mlp, self.w_h4h.dense())
+        o = prompt_product(hip, attn, self.wo_t)
+        inter = prompt_product(hip, xn_mlp, self.w_h4h, _GEMM_GELU if adapter is None else _GEMM_PLAIN)
         if adapter is not None:
             d = adapter.delta("dense", attn)
             if d is not None:
@@ -1212,8 +1256,8 @@ class FalconFastPath(_TPFastPathMixin):
             dh = adapter.delta("h4h", xn_mlp)
             if dh is not None:
                 inter = inter + dh.to(inter.dtype)
-        act = bias_gelu(hip, inter)
-        out = torch.matmul(act, self.w_4hh.dense())
+        act = inter if adapter is None else bias_gelu(hip, inter)
+        out = prompt_product(hip, act, self.w_4hh)
         if adapter is not None:
             d4 = adapter.delta("4hh", act)
             if d4 is not None:

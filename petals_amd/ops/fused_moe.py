@@ -98,6 +98,7 @@ class MixtralFastPath(LlamaFastPath):
     # the router consumes the true ln2-weighted normed activations (softmax is
     # not scale-invariant), so the MLP norm cannot fold into expert weights
     supports_fold_norm = False
+    dense_mlp = False
 
     def _init_mlp_weights(self, block, hip_ops, quant):
         def t(w):

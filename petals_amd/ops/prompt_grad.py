@@ -48,6 +48,31 @@ def aligned(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
+def gemm_matrix(w: torch.Tensor) -> bool:
+    """A matrix [K, N] that ops/csrc/gemm.hip takes, from either side."""
+    return (
+        w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.data_ptr() % 16 == 0
+        and w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and 0 < w.numel() < 1 << 31
+    )
+
+
+def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = False) -> bool:
+    """Whether m rows of k times a matrix with n columns are faster by ops/csrc/gemm.hip than by the
+    library. `fused`: an activation follows, which would be a launch of its own.
+
+    Up to 128 rows weights are what a product reads, and up to half as many tiles of 128 x 256 as there are
+    compute units the library leaves most of these idle: it takes 1.0 to 3.6 times as long (16384 x
+    4096: 139 beside 38 us at 128 rows, 156 beside 121 at 900). With 192 to 512 tiles it takes 0.76 to 1.0 times
+    as long (4096 x 28672: 77 beside 98 us at 283 rows). With a transposed matrix it does as well, but
+    where the sum is long beside the columns (22016 to 4096: 232 beside 162 us at 758 rows)."""
+    if m <= 0 or m * k >= 1 << 31:
+        return False
+    tiles = -(-m // 128) * -(-n // 256)
+    if transposed:
+        return tiles <= 64 and k >= n or tiles <= 128 and k >= 4 * n
+    return m <= 128 or tiles <= (256 if fused else 128)
+
+
 def _by_torch(*grads) -> bool:
     """Whether these gradients are taken through torch operations: those that are to have gradients
     themselves, and those that are watched, which the forward pass need not have been."""
@@ -158,8 +183,38 @@ class _Attention(torch.autograd.Function):
         return (ctx.hip.attn_prompt_grad(aligned(rows), aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 
 
+class _Product(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w, hip):
+        ctx.w, ctx.hip = w, hip  # constant, maybe made in inference mode: such tensors can't be saved
+        return rows_product(x, w, hip)
+
+    @staticmethod
+    def backward(ctx, g):
+        w = ctx.w
+        if _by_torch(g):
+            return torch.matmul(g, w.t()), None, None
+        return rows_product(g, w, ctx.hip, transposed=True), None, None
+
+
+def rows_product(x, w, hip, transposed=False):
+    """x [..., K] times w [K, N], or [..., N] times its transpose: by ops/csrc/gemm.hip where that is
+    the faster one, else the library's."""
+    k, n = w.shape if not transposed else w.shape[::-1]
+    if takes_gemm(x.numel() // k, k, n, transposed):
+        return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
+    return torch.matmul(x, w.t() if transposed else w)
+
+
 def norm(x, w, eps, hip):
     return _Norm.apply(x, w, eps, hip)
+
+
+def product(x, w, hip):
+    """x [..., K] times a frozen matrix [K, N]"""
+    if w.requires_grad or not (fused_training(x) and gemm_matrix(w)):
+        return torch.matmul(x, w)
+    return _Product.apply(x, w, hip)
 
 
 def add_norm(x, y, w, eps, hip):

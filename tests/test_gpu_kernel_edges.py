@@ -848,3 +848,73 @@ def test_decode_attention_edges(hip, hd, gq, kv, alibi, kv_len, lmax):
     delta = (qd.abs() @ kd.abs().transpose(-1, -2) * hd**-0.5).max() * 2.0**-9 + scores.abs().max() * 2.0**-22
     bound = (torch.expm1(2 * delta) + 2.0**-8) * (weights @ vd.abs())
     assert bool(((got - weights @ vd).abs() <= bound).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, -1])
+@pytest.mark.parametrize(
+    "m,k,n",
+    [
+        (1, 64, 64),  # one step, fewer columns than a tile
+        (33, 128, 320),  # fewer steps than buffers; a row and 64 columns beyond a tile
+        (127, 256, 576),  # as many steps as buffers
+        (129, 704, 256),  # a row beyond two tiles, steps that end in the middle of the buffers
+        (300, 4160, 192),  # parts along K, the last one shorter
+        (640, 1024, 3328),  # tiles of a whole wave and some left over, in parts
+    ],
+)
+def test_prompt_product_edges(hip, m, k, n, tile, transposed):
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).to(BF16)
+
+    x, w, residual, bias = normal(m, k), normal(k, n) * 0.125, normal(m, n), normal(n)
+    given = w.t().contiguous() if transposed else w
+    ref = x.double() @ w.double()
+    # one rounding to bf16, and sums of k terms in 32 bits
+    loose = (x.double().abs() @ w.double().abs()) * k * 2.0**-24
+
+    def check(y, want, slack):
+        assert y.shape == want.shape and bool(torch.isfinite(y).all())
+        assert bool(((y.double() - want).abs() <= 2.0**-8 * want.abs() + slack + 1e-6).all())
+
+    check(hip.gemm_rows(x, given, transposed, 0, None, None, tile), ref, loose)
+    check(hip.gemm_rows(x, given, transposed, 1, residual, bias, tile), ref + residual.double() + bias.double(), loose)
+    gelu = torch.nn.functional.gelu(ref + bias.double(), approximate="tanh")
+    check(hip.gemm_rows(x, given, transposed, 2, None, bias, tile), gelu, 1.2 * loose)  # its slope is at most 1.13
+    (g, u), (lg, lu) = ref.chunk(2, dim=-1), loose.chunk(2, dim=-1)
+    # silu's slope is at most 1.1; its exponential is good to 2^-20
+    silu = torch.nn.functional.silu(g)
+    slack = 1.1 * lg * u.abs() + silu.abs() * lu + (silu * u).abs() * 2.0**-20
+    check(hip.gemm_rows(x, given, transposed, 3, None, None, tile), silu * u, slack)
+
+
+@requires_gpu
+@pytest.mark.parametrize("family,rows", [("llama", 40), ("bloom", 40), ("falcon", 40), ("llama", 700)])
+def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
+    """A block's prompt and gradients with and without csrc/gemm.hip."""
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.ops import prompt_grad
+    from petals_amd.server.from_pretrained import build_empty_block, init_random_block_
+
+    config = load_model_config({"llama": "tinyllama-1.1b", "bloom": "bloom-7b1", "falcon": "falcon-7b"}[family])
+    block = build_empty_block(config, 0, torch.device("cuda"), BF16)
+    init_random_block_(block, config, 0)
+    block = block.eval().optimize_for_inference()
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    x, g = (torch.randn(2, rows // 2, config.hidden_size, device="cuda", generator=gen).to(BF16) for _ in range(2))
+
+    def run():
+        with torch.inference_mode():
+            y = block(x)
+        leaf = x.clone().requires_grad_(True)
+        (dx,) = torch.autograd.grad(block(leaf), leaf, g)
+        return y, dx
+
+    got = run()
+    monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *args, **kwargs: False)
+    for a, b in zip(got, run()):
+        # both round every product to bf16: errors of 2^-9 each, over a block's half a dozen
+        assert (a.double() - b.double()).norm() <= 2.0**-6 * b.double().norm()

@@ -58,6 +58,10 @@ class Kernels:
     def swiglu_rows_grad(self, gateup, g):
         return self._pull(lambda t: reference.swiglu(*t.chunk(2, dim=-1)), gateup, g)
 
+    def gemm_rows(self, x, w, transposed=False):
+        x, w = self._plain(x, w)
+        return x @ (w.t() if transposed else w)
+
     def rotate_rows(self, qkv, cos, sin, start, qh, kh, hd):
         (qkv,) = self._plain(qkv)
         self.projection = qkv  # what attn_prompt_grad turns its rows back to
@@ -221,3 +225,36 @@ def test_saved_tensors_from_hooks():
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
         out = through_kernels(x, *weights)
     close(torch.autograd.grad(out.sum(), x)[0], want)
+
+
+def test_products_with_a_frozen_matrix(monkeypatch):
+    """Rows, their gradients, gradients of these and batches of them, whichever kernel multiplies."""
+    w = torch.randn(64, 128, generator=torch.Generator().manual_seed(1), dtype=torch.float64)
+    x, v, u = (torch.randn(2, 3, n, dtype=torch.float64) for n in (64, 128, 64))
+    for takes in (False, True):
+        monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *sizes: takes)
+
+        def product(t):
+            return prompt_grad._Product.apply(t, w, HIP)
+
+        leaf = x.clone().requires_grad_(True)
+        y = product(leaf)
+        torch.testing.assert_close(y, x @ w)
+        (g,) = torch.autograd.grad(y, leaf, v, retain_graph=True)
+        torch.testing.assert_close(g, v @ w.t())
+        cut = v.clone().requires_grad_(True)
+        (g,) = torch.autograd.grad(y, leaf, cut, retain_graph=True, create_graph=True)
+        torch.testing.assert_close(torch.autograd.grad(g, cut, u)[0], u @ w)
+        many = torch.stack([v, 2 * v])
+        (g,) = torch.autograd.grad(y, leaf, many, is_grads_batched=True)
+        torch.testing.assert_close(g, many @ w.t())
+
+
+@pytest.mark.parametrize("rows", [1, 128, 129, 758, 1024, 1025])
+def test_rule_of_products(rows):
+    # many rows of a wide matrix are the library's, few rows and sums that are long are the kernel's
+    assert prompt_grad.takes_gemm(rows, 16384, 4096) == (rows <= 1024)
+    assert prompt_grad.takes_gemm(rows, 4096, 28672) == (rows <= 128)
+    assert prompt_grad.takes_gemm(rows, 22016, 4096, transposed=True) == (rows <= 1024)
+    assert prompt_grad.takes_gemm(rows, 4096, 11008, transposed=True) is False
+    assert not prompt_grad.takes_gemm(0, 64, 64)
