@@ -23,7 +23,10 @@ torch::Tensor qkv_rope_reduce(
 torch::Tensor gemv_bf16(
     torch::Tensor wt, torch::Tensor x, torch::Tensor workspace,
     c10::optional<torch::Tensor> residual, int64_t epilogue, int64_t splits_override,
-    c10::optional<torch::Tensor> bias);
+    c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> sumsq_out);
+torch::Tensor gemv_bf16_normed(
+    torch::Tensor wt, torch::Tensor h, torch::Tensor w, c10::optional<torch::Tensor> sumsq, double eps,
+    torch::Tensor workspace, int64_t epilogue);
 torch::Tensor attn_decode_fused(
     torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor kv_len,
     int64_t gq, int64_t n_splits, torch::Tensor part_o, torch::Tensor part_ml, double scale,
@@ -105,7 +108,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none());
   m.def("gemv_bf16", &gemv_bf16, "split-K bf16 gemv with fused epilogue",
         py::arg("wt"), py::arg("x"), py::arg("workspace"), py::arg("residual"), py::arg("epilogue"),
-        py::arg("splits") = 0, py::arg("bias") = py::none());
+        py::arg("splits") = 0, py::arg("bias") = py::none(), py::arg("sumsq_out") = py::none());
+  m.def("gemv_bf16_normed", &gemv_bf16_normed, "gemv_bf16 of the RMS norm of bf16 rows",
+        py::arg("wt"), py::arg("h"), py::arg("w"), py::arg("sumsq"), py::arg("eps"), py::arg("workspace"),
+        py::arg("epilogue"));
   m.def("attn_decode_fused", &attn_decode_fused, "GQA decode attention (flash-decoding)",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("kv_len"), py::arg("gq"),
         py::arg("n_splits"), py::arg("part_o"), py::arg("part_ml"), py::arg("scale"),

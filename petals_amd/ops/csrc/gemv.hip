@@ -184,7 +184,8 @@ torch::Tensor gemv_bf16(
     c10::optional<torch::Tensor> residual,  // [batch, out] bf16
     int64_t epilogue,
     int64_t splits_override,
-    c10::optional<torch::Tensor> bias) {  // [out] bf16, added pre-activation
+    c10::optional<torch::Tensor> bias,       // [out] bf16, added pre-activation
+    c10::optional<torch::Tensor> sumsq_out) {  // [batch, out/64] f32: sums of the results' squares (residual epilogue)
   TORCH_CHECK(wt.is_cuda() && wt.dtype() == torch::kBFloat16 && wt.dim() == 2);
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.dim() == 2);
   const int in_dim = wt.size(0), out_dim = wt.size(1);
@@ -206,6 +207,20 @@ torch::Tensor gemv_bf16(
     return partials;
   }
   torch::Tensor y = launch_gemv_reduce(
-      partials, residual, bias, splits, batch, out_dim, (int)epilogue, x.options(), wt.options());
+      partials, residual, bias, splits, batch, out_dim, (int)epilogue, x.options(), wt.options(), sumsq_out);
   return y;
+}
+
+// the same for the RMS norm of h [batch, in] bf16 with weight w (gemv_norm.h)
+torch::Tensor gemv_bf16_normed(
+    torch::Tensor wt, torch::Tensor h, torch::Tensor w, c10::optional<torch::Tensor> sumsq, double eps,
+    torch::Tensor workspace, int64_t epilogue) {
+  TORCH_CHECK(wt.is_cuda() && wt.dtype() == torch::kBFloat16 && wt.dim() == 2);
+  const GemvNorm norm = gemv_norm(h, w, sumsq, eps);
+  TORCH_CHECK(h.size(1) == wt.size(0) && h.size(0) >= 1 && h.size(0) <= 8 && gemv_mfma_fits(wt, wt.size(1)));
+  TORCH_CHECK(workspace.numel() == 0 || (workspace.is_cuda() && workspace.dtype() == torch::kFloat32));
+  auto partials = launch_gemv_mfma(wt, h, nullptr, 1, workspace, &norm);
+  if (epilogue < 0) return partials;
+  return launch_gemv_reduce(partials, c10::nullopt, c10::nullopt, (int)partials.size(0), (int)partials.size(1),
+                            (int)partials.size(2), (int)epilogue, partials.options(), wt.options());
 }

@@ -22,6 +22,7 @@
 #pragma once
 
 #include "common.h"
+#include "gemv_norm.h"
 #include "paged.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
@@ -60,14 +61,15 @@ static __device__ __forceinline__ void split_bf16(const float* x, bf16x8* p) {
 
 // Grid: (128 columns, runs of 4 x 32 S inputs, rows of sel or 1). With sel, there is one row,
 // blockIdx.z: that of x[blockIdx.z / k_per_tok] with matrix sel[blockIdx.z].
-template <int S>
+// NORM: inputs are norm's rows instead of x (no sel).
+template <int S, bool NORM>
 static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
     const unsigned short* __restrict__ wt,  // [in, out] or [experts, in, out]
     const float* __restrict__ x,            // [rows, in]
     const int* __restrict__ sel,            // [rows * k_per_tok] or null
     float* __restrict__ partials,           // [splits, rows or gridDim.z, out]
-    int in_dim, int out_dim, int rows, int k_per_tok, int experts, bool by4) {
-  extern __shared__ float gemv_red[];  // [4 waves, rows, 128]
+    int in_dim, int out_dim, int rows, int k_per_tok, int experts, bool by4, GemvNorm norm) {
+  extern __shared__ float gemv_red[];  // [4 waves, rows, 128], and with NORM [4 waves, rows]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 15, hi = lane >> 4;
   const int n0 = blockIdx.x * GEMV_MFMA_COLS, k0 = (blockIdx.y * 4 + wave) * 32 * S;
@@ -79,10 +81,19 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
   }
 
   float xs[S][8];
+  short8 hs[NORM ? S : 1], ws[NORM ? S : 1];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int k = k0 + s * 32 + hi * 8;
     const float* p = x + (size_t)col * in_dim + k;
+    if constexpr (NORM) {  // in_dim is a multiple of 8; expanded when the weights are on their way
+      hs[s] = ws[s] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (col < rows && k < in_dim) {
+        hs[s] = *reinterpret_cast<const short8*>(norm.h + (size_t)col * in_dim + k);
+        ws[s] = *reinterpret_cast<const short8*>(norm.w + k);
+      }
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) xs[s][i] = 0.f;
     if (col < rows) {
@@ -116,6 +127,8 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
       }
   }
   __builtin_amdgcn_sched_barrier(0);
+  float* sq = gemv_red + (size_t)4 * rows * GEMV_MFMA_COLS;
+  if constexpr (NORM) norm_sums(norm, rows, in_dim, sq);
 
   f32x4 acc[8];
 #pragma unroll
@@ -123,6 +136,10 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     bf16x8 xp[3], wf[8];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xs[s][i] = bf16_to_f32((unsigned short)hs[s][i]) * bf16_to_f32((unsigned short)ws[s][i]);
+    }
     split_bf16(xs[s], xp);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -133,7 +150,7 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
       wf[j] = __builtin_bit_cast(bf16x8, v);
     }
 #pragma unroll
-    for (int q = 2; q >= 0; --q)
+    for (int q = NORM ? 1 : 2; q >= 0; --q)  // 16 bits of a product are in two parts
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xp[q], acc[j], 0, 0, 0);
   }
@@ -152,7 +169,8 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
   for (int i = tid; i < n; i += 256) {
     const int c = n0 + i % GEMV_MFMA_COLS;
     if (c >= out_dim) continue;
-    const float sum = (gemv_red[i] + gemv_red[n + i]) + (gemv_red[2 * n + i] + gemv_red[3 * n + i]);
+    float sum = (gemv_red[i] + gemv_red[n + i]) + (gemv_red[2 * n + i] + gemv_red[3 * n + i]);
+    if constexpr (NORM) sum *= norm_factor(norm, rows, i / GEMV_MFMA_COLS, in_dim, sq);
     const size_t row = sel ? (size_t)blockIdx.y * gridDim.z + blockIdx.z : (size_t)blockIdx.y * rows + i / GEMV_MFMA_COLS;
     partials[row * out_dim + c] = sum;
   }
@@ -163,9 +181,10 @@ static bool gemv_mfma_fits(const torch::Tensor& wt, int64_t out_dim) {
   return out_dim % 8 == 0 && reinterpret_cast<uintptr_t>(wt.data_ptr()) % 16 == 0 && wt.is_contiguous();
 }
 
-// sel: [rows] matrices or null; returns [splits, rows, out]
+// sel: [rows] matrices or null; with norm, x are the rows that it is of. Returns [splits, rows, out], f32
 static torch::Tensor launch_gemv_mfma(
-    const torch::Tensor& wt, const torch::Tensor& x, const torch::Tensor* sel, int64_t k_per_tok, torch::Tensor workspace) {
+    const torch::Tensor& wt, const torch::Tensor& x, const torch::Tensor* sel, int64_t k_per_tok, torch::Tensor workspace,
+    const GemvNorm* norm = nullptr) {
   const int lead = sel ? 1 : 0;
   const long in_dim = wt.size(lead), out_dim = wt.size(lead + 1);
   TORCH_CHECK(x.is_contiguous());
@@ -179,19 +198,26 @@ static torch::Tensor launch_gemv_mfma(
   const long splits = std::max(1L, (in_dim + 128 * s - 1) / (128 * s));
   torch::Tensor partials = workspace.numel() >= splits * rows * out_dim
                                ? workspace.view(-1).narrow(0, 0, splits * rows * out_dim).view({splits, rows, out_dim})
-                               : torch::empty({splits, rows, out_dim}, x.options());
+                               : torch::empty({splits, rows, out_dim}, x.options().dtype(torch::kFloat32));
   if (rows == 0 || out_dim == 0) return partials;
   const bool by4 = in_dim % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
   const dim3 grid(columns, splits, z);
-  const size_t lds = sizeof(float) * 4 * batch * GEMV_MFMA_COLS;
+  const size_t lds = sizeof(float) * 4 * batch * (GEMV_MFMA_COLS + (norm ? 1 : 0));
   auto stream = c10::hip::getCurrentHIPStream().stream();
-#define GEMV_MFMA(S)                                                                                                \
-  gemv_mfma_kernel<S><<<grid, 256, lds, stream>>>(                                                                  \
-      reinterpret_cast<const unsigned short*>(wt.data_ptr()), x.data_ptr<float>(), sel ? sel->data_ptr<int>() : nullptr, \
-      partials.data_ptr<float>(), (int)in_dim, (int)out_dim, batch, (int)k_per_tok, sel ? (int)wt.size(0) : 1, by4)
-  if (s == 4) GEMV_MFMA(4);
-  else if (s == 2) GEMV_MFMA(2);
-  else GEMV_MFMA(1);
+#define GEMV_MFMA(S, NORM)                                                                                          \
+  gemv_mfma_kernel<S, NORM><<<grid, 256, lds, stream>>>(                                                            \
+      reinterpret_cast<const unsigned short*>(wt.data_ptr()), NORM ? nullptr : x.data_ptr<float>(),                 \
+      sel ? sel->data_ptr<int>() : nullptr, partials.data_ptr<float>(), (int)in_dim, (int)out_dim, batch,           \
+      (int)k_per_tok, sel ? (int)wt.size(0) : 1, by4, norm ? *norm : GemvNorm())
+#define GEMV_MFMA_EITHER(S)             \
+  do {                                  \
+    if (norm) GEMV_MFMA(S, true);       \
+    else GEMV_MFMA(S, false);           \
+  } while (0)
+  if (s == 4) GEMV_MFMA_EITHER(4);
+  else if (s == 2) GEMV_MFMA_EITHER(2);
+  else GEMV_MFMA_EITHER(1);
+#undef GEMV_MFMA_EITHER
 #undef GEMV_MFMA
   HIP_CHECK_LAST();
   return partials;

@@ -5,7 +5,7 @@
 torch::Tensor gemv_bf16(
     torch::Tensor wt, torch::Tensor x, torch::Tensor workspace,
     c10::optional<torch::Tensor> residual, int64_t epilogue, int64_t splits_override,
-    c10::optional<torch::Tensor> bias);
+    c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> sumsq_out);
 torch::Tensor gemv_bf16_moe(
     torch::Tensor wt_all, torch::Tensor x, torch::Tensor sel, int64_t k_per_tok,
     torch::Tensor workspace, int64_t epilogue, int64_t splits_override, double limit, double alpha);
@@ -31,7 +31,7 @@ torch::Tensor moe_linear_f32(torch::Tensor w, torch::Tensor x, torch::Tensor sel
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemv_bf16", &gemv_bf16, "split-K bf16 gemv with fused epilogue",
         py::arg("wt"), py::arg("x"), py::arg("workspace"), py::arg("residual"), py::arg("epilogue"),
-        py::arg("splits") = 0, py::arg("bias") = py::none());
+        py::arg("splits") = 0, py::arg("bias") = py::none(), py::arg("sumsq_out") = py::none());
   m.def("gemv_bf16_moe", &gemv_bf16_moe, "device-routed expert gemv (bf16 weights)",
         py::arg("wt_all"), py::arg("x"), py::arg("sel"), py::arg("k_per_tok"),
         py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0,

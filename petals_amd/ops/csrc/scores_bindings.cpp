@@ -6,7 +6,7 @@
 torch::Tensor gemv_bf16(
     torch::Tensor wt, torch::Tensor x, torch::Tensor workspace,
     c10::optional<torch::Tensor> residual, int64_t epilogue, int64_t splits_override,
-    c10::optional<torch::Tensor> bias);
+    c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> sumsq_out);
 torch::Tensor batched_linear(torch::Tensor a, torch::Tensor w, bool out_f32, c10::optional<torch::Tensor> out);
 torch::Tensor residual_norm(
     torch::Tensor x, c10::optional<torch::Tensor> y, c10::optional<torch::Tensor> bias,
@@ -36,7 +36,7 @@ void paired_attention(
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemv_bf16", &gemv_bf16, "split-K bf16 gemv with fused epilogue",
         py::arg("wt"), py::arg("x"), py::arg("workspace"), py::arg("residual"), py::arg("epilogue"),
-        py::arg("splits") = 0, py::arg("bias") = py::none());
+        py::arg("splits") = 0, py::arg("bias") = py::none(), py::arg("sumsq_out") = py::none());
   m.def("batched_linear", &batched_linear, "out[t,h,n] = sum_k a[t,h,k] w[h,n,k]",
         py::arg("a"), py::arg("w"), py::arg("out_f32"), py::arg("out") = py::none());
   m.def("residual_norm", &residual_norm, "x += mult (y + bias); RMS norm of x in equal parts",

@@ -918,3 +918,24 @@ def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
     for a, b in zip(got, run()):
         # both round every product to bf16: errors of 2^-9 each, over a block's half a dozen
         assert (a.double() - b.double()).norm() <= 2.0**-6 * b.double().norm()
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("k_in,n_out", [(8, 128), (136, 192), (1088, 64), (2056, 264), (4544, 2560), (8192, 1024)])
+def test_products_of_a_norm(hip, k_in, n_out, batch):
+    """The norm within the product, with its sums of squares given or not, against 64 bits."""
+    gen = torch.Generator(device="cuda").manual_seed(k_in + batch)
+    w = (torch.randn(k_in, n_out, device="cuda", generator=gen) * 0.05).to(BF16)
+    h = torch.randn(batch, k_in, device="cuda", generator=gen).to(BF16)
+    h[:, :: max(1, k_in // 5)] *= 300.0  # loud channels
+    h[batch // 2] *= 1e-10
+    weight = (1 + 0.1 * torch.randn(k_in, device="cuda", generator=gen)).to(BF16)
+    hd = h.double()
+    x = hd * torch.rsqrt(hd.square().mean(-1, keepdim=True) + 1e-5) * weight.double()
+    # and the factor: some dozen roundings
+    bound = sum_bound(x, w.double()) + 16 * 2.0**-24 * (x @ w.double()).abs()
+    parts = torch.stack([c.float().square().sum(-1) for c in h.split(64, dim=-1)], dim=1)
+    for sumsq in (None, parts):
+        y = hip.gemv_bf16_normed(w, h, weight, sumsq, 1e-5, torch.empty(0, device="cuda"), 0)
+        assert bool(((y.double() - x @ w.double()).abs() <= bound).all())
