@@ -24,10 +24,17 @@ __global__ void rms_norm_kernel(
 
   float sumsq = 0.f;
   const int chunk = T * 8;
+  // the first chunk, which is the whole row in decoding, stays in registers, and its weights are
+  // on their way before the sum is awaited
+  short8 first = {0, 0, 0, 0, 0, 0, 0, 0}, first_w = first;
+  if (tid * 8 + 8 <= dim) {
+    first = *reinterpret_cast<const short8*>(xr + tid * 8);
+    first_w = *reinterpret_cast<const short8*>(w + tid * 8);
+  }
   for (int base = 0; base < dim; base += chunk) {
     const int idx = base + tid * 8;
     if (idx + 8 <= dim) {
-      const short8 v = *reinterpret_cast<const short8*>(xr + idx);
+      const short8 v = base == 0 ? first : *reinterpret_cast<const short8*>(xr + idx);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float f = bf16_to_f32((unsigned short)v[j]);
@@ -52,8 +59,8 @@ __global__ void rms_norm_kernel(
   for (int base = 0; base < dim; base += chunk) {
     const int idx = base + tid * 8;
     if (idx + 8 <= dim) {
-      const short8 v = *reinterpret_cast<const short8*>(xr + idx);
-      const short8 wv = *reinterpret_cast<const short8*>(w + idx);
+      const short8 v = base == 0 ? first : *reinterpret_cast<const short8*>(xr + idx);
+      const short8 wv = base == 0 ? first_w : *reinterpret_cast<const short8*>(w + idx);
       if (OUT_F32) {
         float* yr = reinterpret_cast<float*>(y) + (size_t)row * dim + idx;
 #pragma unroll
@@ -143,10 +150,17 @@ __global__ void layer_norm_kernel(
 
   float sum = 0.f, sumsq = 0.f;
   const int chunk = T * 8;
+  // as in rms_norm_kernel
+  short8 first = {0, 0, 0, 0, 0, 0, 0, 0}, first_w = first, first_b = first;
+  if (tid * 8 + 8 <= dim) {
+    first = *reinterpret_cast<const short8*>(xr + tid * 8);
+    first_w = *reinterpret_cast<const short8*>(w + tid * 8);
+    first_b = *reinterpret_cast<const short8*>(bias + tid * 8);
+  }
   for (int base = 0; base < dim; base += chunk) {
     const int idx = base + tid * 8;
     if (idx + 8 <= dim) {
-      const short8 v = *reinterpret_cast<const short8*>(xr + idx);
+      const short8 v = base == 0 ? first : *reinterpret_cast<const short8*>(xr + idx);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float f = bf16_to_f32((unsigned short)v[j]);
@@ -183,9 +197,9 @@ __global__ void layer_norm_kernel(
   for (int base = 0; base < dim; base += chunk) {
     const int idx = base + tid * 8;
     if (idx + 8 <= dim) {
-      const short8 v = *reinterpret_cast<const short8*>(xr + idx);
-      const short8 wv = *reinterpret_cast<const short8*>(w + idx);
-      const short8 bv = *reinterpret_cast<const short8*>(bias + idx);
+      const short8 v = base == 0 ? first : *reinterpret_cast<const short8*>(xr + idx);
+      const short8 wv = base == 0 ? first_w : *reinterpret_cast<const short8*>(w + idx);
+      const short8 bv = base == 0 ? first_b : *reinterpret_cast<const short8*>(bias + idx);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float f = (bf16_to_f32((unsigned short)v[j]) - mean) * inv *
@@ -465,6 +479,19 @@ __global__ __launch_bounds__(64 * G_T) void qkv_rope_reduce_kernel(
   // partner offset: +half for d<half, -half otherwise
   const int partner = rotate ? (d < half ? o + half : o - half) : o;
 
+  // what the sums meet is on its way before they are
+  const int p = *pos_ptr;
+  float c = 0.f, sn = 0.f, add = 0.f, partner_add = 0.f;
+  if (sg == 0 && live) {
+    if (bias) {
+      add = bf16_to_f32(bias[o]);
+      if (rotate) partner_add = bf16_to_f32(bias[partner]);
+    }
+    if (rotate) {
+      c = cos_t[(size_t)p * hd + (d < half ? d : d - half)];
+      sn = sin_t[(size_t)p * hd + (d < half ? d : d - half)];
+    }
+  }
   float a = 0.f, p2 = 0.f;
   if (live) {
     for (int s = sg; s < n_splits; s += G) a += partials[(size_t)s * stride + row + o];
@@ -481,18 +508,12 @@ __global__ __launch_bounds__(64 * G_T) void qkv_rope_reduce_kernel(
     sum += acc_a[k][ol];
     psum += acc_b[k][ol];
   }
-  if (bias) {
-    sum += bf16_to_f32(bias[o]);
-    if (rotate) psum += bf16_to_f32(bias[partner]);
-  }
-
-  const int p = *pos_ptr;
+  sum += add;
+  psum += partner_add;
   float val = sum;
   if (rotate) {
-    const float c = cos_t[(size_t)p * hd + (d < half ? d : d - half)];
-    const float s = sin_t[(size_t)p * hd + (d < half ? d : d - half)];
     // pair (x1, x2) at (d, d+half): out_d = x1*c - x2*s; out_{d+half} = x2*c + x1*s
-    val = (d < half) ? (sum * c - psum * s) : (sum * c + psum * s);
+    val = (d < half) ? (sum * c - psum * sn) : (sum * c + psum * sn);
   }
   if (in_q) {
     q_out[(size_t)bi * qh * hd + o] = val;
