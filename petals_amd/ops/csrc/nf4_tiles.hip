@@ -15,7 +15,8 @@
 // Digits come from v_perm_b32, which looks four codes up in eight bytes at once. Two
 // lookups make up the 16 levels: a code of the other half selects a sign or a constant (0
 // for 12, all ones above), which for given tables is known, and which the other table is
-// xored with below, so that the xor of both lookups is the digit. That costs the same for
+// xored with below, so that the xor of both lookups is the digit; or the tables are made for
+// their sum, and both are multiplied (see SUMMED). That costs the same for
 // one row as for four, and no LDS, where the kernel that it stands for gathers the two
 // levels of a byte from a table: there random indices collide, and every row more is
 // another operation a weight.
@@ -76,6 +77,12 @@ __device__ constexpr unsigned NF4_DIGITS[3][4] = {
     {0x19a4ad3du, 0xffcff138u, 0xddc51d8cu, 0x3c232e57u},
     {0x2e3d5289u, 0xff0a15deu, 0xd71d1309u, 0x88a9bc34u},
 };
+// the same digits as sums of both lookups: less what the other one yields
+__device__ constexpr unsigned NF4_SUMMANDS[3][4] = {
+    {0x715bdb4bu, 0x01d66436u, 0x8a7bb776u, 0xb7da16c6u},
+    {0x1aa5523du, 0x01310f38u, 0x223a1d73u, 0xc4ddd257u},
+    {0xd1c2ad89u, 0x01f6ebdeu, 0x281e140au, 0x78574434u},
+};
 
 __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -129,6 +136,9 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4) {
   const int steps = LONG ? n_steps : 1;
   constexpr int NS = (B + 3) / 4, NCOL = 4 * B, PER = KB * 2;
+  // the two lookups of a digit are multiplied one by one, which saves their xor, where the matrix cores
+  // have little else to do: 8192 x 57344 takes 59.5 instead of 61.8 us with 1 row, 113.7 instead of 111.3 with 8
+  constexpr bool SUMMED = NS == 1;
   __shared__ __align__(16) unsigned char digits[4][KB * 128 * NCOL];
   __shared__ __align__(16) float red[4 * B * 64];  // [waves, rows, columns]
 
@@ -344,13 +354,19 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
           for (int i = 0; i < 4; ++i) up[i] = lo[i] ^ 0x08080808u;
 #pragma unroll
           for (int p = 0; p < 3; ++p) {
-            i32x4 a;
+            constexpr auto& table = SUMMED ? NF4_SUMMANDS : NF4_DIGITS;
+            i32x4 a, b;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              a[i] = (int)(__builtin_amdgcn_perm(NF4_DIGITS[p][1], NF4_DIGITS[p][0], lo[i]) ^
-                           __builtin_amdgcn_perm(NF4_DIGITS[p][3], NF4_DIGITS[p][2], up[i]));
+            for (int i = 0; i < 4; ++i) {
+              a[i] = (int)__builtin_amdgcn_perm(table[p][1], table[p][0], lo[i]);
+              b[i] = (int)__builtin_amdgcn_perm(table[p][3], table[p][2], up[i]);
+            }
+            if (!SUMMED) a ^= b;
 #pragma unroll
-            for (int s = 0; s < NS; ++s) acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xd[s], acc[s][c][p], 0, 0, 0);
+            for (int s = 0; s < NS; ++s) {
+              acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xd[s], acc[s][c][p], 0, 0, 0);
+              if (SUMMED) acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, xd[s], acc[s][c][p], 0, 0, 0);
+            }
           }
         }
       }
