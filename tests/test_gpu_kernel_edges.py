@@ -939,3 +939,16 @@ def test_products_of_a_norm(hip, k_in, n_out, batch):
     for sumsq in (None, parts):
         y = hip.gemv_bf16_normed(w, h, weight, sumsq, 1e-5, torch.empty(0, device="cuda"), 0)
         assert bool(((y.double() - x @ w.double()).abs() <= bound).all())
+
+
+@requires_gpu
+def test_position_of_a_decoding_step():
+    from petals_amd.ops.fused_decode import DecodeContext
+
+    ctx = DecodeContext(torch.device("cuda"))
+    for p in (0, 1, 7900, (1 << 31) - 3):
+        ctx.set_position(p)
+        assert (ctx.pos.tolist(), ctx.kv_len.tolist()) == ([p], [p + 1])
+        ctx.advance()
+        assert (ctx.pos.tolist(), ctx.kv_len.tolist()) == ([p + 1], [p + 2])
+    assert ctx.pos.dtype == ctx.kv_len.dtype == torch.int32
