@@ -7,7 +7,8 @@ layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
       rms_norm_f32out -> gemv(QKV) -> rope_cache_write -> attn_decode_fused
       -> gemv(O, +residual) -> rms_norm_f32out -> gemv(gate|up, SwiGLU epi)
       -> gemv(down, +residual)
-    ... 8 kernel launches per block, every byte of weights read exactly once
+    ... every product followed by the sum of its parts; with bf16 weights the norms are
+    taken within the products that read them (csrc/gemv_norm.h). Every byte of weights read exactly once
     (HBM-bound by design; see profiles/).
 
   prefill (q_len > 1): bf16 GEMMs on the SAME transposed weights (ops/csrc/gemm.hip up to
