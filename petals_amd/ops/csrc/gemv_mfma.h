@@ -173,7 +173,7 @@ static __global__ __launch_bounds__(256) void gemv_mfma_kernel(
     const int c = n0 + i % GEMV_MFMA_COLS;
     if (c >= out_dim) continue;
     float sum = (gemv_red[i] + gemv_red[n + i]) + (gemv_red[2 * n + i] + gemv_red[3 * n + i]);
-    if constexpr (NORM) sum *= norm_factor(norm, rows, i / GEMV_MFMA_COLS, in_dim, sq);
+    if constexpr (NORM) sum = norm_scaled(norm, rows, i / GEMV_MFMA_COLS, in_dim, sq, sum);
     const size_t row = sel ? (size_t)blockIdx.y * gridDim.z + blockIdx.z : (size_t)blockIdx.y * rows + i / GEMV_MFMA_COLS;
     partials[row * out_dim + c] = sum;
   }

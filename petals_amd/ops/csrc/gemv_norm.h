@@ -45,6 +45,20 @@ static __device__ __forceinline__ float norm_factor(const GemvNorm& n, int rows,
   return rsqrtf(((sq[r] + sq[rows + r]) + (sq[2 * rows + r] + sq[3 * rows + r])) / in_dim + n.eps);
 }
 
+// A row's sum times its factor. Where the squares overflow (from 2^64 on they do) the factor is 0, and
+// a norm of finite values is zeros, also where h * w or the sum is infinite; with an infinity among
+// the row's values it is NaN, as that sum times 0. The bits are looked at: -ffast-math knows no
+// infinities.
+static __device__ __forceinline__ float norm_scaled(const GemvNorm& n, int rows, int r, int in_dim, const float* sq, float sum) {
+  const float factor = norm_factor(n, rows, r, in_dim, sq);
+  if (__float_as_uint(factor) == 0u) {
+    bool finite = true;
+    for (int i = 0; i < in_dim; ++i) finite &= (n.h[(size_t)r * in_dim + i] & 0x7FFF) < 0x7F80;
+    if (finite) return 0.f;
+  }
+  return sum * factor;
+}
+
 // h [rows, in], w [in] and the sums of squares, as the kernels read them
 static inline GemvNorm gemv_norm(const torch::Tensor& h, const torch::Tensor& w, const c10::optional<torch::Tensor>& sumsq,
                                  double eps) {

@@ -942,6 +942,33 @@ def test_products_of_a_norm(hip, k_in, n_out, batch):
 
 
 @requires_gpu
+@pytest.mark.parametrize("k_in", [136, 4096])
+def test_products_of_a_norm_of_extreme_rows(hip, k_in):
+    """Infinities, NaNs and values whose squares overflow, as the norm kernel has them."""
+    gen = torch.Generator(device="cuda").manual_seed(k_in)
+    w = (torch.randn(k_in, 192, device="cuda", generator=gen) * 0.05).to(BF16)
+    h = torch.randn(8, k_in, device="cuda", generator=gen).to(BF16)
+    weight = (2 + 0.1 * torch.randn(k_in, device="cuda", generator=gen)).to(BF16)
+    h[1, 3] = float("inf")
+    h[2, 5] = float("nan")
+    h[3] = (h[3].float() * 1e38).clamp(-3e38, 3e38).to(BF16)  # twice these are infinite
+    h[4, 7] = 3e38
+    h[5, ::2] = 2.0**63.5  # no square is infinite, their sum is
+    h[6, 1], h[6, 2] = -3e38, float("-inf")
+    h[7, 7] = 2.0**63
+    empty = torch.empty(0, device="cuda")
+    want = hip.gemv_bf16(w, hip.rms_norm_f32out(h, weight, 1e-5), empty, None, 0)
+    assert want.isnan().all(-1).tolist() == [False, True, True, False, False, False, True, False]
+    assert not bool(want[3:6].any())
+    parts = torch.stack([c.float().square().sum(-1) for c in h.split(64, dim=-1)], dim=1)
+    for sumsq in (None, parts):
+        got = hip.gemv_bf16_normed(w, h, weight, sumsq, 1e-5, empty, 0)
+        assert torch.equal(got.isnan(), want.isnan())
+        kept = ~want.isnan()
+        torch.testing.assert_close(got[kept], want[kept], rtol=1e-4, atol=1e-4)
+
+
+@requires_gpu
 def test_position_of_a_decoding_step():
     from petals_amd.ops.fused_decode import DecodeContext
 
