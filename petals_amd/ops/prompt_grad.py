@@ -186,15 +186,20 @@ class _Attention(torch.autograd.Function):
 class _Product(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, hip):
-        ctx.w, ctx.hip = w, hip  # constant, maybe made in inference mode: such tensors can't be saved
+        # saved as torch's product saves it: hooks see it, and a change before the backward pass is
+        # an error. What was made in inference mode can't be saved
+        ctx.w = w if w.is_inference() else None
+        if ctx.w is None:
+            ctx.save_for_backward(w)
+        ctx.hip = hip
         return rows_product(x, w, hip)
 
     @staticmethod
     def backward(ctx, g):
-        w = ctx.w
-        if _by_torch(g):
+        w = ctx.saved_tensors[0] if ctx.w is None else ctx.w
+        if _by_torch(g, w):
             return torch.matmul(g, w.t()), None, None
-        return rows_product(g, w, ctx.hip, transposed=True), None, None
+        return rows_product(g, aligned(w), ctx.hip, transposed=True), None, None
 
 
 def rows_product(x, w, hip, transposed=False):

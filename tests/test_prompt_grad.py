@@ -250,6 +250,35 @@ def test_products_with_a_frozen_matrix(monkeypatch):
         torch.testing.assert_close(g, many @ w.t())
 
 
+@pytest.mark.parametrize("takes", [False, True])
+def test_frozen_matrix_is_saved(monkeypatch, takes):
+    """As by torch's product: hooks pack and unpack it, maybe to another address, and changing it
+    before the backward pass is an error."""
+    monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *sizes: takes)
+    w = torch.randn(64, 128, dtype=torch.float64)
+    x, v = (torch.randn(3, n, dtype=torch.float64) for n in (64, 128))
+    x.requires_grad_(True)
+
+    def unpack(t):
+        moved = torch.empty(t.numel() + 1, dtype=t.dtype)[1:].view(t.shape)
+        return moved.copy_(t)
+
+    for product in (torch.matmul, lambda a, b: prompt_grad._Product.apply(a, b, HIP)):
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, unpack):
+            y = product(x, w)
+        assert any(t.data_ptr() == w.data_ptr() for t in packed)
+        torch.testing.assert_close(torch.autograd.grad(y, x, v)[0], v @ w.t())
+        y = product(x, w)
+        w.mul_(2)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(y, x, v)
+    with torch.inference_mode():
+        constant = w.clone()
+    y = prompt_grad._Product.apply(x, constant, HIP)
+    torch.testing.assert_close(torch.autograd.grad(y, x, v)[0], v @ w.t())
+
+
 @pytest.mark.parametrize("rows", [1, 128, 129, 758, 1024, 1025])
 def test_rule_of_products(rows):
     # many rows of a wide matrix are the library's, few rows and sums that are long are the kernel's
