@@ -279,6 +279,21 @@ def test_frozen_matrix_is_saved(monkeypatch, takes):
     torch.testing.assert_close(torch.autograd.grad(y, x, v)[0], v @ w.t())
 
 
+def test_products_under_autocast(monkeypatch):
+    """They come in the type that autocast gives torch's products, with gradients."""
+    for rule in ("fused_training", "gemm_matrix"):
+        monkeypatch.setattr(prompt_grad, rule, lambda *tensors: True)
+    w = torch.randn(64, 128).bfloat16()
+    x = torch.randn(2, 3, 64).bfloat16().requires_grad_(True)
+    for kind in (torch.float16, torch.bfloat16):
+        with torch.autocast("cpu", kind):
+            y = prompt_grad.product(x, w, HIP)
+            want = torch.matmul(x, w)
+        assert y.dtype == want.dtype == kind and torch.equal(y, want)
+        g = torch.randn(y.shape).to(kind)
+        assert torch.equal(*(torch.autograd.grad(t, x, g)[0] for t in (y, want)))
+
+
 @pytest.mark.parametrize("rows", [1, 128, 129, 758, 1024, 1025])
 def test_rule_of_products(rows):
     # many rows of a wide matrix are the library's, few rows and sums that are long are the kernel's
