@@ -7,8 +7,8 @@ layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
       rms_norm_f32out -> gemv(QKV) -> rope_cache_write -> attn_decode_fused
       -> gemv(O, +residual) -> rms_norm_f32out -> gemv(gate|up, SwiGLU epi)
       -> gemv(down, +residual)
-    ... every product followed by the sum of its parts; with bf16 weights the norms are
-    taken within the products that read them (csrc/gemv_norm.h). Every byte of weights read exactly once
+    ... every product followed by the sum of its parts; with bf16 weights and few rows the norms
+    are taken within the products that read them (norm_within). Every byte of weights read exactly once
     (HBM-bound by design; see profiles/).
 
   prefill (q_len > 1): bf16 GEMMs on the SAME transposed weights (ops/csrc/gemm.hip up to
@@ -36,9 +36,26 @@ _EPI_RESIDUAL_BF16 = 2
 _EPI_SWIGLU_F32 = 3
 _EPI_GELU_F32 = 4
 
-# rows whose sums of squares every workgroup of the fused projection takes by itself. Width 2048, 1 row:
-# 6.0 us instead of 5.1 and a norm of 2.9; width 4096, 2 rows: 12.7 instead of 11.3 and 4.5
-_SELF_NORM_ROWS = 4
+def norm_within(rows: int, k: int, n: int, summed: bool) -> bool:
+    """Whether the RMS norm of rows of k values is faster within their product with a matrix [k, n] in
+    bf16 (csrc/gemv_norm.h) than ahead of it. `summed`: what wrote the rows left sums of their
+    squares; else every workgroup sums the rows up, and the time for that grows with rows, their length and the
+    workgroups. It saves a launch of 2 to 5 us. MI355X, us, ahead and within:
+
+      by itself   2048 x 2560   1 row 7.2, 5.4    4 rows 7.5, 7.2    5 rows 7.6, 7.8
+                  4096 x 6144   1 row 13.7, 11.5  2 rows 13.8, 12.7  4 rows 14.1, 14.3
+                  4096 x 12288  1 row 21.2, 19.6  2 rows 21.4, 22.4
+                  8192 x 2560   1 row 13.2, 11.4  3 rows 13.6, 13.7
+                  8192 x 10240  1 row 31.5, 33.8  4 rows 32.4, 43.0
+      summed      2048 x 11264  1 row 15.6, 13.0  6 rows 16.7, 15.9  8 rows 17.2, 17.6
+                  4096 x 5504   1 row 15.9, 13.3  5 rows 17.0, 15.4
+                  4096 x 28672  2 rows 44.7, 43.3  3 rows 45.2, 47.7  8 rows 49.9, 61.3
+                  8192 x 57344  2 rows 161, 161    3 rows 167, 174    8 rows 190, 224
+    """
+    if summed:
+        return rows <= 2 and rows * k <= 16384 or rows <= 6 and rows * k * n <= 1 << 27
+    return rows <= 4 and rows * k <= 12288 and rows * k * n <= (48 << 20 if k <= 6144 else 24 << 20)
+
 
 _workspaces: Dict[Tuple[torch.device, str], torch.Tensor] = {}
 _retired_workspaces: list = []  # replaced but possibly graph-captured (see _get_ws)
@@ -187,13 +204,15 @@ class _FastWeight:
         return self._gemv_raw(x, ws, residual, epilogue, self.splits, bias,
                               x_parts=x_parts, fold_eps=fold_eps, sumsq_out=sumsq_out)
 
-    def takes_norm(self, h: torch.Tensor) -> bool:
-        """Whether the RMS norm of these rows is taken within the product (csrc/gemv_norm.h): with bf16
-        weights. NF4's products are bound by vector instructions, not by memory: with the norm, 8192 x
-        57344 takes 65.9 us instead of 62.0 and a norm of 4.5, and 136.7 instead of 111 with 8 rows."""
+    def takes_norm(self, h: torch.Tensor, summed: bool) -> bool:
+        """Whether the RMS norm of these rows is taken within the product: with bf16 weights, by
+        norm_within's rule. NF4's products are bound by vector instructions, not by memory: with the
+        norm, 8192 x 57344 takes 65.9 us instead of 62.0 and a norm of 4.5, and 136.7 instead of 111
+        with 8 rows."""
         if self.t is None or self.t.data_ptr() % 16 or self.out_dim % 8:
             return False
-        return h.dtype == torch.bfloat16 and h.shape[1] % 8 == 0 and h.data_ptr() % 16 == 0
+        fits = h.dtype == torch.bfloat16 and h.shape[1] % 8 == 0 and h.data_ptr() % 16 == 0
+        return fits and norm_within(h.shape[0], self.in_dim, self.out_dim, summed)
 
     def gemv_normed(self, h, w, sumsq, eps, ws, epilogue):
         """gemv of the RMS norm of h [B, in] bf16 with weight w; sumsq [B, parts]: sums of a row's squares, or None"""
@@ -607,7 +626,7 @@ class LlamaFastPath(_TPFastPathMixin):
                 self.qh, self.kh, True,
             )
         elif adapter is None:
-            if B <= _SELF_NORM_ROWS and self.wqkv_t.takes_norm(h):
+            if self.wqkv_t.takes_norm(h, summed=False):
                 parts = self.wqkv_t.gemv_normed(h, self.ln1_w_post, None, self.eps, ws, _EPI_RAW)
             else:
                 xn = self.hip.rms_norm_f32out(h, self.ln1_w_post, self.eps)  # [B, H] f32
@@ -662,7 +681,7 @@ class LlamaFastPath(_TPFastPathMixin):
 
     def _norm_in_mlp(self, h: torch.Tensor) -> bool:
         """Whether the gate and up projection takes the norm ahead of it, of rows like h."""
-        return self.dense_mlp and self.wgateup_t.takes_norm(h) and self.wo_t.out_dim % 64 == 0
+        return self.dense_mlp and self.wgateup_t.takes_norm(h, summed=True) and self.wo_t.out_dim % 64 == 0
 
     def _max_gemv_out(self) -> int:
         return max(self.wgateup_t.shape[1], self.wqkv_t.shape[1], self.wo_t.shape[1])
