@@ -56,20 +56,46 @@ def gemm_matrix(w: torch.Tensor) -> bool:
     )
 
 
-def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = False) -> bool:
+def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = False, added: bool = False) -> bool:
     """Whether m rows of k times a matrix with n columns are faster by ops/csrc/gemm.hip than by the
-    library. `fused`: an activation follows, which would be a launch of its own.
+    library. `fused`: an activation follows, `added`: a residual, which would be a launch of its own.
 
     Up to 128 rows weights are what a product reads, and up to half as many tiles of 128 x 256 as there are
-    compute units the library leaves most of these idle: it takes 1.0 to 3.6 times as long (16384 x
-    4096: 139 beside 38 us at 128 rows, 156 beside 121 at 900). With 192 to 512 tiles it takes 0.76 to 1.0 times
-    as long (4096 x 28672: 77 beside 98 us at 283 rows). With a transposed matrix it does as well, but
-    where the sum is long beside the columns (22016 to 4096: 232 beside 162 us at 758 rows)."""
+    compute units the library leaves most of these idle: it takes 1.3 times as long in the mean (16384 x
+    4096: 139 beside 38 us at 128 rows, 156 beside 121 at 900). A call of the library also takes the
+    host 18 us and the kernel's 8, so that a product alone is the kernel's where it is up to 10 us the
+    slower of the two (2048 x 2560, 2 rows: both 11 us, alone 35 and 21): a small model's launches are
+    what bounds its prompts and gradients. Where it was slower by more, the library has the product: see
+    below, us on MI355X by the library (with what follows) and by the kernel, and
+    profiles/prompt_products.csv for all that was measured."""
     if m <= 0 or m * k >= 1 << 31:
         return False
-    tiles = -(-m // 128) * -(-n // 256)
+    weights, tiles = k * n, -(-m // 128) * -(-n // 256)
+    # three rows of tiles, nearly full, fit the library; the kernel's 96 tiles in two parts each leave a
+    # quarter of the compute units idle. 28672 x 8192: 283 rows 237, 193; 384 rows 200, 210.
+    # 57344 to 8192: 283 rows 331, 391
+    if n >= 8192 and weights >= 1 << 27 and (256 if weights > 1 << 28 else 320) < m <= 384:
+        return False
     if transposed:
+        # 16384 to 16384: 16 rows 97, 140; 128 rows 137, 153. 18432 to 16384: 128 rows 140, 130
+        if weights >= 1 << 28 and 8 * k < 9 * n:
+            return False
+        # 32768 to 8192: 16 rows 100, 132; 64 rows 152, 136. 57344 to 14336: 40 rows 286, 312; 128 rows 411, 335
+        if weights >= 1 << 28 and m <= 40 and 2 * n <= k <= 4 * n:
+            return False
+        if weights > 1 << 29 and m > 128:  # 106496 to 16384: 128 rows 632, 601; 129 rows 666, 1079
+            return False
+        # 12288 to 4096: 256 rows 51, 41; 758 rows 89, 93. 22016 to 4096: 758 rows 231, 160
         return tiles <= 64 and k >= n or tiles <= 128 and k >= 4 * n
+    # 2048 x 2560, where prompts are long enough for the host: 384 rows 14.0, 19.9; 1024 rows 26, 18
+    if 1 << 22 <= weights < 1 << 23 and m > 256 and tiles < 70 and n < 3 * k and not (fused or added and k >= 2 * n):
+        return False
+    # 8192 x 14336: 256 rows 98, 99; 384 rows 109, 135; 512 rows 135, 124
+    if fused and tiles > 128 and 256 < m <= 384 and weights >= 96 << 20:
+        return False
+    if n >= 4 * k and weights > 1 << 29 and m <= 16:  # 16384 x 106496: 16 rows 597, 635; 64 rows 766, 644
+        return False
+    # 8192 x 10240: 128 rows 76, 44; 384 rows 95, 84; 512 rows 108, 109. 4096 x 28672: 256 rows 79, 73; 283 rows 80, 100
     return m <= 128 or tiles <= (256 if fused else 128)
 
 
