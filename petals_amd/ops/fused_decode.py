@@ -96,7 +96,8 @@ class DecodeContext:
         self.kv_len = self._both[1:]  # prefix + 1
 
     def set_position(self, prefix_length: int) -> None:
-        torch.arange(prefix_length, prefix_length + 2, out=self._both)
+        # with its device: torch.set_default_device would put another one in
+        torch.arange(prefix_length, prefix_length + 2, out=self._both, device=self._both.device)
 
     def advance(self) -> None:
         """On-device increment (graph-capturable)."""
