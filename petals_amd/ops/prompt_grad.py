@@ -232,7 +232,7 @@ def rows_product(x, w, hip, transposed=False):
     """x [..., K] times w [K, N], or [..., N] times its transpose: by ops/csrc/gemm.hip where that is
     the faster one, else the library's."""
     k, n = w.shape if not transposed else w.shape[::-1]
-    if takes_gemm(x.numel() // k, k, n, transposed):
+    if x.shape[-1] == k and takes_gemm(x.numel() // k, k, n, transposed):  # torch refuses rows of other lengths
         return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
     return torch.matmul(x, w.t() if transposed else w)
 

@@ -921,6 +921,17 @@ def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
 
 
 @requires_gpu
+@pytest.mark.parametrize("shape", [(2, 3, 128), (4, 32)])
+def test_prompt_product_refuses_rows_that_do_not_fit(hip, shape):
+    from petals_amd.ops.fused_decode import _FastWeight, prompt_product
+
+    weight = _FastWeight(torch.ones(64, 128, device="cuda", dtype=BF16), hip, "none")
+    assert prompt_product(hip, torch.ones(2, 3, 64, device="cuda", dtype=BF16), weight).shape == (2, 3, 128)
+    with pytest.raises(RuntimeError, match="mat"):
+        prompt_product(hip, torch.ones(shape, device="cuda", dtype=BF16), weight)
+
+
+@requires_gpu
 @pytest.mark.parametrize("batch", [1, 3, 4, 5, 8])
 @pytest.mark.parametrize("k_in,n_out", [(8, 128), (136, 192), (1088, 64), (2056, 264), (4544, 2560), (8192, 1024)])
 def test_products_of_a_norm(hip, k_in, n_out, batch):

@@ -279,6 +279,17 @@ def test_frozen_matrix_is_saved(monkeypatch, takes):
     torch.testing.assert_close(torch.autograd.grad(y, x, v)[0], v @ w.t())
 
 
+def test_products_of_rows_that_do_not_fit(monkeypatch):
+    """Rows of another length are refused, also where there are whole ones of the matrix's in all."""
+    monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *sizes, **kinds: True)
+    w = torch.randn(64, 128, dtype=torch.float64)
+    for rows in (torch.randn(2, 3, 128, dtype=torch.float64), torch.randn(4, 32, dtype=torch.float64)):
+        with pytest.raises(RuntimeError, match="mat"):
+            prompt_grad._Product.apply(rows, w, HIP)
+    y = prompt_grad._Product.apply(torch.randn(4, 64, dtype=torch.float64, requires_grad=True), w, HIP)
+    assert y.shape == (4, 128)
+
+
 def test_products_under_autocast(monkeypatch):
     """They come in the type that autocast gives torch's products, with gradients."""
     for rule in ("fused_training", "gemm_matrix"):
