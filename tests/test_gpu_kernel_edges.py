@@ -861,7 +861,10 @@ def test_decode_attention_edges(hip, hd, gq, kv, alibi, kv_len, lmax):
         (127, 256, 576),  # as many steps as buffers
         (129, 704, 256),  # a row beyond two tiles, steps that end in the middle of the buffers
         (300, 4160, 192),  # parts along K, the last one shorter
-        (640, 1024, 3328),  # tiles of a whole wave and some left over, in parts
+        (640, 1024, 3328),  # the lowest tile: a whole wave and some left over, in parts
+        (640, 1024, 13312),  # the same for all tiles: 256, 512 or 1024 and 4, 8 or 16
+        (640, 448, 13312),  # and left over, but not in parts
+        (512, 192, 16384),  # whole waves and none left over
     ],
 )
 def test_prompt_product_edges(hip, m, k, n, tile, transposed):
@@ -892,9 +895,47 @@ def test_prompt_product_edges(hip, m, k, n, tile, transposed):
 
 
 @requires_gpu
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,k,n", [(40, 128, 128), (70, 1024, 320)])  # whole sums, and in parts
+def test_prompt_products_of_extreme_values(hip, m, k, n, transposed):
+    """Infinities, NaNs and large values stay in their rows and columns, and activations and
+    residuals have them as the library's product and the kernels after it do."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    x, residual = (torch.randn(m, c, device="cuda", generator=gen).to(BF16) for c in (k, n))
+    w = (torch.randn(k, n, device="cuda", generator=gen) * 0.125).to(BF16)
+    bias = torch.randn(n, device="cuda", generator=gen).to(BF16)
+    inf, nan = float("inf"), float("nan")
+    x[1, 3], x[2, k - 1], x[5, 0], x[6, 7], x[m - 1, 9] = inf, nan, -inf, 3e38, -3e38
+    w[11, 5], w[12, n // 2 + 5], w[k - 1, n - 1] = inf, nan, -inf
+    residual[3, 2], residual[4, 3], residual[7, 4] = inf, nan, -inf
+    bias[17], bias[18], bias[n - 2] = inf, nan, -inf
+    given = w.t().contiguous() if transposed else w
+    y = torch.matmul(x, w)
+    gelu = y.clone()
+    hip.bias_gelu_rows(gelu, bias)
+    want = [
+        (y, hip.gemm_rows(x, given, transposed, 0)),
+        (hip.add_rows(residual, y, None, bias), hip.gemm_rows(x, given, transposed, 1, residual, bias)),
+        (gelu, hip.gemm_rows(x, given, transposed, 2, None, bias)),
+        (hip.swiglu_rows(y), hip.gemm_rows(x, given, transposed, 3)),
+    ]
+    for ref, got in want:
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+        assert torch.equal(got[got.isinf()], ref[ref.isinf()])
+        finite = got.isfinite()
+        assert 0.5 < finite.float().mean() < 1
+        a, b = got[finite].double(), ref[finite].double()
+        # the reference rounds its product to bf16 (2^-9 of it) before the activation or residual
+        size = y.double().abs().clamp(max=1e30)[:, : got.shape[1]][finite] + 4
+        if got is want[3][1]:
+            size = size * y.double().abs().clamp(max=1e30)[:, n // 2 :][finite] + 4
+        assert bool(((a - b).abs() <= 2.0**-7 * b.abs() + 2.0**-8 * size).all())
+
+
+@requires_gpu
 @pytest.mark.parametrize("family,rows", [("llama", 40), ("bloom", 40), ("falcon", 40), ("llama", 700)])
 def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
-    """A block's prompt and gradients with and without csrc/gemm.hip."""
+    """A block's prompt with and without csrc/gemm.hip, and its gradients where they go through it."""
     from petals_amd.models.config_base import load_model_config
     from petals_amd.ops import prompt_grad
     from petals_amd.server.from_pretrained import build_empty_block, init_random_block_
@@ -905,17 +946,36 @@ def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
     block = block.eval().optimize_for_inference()
     gen = torch.Generator(device="cuda").manual_seed(rows)
     x, g = (torch.randn(2, rows // 2, config.hidden_size, device="cuda", generator=gen).to(BF16) for _ in range(2))
+    calls, gemm_rows = set(), hip.gemm_rows
+
+    def watched(x, w, transposed=False, epilogue=0, *rest):
+        calls.add((transposed, epilogue))
+        return gemm_rows(x, w, transposed, epilogue, *rest)
 
     def run():
         with torch.inference_mode():
             y = block(x)
+        by_prompt = frozenset(calls)
+        calls.clear()
+        if family != "llama":  # their gradients are torch's
+            return by_prompt, y
         leaf = x.clone().requires_grad_(True)
         (dx,) = torch.autograd.grad(block(leaf), leaf, g)
-        return y, dx
+        return by_prompt, y, dx
 
-    got = run()
+    monkeypatch.setattr(hip, "gemm_rows", watched)
+    prompts, *got = run()
+    plain, residual, gelu, swiglu = ((False, epilogue) for epilogue in range(4))
+    assert prompts == {
+        ("llama", 40): {plain, swiglu, residual}, ("llama", 700): {residual},
+        ("bloom", 40): {plain, gelu, residual}, ("falcon", 40): {plain, gelu},
+    }[family, rows]
+    assert calls == ({plain, (True, 0)} if family == "llama" else set())
+    calls.clear()
     monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *args, **kwargs: False)
-    for a, b in zip(got, run()):
+    prompts, *want = run()
+    assert not prompts and not calls
+    for a, b in zip(got, want):
         # both round every product to bf16: errors of 2^-9 each, over a block's half a dozen
         assert (a.double() - b.double()).norm() <= 2.0**-6 * b.double().norm()
 
@@ -940,7 +1000,8 @@ def test_products_of_a_norm(hip, k_in, n_out, batch):
     w = (torch.randn(k_in, n_out, device="cuda", generator=gen) * 0.05).to(BF16)
     h = torch.randn(batch, k_in, device="cuda", generator=gen).to(BF16)
     h[:, :: max(1, k_in // 5)] *= 300.0  # loud channels
-    h[batch // 2] *= 1e-10
+    if batch > 1:  # next to which eps is large, so that it says nothing about the sum of squares
+        h[batch // 2] *= 1e-10
     weight = (1 + 0.1 * torch.randn(k_in, device="cuda", generator=gen)).to(BF16)
     hd = h.double()
     x = hd * torch.rsqrt(hd.square().mean(-1, keepdim=True) + 1e-5) * weight.double()
@@ -950,6 +1011,40 @@ def test_products_of_a_norm(hip, k_in, n_out, batch):
     for sumsq in (None, parts):
         y = hip.gemv_bf16_normed(w, h, weight, sumsq, 1e-5, torch.empty(0, device="cuda"), 0)
         assert bool(((y.double() - x @ w.double()).abs() <= bound).all())
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", [1, 2, 6])
+@pytest.mark.parametrize("k_in,width,inner", [(64, 128, 64), (192, 1024, 136), (136, 1152, 72), (128, 2176, 128), (2048, 4096, 512)])
+def test_products_of_a_norm_of_a_sum(hip, k_in, width, inner, batch):
+    """As a decoding step has them: a product added to the stream leaves sums of squares, and gate and up
+    take the norm with them, in 1, 8, 9, 17 and, wider, 32 parts."""
+    gen = torch.Generator(device="cuda").manual_seed(width + batch)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).to(BF16)
+
+    wo, both, weight = normal(k_in, width) * 0.05, normal(width, 2 * inner) * 0.05, 1 + 0.1 * normal(width)
+    x, h = torch.randn(batch, k_in, device="cuda", generator=gen), normal(batch, width) * 3
+    h[:, :: width // 5] *= 100.0  # loud channels
+    sums = torch.full((batch, width // 64), float("nan"), device="cuda")
+    ws = torch.empty(64 * batch * max(width, 2 * inner), device="cuda")
+    h2 = hip.gemv_bf16(wo, x, ws, h, 2, 0, None, sums)
+    hd = h2.double()
+    squares = hd.square().view(batch, -1, 64).sum(-1)
+    assert bool(((sums.double() - squares).abs() <= 2.0**-20 * squares).all())
+    act = hip.gemv_bf16_normed(both, h2, weight, sums, 1e-5, ws, 3)
+    # and with sums of squares that every workgroup takes
+    alone = hip.gemv_bf16_normed(both, h2, weight, None, 1e-5, torch.empty(0, device="cuda"), 3)
+    n = hd * torch.rsqrt(hd.square().mean(-1, keepdim=True) + 1e-5) * weight.double()
+    gu = n @ both.double()
+    bound = sum_bound(n, both.double()) + 16 * 2.0**-24 * gu.abs()
+    (g, u), (bg, bu) = gu.chunk(2, dim=-1), bound.chunk(2, dim=-1)
+    silu = torch.nn.functional.silu(g)
+    # silu's slope is at most 1.1; its exponential is good to 2^-20
+    bound = 1.1 * bg * (u.abs() + bu) + silu.abs() * bu + (silu * u).abs() * 2.0**-20 + 1e-12
+    for y in (act, alone):
+        assert bool(((y.double() - silu * u).abs() <= bound).all())
 
 
 @requires_gpu
