@@ -7,7 +7,8 @@ inference with server-side KV caches, and parameter-efficient fine-tuning
 (prompt tuning / LoRA) over the swarm.
 
 The compute path is MI355X-first: hand-written HIP/CDNA4 kernels (MFMA + LDS
-tiles) for the hot ops, hipBLASLt/rocBLAS for plain GEMMs, RCCL over xGMI for
+tiles) for the hot ops and for the GEMMs of decoding and of prompts of some hundreds of
+rows, hipBLASLt/rocBLAS for larger plain GEMMs, RCCL over xGMI for
 intra-node activation hand-off and tensor parallelism.
 """
 

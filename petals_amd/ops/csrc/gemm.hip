@@ -35,7 +35,8 @@
 //   28672 x 8192      134, 86     199, 96      352, 216     301, 389
 //   8192 x 57344      161, 161    173, 175     413, 459     602, 651
 //   22016, transposed, to 4096:   114, 52      233, 102     232, 162
-// Which of the two a product takes is ops/prompt_grad.py's rule.
+// A call takes the host 8 us, the library's 18. Which of the two a product takes is ops/prompt_grad.py's rule
+// (takes_gemm); profiles/prompt_products.csv has what it was drawn from.
 
 #include "common.h"
 #include "gemv_reduce.h"

@@ -4,7 +4,8 @@
 // 16-bit products of two bf16 numbers, the factor of a row is known when the weights have arrived, and
 // no launch of its own (2.9 us at width 2048, 4.5 us at 8192, as much as a small product) comes first.
 // A row's sum of squares is either given in parts, by the kernel that wrote the row (gemv_reduce.h), or
-// every workgroup sums the row up, which is 16 KB from L2 at width 8192: for few rows only.
+// every workgroup sums the row up, which is 16 KB from L2 at width 8192: for few rows only. How few is
+// ops/fused_decode.py's rule (norm_within), with times.
 #pragma once
 
 #include "common.h"

@@ -51,16 +51,15 @@ static __device__ __forceinline__ float gelu_tanh_f32(float x) {
   return 0.5f * x * (1.f + t);
 }
 
-// 512 threads = 64 outputs x 8 split groups per workgroup: the one-thread-
+// A workgroup has 64 outputs x G groups of parts, a wave each: the one-thread-
 // per-output version launched only `out/64` single-wave workgroups (0.15
 // waves/SIMD for a 10k-output gemv) and was latency-bound at ~7 us — as much
-// as the small gemvs themselves. Split groups multiply resident waves 8x and
-// cut each thread's serial chain 8x; a tiny LDS tree combines (deterministic
-// order preserved: fixed group partition, fixed add order).
-#define GEMV_REDUCE_GROUPS 16  // 16 split groups x 64 outputs (1024-thread
-// wgs): halves each thread's serial split chain vs the earlier value of 8 —
-// +1.3 tok/s on every alternating A/B pair (profiles/qrr_groups_ab.log);
-// PETALS_REDUCE_GROUPS=8 selects the old width
+// as the small gemvs themselves. Groups multiply resident waves and
+// cut each thread's serial chain; a tiny LDS tree combines (deterministic
+// order preserved: fixed group partition, fixed add order). G is chosen in
+// launch_gemv_reduce.
+#define GEMV_REDUCE_GROUPS 16  // most of them: 1024 threads. Of many parts, half the serial chain
+// that 8 have: +1.3 tok/s on every alternating A/B pair (profiles/qrr_groups_ab.log)
 
 template <int G>
 static __global__ __launch_bounds__(64 * G) void gemv_reduce_kernel_impl(
@@ -201,7 +200,10 @@ static inline torch::Tensor launch_gemv_reduce(
     const char* e = std::getenv("PETALS_REDUCE_GROUPS");
     return e ? std::atoi(e) : 0;
   }();
-  // no more groups than parts: 8 x 57344 in two parts take 4.6 us so, 11.7 with 16. The sums are the same
+  // the fewest of 4, 8 and 16 groups that have a part each at most, 16 beyond that: a group without parts is a wave
+  // that only waits. 8 x 57344 in two parts take 4.6 us with 4, 11.7 with 16; 4096 x 28672 with its product, 8
+  // rows in 8 parts, 46.8 with 8, 48.9 with 16. The sums are the same. PETALS_REDUCE_GROUPS=8 or 16 is
+  // used for all
   const int groups = red_g == 16 || red_g == 8 ? red_g : n_splits <= 4 ? 4 : n_splits <= 8 ? 8 : GEMV_REDUCE_GROUPS;
   int rblocks = (total + 63) / 64;
   auto stream = c10::hip::getCurrentHIPStream().stream();

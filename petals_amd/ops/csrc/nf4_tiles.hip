@@ -35,18 +35,18 @@
 // It is bound by vector instructions (half-rate lookups; the chip lowers its clock under
 // them), not by memory. llama-2-70b, us a product with its reduction, the kernel in
 // nf4.hip and this one, for 1, 4 and 8 rows:
-//   qkv   8192 x 10240   19, 29, 47     20, 23, 31
-//   o     8192 x 8192    22, 30, 49     17, 19, 23
-//   gate  8192 x 57344   64, 96, 160    65, 79, 112
-//   down  28672 x 8192   36, 51, 84     34, 40, 61
-// (Runs of 1024 for one row: 70 and 38 us for the last two; four waves a SIMD: 71, 39.)
+//   qkv   8192 x 10240   19, 29, 47     21, 22, 30
+//   o     8192 x 8192    22, 30, 49     17, 19, 22
+//   gate  8192 x 57344   64, 96, 160    61, 69, 103
+//   down  28672 x 8192   36, 51, 84     34, 41, 60
+// (Before lookups were summed, runs of 1024 for one row: 70 and 38 us for the last two beside 65 and 34; four waves
+// a SIMD: 71, 39.)
 // Cut off instead of rounded, and with the largest input of a run at 2^30 whatever the others
 // are, it took 0 to 5% less (8192 x 8192: 14.7, 16.1, 18.5 us without the reduction for 1, 4,
 // 8 rows beside 14.8, 16.6, 19.5). Runs with inputs beyond 64 times their mean take longer: two
 // of 8192 inputs a thousand times the rest, 15.2, 18.2, 23.6.
-// Weights are read once and marked so (non-temporal): a decoding step of four blocks of width
-// 8192 takes 589 us instead of 601 with one row, 1059 instead of 1071 with eight, one of two
-// blocks of 8 experts 301 instead of 312.
+// Weights are read once and marked so (non-temporal): 2% of a decoding step of four blocks of width
+// 8192 with one row (601 to 589 us when it was measured), 1% with eight, 3.5% of two blocks of 8 experts.
 // Error against 64 bits, of the root mean square result: 0.9e-7 (nf4.hip: 1.6e-7).
 
 #include "common.h"
@@ -137,7 +137,8 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   const int steps = LONG ? n_steps : 1;
   constexpr int NS = (B + 3) / 4, NCOL = 4 * B, PER = KB * 2;
   // the two lookups of a digit are multiplied one by one, which saves their xor, where the matrix cores
-  // have little else to do: 8192 x 57344 takes 59.5 instead of 61.8 us with 1 row, 113.7 instead of 111.3 with 8
+  // have little else to do: 8192 x 57344 takes 59.5 instead of 61.8 us with 1 row, 63.0 instead of 65.0 with 2,
+  // 72.0 instead of 74.0 with 4, but 113.7 instead of 111.3 with 8
   constexpr bool SUMMED = NS == 1;
   __shared__ __align__(16) unsigned char digits[4][KB * 128 * NCOL];
   __shared__ __align__(16) float red[4 * B * 64];  // [waves, rows, columns]

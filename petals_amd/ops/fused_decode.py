@@ -4,12 +4,12 @@
 layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
 
   decode (q_len == 1, any batch <= 8):
-      rms_norm_f32out -> gemv(QKV) -> rope_cache_write -> attn_decode_fused
+      rms_norm_f32out -> gemv(QKV) -> qkv_rope_reduce (sum, rotation, cache) -> attn_decode_fused
       -> gemv(O, +residual) -> rms_norm_f32out -> gemv(gate|up, SwiGLU epi)
       -> gemv(down, +residual)
-    ... every product followed by the sum of its parts; with bf16 weights and few rows the norms
-    are taken within the products that read them (norm_within). Every byte of weights read exactly once
-    (HBM-bound by design; see profiles/).
+    ... every product followed by the sum of its parts, which has its epilogue; with bf16 weights and few
+    rows the norms are taken within the products that read them (norm_within). Every byte of
+    weights is read exactly once (HBM-bound by design; see profiles/).
 
   prefill (q_len > 1): bf16 GEMMs on the SAME transposed weights (ops/csrc/gemm.hip up to
     some hundreds of rows, the library beyond), one kernel for each gap between them
