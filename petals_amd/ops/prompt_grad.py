@@ -243,7 +243,7 @@ def norm(x, w, eps, hip):
 
 def product(x, w, hip):
     """x [..., K] times a frozen matrix [K, N]. Autocast may have torch's product in another type."""
-    if w.requires_grad or torch.is_autocast_enabled(x.device.type) or not (fused_training(x) and gemm_matrix(w)):
+    if w.requires_grad or not (fused_training(x) and gemm_matrix(w)) or torch.is_autocast_enabled(x.device.type):
         return torch.matmul(x, w)
     return _Product.apply(x, w, hip)
 

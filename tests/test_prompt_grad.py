@@ -291,7 +291,10 @@ def test_products_of_rows_that_do_not_fit(monkeypatch):
 
 
 def test_products_under_autocast(monkeypatch):
-    """They come in the type that autocast gives torch's products, with gradients."""
+    """They come in the type that autocast gives torch's products, with gradients. Devices that have
+    no autocast are not asked for it."""
+    shapes = (torch.ones(*s, device="meta", dtype=torch.bfloat16) for s in ((3, 64), (64, 128)))
+    assert prompt_grad.product(*shapes, HIP).shape == (3, 128)
     for rule in ("fused_training", "gemm_matrix"):
         monkeypatch.setattr(prompt_grad, rule, lambda *tensors: True)
     w = torch.randn(64, 128).bfloat16()
