@@ -48,6 +48,12 @@ def aligned(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
+def recast(rows: torch.Tensor) -> bool:
+    """Whether autocast has torch's products of these rows, which are on a GPU, in another type than bf16."""
+    kind = rows.device.type
+    return torch.is_autocast_enabled(kind) and torch.get_autocast_dtype(kind) != torch.bfloat16
+
+
 def gemm_matrix(w: torch.Tensor) -> bool:
     """A matrix [K, N] that ops/csrc/gemm.hip takes, from either side."""
     return (
@@ -242,8 +248,8 @@ def norm(x, w, eps, hip):
 
 
 def product(x, w, hip):
-    """x [..., K] times a frozen matrix [K, N]. Autocast may have torch's product in another type."""
-    if w.requires_grad or not (fused_training(x) and gemm_matrix(w)) or torch.is_autocast_enabled(x.device.type):
+    """x [..., K] times a frozen matrix [K, N]"""
+    if w.requires_grad or not (fused_training(x) and gemm_matrix(w)) or recast(x):
         return torch.matmul(x, w)
     return _Product.apply(x, w, hip)
 

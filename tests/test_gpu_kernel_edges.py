@@ -981,6 +981,22 @@ def test_prompt_products_match_the_library(hip, monkeypatch, family, rows):
 
 
 @requires_gpu
+@pytest.mark.parametrize("kind", [torch.float16, BF16])
+def test_prompt_product_under_autocast(hip, kind):
+    """In the type that autocast gives torch's product, whichever kernel would have it."""
+    from petals_amd.ops.fused_decode import _FastWeight, prompt_product
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x, w = (torch.randn(*s, device="cuda", generator=gen).to(BF16) for s in ((40, 4096), (4096, 4096)))
+    with torch.inference_mode(), torch.autocast("cuda", kind):
+        y = prompt_product(hip, x, _FastWeight(w, hip, "none"))
+        want = torch.matmul(x, w)
+    assert y.dtype == want.dtype == kind
+    if kind != BF16:
+        assert torch.equal(y, want)
+
+
+@requires_gpu
 @pytest.mark.parametrize("shape", [(2, 3, 128), (4, 32)])
 def test_prompt_product_refuses_rows_that_do_not_fit(hip, shape):
     from petals_amd.ops.fused_decode import _FastWeight, prompt_product
