@@ -336,7 +336,7 @@ def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=Non
     fused = epilogue in (_GEMM_GELU, _GEMM_SWIGLU)
     if (
         x.is_cuda and x.dtype == torch.bfloat16 and prompt_grad.gemm_matrix(w) and x.shape[-1] == w.shape[0]
-        and not prompt_grad.recast(x)
+        and not prompt_grad.recast(x) and not torch._C._len_torch_dispatch_stack()  # modes see torch's product
         and prompt_grad.takes_gemm(x.numel() // w.shape[0], *w.shape, fused=fused, added=epilogue == _GEMM_RESIDUAL)
     ):
         rows = prompt_grad.aligned(x).view(-1, w.shape[0])

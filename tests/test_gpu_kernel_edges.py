@@ -997,6 +997,21 @@ def test_prompt_product_under_autocast(hip, kind):
 
 
 @requires_gpu
+def test_modes_see_prompt_products(hip):
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from petals_amd.ops.fused_decode import _FastWeight, prompt_product
+
+    x, w = (torch.ones(*s, device="cuda", dtype=BF16) for s in ((40, 256), (256, 512)))
+    weight = _FastWeight(w, hip, "none")
+    with torch.inference_mode():
+        with FlopCounterMode(display=False) as counter:
+            seen = prompt_product(hip, x, weight)
+        assert torch.equal(seen, prompt_product(hip, x, weight))
+    assert counter.get_total_flops() == 2 * 40 * 256 * 512
+
+
+@requires_gpu
 @pytest.mark.parametrize("shape", [(2, 3, 128), (4, 32)])
 def test_prompt_product_refuses_rows_that_do_not_fit(hip, shape):
     from petals_amd.ops.fused_decode import _FastWeight, prompt_product
