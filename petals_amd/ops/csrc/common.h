@@ -15,12 +15,10 @@ __device__ __forceinline__ float bf16_to_f32(unsigned short u) {
   return v.f;
 }
 
+// to nearest, ties to even. One v_cvt_pk_bf16_f32, of two neighbouring values where both are needed, in the
+// place of four whole-number operations a value
 __device__ __forceinline__ unsigned short f32_to_bf16(float f) {
-  union { float f; uint32_t i; } v;
-  v.f = f;
-  uint32_t lsb = (v.i >> 16) & 1;            // round-to-nearest-even
-  uint32_t r = (v.i + 0x7FFFu + lsb) >> 16;
-  return (unsigned short)r;
+  return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
 // full-wave fp32 sum (64 lanes)

@@ -1116,3 +1116,18 @@ def test_position_of_a_decoding_step():
         ctx.advance()
         assert (ctx.pos.tolist(), ctx.kv_len.tolist()) == ([p + 1], [p + 2])
     assert ctx.pos.dtype == ctx.kv_len.dtype == torch.int32
+
+
+@requires_gpu
+def test_rounding_to_bf16(hip):
+    """Ties, subnormal numbers, overflow, infinities and NaNs: sums of two bf16 values, rounded once, are torch's to the bit."""
+    bits = torch.arange(1 << 16, device="cuda", dtype=torch.int32)
+    x = bits.to(torch.int16).view(BF16).view(256, 256)  # every bf16 value
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    near = torch.randint(-9, 10, (1 << 16,), device="cuda", generator=gen) * 128  # exponents up to nine apart: half of the sums are ties
+    others = [x.flip(0), (bits ^ 1).to(torch.int16).view(BF16).view_as(x), (bits + near).to(torch.int16).view(BF16).view_as(x)]
+    for y in others:
+        got, want = hip.add_rows(x.contiguous(), y.contiguous()), x + y
+        assert torch.equal(got.isnan(), want.isnan())
+        kept = ~want.isnan()
+        assert torch.equal(got[kept].view(torch.int16), want[kept].view(torch.int16))
