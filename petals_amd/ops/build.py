@@ -28,7 +28,7 @@ EXTENSIONS = {
     "core": (
         "_hip_ops.so", "petals_amd_hip_ops", "_build",
         ["bindings.cpp", "elementwise.hip", "gemv.hip", "attention.hip", "nf4.hip", "nf4_tiles.hip", "int8.hip",
-         "prefill_attn.hip", "attn_grad.hip", "prefill_rows.hip", "gemm.hip", "moe.hip"],
+         "prefill_attn.hip", "attn_grad.hip", "prefill_rows.hip", "gemm.hip", "nf4_gemm.hip", "moe.hip"],
     ),
     "latent": (
         "_hip_latent.so", "petals_amd_hip_latent", os.path.join("_build", "latent"),

@@ -58,6 +58,8 @@ torch::Tensor add_rows(torch::Tensor x, torch::Tensor y, c10::optional<torch::Te
 torch::Tensor swiglu_rows(torch::Tensor gu);
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
                         c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile);
+torch::Tensor gemm_nf4_rows(torch::Tensor x, torch::Tensor tiles, torch::Tensor scales, int64_t epilogue,
+                            c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile);
 void bias_gelu_rows(torch::Tensor y, c10::optional<torch::Tensor> bias);
 std::vector<torch::Tensor> nf4_quantize(torch::Tensor w);
 torch::Tensor gemv_int8(
@@ -150,6 +152,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rows", &gemm_rows, "a prompt's rows times a bf16 matrix, and what follows", py::arg("x"), py::arg("w"),
         py::arg("transposed") = false, py::arg("epilogue") = 0, py::arg("residual") = py::none(),
         py::arg("bias") = py::none(), py::arg("tile") = -1);
+  m.def("gemm_nf4_rows", &gemm_nf4_rows, "a prompt's rows times NF4 tiles, and what follows", py::arg("x"), py::arg("tiles"),
+        py::arg("scales"), py::arg("epilogue") = 0, py::arg("residual") = py::none(), py::arg("bias") = py::none(),
+        py::arg("tile") = -1);
   m.def("swiglu_rows", &swiglu_rows, "[..., gate | up] -> silu(gate) * up");
   m.def("bias_gelu_rows", &bias_gelu_rows, "gelu(y + bias), in place", py::arg("y"), py::arg("bias") = py::none());
   m.def("nf4_tile", &nf4_tile, "NF4 in the order of the matrix cores: (packed, absmax) -> (tiles, scales)");

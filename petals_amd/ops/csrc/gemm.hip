@@ -38,78 +38,11 @@
 // A call takes the host 8 us, the library's 18. Which of the two a product takes is ops/prompt_grad.py's rule
 // (takes_gemm); profiles/prompt_products.csv has what it was drawn from.
 
-#include "common.h"
-#include "gemv_reduce.h"
-#include "paged.h"
+#include "gemm.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 
-#define GEMM_THREADS 512
 #define GEMM_BK 64
-#define GEMM_CUS 256
-
-enum GemmEpilogue : int {
-  GEMM_PLAIN = 0,     // y
-  GEMM_RESIDUAL = 1,  // residual + y + bias
-  GEMM_GELU = 2,      // gelu(y + bias)
-  GEMM_SWIGLU = 3,    // silu(y[:N/2]) * y[N/2:]
-};
-
-struct GemmShape {
-  int m, n, k;
-  int row_tiles;  // of a run of columns
-  int whole;      // tiles summed over all of K
-  int rest;       // tiles split along K
-  int splits, per;  // parts of these, and steps of each
-};
-
-struct GemmOut {
-  unsigned short* y;               // [M, N], or [M, N/2] for GEMM_SWIGLU
-  const unsigned short* residual;  // [M, N] or null
-  const unsigned short* bias;      // [N] or null
-  float* parts;                    // [splits, rest, BM, BN]
-  int epilogue;
-};
-
-using gemm_rsrc = __attribute__((ext_vector_type(4))) int;
-
-// where a tile's column comes from: with GEMM_SWIGLU, half of a wave's columns are gates, and
-// the other half the same columns of up
-template <int FN>
-__device__ __forceinline__ int gemm_source_column(int tile, int c, int bn, int n, bool pairs) {
-  if (!pairs) return tile * bn + c;
-  constexpr int HALF = FN * 8;
-  const int in = c % (2 * HALF);
-  return tile * (bn / 2) + c / (2 * HALF) * HALF + in % HALF + (in >= HALF ? n / 2 : 0);
-}
-
-// four neighbouring values of a row, at column c of y's
-__device__ __forceinline__ void gemm_store(const GemmShape& s, const GemmOut& o, int m, int c, f32x4 v) {
-  if (m >= s.m || c >= s.n) return;
-  if (o.bias) {
-    const v4s b = *reinterpret_cast<const v4s*>(o.bias + c);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += bf16_to_f32((unsigned short)b[i]);
-  }
-  const size_t at = (size_t)m * s.n + c;
-  if (o.residual) {
-    const v4s r = *reinterpret_cast<const v4s*>(o.residual + at);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += bf16_to_f32((unsigned short)r[i]);
-  }
-  v4s y;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = (short)f32_to_bf16(o.epilogue == GEMM_GELU ? gelu_tanh_f32(v[i]) : v[i]);
-  *reinterpret_cast<v4s*>(o.y + at) = y;
-}
-
-__device__ __forceinline__ void gemm_store_pair(const GemmShape& s, const GemmOut& o, int m, int c, f32x4 g, f32x4 u) {
-  if (m >= s.m || c >= s.n / 2) return;
-  v4s y;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = (short)f32_to_bf16(g[i] / (1.f + __expf(-g[i])) * u[i]);
-  *reinterpret_cast<v4s*>(o.y + (size_t)m * (s.n / 2) + c) = y;
-}
 
 // byte offset of 16-byte group c in a row of 128 bytes, and of one in a row of W [K, N]
 __device__ __forceinline__ int gemm_row_group(int row, int c) { return row * (GEMM_BK * 2) + ((c ^ (row & 7)) << 4); }
@@ -132,18 +65,9 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 15, hi = lane >> 4;
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  int tile, first = 0, steps = s.k / BK, part = -1;
-  if (local < s.whole / 8) {  // `whole` is a multiple of 8
-    tile = xcd * (s.whole / 8) + local;
-  } else {
-    const int units = s.rest * s.splits, share = (units + 7) / 8, unit = xcd * share + local - s.whole / 8;
-    if (local - s.whole / 8 >= share || unit >= units) return;  // uniform over the workgroup
-    tile = s.whole + unit % s.rest;
-    part = s.splits > 1 ? unit / s.rest : -1;
-    first = unit / s.rest * s.per;
-    steps = min(s.per, steps - first);
-  }
+  GemmSpot spot;
+  if (!gemm_spot(s, s.k / BK, &spot)) return;
+  const int tile = spot.tile, first = spot.first, steps = spot.steps, part = spot.part;
   const bool pairs = o.epilogue == GEMM_SWIGLU;
   const int m0 = tile % s.row_tiles * BM, column_tile = tile / s.row_tiles;
   const int wm = wave / WC * FM * 16, wn = wave % WC * FN * 16;
@@ -304,49 +228,9 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
   }
 }
 
-// four values of a tile per thread
-template <int BM, int BN, int FN>
-__global__ __launch_bounds__(256) void gemm_parts_kernel(GemmShape s, GemmOut o) {
-  const bool pairs = o.epilogue == GEMM_SWIGLU;
-  const int at = blockIdx.x * 256 + threadIdx.x, columns = pairs ? BN / 2 : BN;
-  const int tile = at / (BM * columns / 4), in = at % (BM * columns / 4) * 4;
-  if (tile >= s.rest) return;
-  const int row = in / columns;
-  int c = in % columns;
-  if (pairs) c = c / (FN * 8) * (FN * 16) + c % (FN * 8);
-  const int m = (s.whole + tile) % s.row_tiles * BM + row, column_tile = (s.whole + tile) / s.row_tiles;
-  if (m >= s.m) return;
-  const float* p = o.parts + (size_t)tile * (BM * BN) + row * BN + c;
-  const size_t stride = (size_t)s.rest * (BM * BN);
-  f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f}, up = sum;
-  for (int i = 0; i < s.splits; ++i) {
-    sum += *reinterpret_cast<const f32x4*>(p + i * stride);
-    if (pairs) up += *reinterpret_cast<const f32x4*>(p + i * stride + FN * 8);
-  }
-  const int n = gemm_source_column<FN>(column_tile, c, BN, s.n, pairs);
-  if (pairs) gemm_store_pair(s, o, m, n, sum, up);
-  else gemm_store(s, o, m, n, sum);
-}
-
 // ------------------------------------------------------------------- host
 
-struct GemmTile {
-  int bm, bn;
-  float step;  // us of 64 of K, a tile on every compute unit
-};
 static const GemmTile GEMM_TILES[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
-
-static GemmShape gemm_plan(long m, long n, long k, const GemmTile& t, float* us) {
-  const long row_tiles = (m + t.bm - 1) / t.bm, tiles = row_tiles * ((n + t.bn - 1) / t.bn), steps = k / GEMM_BK;
-  long whole = tiles / GEMM_CUS * GEMM_CUS, rest = tiles - whole, splits = 1;
-  // parts of at least 8 steps
-  if (rest) splits = std::max(1L, std::min(GEMM_CUS / rest, steps / 8));
-  long per = (steps + splits - 1) / splits;
-  splits = (steps + per - 1) / per;
-  *us = t.step * (tiles / GEMM_CUS * steps + (rest ? per : 0));
-  if (splits > 1) *us += 5.f + rest * splits * t.bm * t.bn * 4 * 2 / 8e6f;
-  return GemmShape{(int)m, (int)n, (int)k, (int)row_tiles, (int)whole, (int)rest, (int)splits, (int)per};
-}
 
 // x [M, K] bf16, w [K, N] (or [N, K], transposed) bf16 -> [M, N] bf16 (swiglu: [M, N/2])
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
@@ -382,7 +266,7 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
   for (int i = 0; i < 4; ++i) {
     if (tile >= 0 && tile != i) continue;
     float us;
-    const GemmShape p = gemm_plan(m, n, k, GEMM_TILES[i], &us);
+    const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, GEMM_TILES[i], &us);
     if (s.m == 0 || us < least) best = i, least = us, s = p;
   }
   const GemmTile& t = GEMM_TILES[best];

@@ -12,7 +12,8 @@ layout (transposed [in, out] bf16, QKV and gate/up concatenated) and then runs:
     weights is read exactly once (HBM-bound by design; see profiles/).
 
   prefill (q_len > 1): bf16 GEMMs on the SAME transposed weights (ops/csrc/gemm.hip up to
-    some hundreds of rows, the library beyond), one kernel for each gap between them
+    some hundreds of rows, the library beyond; NF4 weights up to 128 rows by ops/csrc/nf4_gemm.hip,
+    from their codes), one kernel for each gap between them
     (ops/csrc/prefill_rows.hip) and flash attention (prefill_attn.hip).
 
 The original nn.Linear weights are FREED after repacking (a 70B span must not
@@ -332,17 +333,27 @@ _GEMM_SWIGLU = 3
 def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=None):
     """A prompt's rows [..., K] times a _FastWeight, without gradients, and what follows: residual +
     y + bias, gelu(y + bias), or the SwiGLU of [gate | up]."""
-    w = weight.dense()
+    k, n = weight.shape
     fused = epilogue in (_GEMM_GELU, _GEMM_SWIGLU)
-    if (
-        x.is_cuda and x.dtype == torch.bfloat16 and prompt_grad.gemm_matrix(w) and x.shape[-1] == w.shape[0]
+    by_kernel = (
+        x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] == k
         and not prompt_grad.recast(x) and not torch._C._len_torch_dispatch_stack()  # modes see torch's product
-        and prompt_grad.takes_gemm(x.numel() // w.shape[0], *w.shape, fused=fused, added=epilogue == _GEMM_RESIDUAL)
+    )
+
+    def rows():
+        x2 = prompt_grad.aligned(x).view(-1, k)
+        return x2, None if residual is None else prompt_grad.aligned(residual).view(x2.shape[0], -1)
+
+    if by_kernel and weight.tiles is not None and prompt_grad.takes_nf4_gemm(x.numel() // k, k, n):
+        x2, added = rows()
+        return hip.gemm_nf4_rows(x2, weight.tiles, weight.scales, epilogue, added, bias).view(*x.shape[:-1], -1)
+    w = weight.dense()
+    if (
+        by_kernel and prompt_grad.gemm_matrix(w)
+        and prompt_grad.takes_gemm(x.numel() // k, k, n, fused=fused, added=epilogue == _GEMM_RESIDUAL)
     ):
-        rows = prompt_grad.aligned(x).view(-1, w.shape[0])
-        if residual is not None:
-            residual = prompt_grad.aligned(residual).view(rows.shape[0], -1)
-        return hip.gemm_rows(rows, w, False, epilogue, residual, bias).view(*x.shape[:-1], -1)
+        x2, added = rows()
+        return hip.gemm_rows(x2, w, False, epilogue, added, bias).view(*x.shape[:-1], -1)
     y = torch.matmul(x, w)
     if epilogue == _GEMM_RESIDUAL:
         return residual + y if bias is None else hip.add_rows(residual, y, None, bias)

@@ -105,6 +105,22 @@ def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = F
     return m <= 128 or tiles <= (256 if fused else 128)
 
 
+def takes_nf4_gemm(m: int, k: int, n: int) -> bool:
+    """Whether m rows of k times an NF4 matrix with n columns are faster by ops/csrc/nf4_gemm.hip, which reads
+    the codes, than by a product with a copy of it in bf16 that is there already.
+
+    Codes are a quarter of the bytes, but each is looked up and rounded: large matrices gain up to 128 rows, beyond which
+    the matrix cores bound both; smaller ones gain as long as reading a copy takes longer than the
+    launches. us on MI355X, with a copy and from codes: 2048 x 11264, 32 rows 16.0, 15.6, 33 rows 18.4, 20.3;
+    4096 x 4096, 16 rows 12.7, 14.4; 11008 x 4096, 64 rows 28.3, 27.4, 96 rows 33.3, 29.8, 128 rows 32.7, 31.7; 14336 x 4096,
+    64 rows 33.5, 29.2, 128 rows 34.0, 36.3; 8192 x 8192, 128 rows 41.0, 39.2; 8192 x 57344, 128 rows 177, 139, 192 rows
+    207, 264."""
+    if m <= 0 or k % 128:
+        return False
+    weights = k * n
+    return m <= 32 and weights >= 20 << 20 or m <= 64 and weights >= 40 << 20 or m <= 128 and weights >= 64 << 20
+
+
 def _by_torch(*grads) -> bool:
     """Whether these gradients are taken through torch operations: those that are to have gradients
     themselves, and those that are watched, which the forward pass need not have been."""

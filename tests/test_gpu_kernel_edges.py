@@ -1131,3 +1131,100 @@ def test_rounding_to_bf16(hip):
         assert torch.equal(got.isnan(), want.isnan())
         kept = ~want.isnan()
         assert torch.equal(got[kept].view(torch.int16), want[kept].view(torch.int16))
+
+
+@requires_gpu
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2])
+@pytest.mark.parametrize(
+    "m,k,n",
+    [
+        (1, 128, 64),  # one tile of codes, fewer columns than a wave pair's
+        (31, 256, 192), (32, 384, 256), (33, 640, 320),  # edges of 32 rows; fewer tiles of codes than are fetched ahead, odd numbers
+        (65, 1152, 704), (129, 1280, 4160),  # edges of 64 and 128 rows; parts along K, the last one shorter
+        (640, 1024, 3328), (513, 512, 13312),  # whole waves of tiles and some left over
+    ],
+)
+def test_nf4_prompt_product_edges(hip, m, k, n, tile):
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).to(BF16)
+
+    x, residual, bias = normal(m, k), normal(m, n), normal(n)
+    tiles, scales = hip.nf4_tile(*hip.nf4_quantize(normal(k, n) * 0.125))
+    w = hip.nf4_untile(tiles, scales, k)  # the copy in bf16 whose products these are
+    ref = x.double() @ w.double()
+    # one rounding to bf16, and sums of k terms in 32 bits
+    loose = (x.double().abs() @ w.double().abs()) * k * 2.0**-24
+
+    def check(y, want, slack):
+        assert y.shape == want.shape and bool(torch.isfinite(y).all())
+        assert bool(((y.double() - want).abs() <= 2.0**-8 * want.abs() + slack + 1e-6).all())
+
+    def product(*args):
+        return hip.gemm_nf4_rows(x, tiles, scales, *args, tile=tile)
+
+    check(product(0), ref, loose)
+    check(product(1, residual, bias), ref + residual.double() + bias.double(), loose)
+    gelu = torch.nn.functional.gelu(ref + bias.double(), approximate="tanh")
+    check(product(2, None, bias), gelu, 1.2 * loose)  # its slope is at most 1.13
+    (g, u), (lg, lu) = ref.chunk(2, dim=-1), loose.chunk(2, dim=-1)
+    # silu's slope is at most 1.1; its exponential is good to 2^-20
+    silu = torch.nn.functional.silu(g)
+    check(product(3), silu * u, 1.1 * lg * u.abs() + silu.abs() * lu + (silu * u).abs() * 2.0**-20)
+
+
+@requires_gpu
+@pytest.mark.parametrize("m", [5, 70])
+def test_nf4_prompt_products_of_extreme_values(hip, m):
+    """Infinities, NaNs and large values stay in their rows, those of scales in their blocks; blocks of zeros are zeros."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, 256, device="cuda", generator=gen).to(BF16)
+    w = (torch.randn(256, 192, device="cuda", generator=gen) * 0.125).to(BF16)
+    w[7, :64] = 0.0
+    inf, nan = float("inf"), float("nan")
+    x[0, 3], x[1, 255], x[2, 0], x[4, 9] = inf, nan, -inf, 3e38
+    tiles, scales = hip.nf4_tile(*hip.nf4_quantize(w))
+    for scale in (None, inf, nan):
+        if scale is not None:
+            scales[1, 11] = scale
+        dense = hip.nf4_untile(tiles, scales, 256)
+        want, got = x.double() @ dense.double(), hip.gemm_nf4_rows(x, tiles, scales)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        finite = want.isfinite()
+        assert torch.equal(got[got.isinf()].double(), want[want.isinf()]) and 0.2 < finite.float().mean() < 1
+        # one rounding to bf16, and sums of 256 terms in 32 bits
+        loose = (x.double().abs() @ dense.double().abs())[finite] * 2.0**-16
+        assert bool(((got[finite].double() - want[finite]).abs() <= 2.0**-8 * want[finite].abs() + loose).all())
+
+
+@requires_gpu
+def test_nf4_prompts_read_codes(hip, monkeypatch):
+    """Rows that the rule gives to csrc/nf4_gemm.hip make no copy of the matrix, others do; both are the same product.
+    Rows of other lengths and codes of other sizes are refused."""
+    from petals_amd.ops import fused_decode, prompt_grad
+    from petals_amd.ops.fused_decode import _FastWeight, prompt_product
+
+    assert prompt_grad.takes_nf4_gemm(32, 4096, 6144) and not prompt_grad.takes_nf4_gemm(33, 4096, 6144)
+    assert prompt_grad.takes_nf4_gemm(128, 8192, 8192) and not prompt_grad.takes_nf4_gemm(129, 8192, 8192)
+    assert not prompt_grad.takes_nf4_gemm(0, 8192, 8192) and not prompt_grad.takes_nf4_gemm(8, 8192 + 64, 8192)
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    weight = _FastWeight((torch.randn(512, 320, device="cuda", generator=gen) * 0.125).to(BF16), hip, "nf4")
+    x = torch.randn(2, 9, 513, device="cuda", generator=gen).to(BF16)[..., 1:]  # not aligned, not contiguous
+    residual = torch.randn(2, 9, 320, device="cuda", generator=gen).to(BF16)
+    made = []
+    monkeypatch.setattr(fused_decode, "_dequant_cached", lambda w, make: made.append(w) or make())
+    got = []
+    for takes in (True, False):
+        monkeypatch.setattr(prompt_grad, "takes_nf4_gemm", lambda *sizes: takes)
+        got.append((prompt_product(hip, x, weight), prompt_product(hip, x, weight, 1, residual), prompt_product(hip, x, weight, 3)))
+        assert len(made) == (0 if takes else 3)
+    for a, b in zip(*got):
+        assert a.shape == b.shape and (a.double() - b.double()).norm() <= 2.0**-7 * b.double().norm()
+    for bad in (x[0, :, :448].contiguous(), x[0].float().contiguous(), x.contiguous()):
+        with pytest.raises(RuntimeError):
+            hip.gemm_nf4_rows(bad, weight.tiles, weight.scales)
+    with pytest.raises(RuntimeError):
+        hip.gemm_nf4_rows(x[0].contiguous(), weight.tiles, weight.scales[:, :256].contiguous())
+    with pytest.raises(RuntimeError):
+        hip.gemm_nf4_rows(x[0].contiguous(), weight.tiles, weight.scales, 1)  # a residual is missing
