@@ -10,7 +10,7 @@
 // 2^-22 of a mean that they have no part in. Sums of products of digits are exact
 // in 32 bits for runs of 512, and a product of 16 columns with 64 inputs is one
 // v_mfma_i32_16x16x64_i8 per digit of the levels: the four digits of up to four rows are its
-// other 16 columns.
+// other 16 columns. Those of up to eight rows are the other columns of a v_mfma_i32_32x32x32_i8.
 //
 // Digits come from v_perm_b32, which looks four codes up in eight bytes at once. Two
 // lookups make up the 16 levels: a code of the other half selects a sign or a constant (0
@@ -32,15 +32,22 @@
 // the inputs are cut into digits. Five to eight rows stay for up to 1024 inputs, as long
 // as that leaves 2048 waves: their sums are 96 registers to combine at the end.
 //
-// It is bound by vector instructions (half-rate lookups; the chip lowers its clock under
-// them), not by memory. llama-2-70b, us a product with its reduction, the kernel in
-// nf4.hip and this one, for 1, 4 and 8 rows:
-//   qkv   8192 x 10240   19, 29, 47     21, 22, 30
-//   o     8192 x 8192    22, 30, 49     17, 19, 22
-//   gate  8192 x 57344   64, 96, 160    61, 69, 103
-//   down  28672 x 8192   36, 51, 84     34, 41, 60
-// (Before lookups were summed, runs of 1024 for one row: 70 and 38 us for the last two beside 65 and 34; four waves
-// a SIMD: 71, 39.)
+// Loads have no conditions: what is not there lies beyond the end of a buffer, which gives zeros. With
+// conditions a wave's loads were some dozens of branches, each with its own (8192 x 8192, 1 row: 14.9 us, 10.4 now). Digits of
+// one input are written together and made columns by loads that transpose bytes; transposed in registers they
+// were 8 lookups' worth of instructions for 4 inputs, and stores of 4 bytes whose lanes met in the same banks.
+//
+// It is bound by vector instructions, not by memory: of 34 for 16 weights of a lane 24 are lookups. A matrix
+// instruction keeps others from starting for some 9 cycles, whatever its size; they are spread among the lookups
+// (1024 weights took 238 cycles with three waves on a SIMD as the compiler orders them, 197 so; 216 with
+// both lookups xored and half as many). llama-2-70b, us a product without its reduction, before this and now, for
+// 1, 4 and 8 rows:
+//   qkv   8192 x 10240   18.8, 19.7, 27.4     14.6, 15.9, 23.3
+//   o     8192 x 8192    14.9, 16.4, 18.9     10.5, 11.9, 16.4
+//   gate  8192 x 57344   58.8, 69.3, 96.2     51.3, 62.9, 87.7
+//   down  28672 x 8192   31.8, 38.6, 56.6     27.2, 33.7, 50.9
+// Workgroups that stay for several runs of columns, with the next one's weights on their way, keep two waves on a
+// SIMD: 62 us for the third, 1 row, and as long as now with eight. Four waves a SIMD: 71 beside 65 us then.
 // Cut off instead of rounded, and with the largest input of a run at 2^30 whatever the others
 // are, it took 0 to 5% less (8192 x 8192: 14.7, 16.1, 18.5 us without the reduction for 1, 4,
 // 8 rows beside 14.8, 16.6, 19.5). Runs with inputs beyond 64 times their mean take longer: two
@@ -56,11 +63,14 @@
 
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
+using i32x2 = __attribute__((ext_vector_type(2))) int;
 
 #define NF4_UNIT (1.0f / 7783094.0f)
 // times a run's mean size. Channels ten times as loud as the rest stay below it; with 16 they
 // didn't, and 8 rows of 8192 x 57344 took 197 us (the loud ones then in loops of their own)
 #define NF4_GATE 64.f
+#define NF4_ONCE 2           // of a load: non-temporal
+#define NF4_BEYOND (1 << 30)  // bytes, more than a run of columns has
 #define NF4_FINITE 0x7F7FFFFFu  // bits of the largest number
 
 static __device__ __constant__ float NF4_TILE_LEVELS[16] = {
@@ -114,16 +124,6 @@ __device__ __forceinline__ float quad_sum(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));
 }
 
-// the 4 x 4 bytes of w transposed
-__device__ __forceinline__ void transpose_bytes(unsigned* w) {
-  const unsigned a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), b = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-  const unsigned c = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u), d = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-  w[0] = __builtin_amdgcn_perm(b, a, 0x05040100u);
-  w[1] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-  w[2] = __builtin_amdgcn_perm(d, c, 0x05040100u);
-  w[3] = __builtin_amdgcn_perm(d, c, 0x07060302u);
-}
-
 // B rows; a wave takes KB tiles of 128 inputs and 64 columns at a time, `steps` times if LONG.
 // Grid: (out/64, runs of 4 KB `steps` tiles, rows of sel). With sel, B is 1 and row
 // blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z].
@@ -135,18 +135,18 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     float* __restrict__ partials,     // [splits, B or gridDim.z, out]
     int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4) {
   const int steps = LONG ? n_steps : 1;
-  constexpr int NS = (B + 3) / 4, NCOL = 4 * B, PER = KB * 2;
+  constexpr bool WIDE = B > 4;  // 32 columns of digits
+  constexpr int PER = KB * 2;
   // the two lookups of a digit are multiplied one by one, which saves their xor, where the matrix cores
-  // have little else to do: 8192 x 57344 takes 59.5 instead of 61.8 us with 1 row, 63.0 instead of 65.0 with 2,
-  // 72.0 instead of 74.0 with 4, but 113.7 instead of 111.3 with 8
-  constexpr bool SUMMED = NS == 1;
-  __shared__ __align__(16) unsigned char digits[4][KB * 128 * NCOL];
+  // have little else to do
+  constexpr bool SUMMED = !WIDE;
+  static_assert(KB == (WIDE ? 2 : 4));  // a lane's inputs are 8 slots of 16 bytes
+  __shared__ __align__(16) unsigned char digits[4][64 * 128];
   __shared__ __align__(16) float red[4 * B * 64];  // [waves, rows, columns]
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 15, hi = lane >> 4;
   const int nb = blockIdx.x, kb0 = (blockIdx.y * 4 + wave) * KB * steps;
-  const int live_kb = min(KB * steps, n_kb - kb0);  // may be negative
   if (sel) {
     const int e = sel[blockIdx.z];
     if (e < 0 || e >= experts) return;  // uniform over the workgroup
@@ -155,44 +155,62 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     x += (size_t)(blockIdx.z / k_per_tok) * in_dim;
   }
 
+  // loads of what lies beyond a run of columns' inputs, and all of a step that is not there, give zeros
+  auto resource = [&](const void* p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+  };
   // inputs of a step: PER of this lane
-  auto fetch_x = [&](int step, int b, float* v) {
-    const int k = (kb0 + step * KB) * 128 + lane * PER;
-    const float* p = x + (size_t)b * in_dim + k;
-    if (by4 && k + PER <= in_dim) {
+  auto fetch_x = [&](int step, int b, float* v, int beyond = 0) {
+    const auto r = resource(x + (size_t)b * in_dim, (size_t)in_dim * 4);
+    const int at = ((kb0 + step * KB) * 128 + lane * PER) * 4 + beyond;
+    if (by4) {
 #pragma unroll
-      for (int i = 0; i < PER; i += 4) *reinterpret_cast<float4v*>(v + i) = *reinterpret_cast<const float4v*>(p + i);
+      for (int i = 0; i < PER; i += 4)
+        *reinterpret_cast<u32x4*>(v + i) = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at + i * 4, 0, 0));
     } else {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) v[i] = k + i < in_dim ? p[i] : 0.f;
+      for (int i = 0; i < PER; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, at + i * 4, 0, 0));
     }
   };
-  auto fetch_scales = [&](int step, unsigned* v) {
-    const int at = step * KB * 128 + lane * PER;
-#pragma unroll
-    for (int i = 0; i < PER / 2; ++i) v[i] = 0u;
-    if (at < live_kb * 128) {
-      const unsigned* p = reinterpret_cast<const unsigned*>(scales + ((size_t)nb * n_kb + kb0) * 128 + at);
-#pragma unroll
-      for (int i = 0; i < PER / 2; ++i) v[i] = p[i];
+  const auto scale_rsrc = resource(scales + (size_t)nb * n_kb * 128, (size_t)n_kb * 256);
+  auto fetch_scales = [&](int step, unsigned* v, int beyond = 0) {
+    const int at = ((kb0 + step * KB) * 128 + lane * PER) * 2 + beyond;
+    if constexpr (PER == 8) {
+      *reinterpret_cast<u32x4*>(v) = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(scale_rsrc, at, 0, 0));
+    } else {
+      static_assert(PER == 4);
+      using u32x2 = __attribute__((ext_vector_type(2))) unsigned;
+      *reinterpret_cast<u32x2*>(v) = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(scale_rsrc, at, 0, 0));
     }
   };
-  const u32x4* wp = reinterpret_cast<const u32x4*>(tiles) + ((size_t)nb * n_kb + kb0) * 256 + lane;
+  // operands of 64 inputs and 16 columns, or of 32 inputs, in two runs of 16, and 32 columns
+  const auto w_rsrc = resource(tiles + (size_t)nb * n_kb * 256, (size_t)n_kb * 4096);
+  const int w_at = kb0 * 4096 + (WIDE ? (hi & 1) * 64 + (hi >> 1) * 32 + col : lane) * 16;
   u32x4 w[KB][4];
-  auto fetch_w = [&](int step, int j) {
+  auto fetch_w = [&](int step, int j, int beyond = 0) {
+    const int at = w_at + (step * KB + j) * 4096 + beyond;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      w[j][c] = u32x4{0u, 0u, 0u, 0u};
-      if (step * KB + j < live_kb) w[j][c] = __builtin_nontemporal_load(wp + ((step * KB + j) * 4 + c) * 64);
-    }
+    for (int c = 0; c < 4; ++c)
+      w[j][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              w_rsrc, at + (WIDE ? c / 2 * 2048 + c % 2 * 256 : c * 1024), 0, NF4_ONCE));
   };
 
-  // the first step's inputs, then its weights, which are awaited last
+  // all inputs, then the first step's weights, which are awaited last
+  constexpr int STEPS = LONG ? 4 : 1;
+  float later[STEPS][B][PER];  // of steps 1 on
+  unsigned later_scales[STEPS][PER / 2];
   float xs[B][PER];
   unsigned sc[PER / 2];
   fetch_scales(0, sc);
 #pragma unroll
   for (int b = 0; b < B; ++b) fetch_x(0, b, xs[b]);
+#pragma unroll
+  for (int step = 1; step < STEPS; ++step) {
+    if (step >= steps) break;
+    fetch_scales(step, later_scales[step]);
+#pragma unroll
+    for (int b = 0; b < B; ++b) fetch_x(step, b, later[step][b]);
+  }
 #pragma unroll
   for (int j = 0; j < KB; ++j) fetch_w(0, j);
   __builtin_amdgcn_sched_barrier(0);
@@ -217,15 +235,11 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   auto add_all = [&](bool clip) {
 #pragma unroll
     for (int b = 0; b < B; ++b) add_sizes(sc, b, xs[b], clip);
-    for (int step = 1; step < steps; ++step) {
-      unsigned s[PER / 2];
-      fetch_scales(step, s);
 #pragma unroll
-      for (int b = 0; b < B; ++b) {
-        float v[PER];
-        fetch_x(step, b, v);
-        add_sizes(s, b, v, clip);
-      }
+    for (int step = 1; step < STEPS; ++step) {
+      if (step >= steps) break;
+#pragma unroll
+      for (int b = 0; b < B; ++b) add_sizes(later_scales[step], b, later[step][b], clip);
     }
   };
 #pragma unroll
@@ -297,106 +311,142 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     unit[b] = __uint_as_float((254u - up) << 23);
   }
 
-  i32x4 acc[NS][4][3];
+  // Digits of an input's rows are neighbours; loads that transpose bytes make them columns. A lane has 8 slots of 16
+  // bytes, turned by half its number, so that 16 lanes that write the same one use all banks.
+  unsigned char* const mine = digits[wave];
+  auto slot_at = [](int block, int slot) { return block * 128 + ((slot + (block >> 1)) & 7) * 16; };
+  auto put = [&](int i, const unsigned* q) {  // digits of this lane's i-th input
+    if constexpr (WIDE) {
+      *reinterpret_cast<u32x4*>(mine + slot_at(lane, 2 * i)) = u32x4{q[0], q[1], q[2], q[3]};
+      *reinterpret_cast<u32x4*>(mine + slot_at(lane, 2 * i + 1)) =
+          u32x4{q[4], B > 5 ? q[B > 5 ? 5 : 0] : 0u, B > 6 ? q[B > 6 ? 6 : 0] : 0u, B > 7 ? q[B > 7 ? 7 : 0] : 0u};
+    } else {
+      *reinterpret_cast<u32x4*>(mine + slot_at(lane, i)) =
+          u32x4{q[0], B > 1 ? q[B > 1 ? 1 : 0] : 0u, B > 2 ? q[B > 2 ? 2 : 0] : 0u, B > 3 ? q[B > 3 ? 3 : 0] : 0u};
+    }
+  };
+  // a lane's column of 16 inputs: those of tile j, half, and run hi, or (h * 2 + run), in two loads
+  int from[WIDE ? 4 : 2];
+  if constexpr (WIDE) {
+    const int row = col / 2, h = hi >> 1;
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
+    for (int i = 0; i < 4; ++i)  // 2 run + which of the loads
+      from[i] = h * 8 * 128 + row / 4 * 128 + ((row % 4 * 2 + (hi & 1) + h * 4 + i) & 7) * 16 + (col & 1) * 8;
+  } else {
+    const int row = col / 2;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int i = 0; i < 2; ++i)  // half
+      from[i] = hi * 2 * 128 + ((row + hi + i * 4) & 7) * 16 + (col & 1) * 8;
+  }
+  auto column = [&](int j, int half, int run) {
+    using lds_two = __attribute__((address_space(3))) i32x2;
+    i32x2 v[2];
 #pragma unroll
-      for (int p = 0; p < 3; ++p) acc[s][c][p] = i32x4{0, 0, 0, 0};
+    for (int i = 0; i < 2; ++i) {
+      const int at = WIDE ? from[2 * run + i] + (j * 32 + half * 16 + run * 4 + i * 2) * 128 : from[half] + (j * 16 + half * 8 + i) * 128;
+      v[i] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_two*)(mine + at));
+    }
+    return i32x4{v[0][0], v[0][1], v[1][0], v[1][1]};
+  };
+  // the digits of four codes in a byte each, or what makes them up
+  auto look_up = [&](unsigned w0, unsigned w1, int p, i32x4& a, i32x4& b) {
+    constexpr auto& table = SUMMED ? NF4_SUMMANDS : NF4_DIGITS;
+    // codes 0-7 select below 8; the others do with bit 3 turned
+    const unsigned lo[4] = {w0 & 0x0F0F0F0Fu, (w0 >> 4) & 0x0F0F0F0Fu, w1 & 0x0F0F0F0Fu, (w1 >> 4) & 0x0F0F0F0Fu};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] = (int)__builtin_amdgcn_perm(table[p][1], table[p][0], lo[i]);
+      b[i] = (int)__builtin_amdgcn_perm(table[p][3], table[p][2], lo[i] ^ 0x08080808u);
+    }
+  };
+
+  using sums = __attribute__((ext_vector_type(WIDE ? 16 : 4))) int;
+  constexpr int G = WIDE ? 2 : 4;  // runs of 32 or 16 columns
+  sums acc[G][3];
+#pragma unroll
+  for (int c = 0; c < G; ++c)
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int r = 0; r < (WIDE ? 16 : 4); ++r) acc[c][p][r] = 0;
 
   for (int step = 0; step < steps; ++step) {
     if (__builtin_expect(loud, 0)) strip(step);
 #pragma unroll
-    for (int b = 0; b < B; ++b)
+    for (int i = 0; i < PER; ++i) {
+      const float s = __uint_as_float(i & 1 ? sc[i / 2] & 0xFFFF0000u : sc[i / 2] << 16);
+      unsigned q[B];
 #pragma unroll
-      for (int i = 0; i < PER; i += 4) {
-        unsigned q[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const unsigned s = (i + j) & 1 ? sc[(i + j) / 2] & 0xFFFF0000u : sc[(i + j) / 2] << 16;
-          const float v = xs[b][i + j] * __uint_as_float(s);
-          q[j] = ((unsigned)(int)rintf(v * factor[b]) + 0x00808080u) ^ 0x00808080u;
-        }
-        transpose_bytes(q);
-        const int at = lane * PER + i;  // of the step: group of 16, then column, then place
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-          *reinterpret_cast<unsigned*>(&digits[wave][((at / 16) * NCOL + b * 4 + d) * 16 + at % 16]) = q[d];
+      for (int b = 0; b < B; ++b) {
+        const float v = xs[b][i] * s;
+        q[b] = ((unsigned)(int)rintf(v * factor[b]) + 0x00808080u) ^ 0x00808080u;
       }
+      put(i, q);
+    }
     wave_fence();
-    const bool next = step + 1 < steps;
-    if (next) {
-      fetch_scales(step + 1, sc);
+    const int beyond = step + 1 < steps ? 0 : NF4_BEYOND;
+    if (LONG) {
+      fetch_scales(step + 1, sc, beyond);
 #pragma unroll
-      for (int b = 0; b < B; ++b) fetch_x(step + 1, b, xs[b]);
+      for (int b = 0; b < B; ++b) fetch_x(step + 1, b, xs[b], beyond);
     }
 #pragma unroll
     for (int j = 0; j < KB; ++j) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        i32x4 xd[NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          // columns without a row are zero, which takes less power than repeating others
-          const int n = s * 16 + col, live = n < NCOL ? -1 : 0;
-          xd[s] = *reinterpret_cast<const i32x4*>(&digits[wave][((j * 8 + half * 4 + hi) * NCOL + n % NCOL) * 16]);
-          if (NCOL % 16) xd[s] &= live;
-        }
+        for (int run = 0; run < (WIDE ? 2 : 1); ++run) {
+          const i32x4 xd = column(j, half, run);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const unsigned w0 = half ? w[j][c].z : w[j][c].x, w1 = half ? w[j][c].w : w[j][c].y;
-          unsigned lo[4], up[4];  // codes 0-7 select below 8; the others do with bit 3 turned
-          lo[0] = w0 & 0x0F0F0F0Fu;
-          lo[1] = (w0 >> 4) & 0x0F0F0F0Fu;
-          lo[2] = w1 & 0x0F0F0F0Fu;
-          lo[3] = (w1 >> 4) & 0x0F0F0F0Fu;
+          for (int c = 0; c < G; ++c) {
+            const u32x4& codes = w[j][WIDE ? 2 * c + run : c];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) up[i] = lo[i] ^ 0x08080808u;
-#pragma unroll
-          for (int p = 0; p < 3; ++p) {
-            constexpr auto& table = SUMMED ? NF4_SUMMANDS : NF4_DIGITS;
-            i32x4 a, b;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              a[i] = (int)__builtin_amdgcn_perm(table[p][1], table[p][0], lo[i]);
-              b[i] = (int)__builtin_amdgcn_perm(table[p][3], table[p][2], up[i]);
+            for (int p = 0; p < 3; ++p) {
+              i32x4 a, b;
+              look_up(half ? codes.z : codes.x, half ? codes.w : codes.y, p, a, b);
+              if constexpr (WIDE) {
+                acc[c][p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a ^ b, xd, acc[c][p], 0, 0, 0);
+              } else {
+                acc[c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xd, acc[c][p], 0, 0, 0);
+                acc[c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, xd, acc[c][p], 0, 0, 0);
+              }
             }
-            if (!SUMMED) a ^= b;
+            if constexpr (!WIDE)
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-              acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, xd[s], acc[s][c][p], 0, 0, 0);
-              if (SUMMED) acc[s][c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, xd[s], acc[s][c][p], 0, 0, 0);
-            }
+              for (int i = 0; i < 6; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+              }
           }
         }
       }
-      if (next) fetch_w(step + 1, j);
+      if (LONG) fetch_w(step + 1, j, beyond);
     }
     wave_fence();
   }
 
+  // this lane's column of digits is that of a row and, in it, of the digit n % 4; it has four neighbouring
+  // columns of weights at a time
+  const int n = WIDE ? lane & 31 : col, row = n / 4, first = WIDE ? (hi >> 1) * 4 : hi * 4;
+  float last = 0.f;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int row = s * 4 + col / 4;  // this lane's row and, col % 4, digit of its inputs
-    float last = 0.f;
+  for (int b = 0; b < B; ++b) last = row == b ? unit[b] : last;
+  const float place = __uint_as_float((127u + 8u * (n & 3)) << 23) * NF4_UNIT;
 #pragma unroll
-    for (int b = s * 4; b < B && b < s * 4 + 4; ++b) last = row == b ? unit[b] : last;
-    const float place = __uint_as_float((127u + 8u * (col & 3)) << 23) * NF4_UNIT;
+  for (int c = 0; c < G; ++c)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int f = 0; f < (WIDE ? 4 : 1); ++f) {
       float4v v;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float sum = fmaf((float)acc[s][c][2][r], 65536.f, fmaf((float)acc[s][c][1][r], 256.f, (float)acc[s][c][0][r]));
+        const float sum = fmaf((float)acc[c][2][4 * f + r], 65536.f, fmaf((float)acc[c][1][4 * f + r], 256.f, (float)acc[c][0][4 * f + r]));
         v[r] = quad_sum(sum * place) * last;
       }
-      if ((col & 3) == 0 && row < B) {
-        float4v* sum = reinterpret_cast<float4v*>(&red[(wave * B + row) * 64 + c * 16 + hi * 4]);
+      if ((n & 3) == 0 && row < B) {
+        float4v* sum = reinterpret_cast<float4v*>(&red[(wave * B + row) * 64 + c * (64 / G) + f * 8 + first]);
         *sum = loud ? *sum + v : v;
       }
     }
-  }
   __syncthreads();
   for (int i = tid; i < B * 64; i += 256) {
     const float sum = (red[i] + red[B * 64 + i]) + (red[2 * B * 64 + i] + red[3 * B * 64 + i]);
@@ -521,6 +571,7 @@ static torch::Tensor launch_nf4_tiles(
   const int batch = sel ? 1 : (int)x.size(0);
   const long rows = sel ? sel->numel() : batch, z = sel ? rows : 1;
   TORCH_CHECK(batch >= 1 && batch <= 8, "NF4 products of few rows take at most 8");
+  TORCH_CHECK(n_kb * 4096 < NF4_BEYOND, "too many inputs");  // 33 million
   const int kb = batch <= 4 ? 4 : 2;
   // longer runs combine their sums once, but only where enough waves remain
   const long units = nb * z * ((n_kb + kb - 1) / kb);
