@@ -127,13 +127,14 @@ __device__ __forceinline__ float quad_sum(float v) {
 // B rows; a wave takes KB tiles of 128 inputs and 64 columns at a time, `steps` times if LONG.
 // Grid: (out/64, runs of 4 KB `steps` tiles, rows of sel). With sel, B is 1 and row
 // blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z].
-template <int B, int KB, bool LONG>
+template <int B, int KB>
 __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     const uint4* __restrict__ tiles, const unsigned short* __restrict__ scales,
     const float* __restrict__ x,      // [rows, in]
     const int* __restrict__ sel,      // [rows * k_per_tok] or null
     float* __restrict__ partials,     // [splits, B or gridDim.z, out]
     int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4) {
+  constexpr bool LONG = B > 4;
   const int steps = LONG ? n_steps : 1;
   constexpr bool WIDE = B > 4;  // 32 columns of digits
   constexpr int PER = KB * 2;
@@ -587,7 +588,7 @@ static torch::Tensor launch_nf4_tiles(
   const dim3 grid(nb, splits, z);
   auto stream = at::cuda::getCurrentCUDAStream();
 #define NF4_TILES(B, KB)                                                                                       \
-  gemv_nf4_tiles_kernel<B, KB, (B > 4)><<<grid, 256, 0, stream>>>(                                                      \
+  gemv_nf4_tiles_kernel<B, KB><<<grid, 256, 0, stream>>>(                                                      \
       reinterpret_cast<const uint4*>(tiles.data_ptr()), reinterpret_cast<const unsigned short*>(scales.data_ptr()), \
       x.data_ptr<float>(), sel ? sel->data_ptr<int>() : nullptr, partials.data_ptr<float>(), (int)in_dim,      \
       (int)out_dim, (int)n_kb, (int)steps, (int)k_per_tok, sel ? (int)tiles.size(0) : 1, by4)
