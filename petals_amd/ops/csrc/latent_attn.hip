@@ -32,6 +32,10 @@
 // LDS row padding (elements): 16, or 8 where two workgroups would not fit in a CU otherwise
 constexpr int lds_pad(int rc) { return rc > 16 ? 8 : 16; }
 
+// 2 waves of a SIMD hide each other's softmax, where their registers fit: 256 hold the sums of 16 chunks if the next
+// tile goes straight to LDS (RC == 16), those of 12 with 4 groups of rows not
+constexpr int waves_per_simd(int rc, int dg) { return rc <= 10 || rc == 16 || (rc < 16 && dg > 1) ? 2 : 1; }
+
 // what is done to a row's weighted sum at the end
 struct LatentEnd {
   const float* sink;    // [H] score of one more entry of the softmax, without a value; or null
@@ -56,10 +60,14 @@ __device__ __forceinline__ float end_factor(const LatentEnd& e, size_t flat, int
 // one is loaded while the current one is used. The same staged tile is the keys
 // (row-major fragments) and the values (transposing LDS loads).
 //
+// Bound by the wave that waits: with one wave a SIMD nothing runs while a tile's scores become probabilities. 583 rows
+// of 32 heads after 0 to 3000 keys, 512 values: 260 us with conditional loads to registers and one wave, 241 with loads
+// without conditions, 144 with rows that go straight to LDS, which leaves registers for two waves.
+//
 // RC = row size in 32-wide MFMA k-chunks (columns past RP read as zero), VC = those
 // of them that are values. Grid: (token runs, groups of 16*RG rows, key splits).
 template <int RC, int VC, int DG>
-__global__ __launch_bounds__(256) void latent_attn_kernel(
+__global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kernel(
     const unsigned short* __restrict__ q,      // [T, H, RP]
     const unsigned short* __restrict__ cache,  // [num_pages, PAGE, RP]
     unsigned short* __restrict__ out,          // [T, H, VP] (n_splits == 1)
@@ -80,6 +88,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(
   constexpr int ROW = R + lds_pad(RC);           // LDS row in elements
   constexpr int LOADS = LKVT * (R / 8);          // 16-byte loads per tile
   constexpr int NLD = (LOADS + 255) / 256;       // per thread
+  constexpr bool DIRECT = RC == 16;              // a wave loads a row at once, from memory to LDS
   constexpr int DB = (VC * 2 + DG - 1) / DG;     // 16-wide dim blocks per wave
   const int tok0 = tiles[2 * blockIdx.x];
   const int ntok = tiles[2 * blockIdx.x + 1];
@@ -89,7 +98,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(
   const int g1 = min(g0 + 16 * RG, rows);
 
   const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = tid & (WAVE - 1);
   const int col = lane & 15;
   const int hi = lane >> 4;
@@ -142,18 +151,44 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(
   const int all_lo = full_wave && window > 0 ? b.pos[tok0 + (r0 + 15) / heads] - window + 1 : 0;
 
   bf16x8 next[NLD];
+  int next_at[NLD];  // in a tile, in bytes; columns past rp lie beyond it
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int idx = tid + i * 256, row = idx / (R / 8), c8 = (idx - row * (R / 8)) * 8;
+    next_at[i] = (row * rp + c8) * 2 + (c8 < rp && row < LKVT ? 0 : BEYOND_ROWS);
+  }
   // rows of tile j0 that lie in [0, j_end); zero elsewhere and past rp
   auto fetch = [&](int j0) {
-    const long at = cache_row(b, seq, j0);
+    const auto rows_of = cached_rows(cache, cache_row(b, seq, j0), min(j_end - j0, LKVT), rp);
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / (R / 8);
-      const int c8 = (idx - row * (R / 8)) * 8;
-      next[i] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if ((LOADS % 256 == 0 || idx < LOADS) && at >= 0 && j0 + row < j_end && c8 < rp)
-        next[i] = *reinterpret_cast<const bf16x8*>(cache + ((size_t)at + row) * rp + c8);
+    for (int i = 0; i < NLD; ++i) next[i] = load_cached(rows_of, next_at[i]);
+  };
+  // DIRECT: the 8 rows of this wave. Rows beyond the end repeat the last one, which no row of the softmax sees
+  // there; columns past rp stay what they are.
+  auto load_rows = [&](int j0, int which) {
+    const long at = cache_row(b, seq, j0);
+    const int row = which * LKVT + wave * 8;
+    const unsigned to = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned short*)smem + row * ROW * 2;
+    if (at < 0) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        *reinterpret_cast<bf16x8*>(&smem[(row + i) * ROW + lane * 8]) = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    } else if (lane * 8 < rp) {
+      const size_t p = (size_t)(cache + (size_t)at * rp);
+      using i32x4 = __attribute__((ext_vector_type(4))) int;
+      const i32x4 rows_of{__builtin_amdgcn_readfirstlane((int)p), __builtin_amdgcn_readfirstlane((int)(p >> 32) & 0xFFFF),
+                          LKVT * rp * 2, 0x00020000};
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(to + i * ROW * 2), "v"(min(wave * 8 + i, j_end - 1 - j0) * (rp * 2) + lane * 16), "s"(rows_of)
+                     : "memory", "m0");
     }
+  };
+  auto arrive = [&] {
+    if (DIRECT) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   };
   auto stage = [&](unsigned short* buf) {
 #pragma unroll
@@ -166,15 +201,27 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(
   };
 
   if (j_begin < j_end) {
-    fetch(j_begin);
-    stage(smem);
+    if constexpr (DIRECT) {
+      if (lane * 8 >= rp) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          *reinterpret_cast<bf16x8*>(&smem[((i & 8) * (LKVT / 8) + wave * 8 + (i & 7)) * ROW + lane * 8]) = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+      load_rows(j_begin, 0);
+    } else {
+      fetch(j_begin);
+      stage(smem);
+    }
   }
-  __syncthreads();
+  arrive();
   int which = 0;
   for (int j0 = j_begin; j0 < j_end; j0 += LKVT, which ^= 1) {
     const unsigned short* k_lds = smem + which * LKVT * ROW;
     const bool more = j0 + LKVT < j_end;
-    if (more) fetch(j0 + LKVT);
+    if (more) {
+      if constexpr (DIRECT) load_rows(j0 + LKVT, which ^ 1);
+      else fetch(j0 + LKVT);
+    }
 
     f32x4 s_acc[2];
 #pragma unroll
@@ -231,8 +278,8 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(
       acc_o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
           p_frag, load_keys(v_lds + (d0 + d) * 16, ROW), acc_o[d], 0, 0, 0);
     }
-    if (more) stage(smem + (which ^ 1) * LKVT * ROW);
-    __syncthreads();
+    if (!DIRECT && more) stage(smem + (which ^ 1) * LKVT * ROW);
+    arrive();
   }
 
 #pragma unroll

@@ -27,6 +27,20 @@ static __device__ __forceinline__ long cache_row(const PagedRows& b, int seq, in
   return (long)page * PAGE + (key - slot * PAGE);
 }
 
+// `rows` cached rows from `at` on (the same for the whole wave): loads of what lies beyond them, or of any if
+// there is none (at < 0), give zeros. They have no conditions, which would be branches between the loads.
+#define BEYOND_ROWS (1 << 30)  // bytes, more than the rows of a page have
+static __device__ __forceinline__ auto cached_rows(const unsigned short* cache, long at, int rows, int width) {
+  const size_t p = (size_t)(cache + (at < 0 ? 0 : at) * width);
+  const size_t base = (unsigned)__builtin_amdgcn_readfirstlane((int)p) | (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32;
+  const int bytes = __builtin_amdgcn_readfirstlane(at < 0 ? 0 : max(rows, 0) * width * 2);
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base), 0, bytes, 0x00020000);
+}
+template <typename R>
+static __device__ __forceinline__ bf16x8 load_cached(R rows, int byte) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rows, byte, 0, 0));
+}
+
 template <typename T> __device__ __forceinline__ float load_f32(const T* p);
 template <> __device__ __forceinline__ float load_f32<float>(const float* p) { return *p; }
 template <> __device__ __forceinline__ float load_f32<unsigned short>(const unsigned short* p) { return bf16_to_f32(*p); }

@@ -463,6 +463,42 @@ def test_latent_attention_kernel(heads, rank, window, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads", [3, 17, 40])
+@pytest.mark.parametrize("rank", [416, 480, 512])
+def test_latent_rows_straight_to_lds(heads, rank):
+    """Rows of 13 to 16 chunks go to LDS without registers: the columns past them and a page that is not in the pool
+    count as zeros, and what is cached beyond the end does not count at all."""
+    from petals_amd.ops import latent
+
+    torch.manual_seed(0)
+    starts, lens = [0, 130, 63], [40, 1, 70]
+    cache = torch.randn(9, PAGE_SIZE, rank, device="cuda").bfloat16()
+    pages = [[3], [5, 0, 7], [8, 1, 2]]
+    batch = PagedBatch(pages, starts, lens, torch.device("cuda"))
+    q = torch.randn(batch.tokens, heads, rank, device="cuda").bfloat16()
+    scale = 1.5 * rank**-0.5
+    seen_rows = []
+    for p, s, n in zip(pages, starts, lens):
+        rows = cache[p].reshape(-1, rank)
+        rows[s + n :] = float("nan")
+        cache[p] = rows.view(-1, PAGE_SIZE, rank)
+        seen_rows.append(rows[: s + n].double().cpu())
+    batch.tables[1, 1] = 9
+    seen_rows[1][PAGE_SIZE : 2 * PAGE_SIZE] = 0
+    run = batch.run_tokens(heads)
+    for splits in (1, 3):
+        got = latent.hip().latent_attention(
+            q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(run), run, batch.max_end, 0, scale, splits
+        )
+        for (lo, hi), c, s in zip(batch.row_ranges(), seen_rows, starts):
+            score = torch.einsum("thr,kr->htk", q[lo:hi].double().cpu(), c) * scale
+            seen = oracle.window_mask(len(c), len(c))[s:]
+            want = torch.einsum("htk,kr->thr", score.masked_fill(~seen, -float("inf")).softmax(-1), c)
+            # probabilities and results are rounded to 8 bits: 2^-8 of the largest value, 5, each
+            assert (got[lo:hi].double().cpu() - want).abs().max() < 4e-2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("t,experts,top,d", [(1, 1, 1, 7), (3, 8, 2, 128), (70, 300, 9, 1000), (65, 5, 5, 129)])
 @pytest.mark.parametrize("slots", [0, 3])
 def test_sublayer_out_kernel(t, experts, top, d, slots):
