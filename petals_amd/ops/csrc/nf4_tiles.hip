@@ -70,7 +70,8 @@ using i32x2 = __attribute__((ext_vector_type(2))) int;
 // didn't, and 8 rows of 8192 x 57344 took 197 us (the loud ones then in loops of their own)
 #define NF4_GATE 64.f
 #define NF4_ONCE 2           // of a load: non-temporal
-#define NF4_BEYOND (1 << 30)  // bytes, more than a run of columns has
+#define NF4_BEYOND (1 << 30)  // bytes, more than a launch has of a run of columns
+#define NF4_LAUNCH (1 << 17)  // tiles of 128 inputs, a multiple of a workgroup's, that offsets of 32 bits hold with room for the former
 #define NF4_FINITE 0x7F7FFFFFu  // bits of the largest number
 
 static __device__ __constant__ float NF4_TILE_LEVELS[16] = {
@@ -126,14 +127,15 @@ __device__ __forceinline__ float quad_sum(float v) {
 
 // B rows; a wave takes KB tiles of 128 inputs and 64 columns at a time, `steps` times if LONG.
 // Grid: (out/64, runs of 4 KB `steps` tiles, rows of sel). With sel, B is 1 and row
-// blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z].
+// blockIdx.z is that of x[blockIdx.z / k_per_tok] and expert sel[blockIdx.z]. A launch has in_dim inputs
+// of x_stride, and n_kb tiles of kb_stride.
 template <int B, int KB>
 __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     const uint4* __restrict__ tiles, const unsigned short* __restrict__ scales,
     const float* __restrict__ x,      // [rows, in]
     const int* __restrict__ sel,      // [rows * k_per_tok] or null
     float* __restrict__ partials,     // [splits, B or gridDim.z, out]
-    int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4) {
+    int in_dim, int out_dim, int n_kb, int n_steps, int k_per_tok, int experts, bool by4, int x_stride, int kb_stride) {
   constexpr bool LONG = B > 4;
   const int steps = LONG ? n_steps : 1;
   constexpr bool WIDE = B > 4;  // 32 columns of digits
@@ -151,9 +153,9 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   if (sel) {
     const int e = sel[blockIdx.z];
     if (e < 0 || e >= experts) return;  // uniform over the workgroup
-    tiles += (size_t)e * (out_dim / 64) * n_kb * 256;
-    scales += (size_t)e * (out_dim / 64) * n_kb * 128;
-    x += (size_t)(blockIdx.z / k_per_tok) * in_dim;
+    tiles += (size_t)e * (out_dim / 64) * kb_stride * 256;
+    scales += (size_t)e * (out_dim / 64) * kb_stride * 128;
+    x += (size_t)(blockIdx.z / k_per_tok) * x_stride;
   }
 
   // loads of what lies beyond a run of columns' inputs, and all of a step that is not there, give zeros
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
   };
   // inputs of a step: PER of this lane
   auto fetch_x = [&](int step, int b, float* v, int beyond = 0) {
-    const auto r = resource(x + (size_t)b * in_dim, (size_t)in_dim * 4);
+    const auto r = resource(x + (size_t)b * x_stride, (size_t)in_dim * 4);
     const int at = ((kb0 + step * KB) * 128 + lane * PER) * 4 + beyond;
     if (by4) {
 #pragma unroll
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
       for (int i = 0; i < PER; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, at + i * 4, 0, 0));
     }
   };
-  const auto scale_rsrc = resource(scales + (size_t)nb * n_kb * 128, (size_t)n_kb * 256);
+  const auto scale_rsrc = resource(scales + (size_t)nb * kb_stride * 128, (size_t)n_kb * 256);
   auto fetch_scales = [&](int step, unsigned* v, int beyond = 0) {
     const int at = ((kb0 + step * KB) * 128 + lane * PER) * 2 + beyond;
     if constexpr (PER == 8) {
@@ -185,7 +187,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
     }
   };
   // operands of 64 inputs and 16 columns, or of 32 inputs, in two runs of 16, and 32 columns
-  const auto w_rsrc = resource(tiles + (size_t)nb * n_kb * 256, (size_t)n_kb * 4096);
+  const auto w_rsrc = resource(tiles + (size_t)nb * kb_stride * 256, (size_t)n_kb * 4096);
   const int w_at = kb0 * 4096 + (WIDE ? (hi & 1) * 64 + (hi >> 1) * 32 + col : lane) * 16;
   u32x4 w[KB][4];
   auto fetch_w = [&](int step, int j, int beyond = 0) {
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
           over |= 1u << (b * PER + i);
         }
       }
-    const unsigned char* bytes = reinterpret_cast<const unsigned char*>(tiles + ((size_t)nb * n_kb + kb0) * 256);
+    const unsigned char* bytes = reinterpret_cast<const unsigned char*>(tiles + ((size_t)nb * kb_stride + kb0) * 256);
     for (unsigned long long lanes = __ballot(over != 0); lanes; lanes &= lanes - 1) {
       const int from = __ffsll((long long)lanes) - 1;
       for (unsigned left = __builtin_amdgcn_readlane((int)over, from); left; left &= left - 1) {
@@ -297,9 +299,9 @@ __global__ __launch_bounds__(256, B <= 4 ? 3 : 2) void gemv_nf4_tiles_kernel(
         const int at = i % 16, half = i % 128 / 64;
         const int byte = (((i / 128) * 4 + lane / 16) * 64 + i % 64 / 16 * 16 + lane % 16) * 16 + half * 8 + at / 8 * 4 + at % 4;
         const float level = NF4_TILE_LEVELS[at & 4 ? bytes[byte] >> 4 : bytes[byte] & 15];
-        const float weight = level * bf16_to_f32(scales[((size_t)nb * n_kb + kb0) * 128 + i]);
+        const float weight = level * bf16_to_f32(scales[((size_t)nb * kb_stride + kb0) * 128 + i]);
         float* sum = &red[(wave * B + b) * 64 + lane];
-        *sum = fmaf(weight, x[(size_t)b * in_dim + kb0 * 128 + i], *sum);
+        *sum = fmaf(weight, x[(size_t)b * x_stride + kb0 * 128 + i], *sum);
       }
     }
   };
@@ -572,7 +574,6 @@ static torch::Tensor launch_nf4_tiles(
   const int batch = sel ? 1 : (int)x.size(0);
   const long rows = sel ? sel->numel() : batch, z = sel ? rows : 1;
   TORCH_CHECK(batch >= 1 && batch <= 8, "NF4 products of few rows take at most 8");
-  TORCH_CHECK(n_kb * 4096 < NF4_BEYOND, "too many inputs");  // 33 million
   const int kb = batch <= 4 ? 4 : 2;
   // longer runs combine their sums once, but only where enough waves remain
   const long units = nb * z * ((n_kb + kb - 1) / kb);
@@ -585,25 +586,30 @@ static torch::Tensor launch_nf4_tiles(
                                : torch::empty({splits, rows, out_dim}, x.options());
   if (z == 0) return partials;
   const bool by4 = in_dim % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
-  const dim3 grid(nb, splits, z);
   auto stream = at::cuda::getCurrentCUDAStream();
-#define NF4_TILES(B, KB)                                                                                       \
-  gemv_nf4_tiles_kernel<B, KB><<<grid, 256, 0, stream>>>(                                                      \
-      reinterpret_cast<const uint4*>(tiles.data_ptr()), reinterpret_cast<const unsigned short*>(scales.data_ptr()), \
-      x.data_ptr<float>(), sel ? sel->data_ptr<int>() : nullptr, partials.data_ptr<float>(), (int)in_dim,      \
-      (int)out_dim, (int)n_kb, (int)steps, (int)k_per_tok, sel ? (int)tiles.size(0) : 1, by4)
-  switch (batch) {
-    case 1: NF4_TILES(1, 4); break;
-    case 2: NF4_TILES(2, 4); break;
-    case 3: NF4_TILES(3, 4); break;
-    case 4: NF4_TILES(4, 4); break;
-    case 5: NF4_TILES(5, 2); break;
-    case 6: NF4_TILES(6, 2); break;
-    case 7: NF4_TILES(7, 2); break;
-    case 8: NF4_TILES(8, 2); break;
-  }
+  for (long first = 0; first < n_kb; first += NF4_LAUNCH) {
+    const long run = std::min<long>(n_kb - first, NF4_LAUNCH), inputs = std::min<long>(in_dim - first * 128, NF4_LAUNCH * 128);
+    const dim3 grid(nb, (run + 4 * kb * steps - 1) / (4 * kb * steps), z);
+#define NF4_TILES(B, KB)                                                                                            \
+  gemv_nf4_tiles_kernel<B, KB><<<grid, 256, 0, stream>>>(                                                           \
+      reinterpret_cast<const uint4*>(tiles.data_ptr()) + first * 256,                                               \
+      reinterpret_cast<const unsigned short*>(scales.data_ptr()) + first * 128, x.data_ptr<float>() + first * 128,  \
+      sel ? sel->data_ptr<int>() : nullptr, partials.data_ptr<float>() + first / (4 * kb * steps) * rows * out_dim, \
+      (int)inputs, (int)out_dim, (int)run, (int)steps, (int)k_per_tok, sel ? (int)tiles.size(0) : 1, by4,           \
+      (int)in_dim, (int)n_kb)
+    switch (batch) {
+      case 1: NF4_TILES(1, 4); break;
+      case 2: NF4_TILES(2, 4); break;
+      case 3: NF4_TILES(3, 4); break;
+      case 4: NF4_TILES(4, 4); break;
+      case 5: NF4_TILES(5, 2); break;
+      case 6: NF4_TILES(6, 2); break;
+      case 7: NF4_TILES(7, 2); break;
+      case 8: NF4_TILES(8, 2); break;
+    }
 #undef NF4_TILES
-  HIP_CHECK_LAST();
+    HIP_CHECK_LAST();
+  }
   return partials;
 }
 

@@ -148,6 +148,28 @@ def test_nf4_tiles_of_a_wide_range(hip, batch, loud):
 
 @requires_gpu
 @pytest.mark.parametrize("batch", [1, 5])
+def test_nf4_tiles_of_many_inputs(hip, batch):
+    """2^30 bytes of codes for a run of columns and more: inputs at both ends and around 2^29 and 2^30 bytes count."""
+    n_kb = (1 << 18) + 5
+    k_in = n_kb * 128 - 84
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    tiles = torch.zeros(1, n_kb, 4, 64, 16, device="cuda", dtype=torch.uint8)
+    scales = torch.zeros(1, n_kb * 128, device="cuda", dtype=BF16)
+    x = torch.zeros(batch, k_in, device="cuda")
+    want = bound = 0.0
+    for at in (0, (1 << 17) - 2, (1 << 18) - 2, n_kb - 2):
+        size = min(512, k_in - at * 128)
+        (t, s), w, scale = nf4_weights(hip, size, 64, gen)
+        tiles[:, at : at + t.shape[1]], scales[:, at * 128 : at * 128 + s.shape[1]] = t, s
+        x[:, at * 128 : at * 128 + size] = torch.randn(batch, size, device="cuda", generator=gen)
+        xd = x[:, at * 128 : at * 128 + size].double()
+        want, bound = want + xd @ w, bound + nf4_bound(xd, w, scale)
+    y = hip.gemv_nf4_tiles(tiles, scales, k_in, x, torch.empty(0, device="cuda"), None, 0).double()
+    assert bool(((y - want).abs() <= bound).all()) and bool((want.abs() > 100 * bound).any())
+
+
+@requires_gpu
+@pytest.mark.parametrize("batch", [1, 5])
 def test_nf4_tiles_of_the_largest_numbers(hip, batch):
     """An input that overflows with its block's scale is multiplied by its weight, which may be zero."""
     gen = torch.Generator(device="cuda").manual_seed(batch)
