@@ -543,32 +543,42 @@ __global__ __launch_bounds__(256) void paged_attn_decode(
   const int width = a.kv_heads * (MAPS * a.dk + a.dv);
   // A tile's keys and values; the next one's are asked for as soon as these have been used (8 tokens of 16 pairs of
   // heads at 2048 keys, each a tile that was waited for whole: 63.2 us, now 57.7). A second set of registers
-  // for it would not fit (256 values for each of two maps: 162 registers spilled)
-  bf16x8 vals[NLD], kt[MAPS][2][RC];
+  // for it would not fit (256 values for each of two maps: 162 registers spilled). Two maps of 256 with 256 values
+  // do not even leave them for one set and its addresses (183 spilled; 24 now): the second map's keys are asked for
+  // once the first's are used, addresses are made each time, and no tile is asked for that is not there. us, 8 heads, 8 x
+  // 2049, 1 x 2049 and 8 x 300 keys: waited for whole 80.1, 27.2, 28.2; all asked for ahead 102.0, 34.3, 35.9; so 47.2,
+  // 17.1, 16.7. One map of 256 has the registers: sigmoid weights of 8 heads 28.1, 10.1, 10.8 and 26.8, 10.3, 11.1.
+  constexpr int TOGETHER = 4 * (3 * MAPS * RC + NLD + MAPS * VB) > 320 ? 1 : MAPS;  // maps whose keys are held
+  constexpr bool APART = TOGETHER < MAPS;
+  bf16x8 vals[NLD], kt[TOGETHER][2][RC];
   auto tile_rows = [&](int j0) {
     return cached_rows(cache, j0 < j_end ? cache_row(b, seq, j0) : -1, min(j_end - j0, KVT), width);
   };
-  auto fetch_keys = [&](const auto& rows) {
+  int from = lane;  // the lane, as a value that addresses cannot be made ahead from if APART
+  auto fetch_keys = [&](const auto& rows, int first) {  // of TOGETHER maps
+    if constexpr (APART) asm volatile("" : "+v"(from));
 #pragma unroll
-    for (int u = 0; u < MAPS; ++u)
+    for (int u = 0; u < TOGETHER; ++u)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int kc = 0; kc < RC; ++kc)
-          kt[u][nb][kc] = load_cached(rows, ((nb * 16 + col) * width + (kvh * MAPS + u) * a.dk + kc * 32 + hi * 8) * 2 +
-                                                (kc * 32 < a.dk ? 0 : BEYOND_ROWS));
+          kt[u][nb][kc] = load_cached(
+              rows, ((nb * 16 + (APART ? from & 15 : col)) * width + (kvh * MAPS + first + u) * a.dk + kc * 32 +
+                     (APART ? from >> 4 : hi) * 8) * 2 + (kc * 32 < a.dk ? 0 : BEYOND_ROWS));
   };
   auto fetch_values = [&](const auto& rows) {
+    if constexpr (APART) asm volatile("" : "+v"(from));
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int idx = lane + i * WAVE, row = idx / V8, c8 = idx % V8 * 8;
+      const int idx = (APART ? from : lane) + i * WAVE, row = idx / V8, c8 = idx % V8 * 8;
       vals[i] = load_cached(rows, (row * width + a.kv_heads * MAPS * a.dk + kvh * a.dv + c8) * 2 + (c8 < a.dv ? 0 : BEYOND_ROWS));
     }
   };
   int j0 = j_begin + wave * KVT;
   if (j0 < j_end) {  // uniform over the wave
     const auto rows = tile_rows(j0);
-    fetch_keys(rows);
+    fetch_keys(rows, 0);
     fetch_values(rows);
   }
   for (; j0 < j_end; j0 += 4 * KVT) {
@@ -578,15 +588,21 @@ __global__ __launch_bounds__(256) void paged_attn_decode(
 #pragma unroll
     for (int u = 0; u < MAPS; ++u) {
       f32x4(&s)[2] = scores[u];
+      if constexpr (APART)
+        if (u > 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          fetch_keys(tile_rows(j0), u);
+        }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
         s[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kc = 0; kc < RC; ++kc)
-          s[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[u][nb][kc], q_frag[u][kc], s[nb], 0, 0, 0);
+          s[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[APART ? 0 : u][nb][kc], q_frag[u][kc], s[nb], 0, 0, 0);
       }
     }
-    fetch_keys(next);
+    if constexpr (APART) __builtin_amdgcn_sched_barrier(0);
+    if (!APART || j0 + 4 * KVT < j_end) fetch_keys(next, 0);
 #pragma unroll
     for (int u = 0; u < MAPS; ++u) {
       f32x4(&s)[2] = scores[u];
@@ -603,7 +619,7 @@ __global__ __launch_bounds__(256) void paged_attn_decode(
       const int idx = lane + i * WAVE, row = idx / V8, c8 = idx % V8 * 8;
       *reinterpret_cast<bf16x8*>(&v_tile[row * VROW + c8]) = vals[i];
     }
-    fetch_values(next);
+    if (!APART || j0 + 4 * KVT < j_end) fetch_values(next);
     wave_lds_fence();
     const unsigned short* v_lds = v_tile + (hi * 4 + col / 4) * VROW + (col & 3) * 4;
 #pragma unroll

@@ -684,6 +684,38 @@ def test_attention_kernels(kind, heads, kv_heads, dk, dv, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads,dk,dv", [(2, 2, 256, 256), (16, 1, 256, 256), (3, 3, 160, 144), (4, 2, 256, 128), (2, 2, 128, 256)])
+@pytest.mark.parametrize("keys", [(1, 32, 33), (128, 129, 160), (600, 511, 385)])
+def test_pairs_of_wide_heads(heads, kv_heads, dk, dv, keys):
+    """A wave has one tile of keys, two and several, the last in part, whether it holds both maps' keys at a time or one's;
+    a page that is not in the pool counts as zeros."""
+    from petals_amd.ops import scores
+
+    torch.manual_seed(0)
+    wide, group, scale = kv_heads * 2 * dk, heads // kv_heads, 1.5 * dk**-0.5
+    starts, n = [k - 1 for k in keys], -(-max(keys) // PAGE_SIZE)
+    pages = torch.randperm(3 * n).view(3, n).tolist()
+    cache = torch.randn(3 * n, PAGE_SIZE, wide + kv_heads * dv, device="cuda").bfloat16()
+    batch = PagedBatch(pages, starts, [1, 1, 1], torch.device("cuda"))
+    q = torch.randn(3, heads, 2, dk, device="cuda").bfloat16()
+    rows = [cache[p].reshape(-1, cache.shape[-1]).double().cpu() for p in pages]
+    if n > 1:
+        batch.tables[1, 0] = 3 * n
+        rows[1][:PAGE_SIZE] = 0
+    want = torch.empty(3, heads, dv, dtype=F64)
+    for i, k in enumerate(keys):
+        held, values = rows[i][:k, :wide].unflatten(1, (kv_heads, 2, dk)), rows[i][:k, wide:].unflatten(1, (kv_heads, dv))
+        for h in range(heads):
+            one, two = (torch.softmax(held[:, h // group, u] @ q[i, h, u].double().cpu() * scale, 0) @ values[:, h // group] for u in range(2))
+            want[i, h] = oracle.rms(one - 0.7 * two, 1e-3) * 0.4
+    for splits in (0, 1, 3):
+        out = torch.empty(3, heads * dv, device="cuda", dtype=torch.bfloat16)
+        scores.hip().paired_attention(q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(1), 1, batch.max_end, kv_heads, dv, 0,
+                                      scale, 0.7, 0.4, 1e-3, dv, None, out, splits)
+        assert max_error(out.view(3, heads, dv), want) < 3e-2, splits
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("y_dtype,dtype", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "bfloat16")])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,taps,rot,ff", [
     (1, 1, 1, 1, 0, 0, 0), (4, 2, 12, 20, 3, 8, 30), (6, 3, 48, 16, 4, 48, 256), (33, 1, 80, 40, 2, 12, 1000),
