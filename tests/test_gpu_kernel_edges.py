@@ -147,6 +147,44 @@ def test_nf4_tiles_of_a_wide_range(hip, batch, loud):
 
 
 @requires_gpu
+@pytest.mark.parametrize("batch", range(5, 9))
+@pytest.mark.parametrize(
+    "k_in,n_out,parts",
+    [
+        (4440, 18176, 3),  # two steps of 256 inputs; the last run has 3 of 4 tiles, the three after it none
+        (4440, 29184, 2),  # four steps; the last run's second one is half there
+        (4097, 32768, 2),  # four steps; one input in the last run
+    ],
+)
+@pytest.mark.parametrize("loud", [[50.0], [1e4, 1e9]])
+def test_nf4_tiles_of_long_runs(hip, batch, k_in, n_out, parts, loud):
+    """Runs of several steps, which end within one: loud inputs in each step cost the quiet ones nothing
+    where they meet a weight of zero."""
+    gen = torch.Generator(device="cuda").manual_seed(k_in + n_out + batch)
+    w = (torch.randn(k_in, 192, device="cuda", generator=gen) * 0.05).to(BF16)
+    at = torch.tensor([*range(17, k_in, 251), k_in - 1], device="cuda")
+    w[at, ::2] = 0.0
+    packed, absmax = hip.nf4_quantize(w)
+    scale = absmax.double().repeat_interleave(64, dim=1)
+    held = NF4_LEVELS.cuda().double()[torch.stack([packed & 15, packed >> 4], dim=-1).view(k_in, 192).long()] * scale
+    which = torch.randint(0, 3, (n_out // 64,), device="cuda", generator=gen)  # each run of 64 columns one of three
+    tiles, scales = (t[which].contiguous() for t in hip.nf4_tile(packed, absmax))
+    x = torch.randn(batch, k_in, device="cuda", generator=gen)
+    for i, k in enumerate(at.tolist()):
+        x[i % batch, k] = loud[i % len(loud)]
+    empty = torch.empty(0, device="cuda")
+    assert hip.gemv_nf4_tiles(tiles, scales, k_in, x, empty, None, -1).shape[0] == parts
+    y = hip.gemv_nf4_tiles(tiles, scales, k_in, x, empty, None, 0).double().view(batch, -1, 64)
+    xd, quiet = x.double(), x.double()
+    quiet[:, at] = 0.0
+    want, bound, still = ((v.view(batch, 3, 64)[:, which]) for v in (xd @ held, nf4_bound(xd, held, scale), nf4_bound(quiet, held, scale)))
+    error = (y - want).abs()
+    assert bool((error <= bound).all())
+    if loud[0] > 100:  # beyond what digits hold; 50 times the mean is not, and takes the others' last places
+        assert bool((error[..., ::2] <= still[..., ::2]).all())
+
+
+@requires_gpu
 @pytest.mark.parametrize("batch", [1, 5])
 def test_nf4_tiles_of_many_inputs(hip, batch):
     """2^30 bytes of codes for a run of columns and more: inputs at both ends and around 2^29 and 2^30 bytes count."""
@@ -1146,8 +1184,15 @@ def test_rounding_to_bf16(hip):
     bits = torch.arange(1 << 16, device="cuda", dtype=torch.int32)
     x = bits.to(torch.int16).view(BF16).view(256, 256)  # every bf16 value
     gen = torch.Generator(device="cuda").manual_seed(0)
-    near = torch.randint(-9, 10, (1 << 16,), device="cuda", generator=gen) * 128  # exponents up to nine apart: half of the sums are ties
+    near = torch.randint(-9, 10, (1 << 16,), device="cuda", generator=gen) * 128  # exponents up to nine apart
     others = [x.flip(0), (bits ^ 1).to(torch.int16).view(BF16).view_as(x), (bits + near).to(torch.int16).view(BF16).view_as(x)]
+    for apart in range(1, 9):  # y's last digits make up half of a place of x: ties wherever the sum's place is x's
+        digits = torch.randint(0, 128, (1 << 16,), device="cuda", generator=gen) >> apart << apart | 1 << (apart - 1)
+        exponent = ((bits >> 7 & 255) - apart).clamp(min=1)
+        y = (bits & 0x8000 | exponent << 7 | digits & 127).to(torch.int16).view(BF16).view_as(x)
+        ties = (x.float() + y.float()).view(torch.int32) & 0xFFFF == 0x8000  # of two bf16 values so close, exact in 32 bits
+        assert ties.float().mean() > 0.2
+        others.append(y)
     for y in others:
         got, want = hip.add_rows(x.contiguous(), y.contiguous()), x + y
         assert torch.equal(got.isnan(), want.isnan())
