@@ -464,10 +464,14 @@ def test_latent_attention_kernel(heads, rank, window, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads", [3, 17, 40])
-@pytest.mark.parametrize("rank", [416, 480, 512])
-def test_latent_rows_straight_to_lds(heads, rank):
-    """Rows of 13 to 16 chunks go to LDS without registers: the columns past them and a page that is not in the pool
-    count as zeros, and what is cached beyond the end does not count at all."""
+@pytest.mark.parametrize("rank,values,window", [
+    (416, 0, 0), (480, 0, 0), (512, 0, 0), (480, 0, 50), (512, 0, 50), (416, 400, 50), (512, 448, 50),  # straight to LDS
+    (384, 0, 0), (384, 320, 50), (448, 384, 0), (448, 384, 50), (576, 512, 50),  # through registers
+])
+def test_latent_rows_straight_to_lds(heads, rank, values, window):
+    """Rows of 13 to 16 chunks of 32 go to LDS without registers, those of 13 and 14 if more than 12 of them are values: the
+    columns past them and a page that is not in the pool count as zeros, and what is cached beyond the end does not
+    count at all. Wide rows that go through registers are held to the same."""
     from petals_amd.ops import latent
 
     torch.manual_seed(0)
@@ -488,12 +492,12 @@ def test_latent_rows_straight_to_lds(heads, rank):
     run = batch.run_tokens(heads)
     for splits in (1, 3):
         got = latent.hip().latent_attention(
-            q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(run), run, batch.max_end, 0, scale, splits
+            q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(run), run, batch.max_end, window, scale, splits, values
         )
         for (lo, hi), c, s in zip(batch.row_ranges(), seen_rows, starts):
             score = torch.einsum("thr,kr->htk", q[lo:hi].double().cpu(), c) * scale
-            seen = oracle.window_mask(len(c), len(c))[s:]
-            want = torch.einsum("htk,kr->thr", score.masked_fill(~seen, -float("inf")).softmax(-1), c)
+            seen = oracle.window_mask(len(c), window or len(c))[s:]
+            want = torch.einsum("htk,kr->thr", score.masked_fill(~seen, -float("inf")).softmax(-1), c[:, : values or rank])
             # probabilities and results are rounded to 8 bits: 2^-8 of the largest value, 5, each
             assert (got[lo:hi].double().cpu() - want).abs().max() < 4e-2
 
