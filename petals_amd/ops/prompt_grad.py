@@ -111,14 +111,22 @@ def takes_nf4_gemm(m: int, k: int, n: int) -> bool:
 
     Codes are a quarter of the bytes, but each is looked up and rounded: large matrices gain up to 128 rows, beyond which
     the matrix cores bound both; smaller ones gain as long as reading a copy takes longer than the
-    launches. us on MI355X, with a copy and from codes: 2048 x 11264, 32 rows 16.0, 15.6, 33 rows 18.4, 20.3;
-    4096 x 4096, 16 rows 12.7, 14.4; 11008 x 4096, 64 rows 28.3, 27.4, 96 rows 33.3, 29.8, 128 rows 32.7, 31.7; 14336 x 4096,
-    64 rows 33.5, 29.2, 128 rows 34.0, 36.3; 8192 x 8192, 128 rows 41.0, 39.2; 8192 x 57344, 128 rows 177, 139, 192 rows
-    207, 264."""
+    launches. Matrices of few columns have few tiles, which are cut into more parts along K that have to be added up. us on
+    MI355X, with a copy and from codes (profiles/nf4_prompt_products.csv has all that was measured): 2048 x 11264, 32 rows
+    17.1, 16.0, 64 rows 19.4, 20.8; 11008 x 4096, 64 rows 28.9, 27.7, 128 rows 29.4, 33.3; 16384 x 4096, 128 rows
+    37.7, 39.4; 18176 x 4544, 128 rows 42.9, 43.2; 8192 x 57344, 128 rows 178, 150, 192 rows 204, 282.
+
+    Where there is no copy, making one comes on top (33 us for 8192 x 8192, 230 for 8192 x 57344): in the first prompt, and in
+    every prompt of a span whose copies together are more than the cache of them holds. So 8192 x 8192, and other
+    matrices of 64 << 20 to 76 << 20 weights that are not narrow, are read as codes up to 128 rows, though with a copy
+    they would take up to 4 us less (112 rows 36.2, 40.1; 5120 x 13824, 96 rows 38.9, 41.2). From 129 rows on it is not
+    looked at whether there is one: 8192 x 57344 with 192 rows would take less from codes in such a span."""
     if m <= 0 or k % 128:
         return False
     weights = k * n
-    return m <= 32 and weights >= 20 << 20 or m <= 64 and weights >= 40 << 20 or m <= 128 and weights >= 64 << 20
+    if m <= 64:
+        return weights >= (20 << 20 if m <= 32 else 40 << 20)
+    return m <= 128 and weights >= (64 << 20 if n > 4608 else 76 << 20)
 
 
 def _by_torch(*grads) -> bool:

@@ -1274,6 +1274,9 @@ def test_nf4_prompts_read_codes(hip, monkeypatch):
 
     assert prompt_grad.takes_nf4_gemm(32, 4096, 6144) and not prompt_grad.takes_nf4_gemm(33, 4096, 6144)
     assert prompt_grad.takes_nf4_gemm(128, 8192, 8192) and not prompt_grad.takes_nf4_gemm(129, 8192, 8192)
+    # few columns: 2 us slower from codes beyond 64 rows
+    assert prompt_grad.takes_nf4_gemm(64, 16384, 4096) and not prompt_grad.takes_nf4_gemm(65, 16384, 4096)
+    assert not prompt_grad.takes_nf4_gemm(128, 16384, 4608) and prompt_grad.takes_nf4_gemm(128, 18176, 4544)
     assert not prompt_grad.takes_nf4_gemm(0, 8192, 8192) and not prompt_grad.takes_nf4_gemm(8, 8192 + 64, 8192)
     gen = torch.Generator(device="cuda").manual_seed(0)
     weight = _FastWeight((torch.randn(512, 320, device="cuda", generator=gen) * 0.125).to(BF16), hip, "nf4")
