@@ -13,12 +13,12 @@
 // combination, before (values through LDS, transposed one by one; every load waited for;
 // weights through LDS) and now:
 //   kv heads x queries each, head size, keys: 8 x 8, 128, 154           12.9 ->  6.2
-//   8 x 8, 128, 2004                                                    18.8 -> 11.3
-//   64 x 8, 128, 2004                                                   41.4 -> 20.6   3.2 TB/s
-//   16 x 4, 128, 7901                                                   44.0 -> 22.4   2.9 TB/s
-//   8 x 4, 128, 32000                                                   73.3 -> 37.9   3.5 TB/s
-//   256 x 1, 128, 1000                                                  44.6 -> 27.1   4.8 TB/s
-//   1 x 71, 64, 1000 (in cache)                                         39.8 -> 20.3
+//   8 x 8, 128, 2004                                                    18.8 ->  9.1
+//   64 x 8, 128, 2004                                                   41.4 -> 18.9   3.5 TB/s
+//   16 x 4, 128, 7901                                                   44.0 -> 18.0   3.6 TB/s
+//   8 x 4, 128, 32000                                                   73.3 -> 32.7   4.0 TB/s
+//   256 x 1, 128, 1000                                                  44.6 -> 25.3   5.2 TB/s
+//   1 x 71, 64, 1000 (in cache)                                         39.8 -> 19.0
 //
 // The original VALU kernel (attn_decode_kernel: 16-lane-group dot products,
 // online softmax in registers) is kept behind PETALS_DECODE_KERNEL=valu.
@@ -453,10 +453,10 @@ torch::Tensor attn_decode_fused(
       n_splits = std::max(1, std::min(1024 / bkv, (lmax + 63) / 64));
     } else {
       // One workgroup for each of the 256 compute units, parts of 128 rows or more of a full
-      // cache: two or three per unit were slower (32000 keys of 8 heads: 16 parts 37.5 us, 32
-      // parts 37.9, 62 parts 48.3; 256 heads: 1 part 27.1, 2 parts 30.6). Up to 384 rows one
-      // part, as the second launch costs more than the longer chain (300 keys of 8 heads: 8.0
-      // us, 8.6 with 4 parts; 500 of 32 heads: 9.7, 9.2). Rows are those that the cache can
+      // cache: two or three per unit were slower (32000 keys of 8 heads: 32 parts 31.7
+      // us, 62 parts 39.6; 256 heads: 1 part 24.4, 2 parts 27.6). Up to 384 rows one
+      // part, as the second launch costs more than the longer chain (300 keys of 8 heads: 8.1
+      // us, 8.6 with 3 parts; of 32 heads 8.2, 8.7; 500 of 32 heads: 10.1, 8.8 with 4). Rows are those that the cache can
       // hold, as a captured launch stays while it fills; a short text in a long cache is read
       // in as many parts, of few rows each.
       static const int short_max = [] {

@@ -1,7 +1,7 @@
 // Products of a prompt's rows with NF4 weights for CDNA4 (gfx950): X [M, K] in bf16 times tiles of codes
 // (nf4_tiles.hip has their order), and what follows them, as in gemm.hip. A weight is level * scale, rounded to
 // bf16, as a copy of the matrix in bf16 would hold it: no such copy is made, kept or read, which is what bounds
-// products of up to 128 rows by gemm.hip (4.9 TB/s; a copy's first use also waits for its making, 35 to 200 us).
+// products of up to 128 rows by gemm.hip (4.9 TB/s; where there is no copy, its making comes first, 33 us for 8192 x 8192, 230 for 8192 x 57344).
 //
 // A workgroup of 8 waves has 32 FM rows and 256 columns, 32 of each wave, whose weights that wave makes in its
 // registers, where they are the matrix cores' operand: of 16 bytes of codes a lane has two runs of 8 inputs of
@@ -11,7 +11,7 @@
 // operations a tile: 5 to 10% slower).
 //
 // Matrix instructions of 32 x 32, as vector instructions run beside these (6 in 32 cycles at no cost) and hardly
-// beside those of 16 x 16 (3 in 16 cycles cost what they cost alone: 128 x 8192 x 57344 took 174 us with them, 139 now).
+// beside those of 16 x 16 (3 in 16 cycles cost what they cost alone: 128 x 8192 x 57344 took 174 us with them, 139 now, 150 among a prompt's other launches).
 // A step is 16 inputs: its products, among which the next step's weights are rounded, those of the third
 // after it looked up, and rows read. Up to 32 rows it is bound by LDS (look-ups and scales: 2000 of 2600 cycles a tile of
 // 128 inputs), with 128 by the matrix cores with vector instructions beside them (0.86 PFLOP/s, 1.0 in the workgroups
@@ -19,11 +19,11 @@
 // SIMD: 236 us.
 //
 // MI355X, us, gemm.hip or the library with copies that are there already, and this one with its sum of parts:
-//   rows                    16            64           128          256
-//   8192 x 10240        37.2, 22.8    39.8, 30.8   44.1, 39.8   62.6, 59.4
-//   8192 x 57344 gated   170, 78       170, 97      177, 139     236, 264
-//   28672 x 8192        85.0, 43.3    95.0, 52.0   96.1, 78.6    136, 134
-//   4096 x 4096         12.7, 14.4    13.5, 17.4   17.2, 23.6
+//   rows                    16            64           128          192
+//   8192 x 10240        37.8, 24.9    39.8, 31.5   44.9, 42.8   62.9, 54.9
+//   8192 x 57344 gated   168, 78       170, 96      178, 150     204, 282
+//   28672 x 8192        85.2, 44.8    89.2, 54.7   96.6, 79.4    131, 136
+//   4096 x 6144         17.1, 16.4    19.9, 21.7   21.9, 26.5   28.6, 29.6
 
 #include "gemm.h"
 #include <torch/extension.h>
