@@ -543,11 +543,12 @@ __global__ __launch_bounds__(256) void paged_attn_decode(
   const int width = a.kv_heads * (MAPS * a.dk + a.dv);
   // A tile's keys and values; the next one's are asked for as soon as these have been used (8 tokens of 16 pairs of
   // heads at 2048 keys, each a tile that was waited for whole: 63.2 us, now 57.7). A second set of registers
-  // for it would not fit (256 values for each of two maps: 162 registers spilled). Two maps of 256 with 256 values
+  // for it would not fit (two maps of 128 with 256 values: 162 registers spilled, 2 with this one). Two maps of 256 with 256 values
   // do not even leave them for one set and its addresses (183 spilled; 24 now): the second map's keys are asked for
   // once the first's are used, addresses are made each time, and no tile is asked for that is not there. us, 8 heads, 8 x
   // 2049, 1 x 2049 and 8 x 300 keys: waited for whole 80.1, 27.2, 28.2; all asked for ahead 102.0, 34.3, 35.9; so 47.2,
   // 17.1, 16.7. One map of 256 has the registers: sigmoid weights of 8 heads 28.1, 10.1, 10.8 and 26.8, 10.3, 11.1.
+  // All sizes and kinds of weights: profiles/paged_decode_attention.csv.
   constexpr int TOGETHER = 4 * (3 * MAPS * RC + NLD + MAPS * VB) > 320 ? 1 : MAPS;  // maps whose keys are held
   constexpr bool APART = TOGETHER < MAPS;
   bf16x8 vals[NLD], kt[TOGETHER][2][RC];
