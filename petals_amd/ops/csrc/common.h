@@ -21,6 +21,20 @@ __device__ __forceinline__ unsigned short f32_to_bf16(float f) {
   return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
+// GELU by its tanh form, 0.5 x (1 + tanh(u)) with u = sqrt(2 / pi) (x + 0.044715 x^3): x times the logistic function of 2u,
+// from exp(-2|u|), which neither overflows nor takes numbers off each other that are nearly equal. Thirteen
+// instructions where the library's tanh has two branches of some twenty: within a product's sums, where a wave
+// has nobody to hide them, 513 us to 495 (4096 x 4096 x 16384). Error against 64 bits, relative in the 2-norm, here and by tanhf:
+// 2.9e-8 and 3.1e-8 for normal values, 1.0e-7 and 3.8e-7 from -4 to -1, 5e-7 and 2e-3 below
+__device__ __forceinline__ float gelu_tanh_f32(float x) {
+  // -2 sqrt(2 / pi) log2(e), and 0.044715 times that
+  const float t = __builtin_amdgcn_exp2f(-fabsf(x * fmaf(x * x, -0.10294324f, -2.3022082f))), d = 1.f + t;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  const float q = t * r;
+  return x > 0.f ? fmaf(-fminf(x, 1e30f), q, x) : x * q;
+}
+
 // full-wave fp32 sum (64 lanes)
 __device__ __forceinline__ float wave_reduce_sum(float x) {
 #pragma unroll

@@ -44,13 +44,6 @@ static __device__ __forceinline__ float reduce_splits(
   return (s0 + s1) + (s2 + s3);
 }
 
-static __device__ __forceinline__ float gelu_tanh_f32(float x) {
-  // matches torch F.gelu(approximate="tanh") (= HF BLOOM/Falcon GELU)
-  const float c = 0.79788456080286535588f;  // sqrt(2/pi)
-  const float t = tanhf(c * (x + 0.044715f * x * x * x));
-  return 0.5f * x * (1.f + t);
-}
-
 // A workgroup has 64 outputs x G groups of parts, a wave each: the one-thread-
 // per-output version launched only `out/64` single-wave workgroups (0.15
 // waves/SIMD for a 10k-output gemv) and was latency-bound at ~7 us — as much

@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void bias_gelu_rows_kernel(
     for (int e = 0; e < 8; ++e) v[e] += c[e];
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = 0.5f * v[e] * (1.f + tanhf(0.79788456080286535588f * (v[e] + 0.044715f * v[e] * v[e] * v[e])));
+  for (int e = 0; e < 8; ++e) v[e] = gelu_tanh_f32(v[e]);
   store8f(y + g * 8, v);
 }
 

@@ -73,6 +73,25 @@ def test_expert_gemm_group_edges(hip, quant, counts, k_in, n_out):
             assert bool(((out[rows] - ref).abs() <= bound).all()), e
 
 
+@requires_gpu
+def test_gelu_over_all_of_bf16(hip):
+    """GELU of every finite bf16 number, infinities and NaN, beside 64 bits."""
+    x = torch.arange(1 << 16, device="cuda", dtype=torch.int32).to(torch.int16).view(BF16)
+    y = x.clone().view(-1, 1024)
+    hip.bias_gelu_rows(y, None)
+    y, xd = y.flatten().double(), x.double()
+    u = (2 / torch.pi) ** 0.5 * (xd + 0.044715 * xd**3)
+    want = torch.where(xd > 0, xd / (1 + torch.exp(-2 * u)), xd * torch.exp(2 * u) / (1 + torch.exp(2 * u)))
+    small = xd.abs() <= 2.0**20
+    # one rounding to bf16, whose 8 bits are good to 2^-8; 32-bit: 2u has an error of 2^-22 of itself, which is that of a small exponential, flushed below 2^-126
+    slack = want.abs() * (2.0**-8 + 2.0**-22 * (2 + 2 * u.abs())) + 2.0**-125 * xd.abs().clamp(min=1.0)
+    assert bool(((y - want).abs() <= slack)[small].all())
+    large = xd.isfinite() & ~small
+    assert torch.equal(y[large & (xd > 0)], xd[large & (xd > 0)]) and not y[large & (xd < 0)].any()
+    assert y[xd == float("inf")].isposinf().all()
+    assert y[xd.isnan() | (xd == float("-inf"))].isnan().all()  # 0 times infinity
+
+
 NF4_LEVELS = torch.tensor([
     -1.0, -0.6961928009986877, -0.5250730514526367, -0.39491748809814453, -0.28444138169288635,
     -0.18477343022823334, -0.09105003625154495, 0.0, 0.07958029955625534, 0.16093020141124725,
