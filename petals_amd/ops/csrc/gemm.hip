@@ -2,43 +2,39 @@
 // or W [N, K] transposed (a backward pass), and what follows them: a bias and GELU, a
 // residual, or the SwiGLU of a fused gate and up projection.
 //
-// For tens to some hundreds of rows: there the library's kernels leave many compute units
+// For tens to some thousands of rows: the library's kernels leave many compute units
 // without a tile (758 x 4096 has 48 tiles of 256 x 256) or one with twice the others' work,
 // and read weights at 2 TB/s where a prompt of 128 tokens is bound by reading them.
 //
-// A workgroup of 8 waves has a tile of BM x BN and K in steps of 64, through ST buffers of LDS
-// that are filled straight from memory (buffer_load ... lds: no registers, no stores, and
+// Two kinds of tiles. Those of 96 to 256 rows and 256 columns are four waves' (gemm_wide.h), bound by the way from L2 to
+// LDS and by the matrix cores. Smaller ones, for few rows or columns, are those of 8 waves: BM x BN and K in steps of 64,
+// through ST buffers of LDS that are filled straight from memory (buffer_load ... lds: no registers, no stores, and
 // what lies beyond the rows or columns repeats the last ones). A step is two phases of 32 of K;
 // in each, the matrix cores work on one set of fragments while the next set is read from LDS
 // and some of the loads of the step ST - 1 ahead are issued. All loads of a step issued at
-// once, behind the barrier, block the waves until the caches' queues have taken them: 512 x
-// 4096 x 16384 took 70.3 instead of 60.5 us then. The barrier leaves the loads of later steps
-// in flight.
+// once, behind the barrier, block the waves until the caches' queues have taken them. The barrier leaves the loads of
+// later steps in flight. 16-byte groups of LDS rows are permuted by the row, so that the rows that a load
+// touches lie in different banks; W [K, N] is read by transposing loads. These are bound by reading weights.
 //
 // Tiles that fill all compute units are summed over all of K; those left over in the last wave
 // of workgroups are split along K, so that it is as full as the others, and a second
 // kernel adds their parts up. Each chiplet has its own consecutive run of tiles, rows first: they find
-// a run of columns' weights in its L2.
+// a run of columns' weights in its L2. The product is W^T X^T, so that a lane ends with 4 neighbouring columns of one row.
 //
-// The product is W^T X^T, so that a lane ends with 4 neighbouring columns of one row. 16-byte groups of
-// LDS rows are permuted by the row, so that the rows that a load touches lie in different
-// banks; W [K, N] is read by transposing loads.
-//
-// Bound by reading weights for up to 128 rows (28672 x 8192: 4.9 TB/s), beyond that by the
-// matrix cores waiting for fragments (1.0 to 1.1 PFLOP/s where tiles fill all compute units; without
-// loads 1.3, without loads and fragments 1.7). MI355X, us, the library's kernels and this one with its sum of
+// MI355X, us, the library's kernels, those of 8 waves alone (tiles of 128 x 256 at most), and these, with their sum of
 // parts, weights from memory:
-//   rows                 16          128          512          758
-//   4096 x 4096        19, 14      33, 18       34, 28       39, 36
-//   8192 x 10240       48, 37      76, 45      112, 110     134, 121
-//   16384 x 4096       79, 34     139, 38      139, 74      149, 119
-//   28672 x 8192      134, 86     199, 96      352, 216     301, 389
-//   8192 x 57344      161, 161    173, 175     413, 459     602, 651
-//   22016, transposed, to 4096:   114, 52      233, 102     232, 162
-// A call takes the host 8 us, the library's 18. Which of the two a product takes is ops/prompt_grad.py's rule
-// (takes_gemm); profiles/prompt_products.csv has what it was drawn from.
+//   rows                 16        128         512              758              1024
+//   4096 x 4096        19, 14    33, 18    31, 28, 26       35, 36, 29       39, 38, 33
+//   4096 x 22016                           89, 97, 91      133, 138, 121    167, 185, 160
+//   11008 x 4096                           96, 58, 54      103, 85, 68      110, 98, 86
+//   16384 x 4096       79, 34   139, 38   139, 74, 70      147, 119, 91
+//   28672 x 8192      134, 86   199, 96   349, 216, 188    299, 389, 272    370, 423, 344
+//   22016, transposed, to 4096:           229, 102, 87     231, 162, 119    248, 180, 143
+//   12288, transposed, to 4096:            79, 62, 55       91, 96, 73      112, 112, 90
+// A call takes the host 8 us, the library's 18. Which of the two a product takes are ops/prompt_grad.py's rules
+// (takes_gemm, takes_wide_gemm); profiles/prompt_products.csv and prompt_products_wide.csv have what they were drawn from.
 
-#include "gemm.h"
+#include "gemm_wide.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 
@@ -69,7 +65,8 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
   if (!gemm_spot(s, s.k / BK, &spot)) return;
   const int tile = spot.tile, first = spot.first, steps = spot.steps, part = spot.part;
   const bool pairs = o.epilogue == GEMM_SWIGLU;
-  const int m0 = tile % s.row_tiles * BM, column_tile = tile / s.row_tiles;
+  const GemmPlace place = gemm_place<BN>(s, tile);
+  const int m0 = place.row * BM, column_tile = place.column;
   const int wm = wave / WC * FM * 16, wn = wave % WC * FN * 16;
 
   // this wave's loads: byte offsets of each lane, of the step, and what a step adds
@@ -228,9 +225,127 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
   }
 }
 
+// ------------------------------------------------------- tiles of four waves
+
+// rows of 16 of a tile of 256 columns. Two rows of waves read less from LDS where rows are many; W [K, N] with few
+// rows is 5% faster with one (758 x 4096 x 22016 in tiles of 160 rows: 134.7 us, 143)
+template <bool WT, int ROWS>
+struct WideGemm {
+  static constexpr int WR = ROWS % 2 == 0 && (WT || ROWS > 10) ? 2 : 1, FM = ROWS / WR;
+  using Tile = WideTile<WT, WR, FM>;
+};
+
+template <bool WT, int ROWS>
+__global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_wide_kernel(
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, GemmShape s, GemmOut o) {
+  using Gemm = WideGemm<WT, ROWS>;
+  using Tile = typename Gemm::Tile;
+  constexpr int FM = Gemm::FM, FN = Tile::FN, BM = Tile::BM, BN = Tile::BN;
+  extern __shared__ __align__(1024) unsigned char gemm_lds[];
+  GemmSpot spot;
+  if (!gemm_spot(s, s.k / GEMM_BK, &spot)) return;
+  const bool pairs = o.epilogue == GEMM_SWIGLU;
+  const GemmPlace place = gemm_place<BN>(s, spot.tile);
+  const int m0 = place.row * BM, column_tile = place.column;
+  f32x4 acc[FN][FM];
+  wide_product<WT, Gemm::WR, FM>(
+      gemm_lds, acc, wide_resource(x, (unsigned)s.m * s.k * 2), wide_resource(w, (unsigned)s.k * s.n * 2),
+      [&](int row) { return (unsigned)min(m0 + row, s.m - 1) * s.k * 2; },
+      [&](int c) { return (unsigned)min(gemm_source_column<FN>(column_tile, c, BN, s.n, pairs), s.n - (WT ? 1 : 8)); },
+      (unsigned)(WT ? s.k : s.n) * 2, spot.first, spot.steps);
+  if (spot.part >= 0) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x & (WAVE - 1);
+    float* to = o.parts + ((size_t)spot.part * s.rest + spot.tile - s.whole) * (BM * BN) + (wave * FM * FN * WAVE + lane) * 4;
+    wide_each<FM>([&](auto j_) {
+      constexpr int j = decltype(j_)::value;
+      wide_each<FN>([&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        wide_pin<(j * FN + i < 56)>(acc[i][j]);
+        *reinterpret_cast<f32x4*>(to + (j * FN + i) * WAVE * 4) = acc[i][j];
+      });
+    });
+    return;
+  }
+  // loads of residuals that follow stores wait for a trip to memory each: 16 to 32 of them
+  const int row = m0 + wide_row<WT, Gemm::WR, FM>(), c = wide_column<WT, Gemm::WR, FM>();
+  int n[FN / 2];
+  Gemm8 bias[FN / 2] = {}, residual[2][FN / 2] = {};
+#pragma unroll
+  for (int i = 0; i < FN / 2; ++i) {
+    n[i] = gemm_source_column<FN>(column_tile, c + i * 32, BN, s.n, pairs);
+    if (o.bias) bias[i] = gemm_load8(o.bias + min(n[i], s.n - 8));
+  }
+  wide_store<WT, Gemm::WR, FM>(
+      pairs, acc,
+      [&](auto j) {
+        if (o.residual)
+#pragma unroll
+          for (int i = 0; i < FN / 2; ++i)
+            residual[j & 1][i] = gemm_load8(o.residual + (size_t)min(row + j * 16, s.m - 1) * s.n + min(n[i], s.n - 8));
+      },
+      [&](auto j, auto i, float (&v)[8], float (&u)[8]) {
+        if (pairs) gemm_store_pair(s, o, row + j * 16, n[i], v, u);
+        else gemm_store(s, o, row + j * 16, n[i], v, bias[i], residual[j & 1][i]);
+      });
+}
+
+// parts [splits, rest, waves, FM, FN, 64, 4]: two fragments, with pairs four, per thread
+template <bool WT, int ROWS>
+__global__ __launch_bounds__(256) void gemm_wide_parts_kernel(GemmShape s, GemmOut o) {
+  using Gemm = WideGemm<WT, ROWS>;
+  using Tile = typename Gemm::Tile;
+  constexpr int FM = Gemm::FM, FN = Tile::FN, BM = Tile::BM, BN = Tile::BN;
+  const bool pairs = o.epilogue == GEMM_SWIGLU;
+  const int unit = __builtin_amdgcn_readfirstlane((blockIdx.x * 256 + threadIdx.x) / WAVE), lane = threadIdx.x & (WAVE - 1);
+  const int each = pairs ? FN / 4 : FN / 2, i = unit % each * 2, j = unit / each % FM, wave = unit / each / FM % 4;
+  const int tile = unit / each / FM / 4;
+  if (tile >= s.rest) return;
+  const float* p = o.parts + (size_t)tile * (BM * BN) + (((wave * FM + j) * FN + i) * WAVE + lane) * 4;
+  const size_t stride = (size_t)s.rest * (BM * BN);
+  f32x4 sum[4] = {};
+  for (int k = 0; k < s.splits; ++k)
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+      if (f < 2 || pairs) sum[f] += *reinterpret_cast<const f32x4*>(p + k * stride + ((f >> 1) * (FN / 2) + (f & 1)) * WAVE * 4);
+  const GemmPlace place = gemm_place<BN>(s, s.whole + tile);
+  const int hi = lane >> 4, m = place.row * BM + (wave / Tile::WC * FM + j) * 16 + (lane & 15);
+  const int n = gemm_source_column<FN>(place.column, (wave % Tile::WC * FN + i + (hi & 1)) * 16 + (hi >> 1) * 8, BN, s.n, pairs);
+  float v[8];
+  wide_join(sum[0], sum[1], v);
+  if (pairs) {
+    float u[8];
+    wide_join(sum[2], sum[3], u);
+    gemm_store_pair(s, o, m, n, v, u);
+  } else {
+    Gemm8 bias = {}, residual = {};
+    if (o.bias) bias = gemm_load8(o.bias + min(n, s.n - 8));
+    if (o.residual) residual = gemm_load8(o.residual + (size_t)min(m, s.m - 1) * s.n + min(n, s.n - 8));
+    gemm_store(s, o, m, n, v, bias, residual);
+  }
+}
+
+template <bool WT, int ROWS>
+static void launch_gemm_wide(const unsigned short* x, const unsigned short* w, const GemmShape& s, const GemmOut& o, long blocks, hipStream_t stream) {
+  using Tile = typename WideGemm<WT, ROWS>::Tile;
+  const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WT, ROWS>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, Tile::LDS);
+  TORCH_CHECK(fits == hipSuccess, "gemm_rows: ", hipGetErrorString(fits));
+  gemm_wide_kernel<WT, ROWS><<<blocks, WIDE_THREADS, Tile::LDS, stream>>>(x, w, s, o);
+  HIP_CHECK_LAST();
+  if (s.splits > 1) {
+    const long threads = (long)s.rest * Tile::BM * Tile::BN / (o.epilogue == GEMM_SWIGLU ? 16 : 8);
+    gemm_wide_parts_kernel<WT, ROWS><<<(threads + 255) / 256, 256, 0, stream>>>(s, o);
+    HIP_CHECK_LAST();
+  }
+}
+
 // ------------------------------------------------------------------- host
 
-static const GemmTile GEMM_TILES[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
+// step, fixed and alone by least squares over 780 products of the presets, 17 to 4096 rows, in either direction: 12% off in
+// the mean; the tile that they choose takes 1.1% more than the best one
+static const GemmTile GEMM_TILES[] = {{128, 256, 0.83f, 4.6f, 0.72f}, {128, 128, 0.54f, 2.2f, 0.81f}, {64, 256, 0.66f, 6.f, 0.88f},
+                                      {32, 256, 0.57f, 3.7f, 1.f},    {256, 256, 1.42f, 2.f, 0.68f},  {192, 256, 1.15f, 2.7f, 0.69f},
+                                      {160, 256, 0.94f, 4.4f, 0.65f}, {96, 256, 0.74f, 3.9f, 0.82f}};
 
 // x [M, K] bf16, w [K, N] (or [N, K], transposed) bf16 -> [M, N] bf16 (swiglu: [M, N/2])
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
@@ -263,7 +378,7 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
   int best = 0;
   float least = 0.f;
   GemmShape s{};
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < (int)(sizeof(GEMM_TILES) / sizeof(GemmTile)); ++i) {
     if (tile >= 0 && tile != i) continue;
     float us;
     const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, GEMM_TILES[i], &us);
@@ -298,12 +413,23 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
     if (transposed) GEMM(true, __VA_ARGS__);   \
     else GEMM(false, __VA_ARGS__);             \
   } while (0)
+#define GEMM_WIDE(ROWS)                                                                             \
+  do {                                                                                              \
+    TORCH_CHECK(ROWS * 16 == t.bm);                                                                 \
+    if (transposed) launch_gemm_wide<true, ROWS>(BF16P(x), BF16P(w), s, o, blocks, stream);         \
+    else launch_gemm_wide<false, ROWS>(BF16P(x), BF16P(w), s, o, blocks, stream);                   \
+  } while (0)
   switch (best) {
-    case 0: GEMM_EITHER(2, 4, 4, 4, 3); break;
     case 1: GEMM_EITHER(2, 4, 4, 2, 4); break;
     case 2: GEMM_EITHER(2, 4, 2, 4, 4); break;
     case 3: GEMM_EITHER(1, 8, 2, 2, 4); break;
+    case 0: GEMM_WIDE(8); break;
+    case 4: GEMM_WIDE(16); break;
+    case 5: GEMM_WIDE(12); break;
+    case 6: GEMM_WIDE(10); break;
+    case 7: GEMM_WIDE(6); break;
   }
+#undef GEMM_WIDE
 #undef GEMM_EITHER
 #undef GEMM
   return y;

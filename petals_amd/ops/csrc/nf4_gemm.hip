@@ -61,7 +61,8 @@ __global__ __launch_bounds__(512, 2) void nf4_gemm_kernel(
   if (!gemm_spot(s, s.k / NF4_BK, &spot)) return;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 31, hi = lane >> 5;
-  const int m0 = spot.tile % s.row_tiles * BM, column_tile = spot.tile / s.row_tiles;
+  const GemmPlace place = gemm_place<NF4_BN>(s, spot.tile);
+  const int m0 = place.row * BM, column_tile = place.column;
   const int n_kb = s.k / NF4_BK, last = spot.first + spot.steps - 1;
 
   // of a tile of codes, this lane has 2 of the 4 runs of 16 inputs (in either half of the tile) of one column

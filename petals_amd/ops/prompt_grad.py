@@ -105,6 +105,30 @@ def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = F
     return m <= 128 or tiles <= (256 if fused else 128)
 
 
+def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: bool = False) -> bool:
+    """Whether m rows of k times a large matrix with n columns, which `takes_gemm` leaves to the library, are
+    faster by the tiles of 256 columns that four waves have in ops/csrc/gemm.hip. `followed`: by a residual or a
+    SwiGLU, which would be launches of their own.
+
+    These are products that the GPU is waited for. Up to 1536 rows the library's tiles leave compute units idle, and
+    it takes 1.13 times as long in the mean; beyond, tiles fill the chip either way, and it is slower only by what
+    follows, or at sizes that are no multiples of 128, for which it has no good kernel. us on MI355X by the library (with what follows) and by the
+    kernel: 4096 x 12288, 758 rows 72, 66; 4096 x 22016, 758 rows 133, 121; 28672 x 8192 with a residual, 758 rows 321, 285;
+    4096 x 28672, 4096 rows 743, 747, with SwiGLU 814, 741; 18176 x 4544, 2048 rows 355, 272.
+    Transposed: 22016 to 4096, 758 rows 231, 119, 4096 rows 540, 620; 8192 to 8192, 512 rows 74, 69, 1024 rows
+    112, 114; 4096 to 11008, 256 rows 50, 44, 512 rows 51, 56. All that was measured: profiles/prompt_products_wide.csv."""
+    weights = k * n
+    if not 128 < m < (1 << 31) // k or weights > 1 << 29:
+        return False
+    # smaller ones, long or wide ones above all (2048 x 11264, 900 rows: 43, 42), are bound by launches
+    if weights < 3 << 23 and (weights < 1 << 24 or max(k, n) >= 4 * min(k, n)):
+        return False
+    odd = k % 128 > 0 or n % 128 > 0
+    if transposed:
+        return m <= 1536 and k > n or m <= 640 and k == n or m <= 320 and n < 3 * k or odd
+    return m <= 1536 or followed or odd
+
+
 def takes_nf4_gemm(m: int, k: int, n: int) -> bool:
     """Whether m rows of k times an NF4 matrix with n columns are faster by ops/csrc/nf4_gemm.hip, which reads
     the codes, than by a product with a copy of it in bf16 that is there already.
@@ -262,7 +286,9 @@ def rows_product(x, w, hip, transposed=False):
     """x [..., K] times w [K, N], or [..., N] times its transpose: by ops/csrc/gemm.hip where that is
     the faster one, else the library's."""
     k, n = w.shape if not transposed else w.shape[::-1]
-    if x.shape[-1] == k and takes_gemm(x.numel() // k, k, n, transposed):  # torch refuses rows of other lengths
+    m = x.numel() // k
+    # torch refuses rows of other lengths
+    if x.shape[-1] == k and (takes_gemm(m, k, n, transposed) or takes_wide_gemm(m, k, n, transposed)):
         return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
     return torch.matmul(x, w.t() if transposed else w)
 

@@ -975,6 +975,25 @@ def test_prompt_product_edges(hip, m, k, n, tile, transposed):
 
 @requires_gpu
 @pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("tile", [0, 4, 5, 6, 7])  # 128, 256, 192, 160 and 96 rows
+@pytest.mark.parametrize(
+    "m,k,n",
+    [
+        (1, 64, 16),  # one step, two groups of columns
+        (95, 128, 272),  # a row less than a tile, two steps; 16 columns beyond a tile
+        (193, 192, 528),  # a row beyond, as many steps as stages
+        (257, 2112, 304),  # parts along K, the last one shorter, of two tiles of columns
+        (2049, 256, 1040),  # bands of rows, the last one shorter
+        (4100, 64, 4112),  # the same with whole turns of workgroups and some left over
+        (1030, 1088, 4624),  # left over, in parts
+    ],
+)
+def test_prompt_products_of_four_waves(hip, m, k, n, tile, transposed):
+    test_prompt_product_edges(hip, m, k, n, tile, transposed)
+
+
+@requires_gpu
+@pytest.mark.parametrize("transposed", [False, True])
 @pytest.mark.parametrize("m,k,n", [(40, 128, 128), (70, 1024, 320)])  # whole sums, and in parts
 def test_prompt_products_of_extreme_values(hip, m, k, n, transposed):
     """Infinities, NaNs and large values stay in their rows and columns, and activations and
