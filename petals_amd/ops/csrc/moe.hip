@@ -17,9 +17,8 @@
 // token); experts whose rows are aligned to 16 bytes take gemv_mfma.h's.
 
 #include "common.h"
+#include "gemm_wide.h"
 #include "gemv_mfma.h"
-#include "gemv_reduce.h"
-#include "paged.h"
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 
@@ -275,6 +274,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
 // pairs by expert with each expert's segment padded to a multiple of MT rows, so every
 // MT-row tile belongs to ONE expert (tile_expert[tile], -1 = pure padding).
 //
+// NF4 weights, and bf16 beyond offsets of 32 bits (the others: moe_wide_kernel below).
 // Up to four tiles of one expert (128 rows) and 256 columns are a workgroup's: an
 // expert's weights are read once per 128 of its rows, and the rows once per 256 columns.
 // With a tile of 32 rows and 128 columns each, weights crossed the caches four times as
@@ -542,6 +542,100 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_kernel(
   }
 }
 
+// bf16 weights, rows in groups of up to 256 that are as equal as tiles of 32 allow, by gemm_wide.h: two groups of 145
+// rows are two tiles of 160 where groups of 128 rows were three, the last one nearly empty, and four waves take less
+// from LDS for a product. Both products of a layer of 8 experts, width 4096 and inner size 14336, with 290 rows an expert
+// and routing as it comes: from 698 and 405 to 571 and 310 us. With 71 rows weights are what bounds either (5.0 TB/s).
+struct MoeGroup {
+  int tile, tiles, column;  // first tile and number of tiles (0: none); run of columns
+};
+// as moe_spot, with groups of up to `most` tiles
+__device__ __forceinline__ MoeGroup moe_group_spot(const int* __restrict__ tile_expert, int n_tiles, int slot, int columns, int most) {
+  const int lane = threadIdx.x & (WAVE - 1), which = slot / columns;
+  int seen = 0, open = 0, open_expert = -1;  // groups so far; first tile of the run that is not closed yet, and whose
+  for (int base = 0; base <= n_tiles; base += WAVE) {
+    const int i = base + lane;
+    const int e = i < n_tiles ? tile_expert[i] : -1;
+    const int before = i > 0 && i <= n_tiles ? tile_expert[i - 1] : -1;
+    const unsigned long long starts = __ballot(i <= n_tiles && (e != before || i == 0 || i == n_tiles));
+    if (starts == 0) continue;
+    // a run counts where it is closed: at the next one's start. Lane l has the run that ends at start l
+    const bool closes = (starts >> lane) & 1;
+    const unsigned long long below = starts & ((1ull << lane) - 1);
+    const int from = below ? WAVE - 1 - __clzll((long long)below) : -1;
+    const int run_expert = __shfl(e, max(from, 0));
+    const int first = from >= 0 ? base + from : open, expert = from >= 0 ? run_expert : open_expert;
+    const int length = closes && expert >= 0 ? i - first : 0, groups = (length + most - 1) / most;
+    int upto = groups;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const int other = __shfl_up(upto, off);
+      if (lane >= off) upto += other;
+    }
+    const unsigned long long here = __ballot(which < seen + upto);
+    if (here) {
+      const int at = __ffsll((long long)here) - 1;
+      const int n = __shfl(groups, at), start = __shfl(first, at), size = __shfl(length, at), ahead = seen + __shfl(upto, at) - n;
+      const int chunk = (which - ahead) & ~(MOE_SHARE - 1), share = min(MOE_SHARE, n - chunk);
+      const int r = slot - columns * (ahead + chunk), group = chunk + r % share;
+      const int each = size / n, more = size % n;  // the first `more` groups have one tile more
+      return {start + group * each + min(group, more), each + (group < more), r / share};
+    }
+    seen += __shfl(upto, WAVE - 1);
+    const int last = WAVE - 1 - __clzll((long long)starts);
+    open = base + last;
+    open_expert = __shfl(e, last);
+  }
+  return {-1, 0, 0};
+}
+
+template <int TILES>
+__device__ __forceinline__ void moe_wide_tile(
+    unsigned char* lds, const unsigned short* w, const unsigned short* x, const int* pairs, unsigned short* c, int n0, int tokens,
+    int in_dim, int out_dim, int k_per_tok) {
+  constexpr int WR = TILES > 5 ? 2 : 1, FM = 2 * TILES / WR;
+  f32x4 acc[WideTile<false, WR, FM>::FN][FM];
+  wide_product<false, WR, FM>(
+      lds, acc, wide_resource(x, (unsigned)tokens * in_dim * 2), wide_resource(w, (unsigned)in_dim * out_dim * 2),
+      [&](int row) { return (unsigned)(max(pairs[row], 0) / k_per_tok) * in_dim * 2; },
+      [&](int column) { return (unsigned)min(n0 + column, out_dim - 8); }, (unsigned)out_dim * 2, 0, in_dim / MOE_BK);
+  const int row = wide_row<false, WR, FM>(), n = n0 + wide_column<false, WR, FM>();
+  int pr[FM];
+#pragma unroll
+  for (int j = 0; j < FM; ++j) pr[j] = pairs[row + j * 16];
+  wide_store<false, WR, FM>(false, acc, [](auto) {}, [&](auto j, auto i, float (&v)[8], float (&)[8]) {
+    if (pr[j] >= 0 && n + i * 32 < out_dim) store8(c + (size_t)pr[j] * out_dim + n + i * 32, v);
+  });
+}
+
+__global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void moe_wide_kernel(
+    const unsigned short* __restrict__ wt_all, const unsigned short* __restrict__ x, const int* __restrict__ sorted_pairs,
+    const int* __restrict__ tile_expert, unsigned short* __restrict__ c, int tokens, int in_dim, int out_dim, int k_per_tok,
+    int n_tiles, int experts, int columns, int most) {
+  extern __shared__ __align__(1024) unsigned char smem[];
+  const MoeGroup spot = moe_group_spot(tile_expert, n_tiles, blockIdx.x >> 3, columns, most);
+  const int tiles = __builtin_amdgcn_readfirstlane(spot.tiles), tile = __builtin_amdgcn_readfirstlane(spot.tile);
+  const int n0 = __builtin_amdgcn_readfirstlane(spot.column * 8 + (blockIdx.x & 7)) * MOE_BN;
+  if (tiles == 0 || n0 >= out_dim) return;
+  const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]);
+  if (e >= experts) return;
+  const unsigned short* w = wt_all + (size_t)e * in_dim * out_dim;
+  const int* pairs = sorted_pairs + tile * MOE_MT;
+#define MOE_TILES(N) \
+  case N: moe_wide_tile<N>(smem, w, x, pairs, c, n0, tokens, in_dim, out_dim, k_per_tok); break
+  switch (tiles) {
+    MOE_TILES(1);
+    MOE_TILES(2);
+    MOE_TILES(3);
+    MOE_TILES(4);
+    MOE_TILES(5);
+    MOE_TILES(6);
+    MOE_TILES(7);
+    MOE_TILES(8);
+  }
+#undef MOE_TILES
+}
+
 // ------------------------------------------------------------------- host
 
 // x [T, dim] f32 or bf16, w [experts, dim] bf16 -> (weights [T, top] f32, experts [T, top] int32): the
@@ -610,6 +704,30 @@ std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t
   return {pairs, tiles};
 }
 
+// Most tiles of a group, 3 to 8: as many as possible, as a step of 64 of K takes about 0.35 us and 0.115 for each tile (what
+// its weights take to come is shared by all), but with few columns a turn of all compute units is as long as its
+// largest group. What routing gives is not known here: experts have 0.8 to 1.2 times the mean.
+static int moe_most_tiles(long pairs, long experts, long columns) {
+  int best = 8;
+  float least = 0.f;
+  for (int most = 8; most >= 3; --most) {
+    float sum = 0.f, longest = 0.f;
+    long units = 0;
+    for (int i = 0; i < 5; ++i) {
+      const long tiles = std::max(1L, (long)std::ceil((0.8f + 0.1f * i) * pairs / experts / MOE_MT));
+      const long groups = (tiles + most - 1) / most, largest = (tiles + groups - 1) / groups;
+      const float us = std::max(0.62f, 0.35f + 0.115f * largest);
+      units += groups;
+      sum += us * groups;
+      longest = std::max(longest, us);
+    }
+    const float turns = (float)units * experts * columns / 5 / GEMM_CUS;
+    const float us = turns < 4 ? std::ceil(turns) * longest : sum * experts * columns / 5 / GEMM_CUS + longest / 2;
+    if (most == 8 || us < 0.99f * least) best = most, least = us;
+  }
+  return best;
+}
+
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all,      // [E, in, out] bf16
     c10::optional<torch::Tensor> nf4_all,     // NF4: [E, out/64, ceil(in/128), 4, 64, 16] u8
@@ -649,6 +767,23 @@ torch::Tensor moe_gemm(
 
   auto c = torch::empty({n_rows, (long)out_dim}, x.options());
   const long n_tiles = Rp / MOE_MT, experts = nf4 ? nf4_all->size(0) : wt_all->size(0);
+  // offsets into an expert's weights and into rows are 32-bit there
+  if (!nf4 && (long)in_dim * out_dim < (1L << 31) && x.size(0) * in_dim < (1L << 31)) {
+    const long runs = (out_dim + MOE_BN - 1) / MOE_BN, columns = (runs + 7) / 8;
+    const int most = moe_most_tiles(n_rows, experts, runs);
+    const long groups = std::min(n_tiles, (n_tiles + (most - 1) * experts) / most), blocks = groups * columns * 8;
+    if (groups == 0 || x.size(0) == 0) return c;
+    TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
+    constexpr int lds = std::max(WideTile<false, 2, 8>::LDS, std::max(WideTile<false, 1, 10>::LDS, WideTile<false, 2, 6>::LDS));
+    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_wide_kernel),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));
+    moe_wide_kernel<<<blocks, WIDE_THREADS, lds, at::cuda::getCurrentCUDAStream()>>>(
+        BF16P(*wt_all), BF16P(x), sorted_pairs.data_ptr<int>(), tile_expert.data_ptr<int>(), BF16P(c), (int)x.size(0), in_dim,
+        out_dim, (int)k_per_tok, (int)n_tiles, (int)experts, (int)columns, most);
+    HIP_CHECK_LAST();
+    return c;
+  }
   // an expert's last group may have one tile
   constexpr long per = MOE_BM / MOE_MT;
   const long groups = std::min(n_tiles, (n_tiles + (per - 1) * experts) / per);

@@ -74,6 +74,37 @@ def test_expert_gemm_group_edges(hip, quant, counts, k_in, n_out):
 
 
 @requires_gpu
+@pytest.mark.parametrize(
+    "counts,k_in,n_out",
+    [
+        ([1, 33, 65, 97, 129, 161, 193, 225], 64, 384),  # groups of 1 to 8 tiles, of one row more than the tile before
+        ([256, 257, 0, 480, 512, 513], 128, 256),  # around one and two full groups, an empty expert between
+        ([290] * 8, 192, 4096),  # smaller groups, as few columns are
+        ([40, 0, 700, 31] * 20, 64, 2176),  # runs that end in another chunk of tiles than they start in
+        ([3000], 256, 128),  # a run of one expert longer than a wave's lanes
+    ],
+)
+def test_expert_gemm_equal_groups(hip, counts, k_in, n_out):
+    """Rows of an expert in groups that are as equal as tiles of 32 allow, two rows a token."""
+    from petals_amd.ops.fused_moe import MOE_GEMM_MT
+
+    gen = torch.Generator(device="cuda").manual_seed(len(counts) + n_out)
+    w = (torch.randn(len(counts), k_in, n_out, device="cuda", generator=gen) * 0.05).to(BF16)
+    pairs = torch.cat([torch.full((n,), e, device="cuda", dtype=torch.int32) for e, n in enumerate(counts)])
+    pairs = pairs[torch.randperm(len(pairs), device="cuda", generator=gen)]
+    x = torch.randn((len(pairs) + 1) // 2, k_in, device="cuda", generator=gen).to(BF16)
+    order, tiles = hip.moe_group(pairs, len(counts), MOE_GEMM_MT)
+    out = hip.moe_gemm(w, None, None, x, order, tiles, 2, len(pairs)).double()
+    rows = x.double().repeat_interleave(2, 0)[: len(pairs)]
+    for e in range(len(counts)):
+        mine, we = pairs == e, w[e].double()
+        ref = rows[mine] @ we
+        # 32-bit sums of exact products of bf16, rounded once
+        bound = 2.0**-8 * ref.abs() + k_in * 2.0**-24 * (rows[mine].abs() @ we.abs())
+        assert bool(((out[mine] - ref).abs() <= bound).all()), e
+
+
+@requires_gpu
 def test_gelu_over_all_of_bf16(hip):
     """GELU of every finite bf16 number, infinities and NaN, beside 64 bits."""
     x = torch.arange(1 << 16, device="cuda", dtype=torch.int32).to(torch.int16).view(BF16)
