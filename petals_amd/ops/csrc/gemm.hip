@@ -227,20 +227,20 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_kernel(
 
 // ------------------------------------------------------- tiles of four waves
 
-// rows of 16 of a tile of 256 columns. Two rows of waves read less from LDS where rows are many; W [K, N] with few
+// rows and columns of 16 of a tile. Two rows of waves read less from LDS where rows are many; W [K, N] with few
 // rows is 5% faster with one (758 x 4096 x 22016 in tiles of 160 rows: 134.7 us, 143)
-template <bool WT, int ROWS>
+template <bool WT, int ROWS, int COLUMNS>
 struct WideGemm {
-  static constexpr int WR = ROWS % 2 == 0 && (WT || ROWS > 10) ? 2 : 1, FM = ROWS / WR;
-  using Tile = WideTile<WT, WR, FM>;
+  static constexpr int WR = ROWS % 2 == 0 && (WT || ROWS > 10 || COLUMNS % 8) ? 2 : 1, FM = ROWS / WR, FN = COLUMNS * WR / 4;
+  using Tile = WideTile<WT, WR, FM, FN>;
 };
 
-template <bool WT, int ROWS>
+template <bool WT, int ROWS, int COLUMNS>
 __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_wide_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, GemmShape s, GemmOut o) {
-  using Gemm = WideGemm<WT, ROWS>;
+  using Gemm = WideGemm<WT, ROWS, COLUMNS>;
   using Tile = typename Gemm::Tile;
-  constexpr int FM = Gemm::FM, FN = Tile::FN, BM = Tile::BM, BN = Tile::BN;
+  constexpr int FM = Gemm::FM, FN = Gemm::FN, BM = Tile::BM, BN = Tile::BN;
   extern __shared__ __align__(1024) unsigned char gemm_lds[];
   GemmSpot spot;
   if (!gemm_spot(s, s.k / GEMM_BK, &spot)) return;
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu
   const GemmPlace place = gemm_place<BN>(s, spot.tile);
   const int m0 = place.row * BM, column_tile = place.column;
   f32x4 acc[FN][FM];
-  wide_product<WT, Gemm::WR, FM>(
+  wide_product<WT, Gemm::WR, FM, FN>(
       gemm_lds, acc, wide_resource(x, (unsigned)s.m * s.k * 2), wide_resource(w, (unsigned)s.k * s.n * 2),
       [&](int row) { return (unsigned)min(m0 + row, s.m - 1) * s.k * 2; },
       [&](int c) { return (unsigned)min(gemm_source_column<FN>(column_tile, c, BN, s.n, pairs), s.n - (WT ? 1 : 8)); },
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu
     return;
   }
   // loads of residuals that follow stores wait for a trip to memory each: 16 to 32 of them
-  const int row = m0 + wide_row<WT, Gemm::WR, FM>(), c = wide_column<WT, Gemm::WR, FM>();
+  const int row = m0 + wide_row<WT, Gemm::WR, FM, FN>(), c = wide_column<WT, Gemm::WR, FM, FN>();
   int n[FN / 2];
   Gemm8 bias[FN / 2] = {}, residual[2][FN / 2] = {};
 #pragma unroll
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu
     n[i] = gemm_source_column<FN>(column_tile, c + i * 32, BN, s.n, pairs);
     if (o.bias) bias[i] = gemm_load8(o.bias + min(n[i], s.n - 8));
   }
-  wide_store<WT, Gemm::WR, FM>(
+  wide_store<FM, FN>(
       pairs, acc,
       [&](auto j) {
         if (o.residual)
@@ -290,11 +290,11 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu
 }
 
 // parts [splits, rest, waves, FM, FN, 64, 4]: two fragments, with pairs four, per thread
-template <bool WT, int ROWS>
+template <bool WT, int ROWS, int COLUMNS>
 __global__ __launch_bounds__(256) void gemm_wide_parts_kernel(GemmShape s, GemmOut o) {
-  using Gemm = WideGemm<WT, ROWS>;
+  using Gemm = WideGemm<WT, ROWS, COLUMNS>;
   using Tile = typename Gemm::Tile;
-  constexpr int FM = Gemm::FM, FN = Tile::FN, BM = Tile::BM, BN = Tile::BN;
+  constexpr int FM = Gemm::FM, FN = Gemm::FN, BM = Tile::BM, BN = Tile::BN;
   const bool pairs = o.epilogue == GEMM_SWIGLU;
   const int unit = __builtin_amdgcn_readfirstlane((blockIdx.x * 256 + threadIdx.x) / WAVE), lane = threadIdx.x & (WAVE - 1);
   const int each = pairs ? FN / 4 : FN / 2, i = unit % each * 2, j = unit / each % FM, wave = unit / each / FM % 4;
@@ -324,17 +324,17 @@ __global__ __launch_bounds__(256) void gemm_wide_parts_kernel(GemmShape s, GemmO
   }
 }
 
-template <bool WT, int ROWS>
+template <bool WT, int ROWS, int COLUMNS>
 static void launch_gemm_wide(const unsigned short* x, const unsigned short* w, const GemmShape& s, const GemmOut& o, long blocks, hipStream_t stream) {
-  using Tile = typename WideGemm<WT, ROWS>::Tile;
-  const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WT, ROWS>),
+  using Tile = typename WideGemm<WT, ROWS, COLUMNS>::Tile;
+  const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<WT, ROWS, COLUMNS>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, Tile::LDS);
   TORCH_CHECK(fits == hipSuccess, "gemm_rows: ", hipGetErrorString(fits));
-  gemm_wide_kernel<WT, ROWS><<<blocks, WIDE_THREADS, Tile::LDS, stream>>>(x, w, s, o);
+  gemm_wide_kernel<WT, ROWS, COLUMNS><<<blocks, WIDE_THREADS, Tile::LDS, stream>>>(x, w, s, o);
   HIP_CHECK_LAST();
   if (s.splits > 1) {
     const long threads = (long)s.rest * Tile::BM * Tile::BN / (o.epilogue == GEMM_SWIGLU ? 16 : 8);
-    gemm_wide_parts_kernel<WT, ROWS><<<(threads + 255) / 256, 256, 0, stream>>>(s, o);
+    gemm_wide_parts_kernel<WT, ROWS, COLUMNS><<<(threads + 255) / 256, 256, 0, stream>>>(s, o);
     HIP_CHECK_LAST();
   }
 }
@@ -345,7 +345,13 @@ static void launch_gemm_wide(const unsigned short* x, const unsigned short* w, c
 // the mean; the tile that they choose takes 1.1% more than the best one
 static const GemmTile GEMM_TILES[] = {{128, 256, 0.83f, 4.6f, 0.72f}, {128, 128, 0.54f, 2.2f, 0.81f}, {64, 256, 0.66f, 6.f, 0.88f},
                                       {32, 256, 0.57f, 3.7f, 1.f},    {256, 256, 1.42f, 2.f, 0.68f},  {192, 256, 1.15f, 2.7f, 0.69f},
-                                      {160, 256, 0.94f, 4.4f, 0.65f}, {96, 256, 0.74f, 3.9f, 0.82f}};
+                                      {160, 256, 0.94f, 4.4f, 0.65f}, {96, 256, 0.74f, 3.9f, 0.82f}, {128, 192, 0.72f, 4.4f, 0.7f}};
+
+// Matrices of up to 25 million weights (4096 x 6144): tiles beyond these gain up to 4 us of 40 there, and would split other sums
+// along K. A sum in another order is rounded otherwise now and then, which for the products ahead of routed experts (8 experts
+// of width 4096 among them) sends a token to another of two nearly equal experts. Sizes that are no multiples of 128
+// gain a third and have no such models.
+static const GemmTile GEMM_SMALL[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
 
 // x [M, K] bf16, w [K, N] (or [N, K], transposed) bf16 -> [M, N] bf16 (swiglu: [M, N/2])
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
@@ -375,16 +381,19 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
                 bias->numel() == n && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 8 == 0);
     o.bias = BF16P(*bias);
   }
+  const bool small = tile < 0 && k * n <= 3L << 23 && k % 128 == 0 && n % 128 == 0;
+  const int usable = small ? (int)(sizeof(GEMM_SMALL) / sizeof(GemmTile)) : (int)(sizeof(GEMM_TILES) / sizeof(GemmTile));
   int best = 0;
   float least = 0.f;
   GemmShape s{};
   for (int i = 0; i < (int)(sizeof(GEMM_TILES) / sizeof(GemmTile)); ++i) {
-    if (tile >= 0 && tile != i) continue;
+    if (tile >= 0 ? tile != i : i >= usable || (pairs && GEMM_TILES[i].bn == 192)) continue;
     float us;
-    const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, GEMM_TILES[i], &us);
+    const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, small ? GEMM_SMALL[i] : GEMM_TILES[i], &us);
     if (s.m == 0 || us < least) best = i, least = us, s = p;
   }
   const GemmTile& t = GEMM_TILES[best];
+  TORCH_CHECK(s.m && !(pairs && t.bn == 192), "gemm_rows: no such tile");  // 96 gates would not be whole pairs of fragments
   torch::Tensor parts;
   if (s.splits > 1) {
     parts = torch::empty({(long)s.splits * s.rest * t.bm * t.bn}, x.options().dtype(torch::kFloat32));
@@ -413,21 +422,22 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
     if (transposed) GEMM(true, __VA_ARGS__);   \
     else GEMM(false, __VA_ARGS__);             \
   } while (0)
-#define GEMM_WIDE(ROWS)                                                                             \
+#define GEMM_WIDE(ROWS, COLUMNS)                                                                             \
   do {                                                                                              \
-    TORCH_CHECK(ROWS * 16 == t.bm);                                                                 \
-    if (transposed) launch_gemm_wide<true, ROWS>(BF16P(x), BF16P(w), s, o, blocks, stream);         \
-    else launch_gemm_wide<false, ROWS>(BF16P(x), BF16P(w), s, o, blocks, stream);                   \
+    TORCH_CHECK(ROWS * 16 == t.bm && COLUMNS * 16 == t.bn);                                                          \
+    if (transposed) launch_gemm_wide<true, ROWS, COLUMNS>(BF16P(x), BF16P(w), s, o, blocks, stream);         \
+    else launch_gemm_wide<false, ROWS, COLUMNS>(BF16P(x), BF16P(w), s, o, blocks, stream);                   \
   } while (0)
   switch (best) {
     case 1: GEMM_EITHER(2, 4, 4, 2, 4); break;
     case 2: GEMM_EITHER(2, 4, 2, 4, 4); break;
     case 3: GEMM_EITHER(1, 8, 2, 2, 4); break;
-    case 0: GEMM_WIDE(8); break;
-    case 4: GEMM_WIDE(16); break;
-    case 5: GEMM_WIDE(12); break;
-    case 6: GEMM_WIDE(10); break;
-    case 7: GEMM_WIDE(6); break;
+    case 0: GEMM_WIDE(8, 16); break;
+    case 4: GEMM_WIDE(16, 16); break;
+    case 5: GEMM_WIDE(12, 16); break;
+    case 6: GEMM_WIDE(10, 16); break;
+    case 7: GEMM_WIDE(6, 16); break;
+    case 8: GEMM_WIDE(8, 12); break;
   }
 #undef GEMM_WIDE
 #undef GEMM_EITHER

@@ -38,13 +38,13 @@ __device__ __forceinline__ void wide_each(F&& f) {
 }
 
 // WR x 4 / WR waves of 16 FM rows and 16 FN columns
-template <bool WT, int WR, int FM>
+template <bool WT, int WR, int FM, int FN>
 struct WideTile {
-  static constexpr int WC = 4 / WR, FN = 16 / WC, BM = WR * FM * 16, BN = 256, BK = 64;
+  static constexpr int WC = 4 / WR, BM = WR * FM * 16, BN = WC * FN * 16, BK = 64;
   static constexpr int XB = BM * BK * 2, WB = BN * BK * 2;                           // bytes of a stage
   static constexpr int SX = 3, SW = SX * XB + 3 * WB <= 160 * 1024 ? 3 : 2;          // stages
   static constexpr int LDS = SX * XB + SW * WB;
-  static_assert(FM * FN <= 64 && LDS <= 160 * 1024);
+  static_assert(FM * FN <= 64 && FN % 2 == 0 && LDS <= 160 * 1024);
 };
 
 // sums past the 56th are in ordinary registers: with all 64 x 4 in the accumulation registers none is left to
@@ -70,33 +70,39 @@ __device__ __forceinline__ gemm_rsrc wide_resource(const void* p, unsigned bytes
 
 // byte offset of 16-byte group c in a row of 128 bytes, and what is added to the group in a row of W [K, N]
 __device__ __forceinline__ int wide_group(int row, int c) { return row * 128 + ((c ^ (row & 7)) << 4); }
-__device__ __forceinline__ int wide_swizzle(int row) { return ((row & 3) | ((row >> 1) & 4)) << 1; }
+template <int BN>
+__device__ __forceinline__ int wide_swizzle(int row) {
+  static_assert(BN % 64 == 0 && BN >= 128);
+  constexpr int GROUPS = BN % 128 ? 8 : 16;  // that are permuted among themselves
+  return ((row & 3) | ((row >> 1) & 4)) << 1 & (GROUPS - 1);
+}
 
 // acc[i][j]: sums of `steps` steps from `first` on; 4 neighbouring columns, hi * 4 of fragment i, of row lane % 16 of
 // fragment j. x_row(row of the tile): byte offset of that row in x. w_at(c): which column of W the tile's c is;
 // for W [K, N] c is a multiple of 8 and so are 8 columns there. row_bytes: of a row of W.
-template <bool WT, int WR, int FM, class XRow, class WAt>
+template <bool WT, int WR, int FM, int FN, class XRow, class WAt>
 __device__ __forceinline__ void wide_product(
-    unsigned char* lds, f32x4 (&acc)[WideTile<WT, WR, FM>::FN][FM], gemm_rsrc xr, gemm_rsrc wr, XRow x_row, WAt w_at,
+    unsigned char* lds, f32x4 (&acc)[FN][FM], gemm_rsrc xr, gemm_rsrc wr, XRow x_row, WAt w_at,
     unsigned row_bytes, int first, int steps) {
-  using Tile = WideTile<WT, WR, FM>;
-  constexpr int WC = Tile::WC, FN = Tile::FN, BK = Tile::BK, BN = Tile::BN, XB = Tile::XB, WB = Tile::WB, SX = Tile::SX, SW = Tile::SW;
+  using Tile = WideTile<WT, WR, FM, FN>;
+  constexpr int WC = Tile::WC, BK = Tile::BK, BN = Tile::BN, XB = Tile::XB, WB = Tile::WB, SX = Tile::SX, SW = Tile::SW;
   constexpr int G = 2 * FM;                                                      // groups of a step
   constexpr int WIN = G <= 8 ? G : G % 8 == 0 ? 8 : G % 10 == 0 ? 10 : G % 7 == 0 ? 7 : 6;  // fragments of X
   static_assert(G % WIN == 0);
-  constexpr int D = WR == 2 ? 3 : WIN == 6 ? 4 : FM < 6 ? FM : 6;                // groups that they are read ahead
+  // groups that they are read ahead: some 24 products
+  constexpr int AHEAD = (24 + FN - 1) / FN, D = AHEAD < FM && AHEAD < WIN - 1 ? AHEAD : FM < WIN - 1 ? FM : WIN - 2 > 0 ? WIN - 2 : 1;
   static_assert(D < WIN && D <= FM);
   constexpr int XL = XB / 4096, WL = WB / 4096;                                   // loads of 1 KB of a step, per wave
-  constexpr int XA = WT ? XL : (XL + 1) / 2, WA = WT ? 0 : 4;                     // of its first half
+  constexpr int XA = WT ? XL : (XL + 1) / 2, WA = WT ? 0 : WL / 2;                    // of its first half
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid & (WAVE - 1);
   const int col = lane & 15, hi = lane >> 4;
   const int wm = wave / WC * FM * 16, wn = wave % WC * FN * 16;
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds, wbase = base + SX * XB;
 
-  // a load's place in its stage; a wave's first four of W [K, N] are of the first 32 rows
+  // a load's place in its stage; the first half of a wave's loads of W [K, N] are of the first 32 rows
   auto x_load = [&](int i) { return wave * XL + i; };
-  auto w_load = [&](int i) { return WT ? wave * WL + i : i / 4 * 16 + wave * 4 + i % 4; };
+  auto w_load = [&](int i) { return WT ? wave * WL + i : i / (WL / 2) * (WL * 2) + wave * (WL / 2) + i % (WL / 2); };
   unsigned x_lane[XL], w_lane[WL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
@@ -107,7 +113,7 @@ __device__ __forceinline__ void wide_product(
   for (int i = 0; i < WL; ++i) {
     const int p = w_load(i) * 64 + lane, row = p / (WT ? 8 : BN / 8);
     w_lane[i] = WT ? w_at(row) * row_bytes + (p % 8 ^ (row & 7)) * 16
-                   : row * row_bytes + w_at((p % (BN / 8) ^ wide_swizzle(row)) * 8) * 2;
+                   : row * row_bytes + w_at((p % (BN / 8) ^ wide_swizzle<BN>(row)) * 8) * 2;
   }
   const unsigned w_step = WT ? BK * 2 : BK * row_bytes;
   auto load = [&](unsigned to, unsigned from, gemm_rsrc r, unsigned at) {
@@ -138,7 +144,7 @@ __device__ __forceinline__ void wide_product(
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
       const int row = hi * 8 + col / 4, c = (wn + i * 16) / 8 + ((col >> 1) & 1);
-      wa[i] = wbase + row * (BN * 2) + ((c ^ wide_swizzle(row)) << 4) + (col & 1) * 8;
+      wa[i] = wbase + row * (BN * 2) + ((c ^ wide_swizzle<BN>(row)) << 4) + (col & 1) * 8;
     }
   bf16x8 wf[2][FN], xf[WIN];
   auto read_x = [&](unsigned from, int g) { xf[g % WIN] = *(lds_frag*)(size_t)(xa[g / FM] + from + g % FM * (16 * 128)); };
@@ -240,28 +246,28 @@ __device__ __forceinline__ void wide_join(f32x4 a, f32x4 b, float (&v)[8]) {
 }
 
 // a lane's row and column of a wave's tile, for the first of its groups of 8 columns
-template <bool WT, int WR, int FM>
+template <bool WT, int WR, int FM, int FN>
 __device__ __forceinline__ int wide_row() {
-  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / WideTile<WT, WR, FM>::WC * FM * 16 + (threadIdx.x & 15);
+  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / WideTile<WT, WR, FM, FN>::WC * FM * 16 + (threadIdx.x & 15);
 }
-template <bool WT, int WR, int FM>
+template <bool WT, int WR, int FM, int FN>
 __device__ __forceinline__ int wide_column() {
-  using Tile = WideTile<WT, WR, FM>;
+  using Tile = WideTile<WT, WR, FM, FN>;
   const int hi = (threadIdx.x & (WAVE - 1)) >> 4;
-  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % Tile::WC * Tile::FN * 16 + (hi & 1) * 16 + (hi >> 1) * 8;
+  return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % Tile::WC * FN * 16 + (hi & 1) * 16 + (hi >> 1) * 8;
 }
 
 // store(j, i, 8 values) for all of a lane's groups: of row wide_row() + 16 j and columns from wide_column() + 32 i on.
 // `pairs`: store(j, i, gates, ups), the first half of a wave's columns being gates. ahead(j) is called a row
 // earlier: what it loads is on its way while that one is stored.
-template <bool WT, int WR, int FM, class Ahead, class Store>
-__device__ __forceinline__ void wide_store(bool pairs, f32x4 (&acc)[WideTile<WT, WR, FM>::FN][FM], Ahead ahead, Store store) {
-  constexpr int FN = WideTile<WT, WR, FM>::FN;
+template <int FM, int FN, class Ahead, class Store>
+__device__ __forceinline__ void wide_store(bool pairs, f32x4 (&acc)[FN][FM], Ahead ahead, Store store) {
   ahead(std::integral_constant<int, 0>{});
   wide_each<FM>([&](auto j) {
     if constexpr (j + 1 < FM) ahead(std::integral_constant<int, j + 1>{});
     wide_each<FN>([&](auto i) { wide_pin<(j * FN + i < 56)>(acc[i][j]); });
-    if (pairs) {
+    // halves of an odd number of pairs are nobody's: their callers have none
+    if (pairs && FN % 4 == 0) {
       wide_each<FN / 4>([&](auto i) {
         float g[8], u[8];
         wide_join(acc[2 * i][j], acc[2 * i + 1][j], g);

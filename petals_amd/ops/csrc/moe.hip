@@ -589,45 +589,50 @@ __device__ __forceinline__ MoeGroup moe_group_spot(const int* __restrict__ tile_
   return {-1, 0, 0};
 }
 
-template <int TILES>
+// NARROW: 128 columns
+template <int TILES, bool NARROW>
 __device__ __forceinline__ void moe_wide_tile(
     unsigned char* lds, const unsigned short* w, const unsigned short* x, const int* pairs, unsigned short* c, int n0, int tokens,
     int in_dim, int out_dim, int k_per_tok) {
-  constexpr int WR = TILES > 5 ? 2 : 1, FM = 2 * TILES / WR;
-  f32x4 acc[WideTile<false, WR, FM>::FN][FM];
-  wide_product<false, WR, FM>(
+  constexpr int WR = NARROW || TILES > 5 ? 2 : 1, FM = 2 * TILES / WR, FN = NARROW ? 4 : 4 * WR;
+  f32x4 acc[FN][FM];
+  wide_product<false, WR, FM, FN>(
       lds, acc, wide_resource(x, (unsigned)tokens * in_dim * 2), wide_resource(w, (unsigned)in_dim * out_dim * 2),
       [&](int row) { return (unsigned)(max(pairs[row], 0) / k_per_tok) * in_dim * 2; },
-      [&](int column) { return (unsigned)min(n0 + column, out_dim - 8); }, (unsigned)out_dim * 2, 0, in_dim / MOE_BK);
-  const int row = wide_row<false, WR, FM>(), n = n0 + wide_column<false, WR, FM>();
+      [&](int column) { return (unsigned)min(n0 + column, out_dim - 8); },
+      (unsigned)out_dim * 2, 0, in_dim / MOE_BK);
+  const int row = wide_row<false, WR, FM, FN>(), n = n0 + wide_column<false, WR, FM, FN>();
   int pr[FM];
 #pragma unroll
   for (int j = 0; j < FM; ++j) pr[j] = pairs[row + j * 16];
-  wide_store<false, WR, FM>(false, acc, [](auto) {}, [&](auto j, auto i, float (&v)[8], float (&)[8]) {
+  wide_store<FM, FN>(false, acc, [](auto) {}, [&](auto j, auto i, float (&v)[8], float (&)[8]) {
     if (pr[j] >= 0 && n + i * 32 < out_dim) store8(c + (size_t)pr[j] * out_dim + n + i * 32, v);
   });
 }
 
+template <bool NARROW>
 __global__ __launch_bounds__(WIDE_THREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void moe_wide_kernel(
     const unsigned short* __restrict__ wt_all, const unsigned short* __restrict__ x, const int* __restrict__ sorted_pairs,
-    const int* __restrict__ tile_expert, unsigned short* __restrict__ c, int tokens, int in_dim, int out_dim, int k_per_tok,
-    int n_tiles, int experts, int columns, int most) {
+    const int* __restrict__ tile_expert, unsigned short* __restrict__ c, int tokens, int in_dim, int out_dim, int k_per_tok, int n_tiles, int experts,
+    int columns, int most) {
   extern __shared__ __align__(1024) unsigned char smem[];
   const MoeGroup spot = moe_group_spot(tile_expert, n_tiles, blockIdx.x >> 3, columns, most);
   const int tiles = __builtin_amdgcn_readfirstlane(spot.tiles), tile = __builtin_amdgcn_readfirstlane(spot.tile);
-  const int n0 = __builtin_amdgcn_readfirstlane(spot.column * 8 + (blockIdx.x & 7)) * MOE_BN;
+  const int n0 = __builtin_amdgcn_readfirstlane(spot.column * 8 + (blockIdx.x & 7)) * (NARROW ? 128 : 256);
   if (tiles == 0 || n0 >= out_dim) return;
   const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]);
   if (e >= experts) return;
   const unsigned short* w = wt_all + (size_t)e * in_dim * out_dim;
   const int* pairs = sorted_pairs + tile * MOE_MT;
 #define MOE_TILES(N) \
-  case N: moe_wide_tile<N>(smem, w, x, pairs, c, n0, tokens, in_dim, out_dim, k_per_tok); break
+  case N: moe_wide_tile<N, NARROW>(smem, w, x, pairs, c, n0, tokens, in_dim, out_dim, k_per_tok); break
   switch (tiles) {
     MOE_TILES(1);
     MOE_TILES(2);
     MOE_TILES(3);
     MOE_TILES(4);
+  }
+  if constexpr (!NARROW) switch (tiles) {
     MOE_TILES(5);
     MOE_TILES(6);
     MOE_TILES(7);
@@ -728,6 +733,38 @@ static int moe_most_tiles(long pairs, long experts, long columns) {
   return best;
 }
 
+static void launch_moe_wide(const torch::Tensor& wt_all, const torch::Tensor& x, const torch::Tensor& sorted_pairs,
+                            const torch::Tensor& tile_expert, torch::Tensor& c, int64_t k_per_tok, int64_t n_rows) {
+  const long experts = wt_all.size(0), in_dim = wt_all.size(1), out_dim = wt_all.size(2), n_tiles = tile_expert.size(0);
+  if (n_tiles == 0 || x.size(0) == 0) return;
+  // Few rows of few columns leave compute units without a tile of 256 columns, and weights are what is read: 8 experts of
+  // 14336 x 4096 with 71 rows each, 218 us with 128 workgroups, 166 with 256.
+  const long hit = std::min(experts, n_rows), mean = (long)std::ceil(1.2f * n_rows / experts / MOE_MT);
+  const bool narrow = mean <= 4 && hit * ((out_dim + 255) / 256) <= GEMM_CUS * 5 / 8;
+  const long bn = narrow ? 128 : 256, runs = (out_dim + bn - 1) / bn, columns = (runs + 7) / 8;
+  const int most = narrow ? 4 : moe_most_tiles(n_rows, experts, runs);
+  const long groups = std::min(n_tiles, (n_tiles + (most - 1) * experts) / most), blocks = groups * columns * 8;
+  TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
+#define MOE_WIDE(NARROW, LDS)                                                                                           \
+  do {                                                                                                                  \
+    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_wide_kernel<NARROW>),                \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                       \
+    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));                                             \
+    moe_wide_kernel<NARROW><<<blocks, WIDE_THREADS, LDS, at::cuda::getCurrentCUDAStream()>>>(                           \
+        BF16P(wt_all), BF16P(x), sorted_pairs.data_ptr<int>(), tile_expert.data_ptr<int>(), BF16P(c), (int)x.size(0),          \
+        (int)in_dim, (int)out_dim, (int)k_per_tok, (int)n_tiles, (int)experts, (int)columns, most);                     \
+  } while (0)
+  constexpr int WIDE_LDS = std::max(WideTile<false, 2, 8, 8>::LDS, WideTile<false, 1, 10, 4>::LDS);
+  if (narrow) {
+    constexpr int NARROW_LDS = WideTile<false, 2, 4, 4>::LDS;
+    MOE_WIDE(true, NARROW_LDS);
+  } else {
+    MOE_WIDE(false, WIDE_LDS);
+  }
+#undef MOE_WIDE
+  HIP_CHECK_LAST();
+}
+
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all,      // [E, in, out] bf16
     c10::optional<torch::Tensor> nf4_all,     // NF4: [E, out/64, ceil(in/128), 4, 64, 16] u8
@@ -769,19 +806,7 @@ torch::Tensor moe_gemm(
   const long n_tiles = Rp / MOE_MT, experts = nf4 ? nf4_all->size(0) : wt_all->size(0);
   // offsets into an expert's weights and into rows are 32-bit there
   if (!nf4 && (long)in_dim * out_dim < (1L << 31) && x.size(0) * in_dim < (1L << 31)) {
-    const long runs = (out_dim + MOE_BN - 1) / MOE_BN, columns = (runs + 7) / 8;
-    const int most = moe_most_tiles(n_rows, experts, runs);
-    const long groups = std::min(n_tiles, (n_tiles + (most - 1) * experts) / most), blocks = groups * columns * 8;
-    if (groups == 0 || x.size(0) == 0) return c;
-    TORCH_CHECK(blocks < (1L << 31), "moe_gemm: too many rows");
-    constexpr int lds = std::max(WideTile<false, 2, 8>::LDS, std::max(WideTile<false, 1, 10>::LDS, WideTile<false, 2, 6>::LDS));
-    const hipError_t fits = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_wide_kernel),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    TORCH_CHECK(fits == hipSuccess, "moe_gemm: ", hipGetErrorString(fits));
-    moe_wide_kernel<<<blocks, WIDE_THREADS, lds, at::cuda::getCurrentCUDAStream()>>>(
-        BF16P(*wt_all), BF16P(x), sorted_pairs.data_ptr<int>(), tile_expert.data_ptr<int>(), BF16P(c), (int)x.size(0), in_dim,
-        out_dim, (int)k_per_tok, (int)n_tiles, (int)experts, (int)columns, most);
-    HIP_CHECK_LAST();
+    launch_moe_wide(*wt_all, x, sorted_pairs, tile_expert, c, k_per_tok, n_rows);
     return c;
   }
   // an expert's last group may have one tile
