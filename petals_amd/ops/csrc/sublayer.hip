@@ -53,6 +53,72 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 
 // ---------------------------------------------------------- sublayer output
 
+// the router of a row in LDS, by a workgroup
+template <typename TW>
+__device__ __forceinline__ void route_row(
+    const float* row, float* logit, const TW* __restrict__ router, int experts, int top, int* __restrict__ sel,
+    float* __restrict__ sel_w, int dp, size_t t) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  __syncthreads();
+  const int wave = tid / WAVE, lane = tid & (WAVE - 1);
+  // two experts per wave at a time; row and router are zero between d and dp
+  for (int e = wave * 2; e < experts; e += nt / WAVE * 2) {
+    const bool both = e + 1 < experts;
+    float z0 = 0.f, z1 = 0.f;
+    const TW* r0 = router + (size_t)e * dp;
+    const TW* r1 = both ? r0 + dp : r0;
+#pragma unroll 4
+    for (int c = lane * 8; c < dp; c += WAVE * 8) {
+      float w0[8], w1[8];
+      ld8(r0 + c, w0);
+      ld8(r1 + c, w1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        z0 = fmaf(row[c + i], w0[i], z0);
+        z1 = fmaf(row[c + i], w1[i], z1);
+      }
+    }
+    z0 = wave_reduce_sum(z0);
+    z1 = wave_reduce_sum(z1);
+    if (lane == 0) {
+      logit[e] = z0;
+      if (both) logit[e + 1] = z1;
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  float mx = NEG_SENTINEL;
+  for (int e = lane; e < experts; e += WAVE) mx = fmaxf(mx, logit[e]);
+  mx = wave_reduce_max(mx);
+  float sum = 0.f;
+  for (int e = lane; e < experts; e += WAVE) sum += expf(logit[e] - mx);
+  sum = wave_reduce_sum(sum);
+  for (int j = 0; j < top; ++j) {
+    float best = NEG_SENTINEL * 2.f;
+    int arg = experts;
+    for (int e = lane; e < experts; e += WAVE)
+      if (logit[e] > best) {
+        best = logit[e];
+        arg = e;
+      }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const float ob = __shfl_xor(best, off, WAVE);
+      const int oa = __shfl_xor(arg, off, WAVE);
+      if (ob > best || (ob == best && oa < arg)) {
+        best = ob;
+        arg = oa;
+      }
+    }
+    if (arg >= experts) arg = 0;  // logits that compare with nothing (NaN)
+    if (lane == 0) {
+      sel[t * top + j] = arg;
+      sel_w[t * top + j] = expf(best - mx) / sum;
+    }
+    if ((arg & (WAVE - 1)) == lane) logit[arg] = NEG_SENTINEL * 3.f;  // taken; this lane alone reads it
+  }
+}
+
 // One workgroup per token.
 //   y [T*k, ys]     sublayer rows; a token's k rows are summed with slot_w
 //   x [T, dp]       residual before, xo after (null: the norm alone is written)
@@ -112,65 +178,88 @@ __global__ __launch_bounds__(1024) void sublayer_out_kernel(
       *reinterpret_cast<uint2*>(xb + t * dp + c) = w;
     }
   }
-  if (!router) return;
-  __syncthreads();
-  const int wave = tid / WAVE, lane = tid & (WAVE - 1);
-  // two experts per wave at a time; row and router are zero between d and dp
-  for (int e = wave * 2; e < experts; e += nt / WAVE * 2) {
-    const bool both = e + 1 < experts;
-    float z0 = 0.f, z1 = 0.f;
-    const TW* r0 = router + (size_t)e * dp;
-    const TW* r1 = both ? r0 + dp : r0;
-#pragma unroll 4
-    for (int c = lane * 8; c < dp; c += WAVE * 8) {
-      float w0[8], w1[8];
-      ld8(r0 + c, w0);
-      ld8(r1 + c, w1);
+  if (router) route_row(row, logit, router, experts, top, sel, sel_w, dp, t);
+}
+
+// The same for aligned rows of up to 256 x 8 G values, which stay in registers: what the norm needs (the residual, its
+// weight) is on its way while rows are summed, and only a router reads the row from LDS. 1161 rows of 4096, us: with a router of 8 experts
+// 27.9 to 21.7, weighted sums of two 17.3 to 10.9 (6 TB/s); 4096 rows 69.7 to 56.0, 40.7 to 31.1. The same bits.
+template <typename TY, typename TW, int G>
+__global__ __launch_bounds__(256, G > 2 ? 3 : 6) void sublayer_out_rows_kernel(
+    const TY* __restrict__ y, int ys, int k, const float* __restrict__ slot_w,
+    const float* __restrict__ norm_w, float eps,
+    const float* __restrict__ x, float* __restrict__ xo, unsigned short* __restrict__ xb,
+    const TW* __restrict__ router, int experts, int top, int* __restrict__ sel, float* __restrict__ sel_w, int d) {
+  extern __shared__ float sm[];
+  __shared__ float red[16];
+  const int tid = threadIdx.x;
+  const size_t t = blockIdx.x;
+  float v[G][8], w[G][8], r[G][8], u[2][G][8];
+  int at[G];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        z0 = fmaf(row[c + i], w0[i], z0);
-        z1 = fmaf(row[c + i], w1[i], z1);
-      }
+  for (int g = 0; g < G; ++g) at[g] = min((g * 256 + tid) * 8, d - 8);
+  auto load_y = [&](int j, int to) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) ld8(y + (t * k + j) * ys + at[g], u[to][g]);
+  };
+  auto add_y = [&](int j, int from) {
+    const float s = slot_w ? slot_w[t * k + j] : 1.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[g][i] = fmaf(s, u[from][g][i], v[g][i]);
+  };
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[g][i] = 0.f;
+  load_y(0, 0);
+  if (k > 1) load_y(1, 1);
+#pragma unroll
+  for (int g = 0; g < G; ++g) ld8(norm_w + at[g], w[g]);
+  if (x)
+#pragma unroll
+    for (int g = 0; g < G; ++g) ld8(x + t * d + at[g], r[g]);
+  add_y(0, 0);
+  if (k > 1) add_y(1, 1);
+  for (int j = 2; j < k; ++j) {
+    load_y(j, 0);
+    add_y(j, 0);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if ((g * 256 + tid) * 8 >= d) v[g][i] = 0.f;
+      ss = fmaf(v[g][i], v[g][i], ss);
     }
-    z0 = wave_reduce_sum(z0);
-    z1 = wave_reduce_sum(z1);
-    if (lane == 0) {
-      logit[e] = z0;
-      if (both) logit[e + 1] = z1;
+  const float inv = __builtin_amdgcn_rsqf(fmaf(__builtin_amdgcn_rcpf((float)d), block_sum(ss, red), eps));
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int c = (g * 256 + tid) * 8;
+    if (c >= d) continue;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[g][i] = fmaf(w[g][i], v[g][i], v[g][i]) * inv;
+      asm("" : "+v"(v[g][i]));  // rounded here, as in the kernel above
+      if (x) v[g][i] += r[g][i];
+    }
+    f32x4* to = reinterpret_cast<f32x4*>(xo + t * d + c);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 four = {v[g][4 * h], v[g][4 * h + 1], v[g][4 * h + 2], v[g][4 * h + 3]};
+      to[h] = four;
+      if (router) reinterpret_cast<f32x4*>(sm + c)[h] = four;
+    }
+    if (xb) {
+      bf16x8 b;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) b[i] = (short)f32_to_bf16(v[g][i]);
+      *reinterpret_cast<bf16x8*>(xb + t * d + c) = b;
     }
   }
-  __syncthreads();
-  if (wave != 0) return;
-  float mx = NEG_SENTINEL;
-  for (int e = lane; e < experts; e += WAVE) mx = fmaxf(mx, logit[e]);
-  mx = wave_reduce_max(mx);
-  float sum = 0.f;
-  for (int e = lane; e < experts; e += WAVE) sum += expf(logit[e] - mx);
-  sum = wave_reduce_sum(sum);
-  for (int j = 0; j < top; ++j) {
-    float best = NEG_SENTINEL * 2.f;
-    int arg = experts;
-    for (int e = lane; e < experts; e += WAVE)
-      if (logit[e] > best) {
-        best = logit[e];
-        arg = e;
-      }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, WAVE);
-      const int oa = __shfl_xor(arg, off, WAVE);
-      if (ob > best || (ob == best && oa < arg)) {
-        best = ob;
-        arg = oa;
-      }
-    }
-    if (arg >= experts) arg = 0;  // logits that compare with nothing (NaN)
-    if (lane == 0) {
-      sel[t * top + j] = arg;
-      sel_w[t * top + j] = expf(best - mx) / sum;
-    }
-    if ((arg & (WAVE - 1)) == lane) logit[arg] = NEG_SENTINEL * 3.f;  // taken; this lane alone reads it
-  }
+  if (router) route_row(sm, sm + d, router, experts, top, sel, sel_w, d, t);
 }
 
 // ----------------------------------------------------------- batched linear
@@ -422,15 +511,30 @@ std::vector<torch::Tensor> sublayer_out(
   int* selp = experts ? sel.data_ptr<int>() : nullptr;
   float* selwp = experts ? sel_w.data_ptr<float>() : nullptr;
   if (t > 0) {
-#define SO(TY, TW, YP)                                                                                     \
-  sublayer_out_kernel<TY, TW><<<t, threads, lds, stream>>>(                                                \
-      YP, (int)y.size(1), k, sw, norm_w.data_ptr<float>(), (float)eps, xp, xo.data_ptr<float>(), xbp,      \
-      reinterpret_cast<const TW*>(rp), experts, (int)top, selp, selwp, d, (int)dp, y_wide)
+  // rows that reach to the end of what is written, with a weight that 16-byte loads can read
+  const int groups = (d + 2047) / 2048;
+  const bool rows = t >= 64 && d == dp && y_wide && groups <= 4 && reinterpret_cast<uintptr_t>(norm_w.data_ptr()) % 16 == 0 &&
+                    reinterpret_cast<uintptr_t>(xp) % 16 == 0;
+#define SO_ROWS(TY, TW, YP, G)                                                                               \
+  sublayer_out_rows_kernel<TY, TW, G><<<t, 256, lds, stream>>>(                                              \
+      YP, (int)y.size(1), k, sw, norm_w.data_ptr<float>(), (float)eps, xp, xo.data_ptr<float>(), xbp,        \
+      reinterpret_cast<const TW*>(rp), experts, (int)top, selp, selwp, d)
+#define SO(TY, TW, YP)                                                                                       \
+  do {                                                                                                       \
+    if (rows && groups == 1) SO_ROWS(TY, TW, YP, 1);                                                         \
+    else if (rows && groups == 2) SO_ROWS(TY, TW, YP, 2);                                                    \
+    else if (rows) SO_ROWS(TY, TW, YP, 4);                                                                   \
+    else                                                                                                     \
+      sublayer_out_kernel<TY, TW><<<t, threads, lds, stream>>>(                                              \
+          YP, (int)y.size(1), k, sw, norm_w.data_ptr<float>(), (float)eps, xp, xo.data_ptr<float>(), xbp,    \
+          reinterpret_cast<const TW*>(rp), experts, (int)top, selp, selwp, d, (int)dp, y_wide);              \
+  } while (0)
     if (yf && rf) SO(float, float, y.data_ptr<float>());
     else if (yf) SO(float, unsigned short, y.data_ptr<float>());
     else if (rf) SO(unsigned short, float, BF16P(y));
     else SO(unsigned short, unsigned short, BF16P(y));
 #undef SO
+#undef SO_ROWS
     HIP_CHECK_LAST();
   }
   return {xo, xb, sel, sel_w};

@@ -543,6 +543,35 @@ def test_moe_group_kernel(pairs, experts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d", [8, 1288, 2048, 2056, 4096, 4104, 8192, 8320])  # around 1, 2 and 4 groups of 8 values a thread
+@pytest.mark.parametrize("slots,router", [(1, True), (2, False), (3, True)])
+def test_sublayer_out_of_many_rows(d, slots, router):
+    """Rows in registers beside the general kernel: a width that is not written whole takes that one, one router column more."""
+    from petals_amd.ops import latent
+
+    gen = torch.Generator(device="cuda").manual_seed(d + slots)
+    t, experts = 64, 5
+
+    def normal(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    y, w, x = normal(t * slots, d).bfloat16(), normal(d), normal(t, d)
+    r = normal(experts, d).bfloat16() if router else None
+    weights = torch.rand(t, slots, device="cuda", generator=gen) if slots > 1 else None
+    wide = [torch.nn.functional.pad(v, (0, 8)) if v is not None else None for v in (x, r)]
+    for residual, padded in ((x, wide[0]), (None, None)):
+        got = latent.hip().sublayer_out(y, weights, w, 1e-6, residual, d, True, r, 2)
+        want = latent.hip().sublayer_out(y, weights, w, 1e-6, padded, d + 8, True, wide[1], 2)
+        assert torch.equal(got[0], want[0][:, :d]) and torch.equal(got[1], want[1][:, :d])
+        assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3])
+        total = (y.double().view(t, slots, d) * (1.0 if weights is None else weights.double()[..., None])).sum(1)
+        ref = total * torch.rsqrt(total.square().mean(-1, keepdim=True) + 1e-6) * (1 + w.double())
+        ref = ref if residual is None else ref + x.double()
+        # sums of up to d squares in 32 bits, and a handful of roundings
+        assert bool(((got[0].double() - ref).abs() <= 2.0**-20 * (ref.abs() + 1)).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("t,h,k,n", [(1, 3, 32, 40), (16, 2, 96, 130), (17, 1, 45, 33), (200, 4, 128, 96)])
 @pytest.mark.parametrize("a_dtype", ["float32", "bfloat16"])
 def test_batched_linear_kernel(t, h, k, n, a_dtype):
