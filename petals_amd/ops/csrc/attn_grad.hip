@@ -14,10 +14,12 @@
 //
 // 32 heads of 128, 2 x 379 tokens: from the result's gradient back to the projection's it was
 // 42 launches of torch operations over [heads, rows, keys] in 32 bits and over copies of
-// rows, 419 us; the two kernels take 71 us (61 with the mean of a row's gradients taken from
-// its rounded result, and score gradients of 16 bits). At this size they are bound by the chain
-// of a workgroup's tiles (six, and six times the heads that share keys): 384 workgroups for
-// 256 compute units, 1.3 GFLOP of products.
+// rows, 419 us; the two kernels take 58 us, 29 and 29. (A row's mean taken from its rounded
+// result and score gradients of 16 bits had saved 10 of 71.) Loads have no conditions, which
+// would be branches between them, and a tile's sums and means come through LDS with its rows:
+// the keys' kernel took 44 us with loads of a mean and a sum per score, in the midst of the
+// products. At this size they are bound by the chain of a workgroup's tiles (six, and six times
+// the heads that share keys): 384 workgroups for 256 compute units, 1.3 GFLOP of products.
 
 #include "common.h"
 #include "paged_attn.h"
@@ -38,15 +40,13 @@ struct TilePair {
   static constexpr int ROW = HD + TPAD, D8 = HD / 8, NLD = AG_TILE * D8 / 256;
   bf16x8 a[NLD], b[NLD];
   // rows from j0 below s, zeros from there
-  __device__ __forceinline__ void fetch(const unsigned short* pa, long sa, const unsigned short* pb, long sb, int j0, int s) {
+  __device__ __forceinline__ void fetch(const unsigned short* pa, int sa, const unsigned short* pb, int sb, int j0, int s) {
+    const auto ra = cached_rows(pa, j0, min(s - j0, AG_TILE), sa), rb = cached_rows(pb, j0, min(s - j0, AG_TILE), sb);
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int idx = threadIdx.x + i * 256, row = j0 + idx / D8, c = idx % D8 * 8;
-      a[i] = b[i] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (row < s) {
-        a[i] = *reinterpret_cast<const bf16x8*>(pa + row * sa + c);
-        b[i] = *reinterpret_cast<const bf16x8*>(pb + row * sb + c);
-      }
+      const int idx = threadIdx.x + i * 256, row = idx / D8, c = idx % D8 * 8;
+      a[i] = load_cached(ra, (row * sa + c) * 2);
+      b[i] = load_cached(rb, (row * sb + c) * 2);
     }
   }
   __device__ __forceinline__ void stage(unsigned short* buf) const {
@@ -132,18 +132,18 @@ __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
   const unsigned short* base = qkv + b * a.s * width;
   const unsigned short* kp = base + (a.heads + kvh) * HD;
   const unsigned short* vp = kp + a.kv_heads * HD;
-  const size_t at = ((size_t)b * a.s + row) * out_width + head * HD, stat = ((size_t)b * a.heads + head) * a.s + row;
   const bool live = row < a.s;
+  // a lane without a row reads the last one: conditions would be branches between the loads
+  const int safe = min(row, a.s - 1);
+  const size_t at = ((size_t)b * a.s + safe) * out_width + head * HD, stat = ((size_t)b * a.heads + head) * a.s + safe;
 
   bf16x8 qf[RC], gf[RC];
 #pragma unroll
   for (int kc = 0; kc < RC; ++kc) {
-    qf[kc] = gf[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (!live) continue;
-    qf[kc] = *reinterpret_cast<const bf16x8*>(base + row * width + head * HD + kc * 32 + hi * 8);
+    qf[kc] = *reinterpret_cast<const bf16x8*>(base + safe * width + head * HD + kc * 32 + hi * 8);
     gf[kc] = *reinterpret_cast<const bf16x8*>(go + at + kc * 32 + hi * 8);
   }
-  const float sum = live ? lse[stat] : 0.f;
+  const float sum = lse[stat];
   f32x4 acc[VB];
 #pragma unroll
   for (int d = 0; d < VB; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256, 2) void attn_grad_q_kernel(
   const int key_end = min(a.s, first + 64), tiles = (key_end + AG_TILE - 1) / AG_TILE;
   const float in = a.scale * LOG2E;
   TilePair<HD> tile;
-  auto fetch = [&](int step) { tile.fetch(kp, width, vp, width, step % tiles * AG_TILE, key_end); };
+  auto fetch = [&](int step) { tile.fetch(kp, (int)width, vp, (int)width, step % tiles * AG_TILE, key_end); };
   fetch(0);
   tile.stage(smem);
   __syncthreads();
@@ -226,11 +226,9 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
   const bool live = key < a.s;
 
   bf16x8 kf[RC], vf[RC];
-  const unsigned short* kp = base + key * width + (a.heads + kvh) * HD;
+  const unsigned short* kp = base + min(key, a.s - 1) * width + (a.heads + kvh) * HD;
 #pragma unroll
   for (int kc = 0; kc < RC; ++kc) {
-    kf[kc] = vf[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (!live) continue;
     kf[kc] = *reinterpret_cast<const bf16x8*>(kp + kc * 32 + hi * 8);
     vf[kc] = *reinterpret_cast<const bf16x8*>(kp + a.kv_heads * HD + kc * 32 + hi * 8);
   }
@@ -242,13 +240,21 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
   const int tiles = (a.s - first + AG_TILE - 1) / AG_TILE, steps = tiles * group;
   const float in = a.scale * LOG2E;
   TilePair<HD> tile;
+  // with a tile's rows come their sums and means, 64 of each, which a lane needs 16 of
+  float* const stats = reinterpret_cast<float*>(smem + 2 * BUF);
+  const float* const mine = tid & 64 ? dots : lse;
+  float stat;
   auto fetch = [&](int step) {
-    const int head = kvh * group + step / tiles;
-    tile.fetch(base + head * HD, width, go + (size_t)b * a.s * out_width + head * HD, out_width,
-               first + step % tiles * AG_TILE, a.s);
+    const int head = kvh * group + step / tiles, j0 = first + step % tiles * AG_TILE;
+    tile.fetch(base + head * HD, (int)width, go + (size_t)b * a.s * out_width + head * HD, (int)out_width, j0, a.s);
+    stat = mine[((size_t)b * a.heads + head) * a.s + min(j0 + (tid & 63), a.s - 1)];
+  };
+  auto stage = [&](int which) {
+    tile.stage(smem + which * BUF);
+    if (tid < 2 * AG_TILE) stats[which * 2 * AG_TILE + tid] = stat;
   };
   fetch(0);
-  tile.stage(smem);
+  stage(0);
   __syncthreads();
   for (int step = 0; step < steps; ++step) {
     const unsigned short* q_lds = smem + (step & 1) * BUF;
@@ -256,20 +262,22 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
     const bool more = step + 1 < steps;
     if (more) fetch(step + 1);
     const int j0 = first + step % tiles * AG_TILE;
-    const size_t stat = ((size_t)b * a.heads + kvh * group + step / tiles) * a.s;
     f32x4 s[NB], ds[NB];
     tile_product<HD>(q_lds, kf, col, hi, s);
     tile_product<HD>(g_lds, vf, col, hi, ds);
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int nb = 0; nb < NB; ++nb) {
+      const float* const of = stats + (step & 1) * 2 * AG_TILE + nb * 16 + hi * 4;
+      const f32x4 sums = *reinterpret_cast<const f32x4*>(of), means = *reinterpret_cast<const f32x4*>(of + AG_TILE);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = j0 + nb * 16 + hi * 4 + r, safe = min(row, a.s - 1);
+        const int row = j0 + nb * 16 + hi * 4 + r;
         const bool seen = live && row < a.s && key <= row;
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[nb][r], in, -lse[stat + safe]));
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[nb][r], in, -sums[r]));
         s[nb][r] = seen ? p : 0.f;
-        ds[nb][r] = seen ? p * (ds[nb][r] - dots[stat + safe]) : 0.f;
+        ds[nb][r] = seen ? p * (ds[nb][r] - means[r]) : 0.f;
       }
+    }
 #pragma unroll
     for (int ks = 0; ks < NB / 2; ++ks) {
       const bf16x8 pf = weight_operand(s[2 * ks], s[2 * ks + 1]);
@@ -284,7 +292,7 @@ __global__ __launch_bounds__(256, 2) void attn_grad_kv_kernel(
         for (int i = 2; i >= 0; --i) dk[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qt, parts[i], dk[d], 0, 0, 0);
       }
     }
-    if (more) tile.stage(smem + ((step + 1) & 1) * BUF);
+    if (more) stage((step + 1) & 1);
     __syncthreads();
   }
   if (!live) return;
@@ -319,9 +327,10 @@ torch::Tensor attn_prompt_grad(
   if (b == 0 || s == 0) return grad;
   auto dots = torch::empty_like(lse);
   const long runs = (s + 63) / 64;
-  TORCH_CHECK(runs * b * qh < (1L << 31) && start + s < (1L << 31), "too many rows at once");
+  // a tile's rows are addressed by 32 bits
+  TORCH_CHECK(runs * b * qh < (1L << 31) && start + s < (1L << 31) && (qh + 2 * kh) * hd < (1L << 24), "too many rows at once");
   GradShape a{(int)s, (int)qh, (int)kh, (int)start, runs, b * qh, (float)scale};
-  const size_t lds = 4 * AG_TILE * (hd + TPAD) * sizeof(unsigned short);
+  const size_t lds = 4 * AG_TILE * (hd + TPAD) * sizeof(unsigned short) + 4 * AG_TILE * sizeof(float);
   auto stream = at::cuda::getCurrentCUDAStream();
   auto bf = [](const torch::Tensor& t) { return reinterpret_cast<unsigned short*>(t.data_ptr()); };
 #define ATTN_GRAD(HD)                                                                                               \

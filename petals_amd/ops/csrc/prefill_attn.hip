@@ -9,13 +9,23 @@
 // in flight during a tile's products. (The kernel before staged one tile at a time, wrote
 // values to LDS transposed, one by one, and weights to LDS and back.)
 //
-// Bound by the products' operand loads from LDS and by the softmax's vector instructions.
-// MI355X, causal, before and now:
-//   64 heads of 128 over 8, 8192 tokens    3534 -> 1353 us   311 -> 813 TFLOP/s
-//   32 over 8, 4096 tokens                  542 ->  215 us   254 -> 640
-//   32 over 8, 512 tokens after 3584        266 ->  121 us   121 -> 267
-//   32 over 8, 512 tokens                  33.5 -> 19.5 us
-//   71 heads of 64 over 1, 4 x 509 tokens    61 ->   50 us
+// The loads of a tile are buffer loads, which give zeros beyond the last key, and a lane
+// beyond the last row reads that one: with conditions each load was a branch of its own, and
+// the loads waited for one another. Products have the priority of a SIMD's two waves: the
+// other's softmax then runs beneath them.
+//
+// Bound by the products' operand loads from LDS and by the softmax's vector instructions,
+// short ones by the chain of their tiles. MI355X, causal; loads under conditions, loads
+// without, and with the products' priority:
+//   64 heads of 128 over 8, 8192 tokens    1308   1255   1255 us   876 TFLOP/s
+//   32 over 8, 4096 tokens                  186    181    181      759
+//   32 over 8, 1024 tokens                 32.9   29.6   27.2
+//   32 over 8, 512 tokens after 3584        113    109     98
+//   32 over 8, 512 tokens                  18.5   16.7   15.4
+//   71 heads of 64 over 1, 4 x 509 tokens    52     43     42
+//   4 x 128 tokens, 32 heads of 128         8.3    7.5    7.1
+// (The kernel that staged one tile at a time took 3534, 542, 266, 33.5 and 61 us for the
+// sizes that it was measured at: the first, second, fourth, fifth and sixth.)
 //
 // NOTE: masking and the running maximum stay in separate loops (paged_attn.h
 // weigh_tile). Fused (mask and `mx = fmaxf(mx, s)` in one loop body), amdclang (ROCm 7.2,
@@ -80,10 +90,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     seen[i].lo = 0;
     m[i] = NEG_SENTINEL;
     l[i] = 0.f;
+    // a lane without a row reads the last one: conditions would be branches between the loads
 #pragma unroll
     for (int kc = 0; kc < RC; ++kc)
-      q_frag[i][kc] = live ? *reinterpret_cast<const bf16x8*>(qp + row * q.row + kc * 32 + hi * 8)
-                           : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      q_frag[i][kc] = *reinterpret_cast<const bf16x8*>(qp + min(row, s_q - 1) * q.row + kc * 32 + hi * 8);
 #pragma unroll
     for (int d = 0; d < VB; ++d) acc[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -93,14 +103,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
 
   bf16x8 kn[NLD], vn[NLD];
   auto fetch = [&](int j0) {  // zeros beyond the last key
+    const int rows = min(key_end - j0, KT), k_row = (int)k.row, v_row = (int)v.row;
+    const auto kr = cached_rows(kp, j0, rows, k_row), vr = cached_rows(vp, j0, rows, v_row);
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int idx = tid + i * 256, row = j0 + idx / D8, c = idx % D8 * 8;
-      kn[i] = vn[i] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (row < key_end) {
-        kn[i] = *reinterpret_cast<const bf16x8*>(kp + row * k.row + c);
-        vn[i] = *reinterpret_cast<const bf16x8*>(vp + row * v.row + c);
-      }
+      const int idx = tid + i * 256, row = idx / D8, c = idx % D8 * 8;
+      kn[i] = load_cached(kr, (row * k_row + c) * 2);
+      vn[i] = load_cached(vr, (row * v_row + c) * 2);
     }
   };
   auto stage = [&](unsigned short* buf) {
@@ -125,6 +134,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
       const bool interior = j0 + KT - 1 <= all_hi && j0 + KT <= key_end;
       bf16x8 p_frag[QB][NB / 2];
       f32x4 s[QB][NB];
+      __builtin_amdgcn_s_setprio(1);  // see above
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -136,6 +146,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
           for (int i = 0; i < QB; ++i) s[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt, q_frag[i][kc], s[i][nb], 0, 0, 0);
         }
       }
+      __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int i = 0; i < QB; ++i) {
         float corr;
@@ -147,6 +158,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
         for (int ks = 0; ks < NB / 2; ++ks) p_frag[i][ks] = weight_operand(s[i][2 * ks], s[i][2 * ks + 1]);
       }
       const unsigned short* v_lds = k_lds + KT * ROW + (hi * 4 + col / 4) * ROW + (col & 3) * 4;
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int d = 0; d < VB; ++d)
 #pragma unroll
@@ -155,6 +167,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
 #pragma unroll
           for (int i = 0; i < QB; ++i) acc[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, p_frag[i][ks], acc[i][d], 0, 0, 0);
         }
+      __builtin_amdgcn_s_setprio(0);
     }
     if (more) stage(smem + (which ^ 1) * 2 * KT * ROW);
     __syncthreads();
@@ -175,9 +188,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
   }
 }
 
-// rows that 16-byte loads can read as they lie, else a copy
+// rows that 16-byte loads can read as they lie, one after the other and within 32 bits for a tile, else a copy
 static torch::Tensor readable_rows(const torch::Tensor& t) {
   bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  ok = ok && t.stride(2) >= t.size(3) && t.stride(2) < (1L << 24);
   for (int i = 0; i < 3; ++i) ok = ok && (t.size(i) == 1 || t.stride(i) % 8 == 0);
   return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }

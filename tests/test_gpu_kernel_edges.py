@@ -441,6 +441,23 @@ def test_prompt_attention_edges(hip, hd, b, qh, kh, s, offset, causal, alibi):
 
 
 @requires_gpu
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("length", [63, 64, 65])
+@pytest.mark.parametrize("step", ["0", "8", "half", "wide"])
+def test_prompt_attention_strides(hip, hd, length, step):
+    """Keys and values whose rows overlap, are one row or lie far apart are read like their copies."""
+    gen = torch.Generator(device="cuda").manual_seed(hd + length)
+    row = {"0": 0, "8": 8, "half": hd // 2, "wide": 1 << 17}[step]
+    store = torch.randn(2 * (row * length + hd), device="cuda", generator=gen).to(BF16)
+    k = store.as_strided((1, 2, length, hd), (store.numel(), store.numel() // 2, row, 1))
+    v = store.flip(0).as_strided(k.shape, k.stride())
+    q = torch.randn(1, 4, length, hd, device="cuda", generator=gen).to(BF16)
+    out = hip.attn_prefill_rows(q, k, v, length, 0, hd**-0.5, True, None)
+    k, v = (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
+    assert torch.equal(out, hip.attn_prefill_rows(q, k, v, length, 0, hd**-0.5, True, None))
+
+
+@requires_gpu
 @pytest.mark.parametrize("hd,qh,kh,s,start", [(64, 3, 1, 1, 0), (128, 4, 2, 33, 5), (64, 2, 2, 70, 130)])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("turns", [False, True])
