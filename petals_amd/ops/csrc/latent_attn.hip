@@ -54,6 +54,25 @@ __device__ __forceinline__ float end_factor(const LatentEnd& e, size_t flat, int
 
 // ------------------------------------------------------------ MFMA kernel
 
+// the maximum over 16 neighbouring lanes, without a way through LDS
+__device__ __forceinline__ float max_of_16(float x) {
+#define TURNED(ctrl) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, false))
+  x = fmaxf(x, TURNED(0x128));
+  x = fmaxf(x, TURNED(0x124));
+  x = fmaxf(x, TURNED(0x122));
+  return fmaxf(x, TURNED(0x121));
+#undef TURNED
+}
+
+// The token run (x) and the group of rows (y) of a workgroup. Late rows of a prompt see most and come first; every second
+// 256 are turned round, so that a compute unit that gets two has a long and a short one.
+__device__ __forceinline__ int2 late_first(int nx, int ny) {
+  int at = blockIdx.y * nx + blockIdx.x;
+  if ((at & 256) && (at | 255) < nx * ny) at ^= 255;
+  at = nx * ny - 1 - at;
+  return int2{at / ny, at % ny};
+}
+
 // A workgroup is 4 waves = RG groups of 16 rows x DG slices of the latent's
 // dims: DG > 1 when there are few rows (decoding), so that all waves share the
 // staging and the weighted sum. Tiles are double-buffered in LDS and the next
@@ -63,6 +82,16 @@ __device__ __forceinline__ float end_factor(const LatentEnd& e, size_t flat, int
 // Bound by the wave that waits: with one wave a SIMD nothing runs while a tile's scores become probabilities. 583 rows
 // of 32 heads after 0 to 3000 keys, 512 values: 260 us with conditional loads to registers and one wave, 241 with loads
 // without conditions, 144 with rows that go straight to LDS, which leaves registers for two waves.
+//
+// So what stands between the products is kept short: a row's maximum goes round 16 lanes without LDS, sums are scaled
+// only where a maximum grew, and the products have the priority of a SIMD's two waves. And the queries' loads have no
+// conditions, which had made them wait for one another. us before and now, 512 values:
+//   32 heads, 1021 + 130 + 7 + 1 + 1 + 1 rows after 300 each    162 -> 120
+//   4096 rows of 32 heads                                      1079 -> 734  (817 without late rows first)
+//   195 + 194 + 194 rows after 0, 1000 and 3000                 311 -> 221
+//   333 rows of 128 heads                                        72 ->  48  (63)
+//   8 x 1 row after 2000 (key splits)                          22.6 -> 22.3
+//   300 rows of 128 heads after 900, 576 values, 512 summed     378 -> 358  (387; one wave of a SIMD)
 //
 // RC = row size in 32-wide MFMA k-chunks (columns past RP read as zero), VC = those
 // of them that are values. Grid: (token runs, groups of 16*RG rows, key splits).
@@ -90,10 +119,11 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
   constexpr int NLD = (LOADS + 255) / 256;       // per thread
   constexpr bool DIRECT = RC == 16;              // a wave loads a row at once, from memory to LDS
   constexpr int DB = (VC * 2 + DG - 1) / DG;     // 16-wide dim blocks per wave
-  const int tok0 = tiles[2 * blockIdx.x];
-  const int ntok = tiles[2 * blockIdx.x + 1];
+  const int2 own = late_first(gridDim.x, gridDim.y);
+  const int tok0 = tiles[2 * own.x];
+  const int ntok = tiles[2 * own.x + 1];
   const int rows = ntok * heads;
-  const int g0 = blockIdx.y * 16 * RG;  // first row of this workgroup
+  const int g0 = own.y * 16 * RG;  // first row of this workgroup
   if (g0 >= rows) return;               // uniform over the workgroup
   const int g1 = min(g0 + 16 * RG, rows);
 
@@ -120,15 +150,13 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
 
   bf16x8 q_frag[RC];
   {
-    const int row = r0 + col;
-    const unsigned short* src = q + ((size_t)tok0 * heads + row) * rp;
+    // no conditions, which would be branches between the loads; a lane beyond the last row has that one
+    const unsigned short* src = q + ((size_t)tok0 * heads + min(r0 + col, rows - 1)) * rp;
 #pragma unroll
     for (int kc = 0; kc < RC; ++kc) {
       const int c0 = kc * 32 + hi * 8;
-      if (row < rows && c0 < rp)
-        q_frag[kc] = *reinterpret_cast<const bf16x8*>(src + c0);
-      else
-        q_frag[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      q_frag[kc] = *reinterpret_cast<const bf16x8*>(src + min(c0, rp - 8));
+      if (c0 >= rp) q_frag[kc] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
   }
 
@@ -142,7 +170,8 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
     m_row[r] = NEG_SENTINEL;
     l_row[r] = 0.f;
     const int row = r0 + hi * 4 + r;
-    row_pos[r] = row < rows ? b.pos[tok0 + row / heads] : -1;  // -1: sees nothing
+    const int pos = b.pos[tok0 + min(row, rows - 1) / heads];
+    row_pos[r] = row < rows ? pos : -1;  // -1: sees nothing
     row_lo[r] = window > 0 ? row_pos[r] - window + 1 : 0;
   }
   // keys that every row of this wave sees: [all_lo, all_hi]
@@ -224,6 +253,7 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
     }
 
     f32x4 s_acc[2];
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
       s_acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -234,8 +264,10 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
       }
     }
 
+    __builtin_amdgcn_s_setprio(0);
     const bool interior = j0 >= all_lo && j0 + LKVT - 1 <= all_hi && j0 + LKVT <= j_end;
     float corr[4], p[2][4];
+    bool grew = false;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       // masking and the running max stay in separate loops (see prefill_attn.hip)
@@ -249,10 +281,8 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
           if (key >= j_end || key > row_pos[r] || key < row_lo[r]) s[nb] = NEG_SENTINEL;
         }
       }
-      float mx = fmaxf(s[0], s[1]);
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, WAVE));
-      const float m_new = fmaxf(m_row[r], mx);
+      const float m_new = fmaxf(m_row[r], max_of_16(fmaxf(s[0], s[1])));
+      grew = grew || m_new > m_row[r];
       corr[r] = (m_row[r] <= NEG_THRESHOLD) ? 0.f : exp2f(m_row[r] - m_new);
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) p[nb][r] = (s[nb] <= NEG_THRESHOLD) ? 0.f : exp2f(s[nb] - m_new);
@@ -269,15 +299,21 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const bf16x8 p_frag = *reinterpret_cast<const bf16x8*>(&p_lds[col * (LKVT + 8) + hi * 8]);
 
+    if (RC > 16 || __any(grew)) {  // else all factors are 1; 18 chunks, whose sums move between register files, ran slower with the branch
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc_o[d][r] *= corr[r];
+    }
     const unsigned short* v_lds = k_lds + (hi * 8 + col / 4) * ROW + (col & 3) * 4;
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
       if (VC * 2 % DG != 0 && d0 + d >= VC * 2) break;  // uniform over the wave
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc_o[d][r] *= corr[r];
       acc_o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
           p_frag, load_keys(v_lds + (d0 + d) * 16, ROW), acc_o[d], 0, 0, 0);
     }
+    __builtin_amdgcn_s_setprio(0);
     if (!DIRECT && more) stage(smem + (which ^ 1) * LKVT * ROW);
     arrive();
   }

@@ -503,6 +503,29 @@ def test_latent_rows_straight_to_lds(heads, rank, values, window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,rank,tokens", [(128, 64, 255), (128, 512, 260), (32, 512, 513), (70, 576, 511)])
+def test_latent_attention_of_many_runs(heads, rank, tokens):
+    """Around 256 and 512 workgroups, one or two of them for a run of rows: each has rows of its own, whatever the order."""
+    from petals_amd.ops import latent
+
+    torch.manual_seed(0)
+    pages = -(-tokens // PAGE_SIZE)
+    cache = torch.randn(pages, PAGE_SIZE, rank, device="cuda").bfloat16()
+    batch = PagedBatch([list(range(pages))[::-1]], [0], [tokens], torch.device("cuda"))
+    q = torch.randn(tokens, heads, rank, device="cuda").bfloat16()
+    run = batch.run_tokens(heads)
+    got = latent.hip().latent_attention(
+        q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(run), run, batch.max_end, 0, 1.5 * rank**-0.5, 1
+    )
+    c = cache.flip(0).reshape(-1, rank)[:tokens].double()
+    score = (q.double() @ c.T) * (1.5 * rank**-0.5)
+    seen = torch.arange(tokens, device="cuda") <= torch.arange(tokens, device="cuda")[:, None]
+    want = score.masked_fill(~seen[:, None], -float("inf")).softmax(-1) @ c
+    # probabilities and results are rounded to 8 bits: 2^-8 of the largest value, 5, each
+    assert (got.double() - want).abs().max() < 4e-2
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("t,experts,top,d", [(1, 1, 1, 7), (3, 8, 2, 128), (70, 300, 9, 1000), (65, 5, 5, 129)])
 @pytest.mark.parametrize("slots", [0, 3])
 def test_sublayer_out_kernel(t, experts, top, d, slots):
