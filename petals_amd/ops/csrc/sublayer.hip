@@ -370,6 +370,101 @@ __global__ __launch_bounds__(256) void batched_linear_kernel(
   }
 }
 
+// Many rows of bf16, k a multiple of 64: 128 rows x 128 columns of one head by 4 waves, which share tiles of 64 k in
+// LDS; two tiles are on their way to registers. Products and their order are those of batched_linear_kernel, which
+// reads 64 bytes of a row at a time, every row once for each 64 columns, under conditions that keep its loads apart.
+// Bound by reading and writing rows, or by the chain of k where they are few. 32 heads, us with that kernel and with this:
+//   k x n        17 rows       100          283          1161         4096
+//   128 x 512    6.2  3.5      8.0  4.0    11.9  7.4    27.0 16.3    69.9 40.3   (1161 rows: 48 MB, 2.9 TB/s)
+//   512 x 128   11.3  6.2     16.6  6.4    18.6  6.6    33.2 14.9    61.4 31.2
+//   512 x 64    10.3  6.2     12.8  6.3    18.2  6.5    19.5 13.7    35.7 28.8
+// 1 head, 4096 x 1024, 17 to 4096 rows: 110 to 118 and 32 to 57. MT: 4 for 128 rows a workgroup, 2 for 64 where those
+// of 128 would be fewer than two for each compute unit.
+template <int MT>
+__global__ __launch_bounds__(256, 2) void batched_linear_rows_kernel(
+    const unsigned short* __restrict__ a, long a_t, long a_h, const unsigned short* __restrict__ w,
+    unsigned short* __restrict__ out, long o_t, long o_h, int t_dim, int n_dim, int k_dim, int heads, int jobs) {
+  constexpr int NT = 4, BM = 32 * MT, BN = 128, BK = 64, ROW = BK + 8, NA = BM / 32, NW = BN / 32;
+  __shared__ unsigned short smem[2][(BM + BN) * ROW];
+  // chiplets take heads of their own, whose weights and rows then stay in their caches
+  const int id = blockIdx.x;
+  const bool dealt = heads % 8 == 0;
+  const size_t h = dealt ? id % 8 + id / 8 / jobs * 8 : id / jobs;
+  const int job = dealt ? id / 8 % jobs : id % jobs, n_tiles = (n_dim + BN - 1) / BN;
+  const int n0 = job % n_tiles * BN, t0 = job / n_tiles * BM;
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, col = lane & 15, hi = lane >> 4;
+  const int wm = wave / 2 * 16 * MT, wn = wave % 2 * 16 * NT;  // of this wave
+
+  // rows and columns beyond the last repeat it
+  const unsigned short *ap[NA], *wp[NW];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) ap[i] = a + (size_t)min(t0 + tid / 8 + i * 32, t_dim - 1) * a_t + h * a_h + tid % 8 * 8;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) wp[i] = w + (h * n_dim + min(n0 + tid / 8 + i * 32, n_dim - 1)) * (size_t)k_dim + tid % 8 * 8;
+  bf16x8 next[2][NA + NW];
+  auto fetch = [&](bf16x8* to, int k0) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) to[i] = *reinterpret_cast<const bf16x8*>(ap[i] + k0);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) to[NA + i] = *reinterpret_cast<const bf16x8*>(wp[i] + k0);
+  };
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int which, int k0) {
+    unsigned short* buf = smem[which];
+#pragma unroll
+    for (int i = 0; i < NA + NW; ++i) *reinterpret_cast<bf16x8*>(&buf[(tid / 8 + i * 32) * ROW + tid % 8 * 8]) = next[which][i];
+    __syncthreads();
+    if (k0 + 2 * BK < k_dim) fetch(next[which], k0 + 2 * BK);
+#pragma unroll
+    for (int kc = 0; kc < BK; kc += 32) {
+      bf16x8 af[MT], wf[NT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) af[m] = *reinterpret_cast<const bf16x8*>(&buf[(wm + m * 16 + col) * ROW + kc + hi * 8]);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) wf[n] = *reinterpret_cast<const bf16x8*>(&buf[(BM + wn + n * 16 + col) * ROW + kc + hi * 8]);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], af[m], acc[m][n], 0, 0, 0);
+    }
+  };
+  fetch(next[0], 0);
+  if (BK < k_dim) fetch(next[1], BK);
+  for (int k0 = 0; k0 < k_dim; k0 += 2 * BK) {
+    step(0, k0);
+    if (k0 + BK < k_dim) step(1, k0 + BK);
+  }
+  __syncthreads();
+
+  // acc[m][n][r]: row wm + m*16 + col, column wn + n*16 + hi*4 + r; rows leave through LDS, 128 bytes at a time
+  constexpr int TO = 16 * NT + 8;
+  unsigned short* tile = smem[0] + wave * 16 * TO;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+      *reinterpret_cast<ushort4*>(&tile[col * TO + n * 16 + hi * 4]) = ushort4{
+          f32_to_bf16(acc[m][n][0]), f32_to_bf16(acc[m][n][1]), f32_to_bf16(acc[m][n][2]), f32_to_bf16(acc[m][n][3])};
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = lane; i < 16 * NT * 2; i += WAVE) {
+      const int r = i / (NT * 2), t = t0 + wm + m * 16 + r, c = i % (NT * 2) * 8;
+      if (t < t_dim && n0 + wn + c < n_dim)
+        *reinterpret_cast<bf16x8*>(out + (size_t)t * o_t + h * o_h + n0 + wn + c) = *reinterpret_cast<const bf16x8*>(&tile[r * TO + c]);
+    }
+  }
+}
+
 // Few rows (t_dim <= 16): the 4 waves of a workgroup share 16 columns and split
 // k, so that even a single token spreads a head over many waves.
 template <typename TA, typename TO>
@@ -567,6 +662,23 @@ torch::Tensor batched_linear(torch::Tensor a, torch::Tensor w, bool out_f32, c10
   const bool w_wide = k % 8 == 0;
   const long ob = out_f32 ? 4 : 2;
   const bool o_wide = ot * ob % 16 == 0 && oh * ob % 16 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0;
+  // faster at every size measured (see the kernel); what it does not take: 32 bits, rows or columns out of line
+  if (t > 16 && !af && !out_f32 && n % 8 == 0 && k > 0 && k % 64 == 0 && a_wide && o_wide &&
+      reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0) {
+    const long tall = (t + 127) / 128 * ((n + 127) / 128), flat = (t + 63) / 64 * ((n + 127) / 128);
+    const bool most = tall * h >= 512;
+    const long per = most ? tall : flat;
+    TORCH_CHECK(per * h < (1L << 31), "too many rows at once");
+#define BR(MT) batched_linear_rows_kernel<MT><<<per * h, 256, 0, stream>>>(BF16P(a), at_, ah, BF16P(w), BF16P(out), ot, oh, t, n, k, h, per)
+    if (most) {
+      BR(4);
+    } else {
+      BR(2);
+    }
+#undef BR
+    HIP_CHECK_LAST();
+    return out;
+  }
   const int n_tiles = (n + 63) / 64;
   const long jobs = n_tiles * ((t + 63) / 64);
 #define BL(TA, TO, AP, OP)                                                               \

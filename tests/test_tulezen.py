@@ -503,6 +503,31 @@ def test_latent_rows_straight_to_lds(heads, rank, values, window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,k,n", [(1, 64, 8), (3, 192, 136), (8, 128, 512), (16, 320, 120), (40, 64, 128)])
+@pytest.mark.parametrize("t", [17, 64, 65, 129, 1700])
+def test_batched_linear_of_many_rows(heads, k, n, t):
+    """Rows of bf16 in line share tiles, with the results, to the bit, that rows out of line have, which do not."""
+    from petals_amd.ops import latent
+
+    torch.manual_seed(0)
+    a = torch.randn(t, heads + 2, k, device="cuda").bfloat16()[:, 1:-1]
+    w = torch.randn(heads, n, k, device="cuda").bfloat16()
+    into = torch.full((t, heads + 1, n + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+    latent.hip().batched_linear(a, w, False, into[:, 1:, :n])
+    got = into[:, 1:, :n]
+    assert (into[:, 0] == 7).all() and (into[..., n:] == 7).all()
+    out_of_line = torch.empty(a.numel() + 1, device="cuda", dtype=torch.bfloat16)[1:].view(a.shape).copy_(a)
+    assert torch.equal(got, latent.hip().batched_linear(out_of_line, w, False))
+    x, y = a.double().transpose(0, 1), w.double().transpose(1, 2).contiguous()
+    want, size = (x @ y).transpose(0, 1), (x.abs() @ y.abs()).transpose(0, 1)
+    # k additions of 32 bits, and the result's rounding
+    assert ((got.double() - want).abs() <= k * 2.0**-24 * size + 2.0**-8 * want.abs()).all()
+    every = torch.randn(1, heads, k, device="cuda").bfloat16().expand(t, heads, k)
+    same = latent.hip().batched_linear(every, w, False)
+    assert torch.equal(same, same[:1].expand_as(same))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,rank,tokens", [(128, 64, 255), (128, 512, 260), (32, 512, 513), (70, 576, 511)])
 def test_latent_attention_of_many_runs(heads, rank, tokens):
     """Around 256 and 512 workgroups, one or two of them for a run of rows: each has rows of its own, whatever the order."""
