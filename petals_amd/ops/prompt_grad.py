@@ -125,6 +125,8 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     if weights <= 3 << 23 and not (odd and weights >= 1 << 24):
         return False
     if transposed:
+        # 4544 to 18176: 192 rows 59, 53; 512 rows 81, 96; 758 rows 98, 112; 1200 rows 256, 185; 1500 rows 188, 224; 2048 rows 313, 286
+        odd = odd and (n < 3 * k or m <= 256 or 800 < m <= 1280 or m > 1536)
         return m <= 1536 and k > n or m <= 640 and k == n or m <= 320 and n < 3 * k or odd
     return m <= 1536 or followed or odd
 
