@@ -84,14 +84,16 @@ __device__ __forceinline__ int2 late_first(int nx, int ny) {
 // without conditions, 144 with rows that go straight to LDS, which leaves registers for two waves.
 //
 // So what stands between the products is kept short: a row's maximum goes round 16 lanes without LDS, sums are scaled
-// only where a maximum grew, and the products have the priority of a SIMD's two waves. And the queries' loads have no
-// conditions, which had made them wait for one another. us before and now, 512 values:
-//   32 heads, 1021 + 130 + 7 + 1 + 1 + 1 rows after 300 each    162 -> 120
-//   4096 rows of 32 heads                                      1079 -> 734  (817 without late rows first)
-//   195 + 194 + 194 rows after 0, 1000 and 3000                 311 -> 221
-//   333 rows of 128 heads                                        72 ->  48  (63)
-//   8 x 1 row after 2000 (key splits)                          22.6 -> 22.3
-//   300 rows of 128 heads after 900, 576 values, 512 summed     378 -> 358  (387; one wave of a SIMD)
+// only where a maximum grew, and the queries' loads have no conditions, which had made them wait for one another. Where
+// rows go straight to LDS the products have the priority of a SIMD's two waves; where they wait in registers, bounds
+// between products and the rest cost more than that gives. us before and now, 512 values:
+//   32 heads, 1021 + 130 + 7 + 1 + 1 + 1 rows after 300 each    162 -> 119  (133 without priorities)
+//   4096 rows of 32 heads                                      1079 -> 726  (778; 817 without late rows first)
+//   195 + 194 + 194 rows after 0, 1000 and 3000                 311 -> 220  (256)
+//   333 rows of 128 heads                                        72 ->  47  (48; 63 without late rows first)
+//   8 x 1 row after 2000 (key splits)                          22.6 -> 22.2
+//   1000 + 700 rows of 8 heads after 0 and 50, 128 values      51.6 -> 37.3  (40.4 with priorities)
+//   300 rows of 128 heads after 900, 576 values, 512 summed     378 -> 335  (353 with priorities)
 //
 // RC = row size in 32-wide MFMA k-chunks (columns past RP read as zero), VC = those
 // of them that are values. Grid: (token runs, groups of 16*RG rows, key splits).
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
     }
 
     f32x4 s_acc[2];
-    __builtin_amdgcn_s_setprio(1);
+    if constexpr (DIRECT) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
       s_acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
       }
     }
 
-    __builtin_amdgcn_s_setprio(0);
+    if constexpr (DIRECT) __builtin_amdgcn_s_setprio(0);
     const bool interior = j0 >= all_lo && j0 + LKVT - 1 <= all_hi && j0 + LKVT <= j_end;
     float corr[4], p[2][4];
     bool grew = false;
@@ -306,14 +308,14 @@ __global__ __launch_bounds__(256, waves_per_simd(RC, DG)) void latent_attn_kerne
         for (int r = 0; r < 4; ++r) acc_o[d][r] *= corr[r];
     }
     const unsigned short* v_lds = k_lds + (hi * 8 + col / 4) * ROW + (col & 3) * 4;
-    __builtin_amdgcn_s_setprio(1);
+    if constexpr (DIRECT) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
       if (VC * 2 % DG != 0 && d0 + d >= VC * 2) break;  // uniform over the wave
       acc_o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
           p_frag, load_keys(v_lds + (d0 + d) * 16, ROW), acc_o[d], 0, 0, 0);
     }
-    __builtin_amdgcn_s_setprio(0);
+    if constexpr (DIRECT) __builtin_amdgcn_s_setprio(0);
     if (!DIRECT && more) stage(smem + (which ^ 1) * LKVT * ROW);
     arrive();
   }

@@ -231,6 +231,12 @@ __device__ __forceinline__ bool weigh_tile(
   return grew;
 }
 
+// 8 values of a query from c on, zeros if c is not below its size (both multiples of 32)
+__device__ __forceinline__ bf16x8 query_part(const unsigned short* q, int c, int size) {
+  const bf16x8 v = *reinterpret_cast<const bf16x8*>(q + min(c, size - 32));
+  return c < size ? v : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+}
+
 // weights of 32 keys as an operand
 __device__ __forceinline__ bf16x8 weight_operand(const f32x4& a, const f32x4& b) {
   using f32x8 = __attribute__((ext_vector_type(8))) float;
@@ -267,6 +273,17 @@ __device__ __forceinline__ int2 spread_tiles(int nx, int ny) {
   return int2{(int)(nx - 1 - at % nx), (int)(at / nx)};
 }
 
+// Bound by the products' operands from LDS, the softmax's vector instructions and the loads of the next tile, which must
+// not wait for one another: they have no conditions (buffer loads give zeros). Priority for the products, which helps in
+// prefill_attn.hip and for latent_attn.hip's rows that go straight to LDS, costs 3 to 15% here. us with a condition at
+// each load, and now; 1021 + 130 + 7 + 1 + 1 + 1 rows after 300 each, and 2048 rows:
+//   two maps of 128, values of 256, 32 heads over 8    181 -> 167    358 -> 327
+//   two maps of 256, values of 256, 8 over 8           165 -> 146    241 -> 213
+//   capped, 128 and 128, 32 over 8                    52.4 -> 45.9  95.3 -> 78.9
+//   sigmoid, 96 and 144, 16 over 4                    53.6 -> 44.1   102 ->  86
+//   softmax, 128 and 128, 32 over 8                   55.8 -> 50.4   107 ->  90
+//   softmax, 64 and 64, 32 over 32                    42.2 -> 37.5  66.2 -> 62.3
+//
 // RC: 32-wide chunks of the key size, VB: 16-wide blocks of the value size, at
 // least as many as there are: tiles are filled up with zeros, so that no branch
 // stands between products. A wave holds all maps of its QB blocks of 16 rows; a tile
@@ -322,20 +339,19 @@ __global__ __launch_bounds__(256, QB) void paged_attn_kernel(
   for (int i = 0; i < QB; ++i) {
     const int row = r0 + i * 16 + col;
     const bool live = row < rows;
-    const int head = live ? kvh * group + row % group : 0;
-    const size_t at = ((size_t)(tok0 + (live ? row / group : 0)) * a.heads + head) * MAPS * a.dk;
-    seen[i].pos = live ? b.pos[tok0 + row / group] : -1;  // -1: sees nothing
-    seen[i].lo = live ? first_key(a, seen[i].pos) : 0;
-    lin[i] = live ? linear_term<KIND>(a, head) : 0.f;
+    // a lane without a row has the last one's query: loads under conditions would be branches, and wait for one another
+    const int safe = min(row, rows - 1), head = kvh * group + safe % group;
+    const unsigned short* own_q = q + ((size_t)(tok0 + safe / group) * a.heads + head) * MAPS * a.dk + hi * 8;
+    const int pos = b.pos[tok0 + safe / group];
+    seen[i].pos = live ? pos : -1;  // -1: sees nothing
+    seen[i].lo = live ? first_key(a, pos) : 0;
+    lin[i] = linear_term<KIND>(a, head);
 #pragma unroll
     for (int u = 0; u < MAPS; ++u) {
       m[i][u] = first_maximum(scale);
       l[i][u] = 0.f;
 #pragma unroll
-      for (int kc = 0; kc < RC; ++kc)
-        q_frag[i][u][kc] = live && kc * 32 < a.dk
-                               ? *reinterpret_cast<const bf16x8*>(q + at + u * a.dk + kc * 32 + hi * 8)
-                               : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      for (int kc = 0; kc < RC; ++kc) q_frag[i][u][kc] = query_part(own_q + u * a.dk, kc * 32, a.dk);
 #pragma unroll
       for (int d = 0; d < VB; ++d) acc_o[i][u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -350,23 +366,22 @@ __global__ __launch_bounds__(256, QB) void paged_attn_kernel(
 
   const int width = a.kv_heads * (MAPS * a.dk + a.dv);
   bf16x8 next[NLD];
+  int next_at[NLD];  // in a tile, in bytes; columns past a head's size lie beyond it
+#pragma unroll
+  for (int i = 0; i < NLD; ++i) {
+    const int idx = tid + i * 256;
+    const bool is_v = idx >= K_LOADS;
+    const int row = is_v ? (idx - K_LOADS) / V8 : idx / K8;
+    const int u = is_v ? 0 : idx % K8 / (RC * 4);
+    const int c8 = (is_v ? (idx - K_LOADS) % V8 : idx % (RC * 4)) * 8;
+    const int c = is_v ? a.kv_heads * MAPS * a.dk + kvh * a.dv + c8 : (kvh * MAPS + u) * a.dk + c8;
+    next_at[i] = idx < LOADS && c8 < (is_v ? a.dv : a.dk) ? (row * width + c) * 2 : BEYOND_ROWS;
+  }
   // rows of tile j0 that lie in [0, j_end); zero elsewhere
   auto fetch = [&](int j0) {
-    const long at = cache_row(b, seq, j0);
+    const auto rows_of = cached_rows(cache, cache_row(b, seq, j0), min(j_end - j0, KT), width);
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int idx = tid + i * 256;
-      next[i] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (LOADS % 256 == 0 || idx < LOADS) {
-        const bool is_v = idx >= K_LOADS;
-        const int row = is_v ? (idx - K_LOADS) / V8 : idx / K8;
-        const int u = is_v ? 0 : idx % K8 / (RC * 4);
-        const int c8 = (is_v ? (idx - K_LOADS) % V8 : idx % (RC * 4)) * 8;
-        const int c = is_v ? a.kv_heads * MAPS * a.dk + kvh * a.dv + c8 : (kvh * MAPS + u) * a.dk + c8;
-        if (at >= 0 && j0 + row < j_end && c8 < (is_v ? a.dv : a.dk))
-          next[i] = *reinterpret_cast<const bf16x8*>(cache + ((size_t)at + row) * width + c);
-      }
-    }
+    for (int i = 0; i < NLD; ++i) next[i] = load_cached(rows_of, next_at[i]);
   };
   auto stage = [&](unsigned short* buf) {
 #pragma unroll

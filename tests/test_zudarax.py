@@ -684,6 +684,47 @@ def test_attention_kernels(kind, heads, kv_heads, dk, dv, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,heads,kv_heads,dk,dv", [
+    ("paired", 4, 2, 128, 256), ("paired", 2, 2, 256, 144), ("capped", 8, 2, 128, 128), ("sigmoid", 4, 4, 96, 80), ("sigmoid", 6, 1, 32, 16),
+])
+@pytest.mark.parametrize("rows", [2, 33, 64, 97])
+def test_prompts_read_what_there_is(kind, heads, kv_heads, dk, dv, rows):
+    """What is cached beyond a prompt's end does not count, and a page that is not in the pool counts as one of zeros."""
+    from petals_amd.ops import scores
+
+    torch.manual_seed(0)
+    hip, maps = scores.hip(), 2 if kind == "paired" else 1
+    starts, lens, pages = [PAGE_SIZE + 5, 7], [rows, rows + 30], [[1, 4, 6], [2, 3, 5]]
+    cache = torch.randn(7, PAGE_SIZE, kv_heads * (maps * dk + dv), device="cuda").bfloat16()
+    batch = PagedBatch(pages, starts, lens, torch.device("cuda"))
+    q = torch.randn(batch.tokens, heads, *([2] if maps == 2 else []), dk, device="cuda").bfloat16()
+    run = batch.run_tokens(heads // kv_heads)
+
+    def result(cache, splits):
+        out = torch.empty(batch.tokens, heads * dv, device="cuda", dtype=torch.bfloat16)
+        args = (q, cache, batch.pos, batch.owner, batch.tables, batch.tiles(run), run, batch.max_end, kv_heads, dv, 0, dk**-0.5)
+        if kind == "paired":
+            hip.paired_attention(*args, 0.7, 0.4, 1e-3, dv, None, out, splits)
+        elif kind == "capped":
+            hip.capped_attention(*args, 2.0, out, splits)
+        else:
+            hip.sigmoid_attention(*args, torch.zeros(heads, device="cuda"), out, splits)
+        return out
+
+    for p, s, n in zip(pages, starts, lens):
+        held = cache[p].view(-1, cache.shape[-1])
+        held[s + n :] = float("nan")
+        cache[p] = held.view(-1, PAGE_SIZE, cache.shape[-1])
+    zeros = cache.nan_to_num(0)
+    zeros[0] = 0
+    batch.tables[0, 0] = 0
+    want = [result(zeros, splits) for splits in (1, 3)]
+    batch.tables[0, 0] = 7
+    for w, splits in zip(want, (1, 3)):
+        assert w.isfinite().all() and torch.equal(result(cache, splits), w)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,dk,dv", [(2, 2, 256, 256), (16, 1, 256, 256), (3, 3, 160, 144), (4, 2, 256, 128), (2, 2, 128, 256)])
 @pytest.mark.parametrize("keys", [(1, 32, 33), (128, 129, 160), (600, 511, 385)])
 def test_pairs_of_wide_heads(heads, kv_heads, dk, dv, keys):
