@@ -348,13 +348,14 @@ def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=Non
         x2, added = rows()
         return hip.gemm_nf4_rows(x2, weight.tiles, weight.scales, epilogue, added, bias).view(*x.shape[:-1], -1)
     w = weight.dense()
-    m, followed = x.numel() // k, epilogue in (_GEMM_RESIDUAL, _GEMM_SWIGLU)
-    if by_kernel and prompt_grad.gemm_matrix(w) and (
-        prompt_grad.takes_gemm(m, k, n, fused=fused, added=epilogue == _GEMM_RESIDUAL)
-        or prompt_grad.takes_wide_gemm(m, k, n, followed=followed)
-    ):
-        x2, added = rows()
-        return hip.gemm_rows(x2, w, False, epilogue, added, bias).view(*x.shape[:-1], -1)
+    if by_kernel and prompt_grad.gemm_matrix(w):  # which has rows
+        m, followed = x.numel() // k, epilogue in (_GEMM_RESIDUAL, _GEMM_SWIGLU)
+        if (
+            prompt_grad.takes_gemm(m, k, n, fused=fused, added=epilogue == _GEMM_RESIDUAL)
+            or prompt_grad.takes_wide_gemm(m, k, n, followed=followed)
+        ):
+            x2, added = rows()
+            return hip.gemm_rows(x2, w, False, epilogue, added, bias).view(*x.shape[:-1], -1)
     y = torch.matmul(x, w)
     if epilogue == _GEMM_RESIDUAL:
         return residual + y if bias is None else hip.add_rows(residual, y, None, bias)

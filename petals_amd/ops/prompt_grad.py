@@ -288,10 +288,10 @@ def rows_product(x, w, hip, transposed=False):
     """x [..., K] times w [K, N], or [..., N] times its transpose: by ops/csrc/gemm.hip where that is
     the faster one, else the library's."""
     k, n = w.shape if not transposed else w.shape[::-1]
-    m = x.numel() // k
-    # torch refuses rows of other lengths
-    if x.shape[-1] == k and (takes_gemm(m, k, n, transposed) or takes_wide_gemm(m, k, n, transposed)):
-        return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
+    if k and x.shape[-1] == k:  # torch refuses rows of other lengths
+        m = x.numel() // k
+        if takes_gemm(m, k, n, transposed) or takes_wide_gemm(m, k, n, transposed):
+            return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
     return torch.matmul(x, w.t() if transposed else w)
 
 

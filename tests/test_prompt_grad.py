@@ -290,6 +290,20 @@ def test_products_of_rows_that_do_not_fit(monkeypatch):
     assert y.shape == (4, 128)
 
 
+def test_products_with_a_matrix_without_rows():
+    """Sums of nothing are zeros, as by torch's product; rows of some length don't fit."""
+    from types import SimpleNamespace
+
+    from petals_amd.ops.fused_decode import prompt_product
+
+    w = torch.ones(0, 128, dtype=torch.float64)
+    weight = SimpleNamespace(shape=w.shape, tiles=None, dense=lambda: w)
+    for product in (lambda x: prompt_product(HIP, x, weight), lambda x: prompt_grad._Product.apply(x, w, HIP)):
+        assert torch.equal(product(torch.ones(2, 3, 0, dtype=torch.float64)), torch.zeros(2, 3, 128, dtype=torch.float64))
+        with pytest.raises(RuntimeError, match="mat"):
+            product(torch.ones(3, 64, dtype=torch.float64))
+
+
 def test_products_under_autocast(monkeypatch):
     """They come in the type that autocast gives torch's products, with gradients. Devices that have
     no autocast are not asked for it."""
