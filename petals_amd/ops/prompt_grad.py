@@ -260,7 +260,8 @@ class _Attention(torch.autograd.Function):
     def backward(ctx, g):
         (qkv, rows, sums), (cos, sin) = ctx.saved_tensors, ctx.tables
         none = (None,) * 8
-        if _by_torch(g):
+        # the kernels address a tile's rows by 32 bits
+        if _by_torch(g) or qkv.shape[-1] >= 1 << 24:
             return (*_through_torch(lambda t: torch_attention(t, cos, sin, *ctx.shape), (qkv,), (g,)), *none)
         return (ctx.hip.attn_prompt_grad(aligned(rows), aligned(g), sums, cos, sin, *ctx.shape, ctx.scale), *none)
 

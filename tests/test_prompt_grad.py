@@ -290,6 +290,26 @@ def test_products_of_rows_that_do_not_fit(monkeypatch):
     assert y.shape == (4, 128)
 
 
+def test_attention_gradients_of_the_widest_rows():
+    """Rows of 2^24 numbers, which the kernels' offsets don't reach, have the gradients of torch operations."""
+    hd, kh = 64, 1 << 16
+    qh, tables = 2 * kh, (torch.ones(1, hd), torch.zeros(1, hd))
+
+    class Narrow(Kernels):
+        def attn_prefill_sums(self, q, k, v, scale):
+            return v.repeat_interleave(2, 1).transpose(1, 2).flatten(2), torch.zeros(1)  # one key has all the weight
+
+        def attn_prompt_grad(self, rows, g, *rest):
+            raise RuntimeError("too many rows at once")
+
+    qkv = torch.randn(1, 1, (qh + 2 * kh) * hd, generator=torch.Generator().manual_seed(1)).requires_grad_(True)
+    out = prompt_grad.attention(qkv, *tables, 0, qh, kh, hd, hd**-0.5, Narrow())
+    (got,) = torch.autograd.grad(out, qkv, torch.ones_like(out))
+    want = torch.zeros(qkv.shape)
+    want[..., -kh * hd :] = 2
+    assert torch.equal(got, want)
+
+
 def test_products_with_a_matrix_without_rows():
     """Sums of nothing are zeros, as by torch's product; rows of some length don't fit."""
     from types import SimpleNamespace
