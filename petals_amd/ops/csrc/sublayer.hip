@@ -606,9 +606,10 @@ std::vector<torch::Tensor> sublayer_out(
   int* selp = experts ? sel.data_ptr<int>() : nullptr;
   float* selwp = experts ? sel_w.data_ptr<float>() : nullptr;
   if (t > 0) {
-  // rows that reach to the end of what is written, with a weight that 16-byte loads can read
+  // rows that reach to the end of what is written, with a weight that 16-byte loads can read; the kernel reads the first
+  // of a token's rows whatever their number
   const int groups = (d + 2047) / 2048;
-  const bool rows = t >= 64 && d == dp && y_wide && groups <= 4 && reinterpret_cast<uintptr_t>(norm_w.data_ptr()) % 16 == 0 &&
+  const bool rows = t >= 64 && k > 0 && d > 0 && d == dp && y_wide && groups <= 4 && reinterpret_cast<uintptr_t>(norm_w.data_ptr()) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(xp) % 16 == 0;
 #define SO_ROWS(TY, TW, YP, G)                                                                               \
   sublayer_out_rows_kernel<TY, TW, G><<<t, 256, lds, stream>>>(                                              \

@@ -620,6 +620,19 @@ def test_sublayer_out_of_many_rows(d, slots, router):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("t", [1, 64])
+@pytest.mark.parametrize("d,slots", [(128, 0), (0, 0), (0, 1)])
+def test_sublayer_out_of_nothing(t, d, slots):
+    """No rows to sum, or no columns: the residual, whichever kernel many rows have."""
+    from petals_amd.ops import latent
+
+    y, w, weights = torch.ones(t * slots, d, device="cuda").bfloat16(), torch.ones(d, device="cuda"), torch.ones(t, slots, device="cuda")
+    x = torch.randn(t, d, device="cuda")
+    xo, xb, _, _ = latent.hip().sublayer_out(y, weights, w, 1e-6, x, d, True, None, 1)
+    assert torch.equal(xo, x) and torch.equal(xb, x.bfloat16())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("t,h,k,n", [(1, 3, 32, 40), (16, 2, 96, 130), (17, 1, 45, 33), (200, 4, 128, 96)])
 @pytest.mark.parametrize("a_dtype", ["float32", "bfloat16"])
 def test_batched_linear_kernel(t, h, k, n, a_dtype):
