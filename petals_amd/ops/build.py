@@ -89,6 +89,9 @@ def build(verbose: bool = False, name: str = "core") -> str:
         is_standalone=False,
         keep_intermediates=True,
     )
+    from petals_amd.ops import sums_check
+
+    sums_check.check(build_dir)
     # copy the built .so in-tree under a stable name
     built = os.path.join(build_dir, ext_name + ".so")
     if os.path.exists(built):

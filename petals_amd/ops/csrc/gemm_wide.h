@@ -19,7 +19,8 @@
 //
 // The matrix instructions are in asm: their sums stay in one register each there, where the compiler moved
 // a third of them about in every step. It does not see their hazards, so: operands come from LDS loads only, whose
-// waits it does see; sums are set before a barrier; and none is read within 32 cycles after the last one.
+// waits it does see; sums are set before a barrier; and none is read within 32 cycles after the last one. Nor may it copy or
+// spill a sum within a loop. ops/sums_check.py looks at what was built for all of this, and the build fails if it isn't so.
 #pragma once
 
 #include "gemm.h"
