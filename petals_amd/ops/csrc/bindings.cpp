@@ -91,7 +91,7 @@ std::vector<torch::Tensor> moe_group(torch::Tensor sel, int64_t experts, int64_t
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> nf4_all,
     c10::optional<torch::Tensor> scales_all, torch::Tensor x, torch::Tensor sorted_pairs,
-    torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows);
+    torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows, bool general);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16 -> bf16)");
@@ -173,5 +173,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "grouped MFMA GEMM over expert-sorted (token, slot) pairs (prefill; NF4 dequant fused "
         "into the LDS B-tile staging)",
         py::arg("wt_all"), py::arg("nf4_all"), py::arg("scales_all"), py::arg("x"),
-        py::arg("sorted_pairs"), py::arg("tile_expert"), py::arg("k_per_tok"), py::arg("n_rows"));
+        py::arg("sorted_pairs"), py::arg("tile_expert"), py::arg("k_per_tok"), py::arg("n_rows"), py::arg("general") = false);
 }

@@ -12,7 +12,7 @@ torch::Tensor gemv_bf16_moe(
 torch::Tensor moe_gemm(
     c10::optional<torch::Tensor> wt_all, c10::optional<torch::Tensor> nf4_all,
     c10::optional<torch::Tensor> scales_all, torch::Tensor x, torch::Tensor sorted_pairs,
-    torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows);
+    torch::Tensor tile_expert, int64_t k_per_tok, int64_t n_rows, bool general);
 torch::Tensor latent_attention(
     torch::Tensor q, torch::Tensor cache, torch::Tensor pos, torch::Tensor owner, torch::Tensor tables,
     torch::Tensor tiles, int64_t run_tokens, int64_t max_keys, int64_t window, double scale, int64_t splits,
@@ -36,7 +36,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("wt_all"), py::arg("x"), py::arg("sel"), py::arg("k_per_tok"),
         py::arg("workspace"), py::arg("epilogue"), py::arg("splits") = 0,
         py::arg("limit") = 0.0, py::arg("alpha") = 0.0);
-  m.def("moe_gemm", &moe_gemm, "grouped MFMA GEMM over expert-sorted pairs");
+  m.def("moe_gemm", &moe_gemm, "grouped MFMA GEMM over expert-sorted pairs",
+        py::arg("wt_all"), py::arg("nf4_all"), py::arg("scales_all"), py::arg("x"), py::arg("sorted_pairs"),
+        py::arg("tile_expert"), py::arg("k_per_tok"), py::arg("n_rows"), py::arg("general") = false);
   m.def("latent_attention", &latent_attention, "sliding-window latent attention over a paged cache",
         py::arg("q"), py::arg("cache"), py::arg("pos"), py::arg("owner"), py::arg("tables"), py::arg("tiles"),
         py::arg("run_tokens"), py::arg("max_keys"), py::arg("window"), py::arg("scale"), py::arg("splits") = 0,

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
 // pairs by expert with each expert's segment padded to a multiple of MT rows, so every
 // MT-row tile belongs to ONE expert (tile_expert[tile], -1 = pure padding).
 //
-// NF4 weights, and bf16 beyond offsets of 32 bits (the others: moe_wide_kernel below).
+// NF4 weights, and bf16 beyond offsets of 32 bits or where a call asks for it (the others: moe_wide_kernel below).
 // Up to four tiles of one expert (128 rows) and 256 columns are a workgroup's: an
 // expert's weights are read once per 128 of its rows, and the rows once per 256 columns.
 // With a tile of 32 rows and 128 columns each, weights crossed the caches four times as
@@ -545,7 +545,9 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_kernel(
 // bf16 weights, rows in groups of up to 256 that are as equal as tiles of 32 allow, by gemm_wide.h: two groups of 145
 // rows are two tiles of 160 where groups of 128 rows were three, the last one nearly empty, and four waves take less
 // from LDS for a product. Both products of a layer of 8 experts, width 4096 and inner size 14336, with 290 rows an expert
-// and routing as it comes: from 698 and 405 to 571 and 310 us. With 71 rows weights are what bounds either (5.0 TB/s).
+// and routing as it comes: from 698 and 405 to 571 and 310 us. With fewer rows weights are what bounds it (5.0 TB/s), and what it gains is that
+// 128 columns keep more compute units busy: 10 rows an expert 318 and 318, 185 and 158 us. profiles/expert_products.csv has 1 to 750 rows:
+// 1.5% slower at most, 14% faster in the mean.
 struct MoeGroup {
   int tile, tiles, column;  // first tile and number of tiles (0: none); run of columns
 };
@@ -773,7 +775,8 @@ torch::Tensor moe_gemm(
     torch::Tensor sorted_pairs,               // [Rp] i32 (expert-sorted, MT-padded, -1 = pad)
     torch::Tensor tile_expert,                // [Rp/MT] i32 (-1 = pure padding tile)
     int64_t k_per_tok,
-    int64_t n_rows) {                         // R = T * k_per_tok (C rows)
+    int64_t n_rows,                           // R = T * k_per_tok (C rows)
+    bool general) {                           // by moe_gemm_kernel whatever the sizes, for tests
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16 && x.dim() == 2 && x.is_contiguous());
   TORCH_CHECK(sorted_pairs.dtype() == torch::kInt32 && sorted_pairs.is_contiguous());
   TORCH_CHECK(tile_expert.dtype() == torch::kInt32 && tile_expert.is_contiguous());
@@ -805,7 +808,7 @@ torch::Tensor moe_gemm(
   auto c = torch::empty({n_rows, (long)out_dim}, x.options());
   const long n_tiles = Rp / MOE_MT, experts = nf4 ? nf4_all->size(0) : wt_all->size(0);
   // offsets into an expert's weights and into rows are 32-bit there
-  if (!nf4 && (long)in_dim * out_dim < (1L << 31) && x.size(0) * in_dim < (1L << 31)) {
+  if (!general && !nf4 && (long)in_dim * out_dim < (1L << 31) && x.size(0) * in_dim < (1L << 31)) {
     launch_moe_wide(*wt_all, x, sorted_pairs, tile_expert, c, k_per_tok, n_rows);
     return c;
   }

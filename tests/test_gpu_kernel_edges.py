@@ -107,6 +107,30 @@ def test_expert_gemm_equal_groups(hip, counts, k_in, n_out):
 
 
 @requires_gpu
+@pytest.mark.parametrize(
+    "counts,k_in,n_out",
+    [([1], 64, 128), ([0, 32, 33, 0, 5], 128, 384), ([128, 129, 127, 31], 192, 256), ([2050, 40], 64, 128), ([1100, 40], 192, 2304)],
+)
+def test_expert_gemm_without_limits(hip, counts, k_in, n_out):
+    """The kernel that experts beyond offsets of 32 bits have, which no test is large enough for."""
+    from petals_amd.ops.fused_moe import MOE_GEMM_MT
+
+    gen = torch.Generator(device="cuda").manual_seed(sum(counts))
+    w = (torch.randn(len(counts), k_in, n_out, device="cuda", generator=gen) * 0.05).to(BF16)
+    pairs = torch.cat([torch.full((n,), e, device="cuda", dtype=torch.int32) for e, n in enumerate(counts)])
+    pairs = pairs[torch.randperm(len(pairs), device="cuda", generator=gen)]
+    x = torch.randn(len(pairs), k_in, device="cuda", generator=gen).to(BF16)
+    order, tiles = hip.moe_group(pairs, len(counts), MOE_GEMM_MT)
+    out = hip.moe_gemm(w, None, None, x, order, tiles, 1, len(pairs), general=True).double()
+    for e in range(len(counts)):
+        mine, we = pairs == e, w[e].double()
+        ref = x[mine].double() @ we
+        # 32-bit sums of exact products of bf16, rounded once
+        loose = k_in * 2.0**-24 * (x[mine].double().abs() @ we.abs())
+        assert bool(((out[mine] - ref).abs() <= 2.0**-8 * ref.abs() + loose).all()), e
+
+
+@requires_gpu
 def test_gelu_over_all_of_bf16(hip):
     """GELU of every finite bf16 number, infinities and NaN, beside 64 bits."""
     x = torch.arange(1 << 16, device="cuda", dtype=torch.int32).to(torch.int16).view(BF16)
