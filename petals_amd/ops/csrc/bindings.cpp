@@ -57,7 +57,7 @@ std::vector<torch::Tensor> add_norm_rows(
 torch::Tensor add_rows(torch::Tensor x, torch::Tensor y, c10::optional<torch::Tensor> z, c10::optional<torch::Tensor> bias);
 torch::Tensor swiglu_rows(torch::Tensor gu);
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
-                        c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile);
+                        c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile, bool steady);
 torch::Tensor gemm_nf4_rows(torch::Tensor x, torch::Tensor tiles, torch::Tensor scales, int64_t epilogue,
                             c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile);
 void bias_gelu_rows(torch::Tensor y, c10::optional<torch::Tensor> bias);
@@ -151,7 +151,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x"), py::arg("y"), py::arg("z") = py::none(), py::arg("bias") = py::none());
   m.def("gemm_rows", &gemm_rows, "a prompt's rows times a bf16 matrix, and what follows", py::arg("x"), py::arg("w"),
         py::arg("transposed") = false, py::arg("epilogue") = 0, py::arg("residual") = py::none(),
-        py::arg("bias") = py::none(), py::arg("tile") = -1);
+        py::arg("bias") = py::none(), py::arg("tile") = -1, py::arg("steady") = false);
   m.def("gemm_nf4_rows", &gemm_nf4_rows, "a prompt's rows times NF4 tiles, and what follows", py::arg("x"), py::arg("tiles"),
         py::arg("scales"), py::arg("epilogue") = 0, py::arg("residual") = py::none(), py::arg("bias") = py::none(),
         py::arg("tile") = -1);

@@ -6,8 +6,9 @@
 // without a tile (758 x 4096 has 48 tiles of 256 x 256) or one with twice the others' work,
 // and read weights at 2 TB/s where a prompt of 128 tokens is bound by reading them.
 //
-// Two kinds of tiles. Those of 96 to 256 rows and 256 columns are four waves' (gemm_wide.h), bound by the way from L2 to
-// LDS and by the matrix cores. Smaller ones, for few rows or columns, are those of 8 waves: BM x BN and K in steps of 64,
+// Two kinds of tiles. Those of 160 to 256 rows and 256 columns, of 96 rows, and of 128 x 192, are four waves' (gemm_wide.h), bound by the
+// way from L2 to LDS and by the matrix cores. Those for fewer rows or columns, or short K, are eight waves': up to 128 x 256, where one wave's store
+// runs beneath another's products (by four waves 2048 x 11264 took 40.8 us at 640 rows, not 37.4, and 1.5% longer over all). BM x BN and K in steps of 64,
 // through ST buffers of LDS that are filled straight from memory (buffer_load ... lds: no registers, no stores, and
 // what lies beyond the rows or columns repeats the last ones). A step is two phases of 32 of K;
 // in each, the matrix cores work on one set of fragments while the next set is read from LDS
@@ -21,16 +22,16 @@
 // kernel adds their parts up. Each chiplet has its own consecutive run of tiles, rows first: they find
 // a run of columns' weights in its L2. The product is W^T X^T, so that a lane ends with 4 neighbouring columns of one row.
 //
-// MI355X, us, the library's kernels, those of 8 waves alone (tiles of 128 x 256 at most), and these, with their sum of
+// MI355X, us, the library's kernels, the best of those of eight waves, and the tile that is chosen, with their sum of
 // parts, weights from memory:
-//   rows                 16        128         512              758              1024
-//   4096 x 4096        19, 14    33, 18    31, 28, 26       35, 36, 29       39, 38, 33
-//   4096 x 22016                           89, 97, 91      133, 138, 121    167, 185, 160
-//   11008 x 4096                           96, 58, 54      103, 85, 68      110, 98, 86
-//   16384 x 4096       79, 34   139, 38   139, 74, 70      147, 119, 91
-//   28672 x 8192      134, 86   199, 96   349, 216, 188    299, 389, 272    370, 423, 344
-//   22016, transposed, to 4096:           229, 102, 87     231, 162, 119    248, 180, 143
-//   12288, transposed, to 4096:            79, 62, 55       91, 96, 73      112, 112, 90
+//   rows                   128                 512                758               1024
+//   4096 x 4096         39, 19, 19          39, 31, 31         41, 40, 40         44, 41, 41
+//   4096 x 22016        67, 51, 47          89, 107, 99       134, 134, 128      167, 179, 169
+//   11008 x 4096        96, 29, 29          96, 54, 54        101, 86, 69        110, 90, 87
+//   16384 x 4096       139, 38, 38         138, 74, 71        146, 120, 92       157, 124, 116
+//   28672 x 8192       207, 100, 99        357, 214, 196      307, 376, 295      376, 387, 359
+//   22016, transposed, to 4096:  114, 52, 51    234, 102, 89   231, 160, 117      247, 165, 144
+//   12288, transposed, to 4096:   66, 32, 32     78, 59, 59     89, 97, 76        109, 99, 91
 // A call takes the host 8 us, the library's 18. Which of the two a product takes are ops/prompt_grad.py's rules
 // (takes_gemm, takes_wide_gemm); profiles/prompt_products.csv and prompt_products_wide.csv have what they were drawn from.
 
@@ -341,22 +342,21 @@ static void launch_gemm_wide(const unsigned short* x, const unsigned short* w, c
 
 // ------------------------------------------------------------------- host
 
-// step, fixed and alone by least squares over 780 products of the presets, 17 to 4096 rows, in either direction: 12% off in
-// the mean; the tile that they choose takes 1.1% more than the best one. 192, 160 and 96 rows are 1 to 3% dearer than that fit:
-// with it 65 to 96 rows of 14336 x 4096 had tiles of 96 rows, 34.3 us beside 31.7, and 320 of 4544 x 18176 those of 160, 77 beside 67
-static const GemmTile GEMM_TILES[] = {{128, 256, 0.83f, 4.6f, 0.72f}, {128, 128, 0.54f, 2.2f, 0.81f}, {64, 256, 0.66f, 6.f, 0.88f},
-                                      {32, 256, 0.57f, 3.7f, 1.f},    {256, 256, 1.42f, 2.f, 0.68f},  {192, 256, 1.16f, 2.7f, 0.69f},
-                                      {160, 256, 0.96f, 4.4f, 0.65f}, {96, 256, 0.75f, 4.9f, 0.82f}, {128, 192, 0.72f, 4.4f, 0.7f}};
+// step, fixed and alone by least squares over 1539 products of the presets, 17 to 4096 rows, in either direction, with what
+// follows: 7% off in the mean. The tile that they choose takes 1.0% more than the best one, 1.4% for matrices of up to 25 million
+// weights (profiles/prompt_products_wide.csv)
+static const GemmTile GEMM_TILES[] = {{128, 256, 0.863f, 6.7f, 0.82f}, {128, 128, 0.554f, 4.6f, 0.96f}, {64, 256, 0.668f, 5.9f, 1.f},
+                                      {32, 256, 0.564f, 4.4f, 1.f},    {256, 256, 1.469f, 5.f, 0.84f},  {192, 256, 1.205f, 5.3f, 0.75f},
+                                      {160, 256, 1.032f, 6.f, 0.7f},   {96, 256, 0.782f, 5.5f, 0.92f},  {128, 192, 0.73f, 5.3f, 0.9f}};
 
-// Matrices of up to 25 million weights (4096 x 6144): tiles beyond these gain up to 4 us of 40 there, and would split other sums
-// along K. A sum in another order is rounded otherwise now and then, which for the products ahead of routed experts (8 experts
-// of width 4096 among them) sends a token to another of two nearly equal experts. Sizes that are no multiples of 128
-// gain a third and have no such models.
-static const GemmTile GEMM_SMALL[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
+// For what a router reads: the first four tiles alone, by the cost of their steps alone. A sum that is cut along K elsewhere is as
+// exact but rounds otherwise now and then, which sends a token to the other of two experts that score alike. So these products keep
+// their cuts whatever is measured for the others, and whoever has a router asks for it (`steady`).
+static const GemmTile GEMM_STEADY[] = {{128, 256, 0.92f}, {128, 128, 0.55f}, {64, 256, 0.65f}, {32, 256, 0.5f}};
 
 // x [M, K] bf16, w [K, N] (or [N, K], transposed) bf16 -> [M, N] bf16 (swiglu: [M, N/2])
 torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64_t epilogue,
-                        c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile) {
+                        c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> bias, int64_t tile, bool steady) {
   for (const auto& t : {x, w})
     TORCH_CHECK(t.is_cuda() && t.dtype() == torch::kBFloat16 && t.dim() == 2 && t.is_contiguous() &&
                 reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "gemm_rows takes aligned bf16 matrices");
@@ -382,18 +382,19 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
                 bias->numel() == n && reinterpret_cast<uintptr_t>(bias->data_ptr()) % 8 == 0);
     o.bias = BF16P(*bias);
   }
-  const bool small = tile < 0 && k * n <= 3L << 23 && k % 128 == 0 && n % 128 == 0;
-  const int usable = small ? (int)(sizeof(GEMM_SMALL) / sizeof(GemmTile)) : (int)(sizeof(GEMM_TILES) / sizeof(GemmTile));
   int best = 0;
   float least = 0.f;
   GemmShape s{};
-  for (int i = 0; i < (int)(sizeof(GEMM_TILES) / sizeof(GemmTile)); ++i) {
-    if (tile >= 0 ? tile != i : i >= usable || (pairs && GEMM_TILES[i].bn == 192)) continue;
+  steady = steady && tile < 0;
+  const GemmTile* const tiles = steady ? GEMM_STEADY : GEMM_TILES;
+  const int count = steady ? sizeof(GEMM_STEADY) / sizeof(GemmTile) : sizeof(GEMM_TILES) / sizeof(GemmTile);
+  for (int i = 0; i < count; ++i) {
+    if (tile >= 0 ? tile != i : pairs && tiles[i].bn == 192) continue;
     float us;
-    const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, small ? GEMM_SMALL[i] : GEMM_TILES[i], &us);
+    const GemmShape p = gemm_plan(m, n, k, GEMM_BK, 8, tiles[i], &us);
     if (s.m == 0 || us < least) best = i, least = us, s = p;
   }
-  const GemmTile& t = GEMM_TILES[best];
+  const GemmTile& t = tiles[best];
   TORCH_CHECK(s.m && !(pairs && t.bn == 192), "gemm_rows: no such tile");  // 96 gates would not be whole pairs of fragments
   torch::Tensor parts;
   if (s.splits > 1) {
@@ -430,10 +431,10 @@ torch::Tensor gemm_rows(torch::Tensor x, torch::Tensor w, bool transposed, int64
     else launch_gemm_wide<false, ROWS, COLUMNS>(BF16P(x), BF16P(w), s, o, blocks, stream);                   \
   } while (0)
   switch (best) {
+    case 0: GEMM_EITHER(2, 4, 4, 4, 3); break;
     case 1: GEMM_EITHER(2, 4, 4, 2, 4); break;
     case 2: GEMM_EITHER(2, 4, 2, 4, 4); break;
     case 3: GEMM_EITHER(1, 8, 2, 2, 4); break;
-    case 0: GEMM_WIDE(8, 16); break;
     case 4: GEMM_WIDE(16, 16); break;
     case 5: GEMM_WIDE(12, 16); break;
     case 6: GEMM_WIDE(10, 16); break;

@@ -330,9 +330,10 @@ _GEMM_GELU = 2
 _GEMM_SWIGLU = 3
 
 
-def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=None):
+def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=None, steady=False):
     """A prompt's rows [..., K] times a _FastWeight, without gradients, and what follows: residual +
-    y + bias, gelu(y + bias), or the SwiGLU of [gate | up]."""
+    y + bias, gelu(y + bias), or the SwiGLU of [gate | up]. `steady`: a router reads what comes of it, and its sums
+    stay cut along K as they are, whichever tiles are the faster ones (ops/csrc/gemm.hip)."""
     k, n = weight.shape
     fused = epilogue in (_GEMM_GELU, _GEMM_SWIGLU)
     by_kernel = (
@@ -352,10 +353,10 @@ def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=Non
         m, followed = x.numel() // k, epilogue in (_GEMM_RESIDUAL, _GEMM_SWIGLU)
         if (
             prompt_grad.takes_gemm(m, k, n, fused=fused, added=epilogue == _GEMM_RESIDUAL)
-            or prompt_grad.takes_wide_gemm(m, k, n, followed=followed)
+            or not steady and prompt_grad.takes_wide_gemm(m, k, n, followed=followed)
         ):
             x2, added = rows()
-            return hip.gemm_rows(x2, w, False, epilogue, added, bias).view(*x.shape[:-1], -1)
+            return hip.gemm_rows(x2, w, False, epilogue, added, bias, -1, steady).view(*x.shape[:-1], -1)
     y = torch.matmul(x, w)
     if epilogue == _GEMM_RESIDUAL:
         return residual + y if bias is None else hip.add_rows(residual, y, None, bias)
@@ -582,7 +583,10 @@ class LlamaFastPath(_TPFastPathMixin):
 
     def _matmul(self, x, weight, autograd: bool):
         """x times a weight, differentiable when autograd."""
-        return prompt_grad.product(x, weight.dense(), self.hip) if autograd else prompt_product(self.hip, x, weight)
+        steady = not self.dense_mlp  # routed experts follow, in this block and in all after it
+        if autograd:
+            return prompt_grad.product(x, weight.dense(), self.hip, steady)
+        return prompt_product(self.hip, x, weight, steady=steady)
 
     def _ensure_rope(self, needed: int):
         if self.rope_cos is None or self.rope_cos.shape[0] < needed:

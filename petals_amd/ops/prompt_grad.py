@@ -268,31 +268,32 @@ class _Attention(torch.autograd.Function):
 
 class _Product(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w, hip):
+    def forward(ctx, x, w, hip, steady=False):
         # saved as torch's product saves it: hooks see it, and a change before the backward pass is
         # an error. What was made in inference mode can't be saved
         ctx.w = w if w.is_inference() else None
         if ctx.w is None:
             ctx.save_for_backward(w)
         ctx.hip = hip
-        return rows_product(x, w, hip)
+        return rows_product(x, w, hip, steady=steady)
 
     @staticmethod
     def backward(ctx, g):
         w = ctx.saved_tensors[0] if ctx.w is None else ctx.w
         if _by_torch(g, w):
-            return torch.matmul(g, w.t()), None, None
-        return rows_product(g, aligned(w), ctx.hip, transposed=True), None, None
+            return torch.matmul(g, w.t()), None, None, None
+        return rows_product(g, aligned(w), ctx.hip, transposed=True), None, None, None
 
 
-def rows_product(x, w, hip, transposed=False):
+def rows_product(x, w, hip, transposed=False, steady=False):
     """x [..., K] times w [K, N], or [..., N] times its transpose: by ops/csrc/gemm.hip where that is
-    the faster one, else the library's."""
+    the faster one, else the library's. `steady`: a router reads the result, see there."""
     k, n = w.shape if not transposed else w.shape[::-1]
     if k and x.shape[-1] == k:  # torch refuses rows of other lengths
         m = x.numel() // k
-        if takes_gemm(m, k, n, transposed) or takes_wide_gemm(m, k, n, transposed):
-            return hip.gemm_rows(aligned(x).view(-1, k), w, transposed).view(*x.shape[:-1], n)
+        if takes_gemm(m, k, n, transposed) or not steady and takes_wide_gemm(m, k, n, transposed):
+            rest = (0, None, None, -1, True) if steady else ()
+            return hip.gemm_rows(aligned(x).view(-1, k), w, transposed, *rest).view(*x.shape[:-1], n)
     return torch.matmul(x, w.t() if transposed else w)
 
 
@@ -300,11 +301,11 @@ def norm(x, w, eps, hip):
     return _Norm.apply(x, w, eps, hip)
 
 
-def product(x, w, hip):
+def product(x, w, hip, steady=False):
     """x [..., K] times a frozen matrix [K, N]"""
     if w.requires_grad or not (fused_training(x) and gemm_matrix(w)) or recast(x):
         return torch.matmul(x, w)
-    return _Product.apply(x, w, hip)
+    return _Product.apply(x, w, hip, steady)
 
 
 def add_norm(x, y, w, eps, hip):

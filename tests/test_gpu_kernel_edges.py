@@ -1,6 +1,8 @@
 """HIP kernels at the sizes where their tiles, splits and rules of dispatch change,
 against plain 32-bit or 64-bit references."""
 
+import dataclasses
+
 import pytest
 import torch
 
@@ -1049,7 +1051,7 @@ def test_prompt_product_edges(hip, m, k, n, tile, transposed):
 
 @requires_gpu
 @pytest.mark.parametrize("transposed", [False, True])
-@pytest.mark.parametrize("tile", [0, 4, 5, 6, 7, 8])  # 128, 256, 192, 160 and 96 rows; 128 and 192 columns
+@pytest.mark.parametrize("tile", [0, 4, 5, 6, 7, 8])  # 128 (eight waves), 256, 192, 160 and 96 rows; 128 and 192 columns
 @pytest.mark.parametrize(
     "m,k,n",
     [
@@ -1067,6 +1069,51 @@ def test_prompt_products_of_four_waves(hip, m, k, n, tile, transposed):
         return test_prompt_product_edges(hip, m, k, n, tile, transposed)
     with pytest.raises(RuntimeError, match="no such tile"):  # for gates and ups, which come last
         test_prompt_product_edges(hip, m, k, n, tile, transposed)
+
+
+@requires_gpu
+@pytest.mark.parametrize(
+    "m,k,n,tile,own",
+    [
+        (17, 4096, 4096, 3, True), (64, 4096, 6144, 2, False), (100, 4096, 4096, 1, True), (150, 6144, 8192, 0, False),
+        (200, 4096, 6144, 0, False), (283, 4096, 6144, 2, False),  # `own`: others have that tile too
+    ],
+)
+def test_products_ahead_of_a_router(hip, m, k, n, tile, own):
+    """Their sums are cut along K as the tiles of eight waves cut them, to the bit."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x, w = (torch.randn(*s, device="cuda", generator=gen).to(BF16) for s in ((m, k), (k, n)))
+    steady = hip.gemm_rows(x, w, steady=True)
+    assert torch.equal(steady, hip.gemm_rows(x, w, tile=tile))
+    assert torch.equal(steady, hip.gemm_rows(x, w)) == own
+
+
+@requires_gpu
+@pytest.mark.parametrize("model,routed", [("test-mixtral", True), ("tinyllama-1.1b", False)])
+def test_blocks_with_a_router_ask_for_steady_products(hip, monkeypatch, model, routed):
+    from petals_amd.models.config_base import load_model_config
+    from petals_amd.server.from_pretrained import build_empty_block, init_random_block_
+
+    config = load_model_config(model)
+    if routed:  # heads that the kernels take
+        config = dataclasses.replace(config, hidden_size=256, intermediate_size=256)
+    block = build_empty_block(config, 0, torch.device("cuda"), BF16)
+    init_random_block_(block, config, 0)
+    block = block.eval().optimize_for_inference()
+    asked, gemm_rows = set(), hip.gemm_rows
+
+    def watched(x, w, transposed=False, epilogue=0, residual=None, bias=None, tile=-1, steady=False):
+        asked.add((transposed, steady))
+        return gemm_rows(x, w, transposed, epilogue, residual, bias, tile, steady)
+
+    monkeypatch.setattr(hip, "gemm_rows", watched)
+    x = torch.randn(2, 20, config.hidden_size, device="cuda").to(BF16)
+    with torch.inference_mode():
+        block(x)
+    assert asked == {(False, routed)}
+    leaf = x.clone().requires_grad_(True)
+    block(leaf).sum().backward()
+    assert asked == {(False, routed), (True, False)}  # no router reads gradients
 
 
 @requires_gpu

@@ -290,6 +290,26 @@ def test_products_of_rows_that_do_not_fit(monkeypatch):
     assert y.shape == (4, 128)
 
 
+@pytest.mark.parametrize("takes", [False, True])
+def test_products_ahead_of_a_router(monkeypatch, takes):
+    """Their sums keep their order, and tiles that have another one are not asked; gradients have the fastest ones."""
+    monkeypatch.setattr(prompt_grad, "takes_gemm", lambda *sizes: takes)
+    monkeypatch.setattr(prompt_grad, "takes_wide_gemm", lambda *sizes: True)
+    asked = []
+
+    class Watched(Kernels):
+        def gemm_rows(self, x, w, transposed=False, epilogue=0, residual=None, bias=None, tile=-1, steady=False):
+            asked.append((transposed, steady))
+            return x @ (w.t() if transposed else w)
+
+    w = torch.randn(64, 128, dtype=torch.float64)
+    x = torch.randn(3, 64, dtype=torch.float64, requires_grad=True)
+    y = prompt_grad._Product.apply(x, w, Watched(), True)
+    torch.testing.assert_close(y, x @ w)
+    torch.testing.assert_close(torch.autograd.grad(y, x, y)[0], y @ w.t())
+    assert asked == [(False, True)] * takes + [(True, False)]
+
+
 def test_attention_gradients_of_the_widest_rows():
     """Rows of 2^24 numbers, which the kernels' offsets don't reach, have the gradients of torch operations."""
     hd, kh = 64, 1 << 16
