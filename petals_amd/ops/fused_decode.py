@@ -353,7 +353,7 @@ def prompt_product(hip, x, weight, epilogue=_GEMM_PLAIN, residual=None, bias=Non
         m, followed = x.numel() // k, epilogue in (_GEMM_RESIDUAL, _GEMM_SWIGLU)
         if (
             prompt_grad.takes_gemm(m, k, n, fused=fused, added=epilogue == _GEMM_RESIDUAL)
-            or not steady and prompt_grad.takes_wide_gemm(m, k, n, followed=followed)
+            or not steady and prompt_grad.takes_wide_gemm(m, k, n, followed=followed, gelu=epilogue == _GEMM_GELU)
         ):
             x2, added = rows()
             return hip.gemm_rows(x2, w, False, epilogue, added, bias, -1, steady).view(*x.shape[:-1], -1)

@@ -105,30 +105,41 @@ def takes_gemm(m: int, k: int, n: int, transposed: bool = False, fused: bool = F
     return m <= 128 or tiles <= (256 if fused else 128)
 
 
-def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: bool = False) -> bool:
+def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: bool = False, gelu: bool = False) -> bool:
     """Whether m rows of k times a large matrix with n columns, which `takes_gemm` leaves to the library, are
-    faster by the tiles of 256 columns that four waves have in ops/csrc/gemm.hip. `followed`: by a residual or a
-    SwiGLU, which would be launches of their own.
+    faster by the large tiles of ops/csrc/gemm.hip. `followed`: by a residual or a SwiGLU, which would be launches of
+    their own; `gelu`: by that, which is a shorter one.
 
-    These are products that the GPU is waited for. Up to 1536 rows the library's tiles leave compute units idle, and
-    it takes 1.13 times as long in the mean; beyond, tiles fill the chip either way, and it is slower only by what
-    follows, or at sizes that are no multiples of 128, for which it has no good kernel. us on MI355X by the library (with what follows) and by the
-    kernel: 4096 x 12288, 758 rows 72, 66; 4096 x 22016, 758 rows 133, 121; 28672 x 8192 with a residual, 758 rows 321, 285;
-    4096 x 28672, 4096 rows 743, 747, with SwiGLU 814, 741; 18176 x 4544, 2048 rows 355, 272.
-    Transposed: 22016 to 4096, 758 rows 231, 119, 4096 rows 540, 620; 8192 to 8192, 512 rows 74, 69, 1024 rows
-    112, 114; 4096 to 11008, 256 rows 50, 44, 512 rows 51, 56. All that was measured: profiles/prompt_products_wide.csv."""
+    These are products that the GPU is waited for. Matrices of fewer columns than rows leave the library's tiles of 256 x 256
+    without work for all compute units up to some 1500 rows, and it takes 1.2 times as long in the mean; the more columns
+    there are, the sooner they fill the chip, and beyond that it is slower only by what follows. Sizes that are no multiples
+    of 128 it has no good kernel for, but where columns are so many that rows don't matter. us on MI355X by the library (with what follows) and
+    by the kernel: 758 rows of 28672 x 8192 with a residual 314, 298, of 4096 x
+    22016 with SwiGLU 144, 124; 4096 x 28672 with SwiGLU, 4096 rows 797, 735; plain, 1024 rows 195, 211; 4096 x 12288, 512 rows
+    57.5, 58.7, 1024 rows 88, 100; 18176 x 4544, 2048 rows 368, 284. Transposed: 22016 to 4096, 758 rows 231, 117;
+    8192 to 8192, 512 rows 74, 71, 1024 rows 110, 115; 4096 to 11008, 256 rows 48, 39, 512 rows 52, 54.
+
+    All that was measured, the median of three runs on three cards, is in profiles/prompt_products_wide.csv: what is taken
+    takes 0.89 of the library's time in the mean, and 1.07 at most."""
     weights = k * n
     if not 128 < m < (1 << 31) // k or weights > 1 << 29:
         return False
-    odd = k % 128 > 0 or n % 128 > 0
-    # smaller ones gain little (4096 x 6144, 758 rows: 53, 49), but for sizes that the library does not like (4544 x 4672: 47, 36)
-    if weights <= 3 << 23 and not (odd and weights >= 1 << 24):
+    odd, small = k % 128 > 0 or n % 128 > 0, weights <= 3 << 23
+    # smaller ones gain little (4096 x 6144, 758 rows: 53, 52), but for sizes that the library does not like
+    if small and not (odd and weights >= 1 << 24):
         return False
     if transposed:
-        # 4544 to 18176: 192 rows 59, 53; 512 rows 81, 96; 758 rows 98, 112; 1200 rows 256, 185; 1500 rows 188, 224; 2048 rows 313, 286
-        odd = odd and (n < 3 * k or m <= 256 or 800 < m <= 1280 or m > 1536)
-        return m <= 1536 and k > n or m <= 640 and k == n or m <= 320 and n < 3 * k or odd
-    return m <= 1536 or followed or odd
+        if small:
+            return m <= 960
+        if k > n:
+            return m <= (1536 if n < 8192 else 1024) or odd
+        return m <= 640 if k == n else m <= 320 and (n < 3 * k or odd)
+    if followed:
+        return True
+    if odd:
+        return gelu or n < 3 * k or m <= 512
+    most = 768 if n <= 3 * k else 320 if n <= 6 * k else 128
+    return m <= (1536 if gelu or n < 2 * k or k >= 5120 else most)
 
 
 def takes_nf4_gemm(m: int, k: int, n: int) -> bool:

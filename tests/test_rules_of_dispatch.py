@@ -1,5 +1,8 @@
 """Rules that choose between two ways of computing the same, beside what was measured on MI355X."""
 
+import csv
+import os
+
 import pytest
 
 from petals_amd.ops.fused_decode import norm_within
@@ -106,31 +109,31 @@ def test_products_of_prompts(k, n, kind, times):
         assert all(kernel <= library + 1.5 for rows, (library, kernel) in times.items() if rows > 300 and takes_gemm(rows, k, n))
 
 
-# the same for the tiles of 256 columns that four waves have, where the library had the product
-WIDE = [
-    (4096, 12288, "", {192: (59.2, 46.1), 512: (59.0, 62.1), 758: (72.7, 66.3), 1024: (88.3, 91.5), 4096: (317, 329)}),
-    (4096, 22016, "followed", {512: (104, 98), 1024: (187, 169), 2048: (385, 311), 4096: (740, 604)}),
-    (4096, 28672, "followed", {512: (116, 109), 1024: (223, 205), 2048: (454, 394), 4096: (842, 757)}),
-    (8192, 57344, "followed", {512: (441, 412), 1024: (846, 767), 2048: (1573, 1463), 4096: (3084, 2858)}),
-    (8192, 10240, "", {283: (82.2, 68.1), 512: (110, 82.6), 758: (135, 114), 1200: (194, 188)}),
-    (16384, 4096, "followed", {512: (145, 73), 1024: (177, 126), 2048: (261, 231), 4096: (426, 425)}),
-    (18176, 4544, "", {512: (221, 87), 1024: (257, 147), 2048: (373, 296), 4096: (978, 540)}),
-    (22016, 4096, "transposed", {512: (229, 88.5), 758: (230, 119), 1500: (387, 216), 4096: (540, 620)}),
-    (12288, 4096, "transposed", {758: (91.3, 73.1), 1024: (112, 89.9), 4096: (271, 296)}),
-    (8192, 8192, "transposed", {512: (76.7, 70.6), 1024: (113, 114), 2048: (174, 195), 4096: (357, 397)}),
-    (4096, 11008, "transposed", {283: (48.4, 43.5), 512: (53.3, 58.4), 1024: (76.0, 92.4)}),
-    (8192, 28672, "transposed", {448: (165, 187)}),
-    (4544, 18176, "transposed", {192: (59, 53), 512: (81, 96), 758: (98, 112), 1200: (256, 185), 1500: (188, 224), 2048: (313, 286)}),
-]
+MEASURED = os.path.join(os.path.dirname(__file__), os.pardir, "profiles", "prompt_products_wide.csv")
 
 
-@pytest.mark.parametrize("k,n,kind,times", WIDE)
-def test_wide_products(k, n, kind, times):
-    """Taken where it is faster, and nowhere where it is slower by more than 6%, which is what noise and the host make up."""
-    for rows, (library, kernel) in times.items():
-        taken = takes_wide_gemm(rows, k, n, **({kind: True} if kind else {}))
-        assert taken or kernel > 0.94 * library, rows
-        assert not taken or kernel < 1.06 * library, rows
+@pytest.mark.skipif(not os.path.exists(MEASURED), reason="what was measured is not here")
+def test_rules_beside_all_that_was_measured():
+    """What large products take is no more than 7% slower anywhere, and 10% faster in the mean; what they leave is no
+    faster in the mean. What the others take is slower by less than the 10 us that the library's call takes longer on the
+    host, but for 3%, and the tile that is chosen is 2% slower than the best one in the mean."""
+    with open(MEASURED) as f:
+        products = [(r["follows"], *(int(r[c]) for c in ("rows", "k", "n", "transposed")), r) for r in csv.DictReader(f)]
+    assert len(products) > 1500
+    taken, left, chosen = [], [], {True: [], False: []}
+    for follows, m, k, n, transposed, r in products:
+        library, kernel, tiles = float(r["library"]), float(r["kernel"]), [float(r[f"tile{i}"]) for i in range(9)]
+        chosen[k * n <= 25 << 20].append(kernel / min(t for t in tiles if t))
+        if takes_gemm(m, k, n, bool(transposed), fused=follows in ("gelu", "swiglu"), added=follows == "residual"):
+            assert kernel <= 1.03 * library + 10, r
+        elif takes_wide_gemm(m, k, n, bool(transposed), followed=follows in ("residual", "swiglu"), gelu=follows == "gelu"):
+            assert kernel <= 1.07 * library, r
+            taken.append(kernel / library)
+        elif m > 128 and k * n > 25 << 20:
+            left.append(kernel / library)
+    assert sum(taken) < 0.9 * len(taken) and sum(left) > len(left)
+    for which in chosen.values():
+        assert sum(which) < 1.02 * len(which)
 
 
 @pytest.mark.parametrize("m,k,n", [(128, 8192, 8192), (700, 2048, 11264), (758, 2048, 2560), (512, 16384, 53248), (1 << 19, 4096, 4096)])
