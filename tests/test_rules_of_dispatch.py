@@ -140,3 +140,18 @@ def test_rules_beside_all_that_was_measured():
 def test_what_wide_products_leave(m, k, n):
     """Few rows, small matrices, what offsets of 32 bits don't reach."""
     assert not takes_wide_gemm(m, k, n, followed=True)
+
+
+@pytest.mark.parametrize(
+    "m,k,n,taken",
+    [
+        (758, 4096, 22016, True), (768, 4096, 22016, True), (512, 4096, 22016, False), (769, 4096, 22016, False),  # 258, 172 and 344 tiles
+        (4097, 4096, 4096, True), (4096, 4096, 4096, False), (4353, 4096, 4096, False),  # 272, 256, 288
+        (1700, 3584, 18944, True), (1536, 3584, 18944, False),  # 518, 444
+        (1537, 4096, 28160, False),  # 770
+    ],
+)
+@pytest.mark.parametrize("transposed", [False, True])
+def test_few_tiles_of_the_library_left_over(m, k, n, taken, transposed):
+    """After one or two turns of all compute units they cost it another one, whatever the matrix."""
+    assert takes_wide_gemm(m, k, n, transposed) == taken
