@@ -133,7 +133,7 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     if 256 < tiles < 768 and 0 < tiles % 256 <= 20:
         return True
     odd, small = k % 128 > 0 or n % 128 > 0, weights <= 3 << 23
-    # smaller ones gain little (4096 x 6144, 758 rows: 53, 52), but for sizes that the library does not like
+    # smaller ones gain little (4096 x 6144, 758 rows: 55, 54), but for sizes that the library does not like
     if small and not (odd and weights >= 1 << 24):
         return False
     if transposed:
