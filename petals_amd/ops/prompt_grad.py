@@ -122,7 +122,9 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     The library's tiles are 256 x 256 mostly and never cut along K: where some are left over after one or two turns of all
     compute units, these cost it another turn, whatever the matrix. 258 tiles: 758 rows of 4096 x 22016 134, 128, 1400 of
     4096 x 11008 234, 128; 272: 4200 rows of 4096 x 4096 176, 131; 518: 1700 rows of 3584 x 18944 212, 219; 36 such
-    products took 0.5 to 1.04 of the library's time, 0.8 in the mean.
+    products took 0.5 to 1.04 of the library's time, 0.8 in the mean. Where it has no good kernel either, it is so as long as less
+    than four fifths of these turns have work, and from the fourth turn on: 4544 x 18176, 1024 rows (284 tiles) 229, 154, 2048 rows (568)
+    317, 299, 4096 rows 648, 542, transposed, 1200 rows (355) 257, 184; but 758 rows (213) 104, 111, 1500 rows (426) 205, 227.
 
     All that was measured, the median of three runs on three cards, is in profiles/prompt_products_wide.csv: what is taken
     takes 0.88 of the library's time in the mean, and 1.07 at most."""
@@ -136,6 +138,8 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     # smaller ones gain little (4096 x 6144, 758 rows: 55, 54), but for sizes that the library does not like
     if small and not (odd and weights >= 1 << 24):
         return False
+    if odd and n >= 3 * k and tiles > 256 and (tiles > 768 or 5 * tiles < 4 * 256 * -(-tiles // 256)):
+        return True
     if transposed:
         if small:
             return m <= 960

@@ -109,6 +109,33 @@ def test_products_of_prompts(k, n, kind, times):
         assert all(kernel <= library + 1.5 for rows, (library, kernel) in times.items() if rows > 300 and takes_gemm(rows, k, n))
 
 
+# the same for the tiles of 256 columns that four waves have, where the library had the product
+WIDE = [
+    (4096, 12288, "", {192: (59.2, 46.1), 512: (59.0, 62.1), 758: (72.7, 66.3), 1024: (88.3, 91.5), 4096: (317, 329)}),
+    (4096, 22016, "followed", {512: (104, 98), 1024: (187, 169), 2048: (385, 311), 4096: (740, 604)}),
+    (4096, 28672, "followed", {512: (116, 109), 1024: (223, 205), 2048: (454, 394), 4096: (842, 757)}),
+    (8192, 57344, "followed", {512: (441, 412), 1024: (846, 767), 2048: (1573, 1463), 4096: (3084, 2858)}),
+    (8192, 10240, "", {283: (82.2, 68.1), 512: (110, 82.6), 758: (135, 114), 1200: (194, 188)}),
+    (16384, 4096, "followed", {512: (145, 73), 1024: (177, 126), 2048: (261, 231), 4096: (426, 425)}),
+    (18176, 4544, "", {512: (221, 87), 1024: (257, 147), 2048: (373, 296), 4096: (978, 540)}),
+    (22016, 4096, "transposed", {512: (229, 88.5), 758: (230, 119), 1500: (387, 216), 4096: (540, 620)}),
+    (12288, 4096, "transposed", {758: (91.3, 73.1), 1024: (112, 89.9), 4096: (271, 296)}),
+    (8192, 8192, "transposed", {512: (76.7, 70.6), 1024: (113, 114), 2048: (174, 195), 4096: (357, 397)}),
+    (4096, 11008, "transposed", {283: (48.4, 43.5), 512: (53.3, 58.4), 1024: (76.0, 92.4)}),
+    (8192, 28672, "transposed", {448: (165, 187)}),
+    (4544, 18176, "transposed", {192: (59, 53), 512: (81, 96), 758: (98, 112), 1200: (256, 185), 1500: (188, 224), 2048: (313, 286)}),
+]
+
+
+@pytest.mark.parametrize("k,n,kind,times", WIDE)
+def test_wide_products(k, n, kind, times):
+    """Taken where it is faster, and nowhere where it is slower by more than 6%, which is what noise and the host make up."""
+    for rows, (library, kernel) in times.items():
+        taken = takes_wide_gemm(rows, k, n, **({kind: True} if kind else {}))
+        assert taken or kernel > 0.94 * library, rows
+        assert not taken or kernel < 1.06 * library, rows
+
+
 MEASURED = os.path.join(os.path.dirname(__file__), os.pardir, "profiles", "prompt_products_wide.csv")
 
 
@@ -155,3 +182,15 @@ def test_what_wide_products_leave(m, k, n):
 def test_few_tiles_of_the_library_left_over(m, k, n, taken, transposed):
     """After one or two turns of all compute units they cost it another one, whatever the matrix."""
     assert takes_wide_gemm(m, k, n, transposed) == taken
+
+
+@pytest.mark.parametrize("k,n", [(4544, 18176), (4160, 13120), (7232, 28864)])
+def test_turns_of_the_library_with_little_work(k, n):
+    """Sizes that it has no good kernel for and many columns: the rows at which its tiles leave a fifth of the turns idle."""
+    columns = -(-n // 256)
+    for rows in range(513, 8192, 101):
+        tiles = -(-rows // 256) * columns
+        turns = -(-tiles // 256)
+        taken = turns > 3 or turns > 1 and (tiles < 0.8 * turns * 256 or 0 < tiles % 256 <= 20)
+        for transposed in (False, True):
+            assert takes_wide_gemm(rows, k, n, transposed) == taken, rows
