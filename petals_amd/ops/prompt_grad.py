@@ -120,7 +120,7 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     8192 to 8192, 512 rows 74, 71, 1024 rows 110, 115; 4096 to 11008, 256 rows 48, 39, 512 rows 52, 54.
 
     The library's tiles are 256 x 256 mostly and never cut along K: where some are left over after one or two turns of all
-    compute units, these cost it another turn, whatever the matrix. 258 tiles: 758 rows of 4096 x 22016 134, 128, 1400 of
+    compute units, these cost it another turn, whatever the matrix (measured from 4096 x 4096 on). 258 tiles: 758 rows of 4096 x 22016 134, 128, 1400 of
     4096 x 11008 234, 128; 272: 4200 rows of 4096 x 4096 176, 131; 518: 1700 rows of 3584 x 18944 212, 219; 36 such
     products took 0.5 to 1.04 of the library's time, 0.8 in the mean. Where it has no good kernel either, it is so as long as less
     than four fifths of these turns have work, and from the fourth turn on: 4544 x 18176, 1024 rows (284 tiles) 229, 154, 2048 rows (568)
@@ -132,7 +132,7 @@ def takes_wide_gemm(m: int, k: int, n: int, transposed: bool = False, followed: 
     if not 128 < m < (1 << 31) // k or weights > 1 << 29:
         return False
     tiles = -(-m // 256) * -(-n // 256)
-    if 256 < tiles < 768 and 0 < tiles % 256 <= 20:
+    if weights >= 1 << 24 and 256 < tiles < 768 and 0 < tiles % 256 <= 20:
         return True
     odd, small = k % 128 > 0 or n % 128 > 0, weights <= 3 << 23
     # smaller ones gain little (4096 x 6144, 758 rows: 55, 54), but for sizes that the library does not like

@@ -176,6 +176,7 @@ def test_what_wide_products_leave(m, k, n):
         (4097, 4096, 4096, True), (4096, 4096, 4096, False), (4353, 4096, 4096, False),  # 272, 256, 288
         (1700, 3584, 18944, True), (1536, 3584, 18944, False),  # 518, 444
         (1537, 4096, 28160, False),  # 770
+        (6600, 2048, 2560, False), (33000, 512, 512, False),  # 260, 258 of small matrices, which nothing is known of
     ],
 )
 @pytest.mark.parametrize("transposed", [False, True])
